@@ -117,7 +117,7 @@ struct femgpu_ctx {
 
   bool dirty_mat = true, dirty_fix = true, dirty_diag = true, dirty_rhs = true;
 
-  CgScalars *h_sc = nullptr;  // pinned, h_sc[0..3]: poll ring
+  CgScalars *h_sc = nullptr;  // pinned: [0], [1] poll ring, [2] residual norms
   hipEvent_t ev_poll[4] = {nullptr, nullptr, nullptr, nullptr};
   int emax_req = 0, threads_req = 0;
   int tuned_threads = 256;  // threads per patch of the current plan
@@ -229,12 +229,44 @@ std::vector<double> to_internal(const femgpu_ctx *ctx, const double *u) {
   return v;
 }
 
-void from_internal(const femgpu_ctx *ctx, const std::vector<double> &v, double *u) {
-  const int d = ctx->dim;
-  for (int64_t i = 0; i < ctx->nn; ++i) {
-    const int64_t s = ctx->plan.node_perm[i];
-    for (int c = 0; c < d; ++c) u[size_t(s) * d + c] = v[size_t(i) * d + c];
-  }
+// Host node vector (user order) -> device vector `name` in internal order,
+// permuted on the device.  The caller synchronises the stream before the
+// host vector may change.
+template <typename T>
+int upload_nodes(femgpu_ctx *ctx, const std::string &name, const double *u, T **out) {
+  const size_t nd = size_t(ctx->nn) * ctx->dim;
+  double *io;
+  int st;
+  if ((st = dbuf(ctx, "io_in", nd, &io)) || (st = dbuf(ctx, name, nd, out))) return st;
+  HIPCHK(hipMemcpyAsync(io, u, nd * sizeof(double), hipMemcpyHostToDevice, ctx->stream));
+  femgpu::launch_gather_user<T>(ctx->nn, ctx->dim, ctx->d_node_perm, io, *out, ctx->stream);
+  HIPCHK(hipGetLastError());
+  return FEMGPU_OK;
+}
+
+// Device node vector (internal order) -> host vector in user order, 0 at
+// nodes no element references; synchronises.
+template <typename T>
+int download_nodes(femgpu_ctx *ctx, const T *v, double *u) {
+  const size_t nd = size_t(ctx->nn) * ctx->dim;
+  double *io;
+  int st;
+  if ((st = dbuf(ctx, "io_out", nd, &io))) return st;
+  femgpu::launch_scatter_user<T>(ctx->nn, ctx->dm.n_active, ctx->dim,
+                                 ctx->d_node_perm, v, io, ctx->stream);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(u, io, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  return FEMGPU_OK;
+}
+
+// Device element results (user order, nv per element) -> host; synchronises.
+int download_elems(femgpu_ctx *ctx, const double *v, int nv, double *out) {
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(out, v, size_t(ctx->ne) * nv * sizeof(double), hipMemcpyDeviceToHost,
+                        ctx->stream));
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  return FEMGPU_OK;
 }
 
 void lame(int dim, double E, double nu, double &lam, double &mu) {
@@ -780,30 +812,34 @@ int need_mesh(femgpu_ctx *ctx) {
   return FEMGPU_OK;
 }
 
+// FP64 residual r = f - K x of internal device vectors; ||r||^2 and ||f||^2
+// to the host (the kernels write the sums to pinned memory).
+int residual64(femgpu_ctx *ctx, const double *f, const double *x, double *y, double *r,
+               double *slots, double *rr, double *ff) {
+  double *part;
+  int st;
+  if ((st = dbuf(ctx, "part_res", 2 * size_t(femgpu::grid_blocks(ctx->dm.n_active)), &part)))
+    return st;
+  CgScalars *sums = ctx->h_sc + 2;
+  femgpu::launch_matvec_patch<double>(ctx->dm, x, y, slots, ctx->stream);
+  femgpu::launch_residual64(ctx->dm, f, y, slots, r, sums, part, ctx->stream);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(ctx->stream));
+  *rr = sums->rr;
+  *ff = sums->rr0;
+  return FEMGPU_OK;
+}
+
 // True relative residual ||f - K x|| / ||f|| in FP64 (x, f internal, device).
 int true_rel_res(femgpu_ctx *ctx, const double *f, const double *x, double *out) {
-  double *y, *r, *part, *part_node;
-  CgScalars *sc;
+  double *y, *r, *slots, rr, ff;
   const size_t nd = size_t(ctx->nn) * ctx->dim;
   int st;
   if ((st = dbuf(ctx, "rr_y", nd, &y)) || (st = dbuf(ctx, "rr_r", nd, &r)) ||
-      (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &part)) ||
-      (st = dbuf(ctx, "part_node", NODE_PART, &part_node)) ||
-      (st = dbuf(ctx, "sc_aux", 1, &sc)))
+      (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &slots)) ||
+      (st = residual64(ctx, f, x, y, r, slots, &rr, &ff)))
     return st;
-  // ||f||^2 first: the residual of K x replaced by 0 (y and slots zero).
-  femgpu::launch_reset_scalars(sc, 1, 0.0, 0, ctx->stream);
-  femgpu::launch_fill<double>(y, int64_t(nd), 0.0, ctx->stream);
-  femgpu::launch_fill<double>(part, int64_t(ctx->plan.n_slots) * ctx->dim, 0.0, ctx->stream);
-  femgpu::launch_residual64(ctx->dm, f, y, part, r, sc, part_node, ctx->stream);
-  HIPCHK(hipGetLastError());
-  if ((st = poll(ctx, sc))) return st;
-  const double ff = ctx->h_sc->rr;
-  femgpu::launch_matvec_patch<double>(ctx->dm, x, y, part, ctx->stream);
-  femgpu::launch_residual64(ctx->dm, f, y, part, r, sc, part_node, ctx->stream);
-  HIPCHK(hipGetLastError());
-  if ((st = poll(ctx, sc))) return st;
-  *out = ff > 0 ? std::sqrt(ctx->h_sc->rr / ff) : 0.0;
+  *out = ff > 0 ? std::sqrt(rr / ff) : 0.0;
   return FEMGPU_OK;
 }
 
@@ -884,9 +920,12 @@ int upload_plan(femgpu_ctx *ctx) {
       (st = upload(ctx, "elems_int", P.elems_int, &ei)))
     return st;
   {
-    int32_t *np_;
-    if ((st = upload(ctx, "node_perm", P.node_perm, &np_))) return st;
+    int32_t *np_, *ep_;
+    if ((st = upload(ctx, "node_perm", P.node_perm, &np_)) ||
+        (st = upload(ctx, "elem_perm", P.elem_perm, &ep_)))
+      return st;
     ctx->d_node_perm = np_;
+    dm.elem_perm = ep_;
   }
   dm.patches = pp;
   dm.erec = rec;
@@ -1426,31 +1465,24 @@ int femgpu_matvec(femgpu_ctx *ctx, int precision, const double *x, double *y) {
   if (!x || !y) return FEMGPU_E_ARG;
   if ((st = ensure_diag(ctx))) return st;
   const size_t nd = size_t(ctx->nn) * ctx->dim;
-  std::vector<double> xi = to_internal(ctx, x), yi(nd, 0.0);
-  double *dx, *dy, *part;
-  if ((st = upload(ctx, "mv_x", xi, &dx)) || (st = dbuf(ctx, "mv_y", nd, &dy)) ||
-      (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &part)))
-    return st;
-  femgpu::launch_fill<double>(dy, int64_t(nd), 0.0, ctx->stream);
+  const size_t ns = size_t(ctx->plan.n_slots) * ctx->dim + 1;
   if (precision == FEMGPU_FP64) {
-    femgpu::launch_matvec<double>(ctx->dm, dx, dy, part, ctx->stream);
-  } else if (precision == FEMGPU_FP32) {
-    float *fx, *fy, *fpart;
-    if ((st = dbuf(ctx, "mv_x32", nd, &fx)) || (st = dbuf(ctx, "mv_y32", nd, &fy)) ||
-        (st = dbuf(ctx, "partial32", size_t(ctx->plan.n_slots) * ctx->dim + 1, &fpart)))
+    double *dx, *dy, *part;
+    if ((st = upload_nodes<double>(ctx, "mv_x", x, &dx)) || (st = dbuf(ctx, "mv_y", nd, &dy)) ||
+        (st = dbuf(ctx, "partial64", ns, &part)))
       return st;
-    femgpu::launch_convert<double, float>(dx, fx, int64_t(nd), ctx->stream);
-    femgpu::launch_fill<float>(fy, int64_t(nd), 0.f, ctx->stream);
-    femgpu::launch_matvec<float>(ctx->dm, fx, fy, fpart, ctx->stream);
-    femgpu::launch_convert<float, double>(fy, dy, int64_t(nd), ctx->stream);
-  } else {
-    return fail(ctx, FEMGPU_E_ARG, "precision must be FP64 or FP32");
+    femgpu::launch_matvec<double>(ctx->dm, dx, dy, part, ctx->stream);
+    return download_nodes<double>(ctx, dy, y);
   }
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(yi.data(), dy, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  from_internal(ctx, yi, y);
-  return FEMGPU_OK;
+  if (precision == FEMGPU_FP32) {
+    float *fx, *fy, *fpart;
+    if ((st = upload_nodes<float>(ctx, "mv_x32", x, &fx)) || (st = dbuf(ctx, "mv_y32", nd, &fy)) ||
+        (st = dbuf(ctx, "partial32", ns, &fpart)))
+      return st;
+    femgpu::launch_matvec<float>(ctx->dm, fx, fy, fpart, ctx->stream);
+    return download_nodes<float>(ctx, fy, y);
+  }
+  return fail(ctx, FEMGPU_E_ARG, "precision must be FP64 or FP32");
 }
 
 
@@ -1514,13 +1546,9 @@ int femgpu_diag(femgpu_ctx *ctx, double *d) {
   if (!d) return FEMGPU_E_ARG;
   if ((st = ensure_diag(ctx))) return st;
   const size_t nd = size_t(ctx->nn) * ctx->dim;
-  std::vector<double> v(nd);
   double *dd;
   if ((st = dbuf(ctx, "diag64", nd, &dd))) return st;
-  HIPCHK(hipMemcpyAsync(v.data(), dd, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  from_internal(ctx, v, d);
-  return FEMGPU_OK;
+  return download_nodes<double>(ctx, dd, d);
 }
 
 int femgpu_rhs(femgpu_ctx *ctx, double *f) {
@@ -1563,8 +1591,7 @@ static bool trace_enabled() {
 // u = M^-1 r, w = A u, and s = A p for the kept direction p (or p = s = 0
 // at a restart).
 static int solve_cg1(femgpu_ctx *ctx, const femgpu_solve_opts &o, int max_iter, int block,
-                     const double *f64, double *x64, CgScalars *sc, CgScalars *sc2,
-                     femgpu_stats *S) {
+                     const double *f64, double *x64, CgScalars *sc, femgpu_stats *S) {
   const int64_t nd = ctx->nn * ctx->dim;
   int st, done = 0;
   Cg1Pos pos{0, 0};
@@ -1588,8 +1615,9 @@ static int solve_cg1(femgpu_ctx *ctx, const femgpu_solve_opts &o, int max_iter, 
     femgpu::launch_convert<float, double>(w.x[pos.q], x64, nd, ctx->stream);
   } else if (o.precision == FEMGPU_MIXED) {
     femgpu::Cg1State<float> w;
-    double *r64, *y64, *part64, *part_node;
+    double *r64, *y64, *part64, *part_node, *part_res;
     if ((st = cg1_ws(ctx, "32", w)) || (st = dbuf(ctx, "ir_r", size_t(nd), &r64)) ||
+        (st = dbuf(ctx, "part_res", 2 * size_t(femgpu::grid_blocks(ctx->dm.n_active)), &part_res)) ||
         (st = dbuf(ctx, "ir_y", size_t(nd), &y64)) ||
         (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &part64)) ||
         (st = dbuf(ctx, "part_node", NODE_PART, &part_node)))
@@ -1641,12 +1669,8 @@ static int solve_cg1(femgpu_ctx *ctx, const femgpu_solve_opts &o, int max_iter, 
         break;
       }
       // FP64 residual of the accumulated solution
-      femgpu::launch_reset_scalars(sc2, 1, 0.0, 0, ctx->stream);
-      femgpu::launch_matvec_patch<double>(ctx->dm, x64, y64, part64, ctx->stream);
-      femgpu::launch_residual64(ctx->dm, f64, y64, part64, r64, sc2, part_node, ctx->stream);
-      HIPCHK(hipGetLastError());
-      if ((st = poll(ctx, sc2))) return st;
-      const double rr64 = ctx->h_sc->rr;
+      double rr64, ff64;
+      if ((st = residual64(ctx, f64, x64, y64, r64, part64, &rr64, &ff64))) return st;
       rel = ff > 0 ? std::sqrt(rr64 / ff) : 0.0;
       if (trace_enabled())
         std::fprintf(stderr, "femgpu mixed/single-reduction: %d iterations, stop %d, FP64 rel-res %.3e\n",
@@ -1721,15 +1745,15 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
   if ((st = ensure_diag(ctx))) return st;
   const size_t nd = size_t(ctx->nn) * ctx->dim;
   double *f64, *x64;
-  CgScalars *sc, *sc2;
+  CgScalars *sc;
   if ((st = dbuf(ctx, f_name, nd, &f64)) || (st = dbuf(ctx, "sol64", nd, &x64)) ||
-      (st = dbuf(ctx, "sc_main", 1, &sc)) || (st = dbuf(ctx, "sc_outer", 1, &sc2)))
+      (st = dbuf(ctx, "sc_main", 1, &sc)))
     return st;
   femgpu_stats S{};
   int iters = 0, done = 0;
   HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
   if (o.recurrence == FEMGPU_CG_SINGLE_REDUCTION) {
-    if ((st = solve_cg1(ctx, o, max_iter, block, f64, x64, sc, sc2, &S))) return st;
+    if ((st = solve_cg1(ctx, o, max_iter, block, f64, x64, sc, &S))) return st;
   } else if (o.precision == FEMGPU_FP64) {
     PcgWs<double> w;
     if ((st = pcg_ws(ctx, "c64", w))) return st;
@@ -1762,13 +1786,11 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
     // meets the tolerance.
     PcgWs<float> w;
     double *r64, *y64, *part64, *part_node, *part_patch, *part_res;
-    // part_res: the FP64 residual's partials (apart from the inner
-    // iterations' part_node)
     if ((st = pcg_ws(ctx, "c32", w)) || (st = dbuf(ctx, "ir_r", nd, &r64)) ||
         (st = dbuf(ctx, "ir_y", nd, &y64)) ||
         (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &part64)) ||
         (st = dbuf(ctx, "part_node", NODE_PART, &part_node)) ||
-        (st = dbuf(ctx, "part_res", size_t(femgpu::grid_blocks(ctx->dm.n_active)) + 1, &part_res)) ||
+        (st = dbuf(ctx, "part_res", 2 * size_t(femgpu::grid_blocks(ctx->dm.n_active)), &part_res)) ||
         (st = dbuf(ctx, "part_patch", size_t(ctx->dm.np) + 1, &part_patch)))
       return st;
     w.invD = static_cast<float *>(ctx->bufs["invD32"].p);
@@ -1820,12 +1842,9 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
         break;
       }
       // FP64 residual of the accumulated solution
-      femgpu::launch_reset_scalars(sc2, 1, 0.0, 0, ctx->stream);
-      femgpu::launch_matvec_patch<double>(ctx->dm, x64, y64, part64, ctx->stream);
-      femgpu::launch_residual64(ctx->dm, f64, y64, part64, r64, sc2, part_res, ctx->stream);
-      HIPCHK(hipGetLastError());
-      if ((st = poll(ctx, sc2))) return st;
-      rel = ff > 0 ? std::sqrt(ctx->h_sc->rr / ff) : 0.0;
+      double rr64, ff64;
+      if ((st = residual64(ctx, f64, x64, y64, r64, part64, &rr64, &ff64))) return st;
+      rel = ff > 0 ? std::sqrt(rr64 / ff) : 0.0;
       const double rel_rec = ff > 0 ? std::sqrt(rr_rec / ff) : 0.0;
       if (trace_enabled())
         std::fprintf(stderr, "femgpu mixed: %d iterations, stop %d, FP32 recurrence rel-res %.3e, "
@@ -1853,8 +1872,8 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
       kept_p = !restart;
       if (done) femgpu::launch_pcg_resume(sc, ctx->stream);
       rel_prev = rel;
-      pause_rr = ctx->h_sc->rr * drop * drop;
-      pred.seed(iters, ctx->h_sc->rr, ctx->h_sc->rr);
+      pause_rr = rr64 * drop * drop;
+      pred.seed(iters, rr64, rr64);
       ++replacements;
     }
     S.iterations = iters;
@@ -1871,12 +1890,7 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
   double rr;
   if ((st = true_rel_res(ctx, f64, x64, &rr))) return st;
   S.rel_res = rr;
-  if (u_out) {
-    std::vector<double> xi(nd);
-    HIPCHK(hipMemcpyAsync(xi.data(), x64, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    from_internal(ctx, xi, u_out);
-  }
+  if (u_out && (st = download_nodes<double>(ctx, x64, u_out))) return st;
   if (stats) *stats = S;
   if (S.status != FEMGPU_OK) {
     ctx->err = "solve stopped with status " + std::to_string(S.status);
@@ -1891,8 +1905,9 @@ static int ensure_rhs(femgpu_ctx *ctx) {
   std::vector<double> fu;
   host_rhs(ctx, false, fu);
   double *f64;
-  int st = upload(ctx, "f64", to_internal(ctx, fu.data()), &f64);
+  int st = upload_nodes<double>(ctx, "f64", fu.data(), &f64);
   if (st) return st;
+  HIPCHK(hipStreamSynchronize(ctx->stream));  // fu goes out of scope
   ctx->dirty_rhs = false;
   return FEMGPU_OK;
 }
@@ -1910,13 +1925,14 @@ int femgpu_solve_rhs(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const doubl
   int st = need_mesh(ctx);
   if (st) return st;
   if (!f) return fail(ctx, FEMGPU_E_ARG, "null right-hand side");
-  std::vector<double> fi = to_internal(ctx, f);
-  // rows of nodes no element references carry no equation
-  for (int64_t i = ctx->plan.n_owned + ctx->plan.n_iface; i < ctx->nn; ++i)
-    for (int c = 0; c < ctx->dim; ++c) fi[size_t(i) * ctx->dim + c] = 0.0;
   double *df;
-  if ((st = upload(ctx, "f_user", fi, &df))) return st;
-  return solve_core(ctx, opts, "f_user", u_out, stats);
+  if ((st = upload_nodes<double>(ctx, "f_user", f, &df))) return st;
+  // rows of nodes no element references carry no equation
+  const int64_t na = ctx->dm.n_active * ctx->dim;
+  femgpu::launch_fill<double>(df + na, ctx->nn * ctx->dim - na, 0.0, ctx->stream);
+  st = solve_core(ctx, opts, "f_user", u_out, stats);
+  if (st) (void)hipStreamSynchronize(ctx->stream);  // f may still be on its way
+  return st;
 }
 
 int femgpu_material_grad(femgpu_ctx *ctx, const double *u, const double *w, double *g_out) {
@@ -1924,17 +1940,13 @@ int femgpu_material_grad(femgpu_ctx *ctx, const double *u, const double *w, doub
   if (st) return st;
   if (!u || !w || !g_out) return fail(ctx, FEMGPU_E_ARG, "null argument");
   if ((st = ensure_material(ctx)) || (st = ensure_fix(ctx))) return st;
-  std::vector<double> ui = to_internal(ctx, u), wi = to_internal(ctx, w), g(ctx->ne);
   double *du, *dw, *dg;
-  if ((st = upload(ctx, "st_u", ui, &du)) || (st = upload(ctx, "gr_w", wi, &dw)) ||
-      (st = dbuf(ctx, "en_e", g.size(), &dg)))
+  if ((st = upload_nodes<double>(ctx, "st_u", u, &du)) ||
+      (st = upload_nodes<double>(ctx, "gr_w", w, &dw)) ||
+      (st = dbuf(ctx, "en_e", size_t(ctx->ne), &dg)))
     return st;
   femgpu::launch_bilinear<double>(ctx->dm, du, dw, -1.0, dg, ctx->stream);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(g.data(), dg, g.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (int64_t i = 0; i < ctx->ne; ++i) g_out[ctx->plan.elem_perm[i]] = g[i];
-  return FEMGPU_OK;
+  return download_elems(ctx, dg, 1, g_out);
 }
 
 int femgpu_compliance_grad(femgpu_ctx *ctx, const femgpu_solve_opts *opts, double *u_out,
@@ -1956,15 +1968,13 @@ int femgpu_compliance_grad(femgpu_ctx *ctx, const femgpu_solve_opts *opts, doubl
   // adjoint of C = f'u is u itself: dC/ds_e = -u_e' K~_e^0 u_e.
   femgpu::launch_bilinear<double>(ctx->dm, x64, x64, -1.0, dg, ctx->stream);
   HIPCHK(hipGetLastError());
-  std::vector<double> fh(nd), xh(nd), g(ctx->ne);
+  std::vector<double> fh(nd), xh(nd);
   HIPCHK(hipMemcpyAsync(fh.data(), f64, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   HIPCHK(hipMemcpyAsync(xh.data(), x64, nd * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipMemcpyAsync(g.data(), dg, g.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
+  if ((st = download_elems(ctx, dg, 1, g_out))) return st;
   double c = 0.0;
   for (size_t i = 0; i < nd; ++i) c += fh[i] * xh[i];
   *c_out = c;
-  for (int64_t i = 0; i < ctx->ne; ++i) g_out[ctx->plan.elem_perm[i]] = g[i];
   return FEMGPU_OK;
 }
 
@@ -1976,16 +1986,12 @@ int element_tensor(femgpu_ctx *ctx, const double *u, double *out, bool strain) {
   if (!u || !out) return FEMGPU_E_ARG;
   if ((st = ensure_material(ctx))) return st;
   const int nv = 3 * (ctx->dim - 1);
-  std::vector<double> ui = to_internal(ctx, u), s(size_t(ctx->ne) * nv);
   double *du, *ds;
-  if ((st = upload(ctx, "st_u", ui, &du)) || (st = dbuf(ctx, "st_s", s.size(), &ds))) return st;
+  if ((st = upload_nodes<double>(ctx, "st_u", u, &du)) ||
+      (st = dbuf(ctx, "st_s", size_t(ctx->ne) * nv, &ds)))
+    return st;
   femgpu::launch_stress<double>(ctx->dm, du, ds, ctx->stream, strain);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(s.data(), ds, s.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (int64_t i = 0; i < ctx->ne; ++i)
-    for (int k = 0; k < nv; ++k) out[size_t(ctx->plan.elem_perm[i]) * nv + k] = s[size_t(i) * nv + k];
-  return FEMGPU_OK;
+  return download_elems(ctx, ds, nv, out);
 }
 }  // namespace
 
@@ -2002,15 +2008,12 @@ int femgpu_element_energy(femgpu_ctx *ctx, const double *u, double *e_out) {
   if (st) return st;
   if (!u || !e_out) return FEMGPU_E_ARG;
   if ((st = ensure_material(ctx)) || (st = ensure_fix(ctx))) return st;
-  std::vector<double> ui = to_internal(ctx, u), e(ctx->ne);
   double *du, *de;
-  if ((st = upload(ctx, "st_u", ui, &du)) || (st = dbuf(ctx, "en_e", e.size(), &de))) return st;
+  if ((st = upload_nodes<double>(ctx, "st_u", u, &du)) ||
+      (st = dbuf(ctx, "en_e", size_t(ctx->ne), &de)))
+    return st;
   femgpu::launch_energy<double>(ctx->dm, du, de, ctx->stream);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(e.data(), de, e.size() * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(hipStreamSynchronize(ctx->stream));
-  for (int64_t i = 0; i < ctx->ne; ++i) e_out[ctx->plan.elem_perm[i]] = e[i];
-  return FEMGPU_OK;
+  return download_elems(ctx, de, 1, e_out);
 }
 
 int femgpu_default_dyn_opts(femgpu_dyn_opts *o) {
@@ -2545,12 +2548,8 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   S.run_ms = ms;
   S.steps = steps;
   if (u_out) {
-    std::vector<T> xt(nd);
     const T *dfin = expl ? dbufs[steps & 1] : dd;
-    HIPCHK(hipMemcpyAsync(xt.data(), dfin, nd * sizeof(T), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    std::vector<double> xi(xt.begin(), xt.end());
-    from_internal(ctx, xi, u_out);
+    if ((st = download_nodes<T>(ctx, dfin, u_out))) return st;
   }
   if (nrec) {
     const int ns = std::min(max_samples, steps / every);

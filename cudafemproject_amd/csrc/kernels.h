@@ -35,6 +35,7 @@ struct DevMesh {
   const int32_t *slot_start = nullptr;
   const uint8_t *fixmask = nullptr;   // per internal node: bit c = component c fixed
   const int32_t *elems_int = nullptr; // ne x npe internal node ids
+  const int32_t *elem_perm = nullptr; // internal element -> user element
   const double *coords64 = nullptr;
   const float *coords32 = nullptr;
   const double *escale64 = nullptr;   // per internal element or null
@@ -129,7 +130,8 @@ void launch_pcg_apply_x(const DevMesh &dm, T *x, const T *p, CgScalars *sc, hipS
 constexpr int NODE_PARTS = 512;  // blocks of the node-parallel PCG kernels
 static_assert(NODE_PARTS % 256 == 0, "the patch kernels read the partials in chunks of 256");
 
-// r = f - (interface-finished) K x, rr -> sc->rr (FP64 outer loop of MIXED).
+// r = f - (interface-finished) K x (true residual; FP64 outer loop of MIXED),
+// r'r -> sc->rr, f'f -> sc->rr0; part: 2 x grid_blocks(n_active) doubles.
 void launch_residual64(const DevMesh &dm, const double *f, const double *y, const double *partial,
                        double *r, CgScalars *sc, double *part, hipStream_t s);
 // Mixed solve (reliable updates): x64 += x32, x32 = 0; residual replacement
@@ -151,7 +153,7 @@ void launch_copy(const T *a, T *b, int64_t n, hipStream_t s);
 template <typename TA, typename TB>
 void launch_convert(const TA *a, TB *b, int64_t n, hipStream_t s);
 
-// Per-element outputs in internal element order.
+// Per-element outputs in user element order.
 template <typename T>
 void launch_stress(const DevMesh &dm, const T *u, T *sigma, hipStream_t s, bool strain = false);
 template <typename T>
