@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -26,6 +27,7 @@
 #include "femgpu_internal.h"
 #include "kernels.h"
 #include "noalloc.h"
+#include "resident.h"
 
 using femgpu::CgScalars;
 using femgpu::DevMesh;
@@ -35,6 +37,9 @@ using femgpu::OpShift;
 namespace {
 
 constexpr int NODE_PART = 4 * femgpu::NODE_PARTS;  // partials of node kernels (4 arrays)
+// Iterations of one resident launch (a few ms to tens of ms of device time;
+// a longer solve continues in further launches)
+constexpr int RES_ITER_CAP = 4096;
 
 struct DevBuf {
   void *p = nullptr;
@@ -128,6 +133,11 @@ struct femgpu_ctx {
   std::map<std::string, hipGraphExec_t> graphs;
   uint64_t buf_gen = 0;
   uint64_t graph_gen = 0;
+
+  // resident solves (resident.h): patches the exchange words are zeroed for;
+  // off after a launch that did not complete
+  int res_np = 0;
+  bool res_off = false;
 
   // femgpu_matvec_noalloc: this device's fixed scratch array (device
   // address from hipGetSymbolAddress) and the internal -> user node map
@@ -662,6 +672,115 @@ int replay_until(femgpu_ctx *ctx, const Replay &exec, CgScalars *sc, int block, 
   return FEMGPU_OK;
 }
 
+// Resident launches (resident.h) wait for each other's workgroups, so all
+// workgroups of a launch must reach the device: alone they do when they fit
+// it; beside others they do while the launches' shares and the largest
+// workgroup together stay within it (then some compute unit always has room
+// for the next workgroup).  A launch that would not fit waits here for the
+// others to end.
+class ResidentGate {
+ public:
+  ResidentGate(int device, double share, double block) : g_(gate(device)), share_(share) {
+    std::unique_lock<std::mutex> lock(g_.mu);
+    g_.cv.wait(lock, [&] {
+      return g_.n == 0 || g_.load + share + std::max(g_.block, block) <= 1.0;
+    });
+    ++g_.n;
+    g_.load += share;
+    g_.block = std::max(g_.block, block);
+  }
+  ~ResidentGate() {
+    {
+      std::lock_guard<std::mutex> lock(g_.mu);
+      g_.load -= share_;
+      if (--g_.n == 0) g_.load = g_.block = 0.0;
+    }
+    g_.cv.notify_all();
+  }
+
+ private:
+  struct Gate {
+    std::mutex mu;
+    std::condition_variable cv;
+    int n = 0;
+    double load = 0.0, block = 0.0;
+  };
+  static Gate &gate(int device) {
+    static std::mutex mu;
+    static std::map<int, Gate> gates;
+    std::lock_guard<std::mutex> lock(mu);
+    return gates[device];
+  }
+  Gate &g_;
+  double share_;
+};
+
+// Whether this plan's PCG runs resident (all its workgroups on the chip).
+template <typename T>
+bool pcg_resident(const femgpu_ctx *ctx) {
+  femgpu::ResFit fit;
+  return !ctx->res_off && femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit);
+}
+
+// The exchange words and entries (of 8-byte values), zeroed for this plan.
+int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long **entries) {
+  const size_t n = femgpu::res_words(ctx->dm.np);
+  const size_t ne = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
+  double *w, *e;
+  int st;
+  if ((st = dbuf(ctx, "res_words", n, &w)) || (st = dbuf(ctx, "res_entries", ne, &e))) return st;
+  if (ctx->res_np != ctx->dm.np) {
+    femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
+    femgpu::launch_fill<double>(e, int64_t(ne), 0.0, ctx->stream);
+    ctx->res_np = ctx->dm.np;
+  }
+  *words = reinterpret_cast<unsigned long long *>(w);
+  *entries = reinterpret_cast<unsigned long long *>(e);
+  return FEMGPU_OK;
+}
+
+// Runs a resident PCG until it stops; on return the stream is idle and
+// h_sc[0] holds the scalars.  *ok = false: the launch did not complete (its
+// workgroups did not come together); this context then stays with the
+// launch-per-kernel form.
+template <typename T>
+int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
+  femgpu::ResFit fit;
+  int st;
+  if (!femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit))
+    return fail(ctx, FEMGPU_E_STATE, "internal error: resident PCG does not fit");
+  if ((st = res_buffers(ctx, &a.words, &a.entries))) return st;
+  a.sc = ctx->h_sc;
+  a.cap = RES_ITER_CAP;
+  for (;;) {
+    ctx->h_sc->done = femgpu::RES_ABORTED;
+    {
+      ResidentGate gate(ctx->device, fit.share, fit.block);
+      femgpu::launch_res_pcg<T>(ctx->dm, a, ctx->stream);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    const CgScalars &h = *ctx->h_sc;
+    if (h.done == femgpu::RES_ABORTED) {
+      ctx->res_off = true;
+      ctx->res_np = 0;
+      *ok = false;
+      return FEMGPU_OK;
+    }
+    if (h.done != femgpu::RES_CAP) break;
+    a.fresh = 0;
+    a.r_in = a.r_out;
+    a.gamma0 = h.gamma0;
+    a.rr0 = h.rr0;
+    a.thresh = h.thresh;
+    a.g_prev = h.g[1];
+    a.pause = h.pause;
+    a.it0 = h.iter_final;
+  }
+  *ok = true;
+  return FEMGPU_OK;
+}
+
 // Iterations of the short graph that replays expected to contain the stop run.
 inline int tail_block_of(int block) { return std::max(2, (block / 4) & ~1); }
 
@@ -967,6 +1086,28 @@ int upload_plan(femgpu_ctx *ctx) {
   }
   dm.slot_start = ss;
   dm.elems_int = ei;
+  if (dm.np <= femgpu::RES_PATCHES_MAX) {
+    femgpu::ExchangePlan x;
+    if (femgpu::build_exchange(P, x)) {
+      femgpu::ExchangePatch *xp;
+      uint32_t *oe;
+      uint16_t *os, *ip, *se, *op;
+      if ((st = upload(ctx, "x_patch", x.patches, &xp)) || (st = upload(ctx, "x_oe", x.out_entry, &oe)) ||
+          (st = upload(ctx, "x_os", x.out_src, &os)) || (st = upload(ctx, "x_ip", x.in_pos, &ip)) ||
+          (st = upload(ctx, "x_se", x.src_end, &se)) || (st = upload(ctx, "x_op", x.own_pos, &op)))
+        return st;
+      HIPCHK(hipStreamSynchronize(ctx->stream));  // x goes out of scope
+      dm.xpatch = xp;
+      dm.x_out_entry = oe;
+      dm.x_out_src = os;
+      dm.x_in_pos = ip;
+      dm.x_src_end = se;
+      dm.x_own_pos = op;
+      dm.x_in_max = x.n_in_max;
+      dm.x_src_max = x.n_src_max;
+      dm.x_entries = x.n_entries;
+    }
+  }
   std::vector<double> c64(size_t(n_nodes) * dim);
   std::vector<float> c32(c64.size());
   for (int64_t i = 0; i < n_nodes; ++i)
@@ -982,6 +1123,7 @@ int upload_plan(femgpu_ctx *ctx) {
   dm.coords32 = pc32;
   HIPCHK(hipStreamSynchronize(ctx->stream));
   ctx->have_mesh = true;
+  ctx->res_np = 0;
   ctx->dirty_mat = ctx->dirty_fix = ctx->dirty_diag = ctx->dirty_rhs = true;
   return ensure_fix(ctx);
 }
@@ -1010,6 +1152,7 @@ int femgpu_create(femgpu_ctx **out, int device_ordinal) {
   HIPCHK(femgpu::prepare_kernels());
   HIPCHK(femgpu::prepare_cg1_kernels());
   HIPCHK(femgpu::prepare_bl_kernels());
+  HIPCHK(femgpu::prepare_resident_kernels());
   *out = c.release();
   return FEMGPU_OK;
 }
@@ -1725,6 +1868,128 @@ static int solve_cg1(femgpu_ctx *ctx, const femgpu_solve_opts &o, int max_iter, 
   return FEMGPU_OK;
 }
 
+// solve_core's PCG with the iterations in resident launches, where the plan
+// fits the device (*ran; else nothing has happened): FP64 and FP32 in one
+// launch, MIXED one launch per residual replacement, which pauses on the
+// device as soon as the FP32 residual has dropped by inner_tol.
+static int solve_resident(femgpu_ctx *ctx, const femgpu_solve_opts &o, int max_iter,
+                          const double *f64, double *x64, femgpu_stats *S, bool *ran) {
+  const size_t nd = size_t(ctx->nn) * ctx->dim;
+  const int64_t na = ctx->dm.n_active * ctx->dim;
+  int st;
+  *ran = false;
+  if (o.precision == FEMGPU_FP64 ? !pcg_resident<double>(ctx) : !pcg_resident<float>(ctx))
+    return FEMGPU_OK;
+  // (a mixed solve to a relative residual of 1 or more does no iteration)
+  if (o.precision == FEMGPU_MIXED && !(o.tol < 1.0)) return FEMGPU_OK;
+  auto report = [&](const CgScalars &h) {
+    S->iterations = h.iter_final;
+    S->gamma_ratio = h.gamma0 > 0 ? h.g_final / h.gamma0 : 0.0;
+    S->status = done_status(h.done);
+  };
+  if (o.precision == FEMGPU_FP64) {
+    PcgWs<double> w;
+    if ((st = pcg_ws(ctx, "c64", w))) return st;
+    femgpu::ResPcg<double> a{};
+    a.r_in = f64;
+    a.x = x64;
+    a.p = w.p;
+    a.r_out = w.r;
+    a.invD = static_cast<double *>(ctx->bufs["invD64"].p);
+    a.fresh = 1;
+    a.kind = o.tol_kind;
+    a.eps = o.tol;
+    a.max_iter = max_iter;
+    femgpu::launch_fill<double>(x64 + na, int64_t(nd) - na, 0.0, ctx->stream);
+    if ((st = run_resident<double>(ctx, a, ran)) || !*ran) return st;
+    report(*ctx->h_sc);
+    return FEMGPU_OK;
+  }
+  if (o.precision != FEMGPU_FP32 && o.precision != FEMGPU_MIXED)
+    return fail(ctx, FEMGPU_E_ARG, "unknown precision");
+  PcgWs<float> w;
+  if ((st = pcg_ws(ctx, "c32", w))) return st;
+  femgpu::ResPcg<float> a{};
+  a.r_in = w.r;
+  a.x = w.x;
+  a.p = w.p;
+  a.r_out = w.r;
+  a.invD = static_cast<float *>(ctx->bufs["invD32"].p);
+  a.fresh = 1;
+  a.kind = o.tol_kind;
+  a.eps = o.tol;
+  a.max_iter = max_iter;
+  femgpu::launch_convert<double, float>(f64, w.r, int64_t(nd), ctx->stream);
+  femgpu::launch_fill<float>(w.x + na, int64_t(nd) - na, 0.f, ctx->stream);
+  if (o.precision == FEMGPU_FP32) {
+    if ((st = run_resident<float>(ctx, a, ran)) || !*ran) return st;
+    report(*ctx->h_sc);
+    femgpu::launch_convert<float, double>(w.x, x64, int64_t(nd), ctx->stream);
+    return FEMGPU_OK;
+  }
+  // MIXED: the reliable updates of solve_core's launch-per-kernel form
+  double *r64, *y64, *part64;
+  if ((st = dbuf(ctx, "ir_r", nd, &r64)) || (st = dbuf(ctx, "ir_y", nd, &y64)) ||
+      (st = dbuf(ctx, "partial64", size_t(ctx->plan.n_slots) * ctx->dim + 1, &part64)))
+    return st;
+  const double drop = o.inner_tol > 0 && o.inner_tol < 1 ? o.inner_tol : 0.1;
+  a.pause = drop * drop;
+  femgpu::launch_fill<double>(x64, int64_t(nd), 0.0, ctx->stream);
+  int status = FEMGPU_OK, replacements = 0, stag = 0, iters = 0;
+  bool kept_p = false;
+  double ff = 0.0, rel = 1.0, rel_prev = 1.0;
+  for (;;) {
+    if ((st = run_resident<float>(ctx, a, ran)) || !*ran) return st;
+    const CgScalars h = *ctx->h_sc;
+    if (a.fresh) ff = h.rr0;
+    iters = h.iter_final;
+    if (!(ff > 0.0)) {
+      if (h.done != 1) status = done_status(h.done);
+      break;
+    }
+    femgpu::launch_flush_x(ctx->dm, x64, w.x, ctx->stream);
+    const bool retry = h.done == 3 && kept_p;
+    if (h.done != 1 && h.done != 5 && !retry) {
+      status = done_status(h.done);
+      break;
+    }
+    double rr64, ff64;
+    if ((st = residual64(ctx, f64, x64, y64, r64, part64, &rr64, &ff64))) return st;
+    rel = std::sqrt(rr64 / ff);
+    const double rel_rec = std::sqrt(h.rr_final / ff);
+    if (trace_enabled())
+      std::fprintf(stderr, "femgpu mixed: %d iterations, stop %d, FP32 recurrence rel-res %.3e, "
+                   "FP64 rel-res %.3e\n", iters, h.done, rel_rec, rel);
+    if (rel <= o.tol) break;
+    if (iters >= max_iter || replacements > 1000) {
+      status = FEMGPU_E_MAXIT;
+      break;
+    }
+    stag = replacements > 0 && rel >= rel_prev ? stag + 1 : 0;
+    if (stag >= 2) {
+      status = FEMGPU_E_STAGNATION;
+      break;
+    }
+    femgpu::launch_convert<double, float>(r64, w.r, na, ctx->stream);
+    const bool restart = rel > 2.0 * rel_rec || rel > 0.5 * rel_prev || retry;
+    if (restart) femgpu::launch_fill<float>(w.p, int64_t(nd), 0.f, ctx->stream);
+    kept_p = !restart;
+    rel_prev = rel;
+    a.fresh = 0;
+    a.gamma0 = h.gamma0;
+    a.rr0 = h.rr0;
+    a.thresh = h.thresh;
+    a.g_prev = h.g[1];
+    a.it0 = iters;
+    a.pause = rr64 * drop * drop;
+    ++replacements;
+  }
+  S->iterations = iters;
+  S->outer_iterations = replacements;
+  S->status = status;
+  return FEMGPU_OK;
+}
+
 // Static solve of K x = f with f the device vector `f_name` (n_nodes x dim,
 // internal order); the solution stays in the device buffer "sol64" and is
 // copied to u_out (user order) when u_out is given.
@@ -1752,7 +2017,12 @@ static int solve_core(femgpu_ctx *ctx, const femgpu_solve_opts *opts, const char
   femgpu_stats S{};
   int iters = 0, done = 0;
   HIPCHK(hipEventRecord(ctx->ev0, ctx->stream));
-  if (o.recurrence == FEMGPU_CG_SINGLE_REDUCTION) {
+  bool resident = false;
+  if (o.recurrence == FEMGPU_CG_STANDARD &&
+      (st = solve_resident(ctx, o, max_iter, f64, x64, &S, &resident)))
+    return st;
+  if (resident) {
+  } else if (o.recurrence == FEMGPU_CG_SINGLE_REDUCTION) {
     if ((st = solve_cg1(ctx, o, max_iter, block, f64, x64, sc, &S))) return st;
   } else if (o.precision == FEMGPU_FP64) {
     PcgWs<double> w;

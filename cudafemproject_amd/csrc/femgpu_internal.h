@@ -99,4 +99,31 @@ bool stride_records(const MeshPlan &plan, std::vector<uint32_t> &rec,
 void pack_patch_nodes(const MeshPlan &plan, int stride, std::vector<int32_t> &pgid,
                       std::vector<int32_t> &pslot, std::vector<uint16_t> &pend);
 
+// What a patch sends and receives when every patch finishes its own copy of
+// the interface nodes (resident.hip).  For every interface node each patch
+// holding it sends its partial sum to each of the others: one entry per
+// (sender, receiver, node).  Entries are numbered receiver by receiver
+// (every receiver's range starts at a multiple of 64) and within a receiver
+// sender by sender, so that both the sender's stores and the receiver's loads
+// run along consecutive entries.
+// A patch keeps its interface nodes' contributions node by node, each node's
+// in slot order: places within the patch.
+struct ExchangePatch {      // 12 bytes
+  int32_t in_start;         // the patch's entries: in_start + 0 .. n_in - 1
+  int32_t n_in;             // received, and sent
+  int32_t out_start;        // first in out_entry / out_src / in_pos (n_in of each)
+};
+struct ExchangePlan {
+  int64_t n_entries = 0;               // with the gaps between receivers
+  int n_in_max = 0, n_src_max = 0;     // most entries and places of a patch
+  std::vector<ExchangePatch> patches;
+  std::vector<uint32_t> out_entry;     // entries a patch writes
+  std::vector<uint16_t> out_src;       // the place of the contribution it sends there
+  std::vector<uint16_t> in_pos;        // the place of each entry it receives
+  std::vector<uint16_t> src_end;       // per patch interface node (sh order): end of its places
+  std::vector<uint16_t> own_pos;       // and the place of the patch's own contribution
+};
+// False when a patch exchanges too much for 16-bit indices.
+bool build_exchange(const MeshPlan &plan, ExchangePlan &x);
+
 }  // namespace femgpu

@@ -43,6 +43,13 @@ struct DevMesh {
   const double *diag64 = nullptr;     // assembled diag(K), set before any matvec
   const float *diag32 = nullptr;
   double lam = 0, mu = 0;             // Lame constants (2D: plane stress)
+  // exchange tables of the resident kernels (ExchangePlan; null: none built)
+  const ExchangePatch *xpatch = nullptr;
+  const uint32_t *x_out_entry = nullptr;
+  const uint16_t *x_out_src = nullptr, *x_in_pos = nullptr;
+  const uint16_t *x_src_end = nullptr, *x_own_pos = nullptr;
+  int x_in_max = 0, x_src_max = 0;
+  int64_t x_entries = 0;
 };
 
 // Scalars of one PCG run, device resident.  Iteration j of the fused

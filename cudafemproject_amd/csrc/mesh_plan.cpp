@@ -420,4 +420,74 @@ void pack_patch_nodes(const MeshPlan &plan, int stride, std::vector<int32_t> &pg
   }
 }
 
+bool build_exchange(const MeshPlan &plan, ExchangePlan &x) {
+  const size_t np = plan.patches.size();
+  x = ExchangePlan();
+  x.patches.assign(np, ExchangePatch{});
+  x.src_end.assign(plan.sh_gid.size(), 0);
+  x.own_pos.assign(plan.sh_gid.size(), 0);
+  // the patch of every slot and the place that its node's first slot has there
+  std::vector<int32_t> slot_patch(size_t(plan.n_slots)), slot_place(size_t(plan.n_slots));
+  for (size_t p = 0; p < np; ++p) {
+    const PatchInfo &Q = plan.patches[p];
+    int32_t n = 0;
+    for (int32_t i = Q.sh_start; i < Q.sh_start + Q.n_sh; ++i) {
+      const size_t v = size_t(plan.sh_gid[size_t(i)] - plan.n_owned);
+      const int32_t s = plan.sh_slot[size_t(i)], s0 = plan.slot_start[v];
+      slot_patch[size_t(s)] = int32_t(p);
+      slot_place[size_t(s)] = n;
+      if (n + (plan.slot_start[v + 1] - s0) > 0xffff) return false;
+      x.own_pos[size_t(i)] = uint16_t(n + (s - s0));
+      n += plan.slot_start[v + 1] - s0;
+      x.src_end[size_t(i)] = uint16_t(n);
+    }
+    x.n_src_max = std::max(x.n_src_max, int(n));
+  }
+  // senders in order: a receiver's entries come sender by sender
+  struct Out {
+    int32_t to, entry;  // receiver and its entry (receiver-local)
+    uint16_t src, pos;  // places at the sender and at the receiver
+  };
+  std::vector<std::vector<Out>> out(np);
+  for (size_t p = 0; p < np; ++p) {
+    const PatchInfo &Q = plan.patches[p];
+    for (int32_t i = Q.sh_start; i < Q.sh_start + Q.n_sh; ++i) {
+      const size_t v = size_t(plan.sh_gid[size_t(i)] - plan.n_owned);
+      const int32_t mine = plan.sh_slot[size_t(i)], s0 = plan.slot_start[v];
+      for (int32_t s = s0; s < plan.slot_start[v + 1]; ++s)
+        if (s != mine) {
+          const size_t q = size_t(slot_patch[size_t(s)]);
+          out[p].push_back({int32_t(q), x.patches[q].n_in++, x.own_pos[size_t(i)],
+                            uint16_t(slot_place[size_t(s)] + (mine - s0))});
+        }
+    }
+  }
+  int64_t n_out = 0;
+  for (size_t p = 0; p < np; ++p) {
+    ExchangePatch &E = x.patches[p];
+    E.in_start = int32_t(x.n_entries);
+    E.out_start = int32_t(n_out);
+    x.n_entries += (int64_t(E.n_in) + 63) & ~int64_t(63);
+    n_out += E.n_in;  // (each node's patches send to each other: as many as received)
+    if (x.n_entries > INT32_MAX / 64) return false;
+    x.n_in_max = std::max(x.n_in_max, int(E.n_in));
+  }
+  x.out_entry.resize(size_t(n_out));
+  x.out_src.resize(size_t(n_out));
+  x.in_pos.resize(size_t(n_out));
+  for (size_t p = 0; p < np; ++p) {
+    std::stable_sort(out[p].begin(), out[p].end(),
+                     [](const Out &a, const Out &b) { return a.to < b.to; });
+    size_t k = size_t(x.patches[p].out_start);
+    for (const Out &o : out[p]) {
+      const ExchangePatch &R = x.patches[size_t(o.to)];
+      x.out_entry[k] = uint32_t(R.in_start + o.entry);
+      x.out_src[k] = o.src;
+      x.in_pos[size_t(R.out_start + o.entry)] = o.pos;
+      ++k;
+    }
+  }
+  return true;
+}
+
 }  // namespace femgpu

@@ -1,0 +1,77 @@
+// resident.h -- PCG solves and explicit time steps that stay on the chip: one
+// launch runs many iterations (steps), one workgroup per patch, the patch's
+// mesh data and node state in registers and LDS throughout (resident.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "kernels.h"
+
+namespace femgpu {
+
+// The workgroups' exchange buffer for np patches, in 8-byte words: the tag of
+// the last exchange (advanced by every launch), the abort flag, and the
+// tagged partials in EX_COPIES copies on pages of their own.  The interface
+// entries are tagged words too (res_entry_words).  Both are zeroed when they
+// are allocated or the plan changes, and after an aborted launch.
+constexpr int EX_COPIES = 8;
+constexpr size_t RES_HEAD = 512;
+__host__ __device__ inline size_t res_copy_words(int np) {
+  return (size_t(6) * size_t(np) + 511) & ~size_t(511);
+}
+inline size_t res_words(int np) { return RES_HEAD + EX_COPIES * res_copy_words(np); }
+template <typename T>
+inline size_t res_entry_words(int64_t n_entries, int dim) {
+  return size_t(n_entries) * dim * (sizeof(T) / 4) + 1;
+}
+
+// The largest plan the exchange tables are built for (compute units).
+constexpr int RES_PATCHES_MAX = 256;
+
+// One resident PCG launch.  r, x, p: node vectors in internal order; the
+// solve starts from r_in (x = p = 0) when fresh, else from r_in, x, p and
+// the scalars of an earlier launch.
+template <typename T>
+struct ResPcg {
+  const T *r_in;
+  T *x, *p, *r_out;
+  const T *invD;
+  unsigned long long *entries;  // interface entries (res_entry_words)
+  OpShift<T> sh;
+  unsigned long long *words;  // res_words(np)
+  CgScalars *sc;              // the scalars at the end (host-visible memory)
+  int fresh, kind;
+  double eps;             // fresh: tolerance (threshold formed from the initial residual)
+  double gamma0, rr0, thresh, g_prev;  // not fresh
+  double pause;           // stop with done = 5 once r'r < pause (fresh: times
+                          // the initial r'r; 0: never)
+  int it0, max_iter, cap; // updates done before, in all, and at most in this launch
+};
+
+// done codes of a resident launch besides CgScalars': 6 the launch did not
+// complete (its workgroups were not on the chip together), 7 cap reached.
+constexpr int RES_ABORTED = 6, RES_CAP = 7;
+
+// The part of the device that a resident launch takes, and of one compute
+// unit that a workgroup takes.
+struct ResFit {
+  double share = 0.0, block = 0.0;
+};
+
+// Whether the plan's PCG runs resident: every workgroup on a compute unit of
+// its own.  Several workgroups per unit would fit, and lose to the
+// launch-per-kernel form (a 40^3-hex cube, 500 patches: FP64 32.3 against
+// 18.1 us per iteration, mixed 20.4 against 15.3), whose launches cost
+// less the more work there is between them; at 256 patches (32^3 hexes) the
+// resident form is ahead, 12.0 against 14.4 and 10.5 against 13.7 us.
+template <typename T>
+bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit);
+
+template <typename T>
+void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &a, hipStream_t s);
+
+hipError_t prepare_resident_kernels();
+
+}  // namespace femgpu
