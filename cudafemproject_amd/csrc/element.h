@@ -160,6 +160,18 @@ __device__ __forceinline__ T pcg_dir(T invd, T r, T beta, T p) {
   return fma(beta, p, mul_rn(invd, r));
 }
 
+// GN22 corrector of one DOF (the operations of k_dyn_correct): r = F - K d~,
+// v~ = v + c2 a, (1 + alpha c3) M a' = r - alpha M v~, v' = v~ + c3 a'.
+template <typename T>
+__device__ __forceinline__ void gn22_correct(T cf, T cu, T ff, T fu, T kd, T im, T c2, T c3,
+                                             T alpha, T scale, T &a, T &v) {
+  const T r = cf * ff + cu * fu - kd;
+  const T vp = v + c2 * a;
+  const T av = alpha != T(0) ? (r * im - alpha * vp) * scale : r * im;
+  a = av;
+  v = vp + c3 * av;
+}
+
 // ---------------------------------------------------------------------------
 // Element kernels (registers only).  X, U: node-major (npe x dim).
 // fix: bit (dim*a + c) set when that local DOF is constrained.
@@ -293,30 +305,36 @@ __device__ __forceinline__ T recip(T x) {
 // constrained components of u per node and set the constrained rows from
 // the assembled diagonal): f_a = S(H)' c_a with S(H) scaled by
 // es / (6|det J|) once, and f_0 = -(f_1 + f_2 + f_3) since c_0 = -sum c_a.
-// Returns u'K u of the element.
+// Returns u'K u of the element.  In two halves: the geometry g = (c_1, c_2,
+// c_3, scale), and the force from it.
 template <typename T>
-__device__ __forceinline__ T tet_force_free(const T *X, const T *U, T lam, T mu, T es, T *F) {
+__device__ __forceinline__ void tet_geometry(const T *X, T es, T *g) {
   const T e1x = X[3] - X[0], e1y = X[4] - X[1], e1z = X[5] - X[2];
   const T e2x = X[6] - X[0], e2y = X[7] - X[1], e2z = X[8] - X[2];
   const T e3x = X[9] - X[0], e3y = X[10] - X[1], e3z = X[11] - X[2];
-  T c[4][3];
-  c[1][0] = e2y * e3z - e2z * e3y;
-  c[1][1] = e2z * e3x - e2x * e3z;
-  c[1][2] = e2x * e3y - e2y * e3x;
-  c[2][0] = e3y * e1z - e3z * e1y;
-  c[2][1] = e3z * e1x - e3x * e1z;
-  c[2][2] = e3x * e1y - e3y * e1x;
-  c[3][0] = e1y * e2z - e1z * e2y;
-  c[3][1] = e1z * e2x - e1x * e2z;
-  c[3][2] = e1x * e2y - e1y * e2x;
-  const T det = e1x * c[1][0] + e1y * c[1][1] + e1z * c[1][2];
-  const T s = es * recip<T>(T(6) * fabs(det));
+  g[0] = e2y * e3z - e2z * e3y;
+  g[1] = e2z * e3x - e2x * e3z;
+  g[2] = e2x * e3y - e2y * e3x;
+  g[3] = e3y * e1z - e3z * e1y;
+  g[4] = e3z * e1x - e3x * e1z;
+  g[5] = e3x * e1y - e3y * e1x;
+  g[6] = e1y * e2z - e1z * e2y;
+  g[7] = e1z * e2x - e1x * e2z;
+  g[8] = e1x * e2y - e1y * e2x;
+  const T det = e1x * g[0] + e1y * g[1] + e1z * g[2];
+  g[9] = es * recip<T>(T(6) * fabs(det));
+}
+
+template <typename T>
+__device__ __forceinline__ T tet_force_geo(const T *g, const T *U, T lam, T mu, T *F) {
+  const T *c1 = g, *c2 = g + 3, *c3 = g + 6;
+  const T s = g[9];
   T H[3][3];
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const T d1 = U[3 + i] - U[i], d2 = U[6 + i] - U[i], d3 = U[9 + i] - U[i];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) H[i][j] = d1 * c[1][j] + d2 * c[2][j] + d3 * c[3][j];
+    for (int j = 0; j < 3; ++j) H[i][j] = d1 * c1[j] + d2 * c2[j] + d3 * c3[j];
   }
   const T ls = lam * s, ms = mu * s;
   const T tr = ls * (H[0][0] + H[1][1] + H[2][2]);
@@ -328,9 +346,10 @@ __device__ __forceinline__ T tet_force_free(const T *X, const T *U, T lam, T mu,
   const T S12 = ms * (H[1][2] + H[2][1]);
 #pragma unroll
   for (int a = 1; a < 4; ++a) {
-    F[3 * a + 0] = S00 * c[a][0] + S01 * c[a][1] + S02 * c[a][2];
-    F[3 * a + 1] = S01 * c[a][0] + S11 * c[a][1] + S12 * c[a][2];
-    F[3 * a + 2] = S02 * c[a][0] + S12 * c[a][1] + S22 * c[a][2];
+    const T *c = g + 3 * (a - 1);
+    F[3 * a + 0] = S00 * c[0] + S01 * c[1] + S02 * c[2];
+    F[3 * a + 1] = S01 * c[0] + S11 * c[1] + S12 * c[2];
+    F[3 * a + 2] = S02 * c[0] + S12 * c[1] + S22 * c[2];
   }
 #pragma unroll
   for (int k = 0; k < 3; ++k) F[k] = -(F[3 + k] + F[6 + k] + F[9 + k]);
@@ -341,12 +360,26 @@ __device__ __forceinline__ T tet_force_free(const T *X, const T *U, T lam, T mu,
 }
 
 template <typename T>
-__device__ __forceinline__ T tri_force_free(const T *X, const T *U, T lam, T mu, T es, T *F) {
-  const T e1x = X[2] - X[0], e1y = X[3] - X[1];
-  const T e2x = X[4] - X[0], e2y = X[5] - X[1];
-  // c_1 = (e2y, -e2x), c_2 = (-e1y, e1x)
-  const T det = e1x * e2y - e1y * e2x;
-  const T s = es * recip<T>(T(2) * fabs(det));
+__device__ __forceinline__ T tet_force_free(const T *X, const T *U, T lam, T mu, T es, T *F) {
+  T g[10];
+  tet_geometry<T>(X, es, g);
+  return tet_force_geo<T>(g, U, lam, mu, F);
+}
+
+// Triangles: g = (e1, e2, scale), c_1 = (e2y, -e2x), c_2 = (-e1y, e1x).
+template <typename T>
+__device__ __forceinline__ void tri_geometry(const T *X, T es, T *g) {
+  g[0] = X[2] - X[0];
+  g[1] = X[3] - X[1];
+  g[2] = X[4] - X[0];
+  g[3] = X[5] - X[1];
+  const T det = g[0] * g[3] - g[1] * g[2];
+  g[4] = es * recip<T>(T(2) * fabs(det));
+}
+
+template <typename T>
+__device__ __forceinline__ T tri_force_geo(const T *g, const T *U, T lam, T mu, T *F) {
+  const T e1x = g[0], e1y = g[1], e2x = g[2], e2y = g[3], s = g[4];
   const T dx1 = U[2] - U[0], dy1 = U[3] - U[1], dx2 = U[4] - U[0], dy2 = U[5] - U[1];
   const T H00 = dx1 * e2y - dx2 * e1y, H01 = -dx1 * e2x + dx2 * e1x;
   const T H10 = dy1 * e2y - dy2 * e1y, H11 = -dy1 * e2x + dy2 * e1x;
@@ -365,6 +398,30 @@ __device__ __forceinline__ T tri_force_free(const T *X, const T *U, T lam, T mu,
 #pragma unroll
   for (int i = 0; i < 6; ++i) en += U[i] * F[i];
   return en;
+}
+
+template <typename T>
+__device__ __forceinline__ T tri_force_free(const T *X, const T *U, T lam, T mu, T es, T *F) {
+  T g[5];
+  tri_geometry<T>(X, es, g);
+  return tri_force_geo<T>(g, U, lam, mu, F);
+}
+
+// DIM * DIM + 1 values of geometry.
+template <typename T, int DIM>
+__device__ __forceinline__ void elem_geometry(const T *X, T es, T *g) {
+  if constexpr (DIM == 3)
+    tet_geometry<T>(X, es, g);
+  else
+    tri_geometry<T>(X, es, g);
+}
+
+template <typename T, int DIM>
+__device__ __forceinline__ T elem_force_geo(const T *g, const T *U, T lam, T mu, T *F) {
+  if constexpr (DIM == 3)
+    return tet_force_geo<T>(g, U, lam, mu, F);
+  else
+    return tri_force_geo<T>(g, U, lam, mu, F);
 }
 
 template <typename T, int DIM>

@@ -40,6 +40,7 @@ constexpr int NODE_PART = 4 * femgpu::NODE_PARTS;  // partials of node kernels (
 // Iterations of one resident launch (a few ms to tens of ms of device time;
 // a longer solve continues in further launches)
 constexpr int RES_ITER_CAP = 4096;
+constexpr int RES_STEP_CAP = 16384;  // the same for explicit steps
 
 struct DevBuf {
   void *p = nullptr;
@@ -122,7 +123,7 @@ struct femgpu_ctx {
 
   bool dirty_mat = true, dirty_fix = true, dirty_diag = true, dirty_rhs = true;
 
-  CgScalars *h_sc = nullptr;  // pinned: [0], [1] poll ring, [2] residual norms
+  CgScalars *h_sc = nullptr;  // pinned: [0], [1] poll ring, [2] residual norms, [3] abort flag
   hipEvent_t ev_poll[4] = {nullptr, nullptr, nullptr, nullptr};
   int emax_req = 0, threads_req = 0;
   int tuned_threads = 256;  // threads per patch of the current plan
@@ -137,6 +138,8 @@ struct femgpu_ctx {
   // resident solves (resident.h): patches the exchange words are zeroed for;
   // off after a launch that did not complete
   int res_np = 0;
+  int dyn_np = 0;                // the same for the time steps' entries
+  unsigned dyn_tag[2] = {0, 0};  // and the last tags used in them (FP32, FP64)
   bool res_off = false;
 
   // femgpu_matvec_noalloc: this device's fixed scratch array (device
@@ -193,6 +196,36 @@ int plan_mesh(int dim, int64_t n_nodes, const double *nodes, int64_t n_elems, co
     }
     emax = std::max(64, emax * 7 / 8);
   }
+}
+
+// The plan of a mesh without a requested tuning: 256 threads and 768 elements
+// per patch, or 512 and 1536 where that brings the plan to at most
+// RES_PATCHES_MAX patches and 256 threads do not: the solves and explicit
+// steps then run resident (resident.h), a patch per compute unit.  (Above
+// that size 256 threads: the fastest FP64 iteration in launches, within a few
+// percent of the fastest in FP32.)  The second plan is made beside the first.
+int plan_default(int dim, int64_t n_nodes, const double *nodes, int64_t n_elems,
+                 const int32_t *elems, MeshPlan &plan, int *threads, std::string &msg) {
+  constexpr int64_t NP = femgpu::RES_PATCHES_MAX;
+  MeshPlan wide;
+  int wide_st = FEMGPU_E_STATE;
+  std::thread side;
+  // (a patch of 768 elements has more than 256 nodes in 2D and often in 3D:
+  // from half the elements on, 256 threads may give more than NP patches)
+  if (n_elems > NP * 768 / 2 && n_elems <= NP * 1536)
+    side = std::thread([&] {
+      std::string m;
+      wide_st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 512, wide, m);
+    });
+  const int st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 256, plan, msg);
+  if (side.joinable()) side.join();
+  *threads = 256;
+  if (st == FEMGPU_OK && wide_st == FEMGPU_OK && int64_t(plan.patches.size()) > NP &&
+      int64_t(wide.patches.size()) <= NP) {
+    plan = std::move(wide);
+    *threads = 512;
+  }
+  return st;
 }
 
 void drop_graphs(femgpu_ctx *ctx) {
@@ -722,20 +755,23 @@ bool pcg_resident(const femgpu_ctx *ctx) {
   return !ctx->res_off && femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit);
 }
 
-// The exchange words and entries (of 8-byte values), zeroed for this plan.
+// The exchange words and this precision's entries, zeroed for this plan (an
+// entry's tag is short: words of another precision's layout would not do).
+template <typename T>
 int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long **entries) {
   const size_t n = femgpu::res_words(ctx->dm.np);
-  const size_t ne = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
+  const size_t n64 = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
+  const size_t n32 = femgpu::res_entry_words<float>(ctx->dm.x_entries, ctx->dim);
   double *w, *e;
   int st;
-  if ((st = dbuf(ctx, "res_words", n, &w)) || (st = dbuf(ctx, "res_entries", ne, &e))) return st;
+  if ((st = dbuf(ctx, "res_words", n, &w)) || (st = dbuf(ctx, "res_entries", n64 + n32, &e))) return st;
   if (ctx->res_np != ctx->dm.np) {
     femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
-    femgpu::launch_fill<double>(e, int64_t(ne), 0.0, ctx->stream);
+    femgpu::launch_fill<double>(e, int64_t(n64 + n32), 0.0, ctx->stream);
     ctx->res_np = ctx->dm.np;
   }
   *words = reinterpret_cast<unsigned long long *>(w);
-  *entries = reinterpret_cast<unsigned long long *>(e);
+  *entries = reinterpret_cast<unsigned long long *>(e) + (sizeof(T) == 8 ? 0 : n64);
   return FEMGPU_OK;
 }
 
@@ -749,7 +785,7 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
   int st;
   if (!femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit))
     return fail(ctx, FEMGPU_E_STATE, "internal error: resident PCG does not fit");
-  if ((st = res_buffers(ctx, &a.words, &a.entries))) return st;
+  if ((st = res_buffers<T>(ctx, &a.words, &a.entries))) return st;
   a.sc = ctx->h_sc;
   a.cap = RES_ITER_CAP;
   for (;;) {
@@ -778,6 +814,55 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
     a.it0 = h.iter_final;
   }
   *ok = true;
+  return FEMGPU_OK;
+}
+
+// Explicit steps 1 .. n_steps in resident launches, from rest; d.d, d.v, d.a
+// end with the last state.  *ok as in run_resident (d.d, d.v, d.a are then
+// undefined).
+template <typename T>
+int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *ok) {
+  femgpu::ResFit fit;
+  int st;
+  if (!femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit))
+    return fail(ctx, FEMGPU_E_STATE, "internal error: resident steps do not fit");
+  // two sets of entries per precision, then the abort flag
+  const size_t n64 = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
+  const size_t n32 = femgpu::res_entry_words<float>(ctx->dm.x_entries, ctx->dim);
+  const size_t n = 2 * (n64 + n32) + 1;
+  double *w;
+  if ((st = dbuf(ctx, "dyn_entries", n, &w))) return st;
+  d.entries = reinterpret_cast<unsigned long long *>(w) + (sizeof(T) == 8 ? 0 : 2 * n64);
+  d.entry_words = sizeof(T) == 8 ? n64 : n32;
+  d.abort = reinterpret_cast<unsigned long long *>(w) + n - 1;
+  d.fresh = 1;
+  *ok = true;
+  for (int done = 0; done < n_steps && *ok; done += d.n_steps) {
+    d.n_steps = std::min(n_steps - done, RES_STEP_CAP);
+    if (ctx->dyn_np != ctx->dm.np) {
+      femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
+      ctx->dyn_np = ctx->dm.np;
+      ctx->dyn_tag[0] = ctx->dyn_tag[1] = 0;
+    }
+    unsigned &last_tag = ctx->dyn_tag[sizeof(T) == 8 ? 1 : 0];
+    d.step0 = done + 1;
+    d.tag0 = last_tag + 1u;
+    last_tag += unsigned(d.n_steps);
+    unsigned long long *gave_up = reinterpret_cast<unsigned long long *>(&ctx->h_sc[3]);
+    {
+      ResidentGate gate(ctx->device, fit.share, fit.block);
+      femgpu::launch_res_dyn<T>(ctx->dm, d, ctx->stream);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipMemcpyAsync(gave_up, d.abort, sizeof(*gave_up), hipMemcpyDeviceToHost, ctx->stream));
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    *ok = *gave_up == 0;
+    d.fresh = 0;
+  }
+  if (!*ok) {
+    ctx->res_off = true;
+    ctx->dyn_np = 0;
+  }
   return FEMGPU_OK;
 }
 
@@ -1123,7 +1208,7 @@ int upload_plan(femgpu_ctx *ctx) {
   dm.coords32 = pc32;
   HIPCHK(hipStreamSynchronize(ctx->stream));
   ctx->have_mesh = true;
-  ctx->res_np = 0;
+  ctx->res_np = ctx->dyn_np = 0;
   ctx->dirty_mat = ctx->dirty_fix = ctx->dirty_diag = ctx->dirty_rhs = true;
   return ensure_fix(ctx);
 }
@@ -1209,13 +1294,12 @@ int femgpu_set_mesh(femgpu_ctx *ctx, int dim, int64_t n_nodes, const double *nod
   const int npe = dim + 1;
   // one workgroup thread per patch node and at most EPT = 3 elements per
   // thread: patches of <= 3 * threads elements and <= threads nodes
-  // Default 256 threads (768-element patches): on gfx950 the fastest PCG
-  // iteration in FP64 (no register spills, three workgroups per CU) and
-  // within a few percent of the fastest in FP32 among 256/512/1024.
-  const int threads = ctx->threads_req ? ctx->threads_req : 256;
+  int threads = ctx->threads_req ? ctx->threads_req : 256;
   {
     std::string msg;
-    const int st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, ctx->emax, threads, ctx->plan, msg);
+    const int st = ctx->threads_req || ctx->emax
+                       ? plan_mesh(dim, n_nodes, nodes, n_elems, elems, ctx->emax, threads, ctx->plan, msg)
+                       : plan_default(dim, n_nodes, nodes, n_elems, elems, ctx->plan, &threads, msg);
     if (st) return fail(ctx, st, msg);
   }
   // degenerate elements
@@ -1288,8 +1372,10 @@ int femgpu_plan_info(int dim, int64_t n_nodes, const double *nodes, int64_t n_el
     return FEMGPU_E_ARG;
   MeshPlan plan;
   std::string msg;
-  const int st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, elems_per_patch,
-                           patch_threads ? patch_threads : 256, plan, msg);
+  int threads = patch_threads ? patch_threads : 256;
+  const int st = elems_per_patch || patch_threads
+                     ? plan_mesh(dim, n_nodes, nodes, n_elems, elems, elems_per_patch, threads, plan, msg)
+                     : plan_default(dim, n_nodes, nodes, n_elems, elems, plan, &threads, msg);
   if (st) return st;
   info[0] = int64_t(plan.patches.size());
   info[1] = plan.n_owned;
@@ -2516,8 +2602,51 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   // alternate between two buffers as well, and the interface nodes' v and a
   // lag one step (the displacement does not).
   const bool one_launch = expl && nrec == 0 && !relax;
+  femgpu::ResFit fit;
+  bool resident = expl && !relax && !ctx->res_off &&
+                  femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit);
+  if (resident) {
+    femgpu::ResDyn<T> r{};
+    r.d = dd;
+    r.v = dv;
+    r.a = da;
+    r.f_file = dff;
+    r.f_unit = dfu;
+    r.invM = dinvM;
+    r.coef_file = dcf;
+    r.coef_unit = dcu;
+    r.dt = T(C.dt);
+    r.c1 = T(C.c1);
+    r.c2 = T(C.c2);
+    r.c3 = T(C.c3);
+    r.alpha = T(C.alpha);
+    r.scale = T(C.expl_scale);
+    if (nrec && max_samples > 0) {
+      std::vector<int32_t> of(size_t(ctx->nn), -1), next(size_t(nrec), -1);
+      for (int i = nrec - 1; i >= 0; --i) {
+        int32_t &head = of[size_t(ctx->plan.node_inv[ctx->recv[i]])];
+        next[size_t(i)] = head;
+        head = i;
+      }
+      int32_t *pof, *pnext;
+      if ((st = upload(ctx, "recv_of", of, &pof)) || (st = upload(ctx, "recv_next", next, &pnext)))
+        return st;
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+      r.rec_of = pof;
+      r.rec_next = pnext;
+      r.n_rec = nrec;
+      r.rec_every = every;
+      r.rec_samples = max_samples;
+      r.rec_quantity = ctx->recv_quantity;
+      r.traces = dtr;
+    }
+    if ((st = run_resident_steps<T>(ctx, r, endnt, &resident))) return st;
+    if (!resident) {
+      for (T *p : {dd, dv, da}) femgpu::launch_fill<T>(p, int64_t(nd), T(0), ctx->stream);
+    }
+  }
   T *vbufs[2] = {dv, dv}, *abufs[2] = {da, da}, *pbufs[2] = {dpart, dpart};
-  if (one_launch) {
+  if (one_launch && !resident) {
     T *dv2, *da2, *dpart2;
     if ((st = dbuf(ctx, tg + "v2", nd, &dv2)) || (st = dbuf(ctx, tg + "a2", nd, &da2)) ||
         (st = dbuf(ctx, tg + "part2", size_t(ctx->plan.n_slots) * d + 1, &dpart2)))
@@ -2556,7 +2685,9 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       record(k, dbufs[par ^ 1]);
     }
   };
-  if (expl) {
+  if (resident) {
+    steps = endnt;
+  } else if (expl) {
     // Steps are captured in a HIP graph of G steps (G even, so every replay
     // starts on buffer 0) when at least one full graph fits the run; the
     // remainder (or the whole run, and every step when graphs are disabled)
@@ -2818,7 +2949,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   S.run_ms = ms;
   S.steps = steps;
   if (u_out) {
-    const T *dfin = expl ? dbufs[steps & 1] : dd;
+    const T *dfin = expl && !resident ? dbufs[steps & 1] : dd;
     if ((st = download_nodes<T>(ctx, dfin, u_out))) return st;
   }
   if (nrec) {

@@ -97,18 +97,6 @@ struct PatchArgs {
   T c2, c3, alpha, scale;   // GN22 corrector and mass-damping coefficients
 };
 
-// GN22 corrector of one DOF (the operations of k_dyn_correct): r = F - K d~,
-// v~ = v + c2 a, (1 + alpha c3) M a' = r - alpha M v~, v' = v~ + c3 a'.
-template <typename T>
-__device__ __forceinline__ void gn22_correct(T cf, T cu, T ff, T fu, T kd, T im, T c2, T c3,
-                                             T alpha, T scale, T &a, T &v) {
-  const T r = cf * ff + cu * fu - kd;
-  const T vp = v + c2 * a;
-  const T av = alpha != T(0) ? (r * im - alpha * vp) * scale : r * im;
-  a = av;
-  v = vp + c3 * av;
-}
-
 // One workgroup per patch, one patch node per thread (phases A and C), up to
 // EPT elements per thread (phase B).  The element forces stay in registers
 // and are assembled one component at a time through a single-component LDS

@@ -12,8 +12,8 @@
 namespace femgpu {
 
 // The workgroups' exchange buffer for np patches, in 8-byte words: the tag of
-// the last exchange (advanced by every launch), the abort flag, and the
-// tagged partials in EX_COPIES copies on pages of their own.  The interface
+// the last exchange, the abort flag, the tags of the last trade of entries
+// (FP32, FP64; every launch advances its tags), and the tagged partials in EX_COPIES copies on pages of their own.  The interface
 // entries are tagged words too (res_entry_words).  Both are zeroed when they
 // are allocated or the plan changes, and after an aborted launch.
 constexpr int EX_COPIES = 8;
@@ -22,9 +22,11 @@ __host__ __device__ inline size_t res_copy_words(int np) {
   return (size_t(6) * size_t(np) + 511) & ~size_t(511);
 }
 inline size_t res_words(int np) { return RES_HEAD + EX_COPIES * res_copy_words(np); }
+// Words of an entry: dim values of tb bytes, 48 bits to a word.
+__host__ __device__ constexpr int res_entry_size(int dim, int tb) { return (dim * tb * 8 + 47) / 48; }
 template <typename T>
 inline size_t res_entry_words(int64_t n_entries, int dim) {
-  return size_t(n_entries) * dim * (sizeof(T) / 4) + 1;
+  return size_t(n_entries) * res_entry_size(dim, int(sizeof(T))) + 1;
 }
 
 // The largest plan the exchange tables are built for (compute units).
@@ -60,17 +62,44 @@ struct ResFit {
   double share = 0.0, block = 0.0;
 };
 
-// Whether the plan's PCG runs resident: every workgroup on a compute unit of
-// its own.  Several workgroups per unit would fit, and lose to the
-// launch-per-kernel form (a 40^3-hex cube, 500 patches: FP64 32.3 against
-// 18.1 us per iteration, mixed 20.4 against 15.3), whose launches cost
-// less the more work there is between them; at 256 patches (32^3 hexes) the
-// resident form is ahead, 12.0 against 14.4 and 10.5 against 13.7 us.
+// Whether the plan's PCG runs resident: patches of up to 512 nodes and 1536
+// elements, every workgroup on a compute unit of its own.  Several workgroups
+// per unit would fit, and lose to the launch-per-kernel form (a 40^3-hex cube
+// in 500 patches: FP64 32.3 against 18.1 us per iteration, mixed 20.4 against
+// 15.3), whose launches cost less the more work there is between them; in 256
+// patches of twice the size the resident form is ahead, 16.7 and 12.5 us.
 template <typename T>
 bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit);
 
 template <typename T>
 void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &a, hipStream_t s);
+
+// Explicit GN22 steps step0 .. step0 + n_steps - 1 (1-based) in one launch;
+// from d = v = a = 0 when fresh, else from d, v, a, which hold the state at
+// the end.
+template <typename T>
+struct ResDyn {
+  T *d, *v, *a;
+  const T *f_file, *f_unit, *invM;
+  const double *coef_file, *coef_unit;   // per step
+  T dt, c1, c2, c3, alpha, scale;        // DynCoeffs
+  unsigned long long *entries;           // two sets of entry_words
+  size_t entry_words;
+  unsigned long long *abort;             // zero; nonzero after a launch that did not complete
+  unsigned tag0;                         // tags tag0 .. tag0 + n_steps - 1, following the last launch's
+  int fresh, step0, n_steps;
+  // receivers (rec_of null: none): per node its first receiver or -1, the
+  // receivers of one node linked by rec_next
+  const int32_t *rec_of, *rec_next;
+  int n_rec, rec_every, rec_samples, rec_quantity;
+  T *traces;
+};
+
+template <typename T>
+bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit);
+
+template <typename T>
+void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &a, hipStream_t s);
 
 hipError_t prepare_resident_kernels();
 

@@ -1,19 +1,26 @@
-// resident.hip -- the PCG iteration (femfunc.cpp:59-111) as one launch per
-// solve.
+// resident.hip -- the PCG iteration (femfunc.cpp:59-111) and the explicit time
+// step (femfunc.cpp:247-343) as one launch per solve or run.
 //
 // A launch costs about 4 us on gfx950 even when it does nothing, and the
-// two-launch iteration of kernels.hip pays it twice and re-reads its mesh
-// data and vectors every time.  Here one workgroup per patch stays on its
-// compute unit for the whole solve: element records, coordinates, r, p, x
-// and M^-1 are loaded once and kept in registers and LDS; between
-// workgroups only the interface nodes' partial sums and the dot products'
-// partials travel, through memory, at agent scope.  What bounds an iteration
-// now is those two trips, some 3.5 kcycles each from the first store to the
-// last load (10 workgroups; 4 to 7 at 100), then the element phase of one
-// workgroup on one compute unit (2 to 5 kcycles in FP64).  Measured, us per
-// iteration, launch per kernel -> resident: 12x7 plate FP64 10.2 -> 1.9 (one
-// workgroup, no trips), 64x32 plate FP64 10.2 -> 5.6, 24^3-hex cube FP64
-// 14.0 -> 10.0 and mixed 14.0 -> 8.9, 32^3 hexes FP64 14.4 -> 12.0.
+// launch-per-kernel forms of kernels.hip pay it once a step and twice an
+// iteration, and re-read their mesh data and vectors every time.  Here one
+// workgroup per patch stays on its compute unit throughout: element records
+// and geometry, node state and coordinates are loaded once and kept in
+// registers and LDS; between workgroups only the interface nodes' partial
+// sums and the dot products' partials travel, through memory, at agent scope.
+//
+// What bounds it, in kcycles of 2.4 GHz: an iteration's two trips through
+// memory (3.5 each from the first store to the last load at 10 workgroups, 4
+// to 7 at 100; a step's one: 2.6 at 10, 6 at 229) and the element phase of one
+// patch on one compute unit (FP64 tets: 4 for 768 elements, 12 for 1536, bound
+// by LDS traffic and FP64 issue).  Measured, launch per kernel -> resident:
+//   us per PCG iteration: 12x7 plate FP64 10.2 -> 1.9 (one workgroup, no
+//   trips), 64x32 plate FP64 10.2 -> 5.3, 24^3 hexes FP64 14.0 -> 9.0 and mixed
+//   14.0 -> 8.2, 40^3 hexes (1536 elements per patch) FP64 18.1 -> 16.7 and
+//   mixed 15.3 -> 12.5;
+//   us per explicit step: 63x31 plate FP32 with receivers 9.1 -> 2.0, 160x80
+//   plate FP64 5.7 -> 2.3, 16x16x256 column FP64 15.5 -> 10.1 and FP32
+//   10.7 -> 6.3.
 //
 // Every workgroup forms every scalar itself from all partials in the same
 // order, and every patch holding an interface node carries its own copy of
@@ -61,19 +68,12 @@ __device__ __forceinline__ void st_agent(u64 *p, u64 v) {
 __device__ __forceinline__ u64 ld_agent(const u64 *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// A value as tagged words (one for FP32, two for FP64), and back.
-template <typename T>
-constexpr int NW = sizeof(T) / 4;
-
-__device__ __forceinline__ void tag_words(float v, unsigned tag, u64 (&w)[1]) {
-  w[0] = (u64(tag) << 32) | __float_as_uint(v);
-}
+// A double as two tagged words, and back.
 __device__ __forceinline__ void tag_words(double v, unsigned tag, u64 (&w)[2]) {
   const u64 b = static_cast<u64>(__double_as_longlong(v));
   w[0] = (u64(tag) << 32) | (b & 0xffffffffull);
   w[1] = (u64(tag) << 32) | (b >> 32);
 }
-__device__ __forceinline__ float untag(const u64 (&w)[1]) { return __uint_as_float(unsigned(w[0])); }
 __device__ __forceinline__ double untag(const u64 (&w)[2]) {
   return __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
 }
@@ -93,50 +93,76 @@ struct Patience {
   }
 };
 
-// Interface sums travel as entries (femgpu_internal.h): DIM values of W words,
-// word w of 64 consecutive entries together.
+// Interface sums travel as entries (femgpu_internal.h): the bits of DIM values
+// in words of 48 under a 16-bit tag (a third fewer words than 32 under 32;
+// the traffic of some hundred kilobytes a step per workgroup is what bounds a
+// trade).  The tag counts the trades through a set of entries, and every trade
+// writes them all: a stale word carries the tag before the one awaited.  Word
+// w of 64 consecutive entries lie together.
+template <typename T, int DIM>
+constexpr int EW = res_entry_size(DIM, int(sizeof(T)));
+
 template <typename T, int DIM>
 __device__ __forceinline__ size_t entry_word(unsigned e, int w) {
-  return (size_t(e >> 6) * (DIM * NW<T>) + w) * 64 + (e & 63u);
+  return (size_t(e >> 6) * EW<T, DIM> + w) * 64 + (e & 63u);
 }
 
-// Component c of an entry.
-template <typename T, int DIM>
-__device__ __forceinline__ void send_entry(u64 *entries, unsigned e, int c, unsigned tag, T v) {
-  u64 w[NW<T>];
-  tag_words(v, tag, w);
-#pragma unroll
-  for (int h = 0; h < NW<T>; ++h) st_agent(&entries[entry_word<T, DIM>(e, c * NW<T> + h)], w[h]);
+template <typename T>
+__device__ __forceinline__ void to_bits(T v, unsigned *u) {
+  if constexpr (sizeof(T) == 8) {
+    const u64 b = static_cast<u64>(__double_as_longlong(v));
+    u[0] = unsigned(b);
+    u[1] = unsigned(b >> 32);
+  } else {
+    u[0] = __float_as_uint(v);
+  }
+}
+template <typename T>
+__device__ __forceinline__ T from_bits(const unsigned *u) {
+  if constexpr (sizeof(T) == 8)
+    return __longlong_as_double(static_cast<long long>((u64(u[1]) << 32) | u[0]));
+  else
+    return __uint_as_float(u[0]);
 }
 
-// Component c of the entries e0 + i (i = i0, i0 + 256, ... below n) into
-// v[pos[i] * DIM + c], four of them in flight.  False when the wait ran out.
 template <typename T, int DIM>
-__device__ __forceinline__ bool recv_entries(const u64 *entries, unsigned e0, int i0, int n, int c,
-                                             unsigned tag, u64 *abort, T *v, const uint16_t *pos) {
-  constexpr int W = NW<T>, NB = 4;
-  for (int ib = i0; ib < n; ib += 256 * NB) {
-    u64 h[NB][W];
-    Patience wait{abort};
-    for (int spin = 0;; ++spin) {
-      bool all = true;
+__device__ __forceinline__ void send_entry(u64 *entries, unsigned e, unsigned tag, const T *v) {
+  constexpr int W = EW<T, DIM>, U = sizeof(T) / 4;
+  unsigned u[DIM * U + 2];
 #pragma unroll
-      for (int m = 0; m < NB; ++m)
-        if (ib + 256 * m < n)
+  for (int c = 0; c < DIM; ++c) to_bits<T>(v[c], &u[c * U]);
+  u[DIM * U] = u[DIM * U + 1] = 0u;
+  // 16-bit unit j of the payload: half j & 1 of u[j >> 1]
+  auto unit = [&](int j) { return j >= 2 * DIM * U ? 0u : (j & 1) ? u[j >> 1] >> 16 : u[j >> 1] & 0xffffu; };
 #pragma unroll
-          for (int k = 0; k < W; ++k)
-            h[m][k] = ld_agent(&entries[entry_word<T, DIM>(e0 + ib + 256 * m, c * W + k)]);
+  for (int w = 0; w < W; ++w)
+    st_agent(&entries[entry_word<T, DIM>(e, w)],
+             (u64((tag << 16) | unit(3 * w + 2)) << 32) | (unit(3 * w + 1) << 16) | unit(3 * w));
+}
+
+// Entry e into v; false when the wait ran out.
+template <typename T, int DIM>
+__device__ __forceinline__ bool recv_entry(const u64 *entries, unsigned e, unsigned tag, u64 *abort,
+                                           T *v) {
+  constexpr int W = EW<T, DIM>, U = sizeof(T) / 4;
+  u64 h[W];
+  Patience wait{abort};
+  for (int spin = 0;; ++spin) {
+    bool all = true;
 #pragma unroll
-      for (int m = 0; m < NB; ++m)
-        if (ib + 256 * m < n)
+    for (int w = 0; w < W; ++w) h[w] = ld_agent(&entries[entry_word<T, DIM>(e, w)]);
 #pragma unroll
-          for (int k = 0; k < W; ++k) all = all && unsigned(h[m][k] >> 32) == tag;
-      if (all) break;
-      if (wait.over(spin)) return false;
-    }
+    for (int w = 0; w < W; ++w) all = all && unsigned(h[w] >> 48) == (tag & 0xffffu);
+    if (all) break;
+    if (wait.over(spin)) return false;
+  }
+  auto unit = [&](int j) { return unsigned(h[j / 3] >> (16 * (j % 3))) & 0xffffu; };
 #pragma unroll
-    for (int m = 0; m < NB; ++m)
-      if (ib + 256 * m < n) v[int(pos[ib + 256 * m]) * DIM + c] = untag(h[m]);
+  for (int c = 0; c < DIM; ++c) {
+    unsigned u[U];
+#pragma unroll
+    for (int i = 0; i < U; ++i) u[i] = unit(2 * (c * U + i)) | (unit(2 * (c * U + i) + 1) << 16);
+    v[c] = from_bits<T>(u);
   }
   return true;
 }
@@ -249,18 +275,19 @@ __device__ __forceinline__ bool gather(const Exchange &x, unsigned tag, double (
   return *s_flag == 0;
 }
 
-// LDS of a resident workgroup: node coordinates and vector, the node-sorted
-// element entries of every component, the interface nodes' contributions
+// LDS of a resident workgroup: node coordinates and vector, `comps` components
+// of the node-sorted element entries, the interface nodes' contributions
 // slot by slot, the tables of what the patch sends (entry and place of its
 // own contribution) and where a received entry goes.
 struct ResLds {
   int off_x, off_res, off_in, off_oe, off_os, off_ip, off_red, total;
 };
-__host__ __device__ inline ResLds res_lds(int dim, int tb, int pn, int ent, int n_in, int n_src) {
+__host__ __device__ inline ResLds res_lds(int dim, int tb, int pn, int ent, int comps, int n_in,
+                                          int n_src) {
   ResLds L;
   L.off_x = al32(pn * dim * tb);
   L.off_res = L.off_x + al32(pn * dim * tb);
-  L.off_in = L.off_res + al32(dim * ent * tb);
+  L.off_in = L.off_res + al32(comps * ent * tb);
   L.off_oe = L.off_in + al32(n_src * dim * tb);
   L.off_os = L.off_oe + al32(n_in * 4);
   L.off_ip = L.off_os + al32(n_in * 2);
@@ -269,8 +296,9 @@ __host__ __device__ inline ResLds res_lds(int dim, int tb, int pn, int ent, int 
   return L;
 }
 
+// Resident kernels' view of the mesh.
 template <typename T>
-struct ResArgs {
+struct ResMesh {
   const PatchInfo *patches;
   const uint32_t *erec_s;
   int emax;
@@ -285,7 +313,6 @@ struct ResArgs {
   const uint32_t *out_entry;
   const uint16_t *out_src, *in_pos, *src_end, *own_pos;
   int n_in_max, n_src_max;
-  ResPcg<T> s;
 };
 
 // Sum of the entry run [b0, b1) (multiples of 4) in a fixed order.
@@ -312,115 +339,292 @@ __device__ __forceinline__ T run_sum(const T *s_res, int b0, int b1) {
   return (s0 + s1) + (s2 + s3);
 }
 
-// This thread's DOF (node t / DIM of the patch, component t % DIM) of K x by
-// one thread per element and per DOF: patch_common.h's assemble with every
-// component's entries in LDS at once, one barrier instead of 2 DIM - 1.
-template <typename T, int DIM>
-__device__ __forceinline__ T assemble_dof(const T *s_c, const T *s_x, T *s_res, int ent, uint3 rec,
-                                          T esc, int n_elem, T lam, T mu, int b0, int b1) {
-  constexpr int NPE = DIM + 1, NDE = DIM * NPE;
-  if (int(threadIdx.x) < n_elem) {
-    int l[4], q[4];
-    decode_rec(rec, l, q);
-    T X[NDE], U[NDE], F[NDE];
+// One patch in one workgroup of PT threads for a whole launch.  NE = 1: one
+// element and one DOF per thread (thread t: node t / DIM, component t % DIM),
+// the element entries of every component in LDS at once, one barrier instead
+// of 2 DIM - 1 per product.  NE = 2 (patches of up to 512 nodes): two elements
+// per thread, a node with its DIM DOFs in each of the first threads, the
+// components' entries in turn through one list.
+template <typename T, int DIM, int PT, int NE>
+struct ResPatch {
+  static constexpr bool DOF = NE == 1;
+  static constexpr int ND = DOF ? 1 : DIM;     // DOFs per thread
+  static constexpr int COMPS = DOF ? DIM : 1;  // components in the entry list
+  static constexpr int NPE = DIM + 1, NDE = DIM * NPE;
+  // the elements' geometry in registers for the whole launch, where they hold
+  // it (FP64 with two elements per thread: formed again in every product)
+  static constexpr bool GEOM = DOF || sizeof(T) == 4;
+  static constexpr int NGEO = GEOM ? DIM * DIM + 1 : 1;
+
+  T *s_c, *s_x, *s_res, *s_in;
+  uint32_t *s_oe;
+  uint16_t *s_os, *s_ip;
+  double *s_red;
+  int ent, n_elem, n_in, in_start;
+  T lam, mu;
+  uint3 rec[NE];
+  T esc[NE];
+  bool has, own, first;  // first: this patch accounts for the node
+  unsigned fm;           // fixed DOFs of this thread
+  int go;                // global DOF of this thread's first
+  int gid;               // its node
+  int b0, b1, l0, l1, lo;
+  T dK[ND];              // diagonal of a constrained row
+  T geo[NE][NGEO];
+
+  __device__ __forceinline__ int local(int i) const {
+    return DOF ? int(threadIdx.x) : int(threadIdx.x) * DIM + i;
+  }
+  __device__ __forceinline__ int comp(int i) const { return DOF ? int(threadIdx.x) % DIM : i; }
+  __device__ __forceinline__ bool fixed(int i) const { return ((fm >> i) & 1u) != 0u; }
+
+  // Loads the patch (one barrier; the exchange tables are ready after the
+  // next).
+  __device__ __forceinline__ void load(const ResMesh<T> &a, int pid, unsigned char *lds) {
+    const ResLds L = res_lds(DIM, int(sizeof(T)), a.pn, a.ent, COMPS, a.n_in_max, a.n_src_max);
+    s_c = reinterpret_cast<T *>(lds);
+    s_x = reinterpret_cast<T *>(lds + L.off_x);
+    s_res = reinterpret_cast<T *>(lds + L.off_res);
+    s_in = reinterpret_cast<T *>(lds + L.off_in);
+    s_oe = reinterpret_cast<uint32_t *>(lds + L.off_oe);
+    s_os = reinterpret_cast<uint16_t *>(lds + L.off_os);
+    s_ip = reinterpret_cast<uint16_t *>(lds + L.off_ip);
+    s_red = reinterpret_cast<double *>(lds + L.off_red);
+    const int t = threadIdx.x;
+    const PatchInfo P = a.patches[pid];
+    const ExchangePatch E = a.xpatch[pid];
+    ent = a.ent;
+    n_elem = P.n_elem;
+    n_in = E.n_in;
+    in_start = E.in_start;
+    lam = a.lam;
+    mu = a.mu;
+    const uint3 *prec = reinterpret_cast<const uint3 *>(a.erec_s) + size_t(pid) * unsigned(a.emax);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      const int i = t + e * PT;
+      rec[e] = prec[unsigned(min(i, a.emax - 1))];
+      esc[e] = a.escale && i < n_elem ? a.escale[P.elem_start + i] : T(1);
+    }
+    clear_entries<T, PT>(s_res, COMPS * ent);
+    const int k = DOF ? t / DIM : t;
+    has = k < P.n_own + P.n_sh;
+    first = own = k < P.n_own;
+    fm = 0;
+    go = gid = b0 = b1 = l0 = l1 = lo = 0;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) dK[i] = T(0);
+    if (has) {
+      const size_t pbase = size_t(pid) * a.pstride;
+      gid = a.pgid[pbase + k];
+      go = gid * DIM + (DOF ? t % DIM : 0);
+      b1 = int(a.pend[pbase + k]);
+      b0 = k ? int(a.pend[pbase + k - 1]) : 0;
+      fm = a.fixmask[gid] & ((1u << DIM) - 1u);
+      if constexpr (DOF) fm = (fm >> (t % DIM)) & 1u;
+      if (!own) {
+        const int j = P.sh_start + k - P.n_own;
+        first = a.pslot[pbase + k] < 0;
+        l1 = int(a.src_end[j]);
+        l0 = k > P.n_own ? int(a.src_end[j - 1]) : 0;
+        lo = int(a.own_pos[j]);
+      }
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        s_c[local(i)] = a.coords[go + i];
+        if (fixed(i) && first) dK[i] = a.diagK[go + i];
+      }
+    }
+    __syncthreads();
+    if constexpr (GEOM) {
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        int l[4], q[4];
+        decode_rec(rec[e], l, q);
+        T X[NDE];
+#pragma unroll
+        for (int n = 0; n < NPE; ++n)
+#pragma unroll
+          for (int c = 0; c < DIM; ++c) X[n * DIM + c] = s_c[l[n] * DIM + c];
+        elem_geometry<T, DIM>(X, esc[e], geo[e]);
+      }
+    }
+    for (int i = t; i < n_in; i += PT) {
+      s_oe[i] = a.out_entry[E.out_start + i];
+      s_os[i] = a.out_src[E.out_start + i];
+      s_ip[i] = a.in_pos[E.out_start + i];
+    }
+  }
+
+  __device__ __forceinline__ void force(int e, T *F, int *q) const {
+    int l[4];
+    decode_rec(rec[e], l, q);
+    T U[NDE];
 #pragma unroll
     for (int n = 0; n < NPE; ++n)
 #pragma unroll
-      for (int c = 0; c < DIM; ++c) {
-        X[n * DIM + c] = s_c[l[n] * DIM + c];
-        U[n * DIM + c] = s_x[l[n] * DIM + c];
-      }
-    (void)elem_force_free<T, DIM>(X, U, lam, mu, esc, F);
+      for (int c = 0; c < DIM; ++c) U[n * DIM + c] = s_x[l[n] * DIM + c];
+    if constexpr (GEOM) {
+      (void)elem_force_geo<T, DIM>(geo[e], U, lam, mu, F);
+    } else {
+      T X[NDE];
 #pragma unroll
-    for (int c = 0; c < DIM; ++c)
+      for (int n = 0; n < NPE; ++n)
 #pragma unroll
-      for (int n = 0; n < NPE; ++n) s_res[c * ent + q[n]] = F[n * DIM + c];
+        for (int c = 0; c < DIM; ++c) X[n * DIM + c] = s_c[l[n] * DIM + c];
+      (void)elem_force_free<T, DIM>(X, U, lam, mu, esc[e], F);
+    }
   }
-  __syncthreads();
-  return run_sum<T>(s_res + (int(threadIdx.x) % DIM) * ent, b0, b1);
-}
 
-template <typename T, int DIM, int PT>
-__global__ __launch_bounds__(PT) void k_pcg_resident(ResArgs<T> a) {
+  // y = this patch's part of K x at this thread's DOFs (x: their values; the
+  // other threads' through LDS).  A constrained row is its assembled diagonal,
+  // in the patch that accounts for the node.
+  __device__ __forceinline__ void product(const T (&x)[ND], T (&y)[ND]) {
+    const int t = threadIdx.x;
+    if (has)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) s_x[local(i)] = fixed(i) ? T(0) : x[i];
+    __syncthreads();
+    if constexpr (DOF) {
+      if (t < n_elem) {
+        int q[4];
+        T F[NDE];
+        force(0, F, q);
+#pragma unroll
+        for (int c = 0; c < DIM; ++c)
+#pragma unroll
+          for (int n = 0; n < NPE; ++n) s_res[c * ent + q[n]] = F[n * DIM + c];
+      }
+      __syncthreads();
+      y[0] = run_sum<T>(s_res + (t % DIM) * ent, b0, b1);
+    } else {
+      // (corner 0's force is minus the others', formed again at the scatter:
+      // fewer live registers)
+      T F[NE][NDE - DIM];
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        if (t + e * PT >= n_elem) continue;
+        int q[4];
+        T Fe[NDE];
+        force(e, Fe, q);
+#pragma unroll
+        for (int j = 0; j < NDE - DIM; ++j) F[e][j] = Fe[DIM + j];
+      }
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        if (c) __syncthreads();
+#pragma unroll
+        for (int e = 0; e < NE; ++e)
+          if (t + e * PT < n_elem) {
+            int l[4], q[4];
+            decode_rec(rec[e], l, q);
+            T f0 = F[e][c];
+            s_res[q[1]] = F[e][c];
+#pragma unroll
+            for (int n = 2; n < NPE; ++n) {
+              f0 += F[e][(n - 1) * DIM + c];
+              s_res[q[n]] = F[e][(n - 1) * DIM + c];
+            }
+            s_res[q[0]] = -f0;
+          }
+        __syncthreads();
+        y[c] = run_sum<T>(s_res, b0, b1);
+      }
+    }
+    if (fm)
+#pragma unroll
+      for (int i = 0; i < ND; ++i)
+        if (fixed(i)) y[i] = dK[i] * x[i];
+  }
+
+  // An interface node's contribution of this patch to its place (before a
+  // barrier that precedes trade).
+  __device__ __forceinline__ void put(const T (&y)[ND]) {
+    if (has && !own)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) s_in[lo * DIM + comp(i)] = y[i];
+  }
+
+  // Sends this patch's contributions and receives the others', an entry per
+  // thread.  False when the wait ran out; the contributions are complete after
+  // the next barrier.
+  __device__ __forceinline__ bool trade(u64 *entries, unsigned tag, u64 *abort) {
+    for (int i = threadIdx.x; i < n_in; i += PT)
+      send_entry<T, DIM>(entries, s_oe[i], tag, &s_in[int(s_os[i]) * DIM]);
+    for (int i = threadIdx.x; i < n_in; i += PT)
+      if (!recv_entry<T, DIM>(entries, unsigned(in_start + i), tag, abort, &s_in[int(s_ip[i]) * DIM]))
+        return false;
+    return true;
+  }
+
+  // The interface node's sums from all its patches, in slot order.
+  __device__ __forceinline__ void collect(T (&y)[ND]) const {
+    if (has && !own)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        T q = T(0);
+        for (int l = l0; l < l1; ++l) q += s_in[l * DIM + comp(i)];
+        y[i] = q;
+      }
+  }
+};
+
+template <typename T>
+struct PcgArgs {
+  ResMesh<T> m;
+  ResPcg<T> s;
+};
+
+template <typename T, int DIM, int PT, int NE>
+__global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
+  using Patch = ResPatch<T, DIM, PT, NE>;
+  constexpr int ND = Patch::ND;
   extern __shared__ __align__(16) unsigned char lds[];
   __shared__ int s_flag;
   const int b = blockIdx.x;
-  const int pid = (b & 7) * a.p8 + (b >> 3);
-  if (pid >= a.np) return;
-  const bool alone = a.np == 1;  // no exchange
-  const ResLds L = res_lds(DIM, int(sizeof(T)), a.pn, a.ent, a.n_in_max, a.n_src_max);
-  T *s_c = reinterpret_cast<T *>(lds);
-  T *s_x = reinterpret_cast<T *>(lds + L.off_x);
-  T *s_res = reinterpret_cast<T *>(lds + L.off_res);
-  T *s_in = reinterpret_cast<T *>(lds + L.off_in);
-  uint32_t *s_oe = reinterpret_cast<uint32_t *>(lds + L.off_oe);
-  uint16_t *s_os = reinterpret_cast<uint16_t *>(lds + L.off_os);
-  uint16_t *s_ip = reinterpret_cast<uint16_t *>(lds + L.off_ip);
-  double *s_red = reinterpret_cast<double *>(lds + L.off_red);  // p'q; r'z and r'r
-  double *s_bc = s_red + 48;
+  const int pid = (b & 7) * a.m.p8 + (b >> 3);
+  if (pid >= a.m.np) return;
+  const bool alone = a.m.np == 1;  // no exchange
   const int t = threadIdx.x;
   if (t == 0) s_flag = 0;
-
-  // the patch, this thread's element and DOF (node k, component c)
-  const PatchInfo P = a.patches[pid];
-  const ExchangePatch E = a.xpatch[pid];
-  const size_t pbase = size_t(pid) * a.pstride;
-  const int k = t / DIM, c = t - k * DIM;
-  const bool has = k < P.n_own + P.n_sh;
-  const bool own = k < P.n_own;
-  const uint3 rec = reinterpret_cast<const uint3 *>(
-      a.erec_s)[size_t(pid) * unsigned(a.emax) + unsigned(min(t, a.emax - 1))];
-  const T esc = a.escale && t < P.n_elem ? a.escale[P.elem_start + t] : T(1);
-  clear_entries<T, PT>(s_res, DIM * a.ent);
-  int go = 0, b0 = 0, b1 = 0, l0 = 0, l1 = 0, lo = 0;
-  bool first = own, fixed = false;  // first: this patch accounts for the node
-  T r = T(0), p = T(0), x = T(0), d = T(0);
-  if (has) {
-    const int gid = a.pgid[pbase + k];
-    go = gid * DIM + c;
-    b1 = int(a.pend[pbase + k]);
-    b0 = k ? int(a.pend[pbase + k - 1]) : 0;
-    fixed = ((a.fixmask[gid] >> c) & 1) != 0;
-    if (!own) {
-      const int j = P.sh_start + k - P.n_own;
-      first = a.pslot[pbase + k] < 0;
-      l1 = int(a.src_end[j]);
-      l0 = k > P.n_own ? int(a.src_end[j - 1]) : 0;
-      lo = int(a.own_pos[j]);
-    }
-    s_c[t] = a.coords[go];
-    r = a.s.r_in[go];
-    d = a.s.invD[go];
-    if (!a.s.fresh) {
-      p = a.s.p[go];
-      x = a.s.x[go];
+  Patch P;
+  P.load(a.m, pid, lds);
+  double *s_red = P.s_red;  // p'q; r'z and r'r
+  double *s_bc = s_red + 48;
+  T r[ND], p[ND], x[ND], d[ND], q[ND], cMm[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    r[i] = p[i] = x[i] = d[i] = cMm[i] = T(0);
+    if (P.has) {
+      r[i] = a.s.r_in[P.go + i];
+      d[i] = a.s.invD[P.go + i];
+      if (a.s.sh.m) cMm[i] = a.s.sh.cM * a.s.sh.m[P.go + i];
+      if (!a.s.fresh) {
+        p[i] = a.s.p[P.go + i];
+        x[i] = a.s.x[P.go + i];
+      }
     }
   }
-  // the operator's diagonal of a constrained row, its mass shift
-  const T dK = fixed && first ? a.diagK[go] : T(0);
-  const T cK = a.s.sh.cK, cMm = has && a.s.sh.m ? a.s.sh.cM * a.s.sh.m[go] : T(0);
-  for (int i = t; i < E.n_in; i += PT) {
-    s_oe[i] = a.out_entry[E.out_start + i];
-    s_os[i] = a.out_src[E.out_start + i];
-    s_ip[i] = a.in_pos[E.out_start + i];
-  }
-  const int xc = t >> 8, xi = t & 255;  // entries xi, xi + 256, ... of component xc
-  // (workgroup 0 advances the epoch at its end, after an exchange that every
-  // workgroup took part in with the tag it reads here)
+  const T cK = a.s.sh.cK;
+  // (workgroup 0 advances the tags at its end, after an exchange that every
+  // workgroup took part in with the tags it reads here)
   u64 *const epoch = a.s.words;
-  const size_t stride = res_copy_words(a.np);
-  const Exchange xpq{a.s.words + RES_HEAD, stride, epoch + 1, a.np, b % EX_COPIES};
-  const Exchange xrz{xpq.words + size_t(2) * a.np, stride, epoch + 1, a.np, b % EX_COPIES};
-  unsigned tag = unsigned(ld_agent(epoch));
+  const size_t stride = res_copy_words(a.m.np);
+  const Exchange xpq{a.s.words + RES_HEAD, stride, epoch + 1, a.m.np, b % EX_COPIES};
+  const Exchange xrz{xpq.words + size_t(2) * a.m.np, stride, epoch + 1, a.m.np, b % EX_COPIES};
+  u64 *const etag = epoch + 2 + (sizeof(T) == 8 ? 1 : 0);
+  unsigned tag = unsigned(ld_agent(epoch)), entry_tag = unsigned(ld_agent(etag));
 
   // r'z and r'r over all patches
   double g = 0.0, q2 = 0.0;
   auto dots = [&]() -> bool {
     double v[2] = {0.0, 0.0};
-    if (first) {
-      v[0] = double(r) * double(mul_rn(d, r));
-      v[1] = double(r) * double(r);
-    }
+    if (P.first)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        v[0] += double(r[i]) * double(mul_rn(d[i], r[i]));
+        v[1] += double(r[i]) * double(r[i]);
+      }
     sum_to_wave0<PT, 2>(v, s_red + 16);
     ++tag;
     if (!alone && t < 64) publish<2>(xrz, pid, tag, v);
@@ -458,36 +662,27 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(ResArgs<T> a) {
     }
     const T beta = T(g / g_prev);
     g_prev = g;
-    if (has) {
-      p = pcg_dir(d, r, beta, p);
-      s_x[t] = fixed ? T(0) : p;
-    }
-    __syncthreads();
-    T q = assemble_dof<T, DIM>(s_c, s_x, s_res, a.ent, rec, esc, P.n_elem, a.lam, a.mu, b0, b1);
-    // the row of a constrained DOF: the assembled diagonal only; the mass
-    // shift belongs to the patch that accounts for the node
-    if (fixed) q = dK * p;
-    q = cK * q;
+    if (P.has)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) p[i] = pcg_dir(d[i], r[i], beta, p[i]);
+    P.product(p, q);
     double vpq[1] = {0.0};
-    if (has) {
-      if (own) q += cMm * p;
-      vpq[0] = double(p) * double(q);
-      if (!own) {
-        s_in[lo * DIM + c] = q;
-        if (first) vpq[0] += double(cMm) * double(p) * double(p);
+    if (P.has)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        q[i] = cK * q[i];
+        if (P.own) q[i] += cMm[i] * p[i];
+        vpq[0] += double(p[i]) * double(q[i]);
+        // the mass shift belongs to the patch that accounts for the node
+        if (!P.own && P.first) vpq[0] += double(cMm[i]) * double(p[i]) * double(p[i]);
       }
-    }
+    P.put(q);
     ++tag;
+    ++entry_tag;
     sum_to_wave0<PT, 1>(vpq, s_red);
     if (!alone) {
       if (t < 64) publish<1>(xpq, pid, tag, vpq);
-      if (xc < DIM) {
-        for (int i = xi; i < E.n_in; i += 256)
-          send_entry<T, DIM>(a.s.entries, s_oe[i], xc, tag, s_in[int(s_os[i]) * DIM + xc]);
-        if (!recv_entries<T, DIM>(a.s.entries, unsigned(E.in_start), xi, E.n_in, xc, tag, epoch + 1,
-                                  s_in, s_ip))
-          s_flag = 1;
-      }
+      if (!P.trade(a.s.entries, entry_tag, epoch + 1)) s_flag = 1;
     }
     alive = gather<1>(xpq, tag, vpq, s_bc + 2, &s_flag, alone);
     if (!alive) break;
@@ -498,24 +693,24 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(ResArgs<T> a) {
       break;
     }
     const T alpha = T(alpha_d);
-    if (has) {
-      if (!own) {
-        // the DOF's contributions from all its patches, in slot order
-        q = T(0);
-        for (int l = l0; l < l1; ++l) q += s_in[l * DIM + c];
-        q += cMm * p;
+    P.collect(q);
+    if (P.has)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        if (!P.own) q[i] += cMm[i] * p[i];
+        x[i] = x[i] + alpha * p[i];
+        r[i] = r[i] - alpha * q[i];
       }
-      x = x + alpha * p;
-      r = r - alpha * q;
-    }
     alive = dots();
     ++n_upd;
   }
-  if (first) {
-    a.s.x[go] = x;
-    a.s.p[go] = p;
-    a.s.r_out[go] = r;
-  }
+  if (P.first)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      a.s.x[P.go + i] = x[i];
+      a.s.p[P.go + i] = p[i];
+      a.s.r_out[P.go + i] = r[i];
+    }
   if (pid == 0 && t == 0) {
     CgScalars *sc = a.s.sc;
     sc->gamma0 = gamma0;
@@ -527,14 +722,101 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(ResArgs<T> a) {
     sc->iter_final = n_upd;
     sc->pause = pause;
     st_agent(epoch, u64(tag));
+    st_agent(etag, u64(entry_tag));
     if (ld_agent(epoch + 1) != 0) done = RES_ABORTED;
     sc->done = done;
   }
 }
 
+// Explicit GN22 steps (gn22_correct's operations, the predictor of
+// k_dyn_predict): a step is one product and one trade with the patches that
+// share nodes; no workgroup waits for one it has no node in common with.  The
+// entries alternate between two sets (by the tag's parity): a neighbour may
+// still be reading the previous step's when this patch, with that neighbour's
+// in hand, writes the next.
 template <typename T>
-ResArgs<T> res_args(const DevMesh &dm, const ResPcg<T> &s) {
-  ResArgs<T> a{};
+struct DynArgs {
+  ResMesh<T> m;
+  ResDyn<T> s;
+};
+
+template <typename T, int DIM, int PT, int NE>
+__global__ __launch_bounds__(PT) void k_dyn_resident(DynArgs<T> a) {
+  using Patch = ResPatch<T, DIM, PT, NE>;
+  constexpr int ND = Patch::ND;
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_flag;
+  const int b = blockIdx.x;
+  const int pid = (b & 7) * a.m.p8 + (b >> 3);
+  if (pid >= a.m.np) return;
+  const bool alone = a.m.np == 1;
+  if (threadIdx.x == 0) s_flag = 0;
+  Patch P;
+  P.load(a.m, pid, lds);
+  const ResDyn<T> &s = a.s;
+  T d[ND], v[ND], ac[ND], ff[ND], fu[ND], im[ND];
+  int rec = -1;
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    d[i] = v[i] = ac[i] = ff[i] = fu[i] = im[i] = T(0);
+    if (P.has) {
+      ff[i] = s.f_file[P.go + i];
+      fu[i] = s.f_unit[P.go + i];
+      im[i] = s.invM[P.go + i];
+      if (!s.fresh) {
+        d[i] = s.d[P.go + i];
+        v[i] = s.v[P.go + i];
+        ac[i] = s.a[P.go + i];
+      }
+    }
+  }
+  if (s.rec_of && P.has && P.first) rec = s.rec_of[P.gid];
+  bool alive = true;
+  for (int n = 0; n < s.n_steps; ++n) {
+    const int step = s.step0 + n;
+    const T cf = T(s.coef_file[step]), cu = T(s.coef_unit[step]);
+    T x[ND], kd[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) x[i] = (d[i] + s.dt * v[i]) + s.c1 * ac[i];
+    P.product(x, kd);
+    if (!alone) {
+      P.put(kd);
+      __syncthreads();
+      const unsigned tag = s.tag0 + unsigned(n);
+      if (!P.trade(s.entries + ((tag & 1u) ? s.entry_words : 0), tag, s.abort)) s_flag = 1;
+    }
+    __syncthreads();
+    alive = s_flag == 0;
+    if (!alive) break;
+    if (!alone) P.collect(kd);
+    if (P.has)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        gn22_correct<T>(cf, cu, ff[i], fu[i], kd[i], im[i], s.c2, s.c3, s.alpha, s.scale, ac[i], v[i]);
+        d[i] = x[i];
+      }
+    if (rec >= 0 && step % s.rec_every == 0) {
+      const int smp = step / s.rec_every - 1;
+      if (smp < s.rec_samples)
+        for (int k = rec; k >= 0; k = s.rec_next[k])
+#pragma unroll
+          for (int i = 0; i < ND; ++i)
+            s.traces[(int64_t(smp) * s.n_rec + k) * DIM + P.comp(i)] =
+                s.rec_quantity == 0 ? d[i] : s.rec_quantity == 1 ? v[i] : ac[i];
+    }
+  }
+  if (P.first && alive)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      s.d[P.go + i] = d[i];
+      s.v[P.go + i] = v[i];
+      s.a[P.go + i] = ac[i];
+    }
+}
+
+template <typename T>
+ResMesh<T> res_mesh(const DevMesh &dm) {
+  ResMesh<T> a{};
   a.patches = dm.patches;
   a.erec_s = dm.erec_s;
   a.emax = dm.emax;
@@ -566,26 +848,46 @@ ResArgs<T> res_args(const DevMesh &dm, const ResPcg<T> &s) {
   a.own_pos = dm.x_own_pos;
   a.n_in_max = dm.x_in_max;
   a.n_src_max = dm.x_src_max;
-  a.s = s;
   return a;
 }
 
-// One thread per element and per DOF: patches of up to 256 nodes and 768
-// elements.
-constexpr int RES_NODES = 256, RES_ELEMS = 768;
+// The kernels' forms: 768 threads with one element and one DOF each (patches
+// of up to 256 nodes and 768 elements; 512 threads hold the 2D patches, which
+// mostly run into the node limit first), else two elements each and a node per
+// thread (up to 512 nodes and 1536 elements).
+struct Form {
+  int threads, ne;
+};
+constexpr int RES_NODES[] = {0, 256, 512}, RES_THREADS = 768;
+constexpr int RES_LDS_MAX = 160 * 1024 - 256;
 
-template <typename T>
-using PcgKernel = void (*)(ResArgs<T>);
-
-// 2D patches mostly run into the node limit first: 512 threads hold them.
-int res_threads(const DevMesh &dm) { return dm.dim == 2 && dm.emax <= 512 ? 512 : 768; }
-
-template <typename T>
-PcgKernel<T> pcg_kernel(const DevMesh &dm) {
-  if (dm.dim == 3) return k_pcg_resident<T, 3, 768>;
-  return res_threads(dm) == 512 ? PcgKernel<T>(k_pcg_resident<T, 2, 512>)
-                                : PcgKernel<T>(k_pcg_resident<T, 2, 768>);
+Form res_form(const DevMesh &dm) {
+  if (dm.pn <= RES_NODES[1] && dm.emax <= RES_THREADS)
+    return {dm.dim == 2 && dm.emax <= 512 ? 512 : RES_THREADS, 1};
+  if (dm.pn <= RES_NODES[2] && dm.emax <= 2 * RES_THREADS) return {RES_THREADS, 2};
+  return {0, 0};
 }
+
+int res_lds_bytes(const DevMesh &dm, int tb) {
+  return res_lds(dm.dim, tb, dm.pn, dm.ent, res_form(dm).ne == 1 ? dm.dim : 1, dm.x_in_max, dm.x_src_max)
+      .total;
+}
+
+template <typename T>
+using PcgKernel = void (*)(PcgArgs<T>);
+template <typename T>
+using DynKernel = void (*)(DynArgs<T>);
+
+#define FEMGPU_RES_KERNEL(NAME, KIND)                                                       \
+  template <typename T>                                                                     \
+  KIND<T> NAME##_of(int dim, Form f) {                                                      \
+    if (f.ne == 2) return dim == 3 ? KIND<T>(NAME<T, 3, 768, 2>) : KIND<T>(NAME<T, 2, 768, 2>); \
+    if (dim == 3) return NAME<T, 3, 768, 1>;                                                \
+    return f.threads == 512 ? KIND<T>(NAME<T, 2, 512, 1>) : KIND<T>(NAME<T, 2, 768, 1>);    \
+  }
+FEMGPU_RES_KERNEL(k_pcg_resident, PcgKernel)
+FEMGPU_RES_KERNEL(k_dyn_resident, DynKernel)
+#undef FEMGPU_RES_KERNEL
 
 // Workgroups of a kernel that a compute unit holds, and the device's units
 // (asked of the runtime once per kernel and LDS size).
@@ -620,20 +922,11 @@ int compute_units(int device) {
   return n;
 }
 
-int res_lds_bytes(const DevMesh &dm, int tb) {
-  return res_lds(dm.dim, tb, dm.pn, dm.ent, dm.x_in_max, dm.x_src_max).total;
-}
-
-constexpr int RES_LDS_MAX = 160 * 1024 - 256;
-
-}  // namespace
-
-template <typename T>
-bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit) {
-  const int lds = res_lds_bytes(dm, int(sizeof(T))), cu = compute_units(device);
-  if (!dm.xpatch || cu < 1 || dm.pn > RES_NODES || dm.emax > RES_ELEMS || lds > RES_LDS_MAX)
-    return false;
-  const int per = blocks_per_cu(reinterpret_cast<const void *>(pcg_kernel<T>(dm)), res_threads(dm), lds);
+// Whether a kernel of this form fits the plan, a workgroup per compute unit.
+bool fits(const DevMesh &dm, int device, const void *fn, int lds, ResFit *fit) {
+  const int cu = compute_units(device);
+  if (cu < 1 || lds > RES_LDS_MAX) return false;
+  const int per = blocks_per_cu(fn, res_form(dm).threads, lds);
   const int grid = 8 * ((dm.np + 7) / 8);
   if (per < 1 || grid > cu) return false;
   fit->block = 1.0 / per;
@@ -641,29 +934,61 @@ bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit) {
   return true;
 }
 
+}  // namespace
+
+template <typename T>
+bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit) {
+  const Form f = res_form(dm);
+  return dm.xpatch && f.ne && fits(dm, device, reinterpret_cast<const void *>(k_pcg_resident_of<T>(dm.dim, f)),
+                                   res_lds_bytes(dm, int(sizeof(T))), fit);
+}
+
 template <typename T>
 void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &s, hipStream_t st) {
-  const ResArgs<T> a = res_args<T>(dm, s);
-  hipLaunchKernelGGL(pcg_kernel<T>(dm), dim3(8 * a.p8), dim3(res_threads(dm)),
+  const PcgArgs<T> a{res_mesh<T>(dm), s};
+  const Form f = res_form(dm);
+  hipLaunchKernelGGL(k_pcg_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
                      res_lds_bytes(dm, int(sizeof(T))), st, a);
 }
 
-hipError_t prepare_resident_kernels() {
+template <typename T>
+bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit) {
+  const Form f = res_form(dm);
+  return dm.xpatch && f.ne && fits(dm, device, reinterpret_cast<const void *>(k_dyn_resident_of<T>(dm.dim, f)),
+                                   res_lds_bytes(dm, int(sizeof(T))), fit);
+}
+
+template <typename T>
+void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &s, hipStream_t st) {
+  const DynArgs<T> a{res_mesh<T>(dm), s};
+  const Form f = res_form(dm);
+  hipLaunchKernelGGL(k_dyn_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
+                     res_lds_bytes(dm, int(sizeof(T))), st, a);
+}
+
+template <typename T>
+static hipError_t prepare_t() {
   hipError_t e = hipSuccess, r;
-  for (const void *f : {reinterpret_cast<const void *>(&k_pcg_resident<double, 3, 768>),
-                        reinterpret_cast<const void *>(&k_pcg_resident<double, 2, 768>),
-                        reinterpret_cast<const void *>(&k_pcg_resident<double, 2, 512>),
-                        reinterpret_cast<const void *>(&k_pcg_resident<float, 3, 768>),
-                        reinterpret_cast<const void *>(&k_pcg_resident<float, 2, 768>),
-                        reinterpret_cast<const void *>(&k_pcg_resident<float, 2, 512>)})
-    if ((r = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX)) != hipSuccess)
-      e = r;
+  for (int dim : {2, 3})
+    for (Form f : {Form{512, 1}, Form{768, 1}, Form{768, 2}})
+      for (const void *fn : {reinterpret_cast<const void *>(k_pcg_resident_of<T>(dim, f)),
+                             reinterpret_cast<const void *>(k_dyn_resident_of<T>(dim, f))})
+        if ((r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX)) !=
+            hipSuccess)
+          e = r;
   return e;
 }
 
-#define FEMGPU_RES_INST(T)                                              \
-  template bool res_pcg_fit<T>(const DevMesh &, int, ResFit *);         \
-  template void launch_res_pcg<T>(const DevMesh &, const ResPcg<T> &, hipStream_t);
+hipError_t prepare_resident_kernels() {
+  const hipError_t e = prepare_t<double>(), r = prepare_t<float>();
+  return e != hipSuccess ? e : r;
+}
+
+#define FEMGPU_RES_INST(T)                                                    \
+  template bool res_pcg_fit<T>(const DevMesh &, int, ResFit *);               \
+  template void launch_res_pcg<T>(const DevMesh &, const ResPcg<T> &, hipStream_t); \
+  template bool res_dyn_fit<T>(const DevMesh &, int, ResFit *);               \
+  template void launch_res_dyn<T>(const DevMesh &, const ResDyn<T> &, hipStream_t);
 FEMGPU_RES_INST(double)
 FEMGPU_RES_INST(float)
 

@@ -131,7 +131,9 @@ int femgpu_set_mesh(femgpu_ctx *ctx, int dim, int64_t n_nodes, const double *nod
                     int64_t n_elems, const int32_t *elems);
 /* Launch tuning, applied at the next femgpu_set_mesh: threads per patch
  * workgroup (256, 512 or 1024; 0 = 256), which is also the node limit of a
- * patch, and elements per patch (<= 3 x threads; 0 = 3 x threads).
+ * patch, and elements per patch (<= 3 x threads; 0 = 3 x threads).  Both 0:
+ * chosen by the mesh (256 threads and 768 elements, or 512 and 1536 where
+ * only those give at most 256 patches, one per compute unit).
  * No counterpart in the reference (its kernels use 256 threads and one
  * thread per element, fem_utils_kernels.cu:3). */
 int femgpu_set_tuning(femgpu_ctx *ctx, int elems_per_patch, int patch_threads);

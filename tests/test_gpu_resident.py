@@ -131,3 +131,75 @@ def test_resident_contexts_on_threads():
     finally:
         for c in ctxs:
             c.close()
+
+
+def _run_with(ctx, pb, tuning, fn):
+    ctx.set_tuning(*tuning)
+    try:
+        ctx.set_problem(pb)
+    finally:
+        ctx.set_tuning(0, 0)
+    return fn()
+
+
+# patches of more than 256 nodes (two elements per thread), small ones, and
+# more than 256 patches (a launch per kernel)
+FORMS = [(1536, 512), (64, 256), (16, 256)]
+
+
+@pytest.mark.parametrize("make", [lambda: cube_problem(9), lambda: plate_problem(70, 45)],
+                         ids=["cube9", "plate70x45"])
+def test_resident_wide_patches_solve(ctx, make):
+    pb = make()
+    u = [_run_with(ctx, pb, t, lambda: ctx.solve(F.FP64, tol=1e-11, tol_kind=F.TOL_REL_RES)[0])
+         for t in FORMS]
+    m = _run_with(ctx, pb, FORMS[0], lambda: ctx.solve(F.MIXED, tol=1e-9, tol_kind=F.TOL_REL_RES)[0])
+    assert rel(u[0], u[2]) <= 1e-9 and rel(u[1], u[2]) <= 1e-9
+    assert rel(m, u[2]) <= 1e-6
+
+
+@pytest.mark.parametrize("precision,bound", [(F.FP64, 1e-11), (F.FP32, 2e-5)])
+@pytest.mark.parametrize("quantity", [F.RECV_DISPLACEMENT, F.RECV_VELOCITY, F.RECV_ACCELERATION])
+@pytest.mark.parametrize("make", [lambda: cube_problem(9), lambda: plate_problem(100, 60)],
+                         ids=["cube9", "plate100x60"])
+def test_resident_steps_match_launches(ctx, make, quantity, precision, bound):
+    """Explicit steps in one launch against a launch per kernel, with damping,
+    an odd number of steps, receivers on interface nodes and one node twice;
+    twice in a row (the exchange words keep counting)."""
+    pb = make()
+    h = 1.0 / 9 if pb.dim == 3 else 1.0 / 100
+    dt = 0.1 * h / np.sqrt(3 * 2e7 / 2400.0)
+    opts = dict(rho=2400.0, dt=dt, endtime=61.5 * dt, wavelet_type=F.WAVELET_RICKER,
+                freq=1.0 / (20 * dt), ampl=1e3, precision=precision,
+                mass_convention=F.MASS_PHYSICAL, damping_alpha=0.3 / dt / 61)
+    nodes = np.append(np.linspace(0, pb.n_nodes - 1, 40).astype(np.int32), 3).astype(np.int32)
+    nodes[7] = 3
+
+    def go():
+        ctx.set_receivers(nodes, quantity, 3)
+        ctx.dyn_run(**opts)
+        u, st = ctx.dyn_run(**opts)
+        assert st["steps"] == 61
+        tr = ctx.traces()
+        assert tr.shape[0] == 20 and np.array_equal(tr[:, 7], tr[:, -1])
+        return u, tr
+
+    res = [_run_with(ctx, pb, t, go) for t in FORMS]
+    for u, tr in res[:2]:
+        assert rel(u, res[2][0]) <= bound and rel(tr, res[2][1]) <= bound
+
+
+def test_resident_steps_past_one_launch(ctx):
+    """More steps than one launch holds (16384) equal, bitwise, two thirds of
+    them continued: displacements after n steps do not depend on the launches."""
+    pb = plate_problem(6, 4, convention=F.LOADS_PHYSICAL)
+    ctx.set_problem(pb)
+    dt = 1e-4
+    opts = dict(rho=2400.0, dt=dt, precision=F.FP64, mass_convention=F.MASS_PHYSICAL)
+    ctx.set_receivers(np.arange(pb.n_nodes, dtype=np.int32), F.RECV_DISPLACEMENT, 100)
+    u1, st = ctx.dyn_run(endtime=20000.5 * dt, **opts)
+    tr = ctx.traces()
+    assert st["steps"] == 20000 and tr.shape[0] == 200
+    assert np.array_equal(tr[-1], u1)
+    u2, _ = ctx.dyn_run(endtime=16000.5 * dt, **opts)
+    assert np.array_equal(tr[159], u2) and np.isfinite(u1).all()
