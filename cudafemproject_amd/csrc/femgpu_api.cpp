@@ -817,6 +817,71 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
   return FEMGPU_OK;
 }
 
+// The receivers of a resident run.
+template <typename T>
+int res_receivers(femgpu_ctx *ctx, int max_samples, T *traces, femgpu::ResRecv<T> *r) {
+  const size_t n = ctx->recv.size();
+  std::vector<int32_t> of(size_t(ctx->nn), -1), next(n, -1);
+  for (size_t i = n; i-- > 0;) {
+    int32_t &head = of[size_t(ctx->plan.node_inv[size_t(ctx->recv[i])])];
+    next[i] = head;
+    head = int32_t(i);
+  }
+  int32_t *pof, *pnext;
+  int st;
+  if ((st = upload(ctx, "recv_of", of, &pof)) || (st = upload(ctx, "recv_next", next, &pnext))) return st;
+  HIPCHK(hipStreamSynchronize(ctx->stream));  // the vectors go out of scope
+  r->rec_of = pof;
+  r->rec_next = pnext;
+  r->n_rec = int(n);
+  r->rec_every = ctx->recv_every;
+  r->rec_samples = max_samples;
+  r->rec_quantity = ctx->recv_quantity;
+  r->traces = traces;
+  return FEMGPU_OK;
+}
+
+// Implicit steps step0 .. step0 + n_steps - 1 in resident launches from the
+// state in m.d, m.v, m.a (rest when m.fresh), which end with the last one's;
+// *done and *steps: the last PCG's done code and the steps completed, *iters
+// their PCG iterations.  *ok as in run_resident.
+template <typename T>
+int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int n_steps, int *done,
+                          int *steps, int *iters, bool *ok) {
+  femgpu::ResFit fit;
+  int st;
+  if (!femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit))
+    return fail(ctx, FEMGPU_E_STATE, "internal error: resident steps do not fit");
+  if ((st = res_buffers<T>(ctx, &m.words, &m.entries))) return st;
+  m.sc = ctx->h_sc;
+  m.it_budget = 4 * RES_ITER_CAP;
+  *done = 1;
+  *steps = *iters = 0;
+  *ok = true;
+  while (*steps < n_steps && *done == 1) {
+    m.step0 = step0 + *steps;
+    m.n_steps = n_steps - *steps;
+    ctx->h_sc->done = femgpu::RES_ABORTED;
+    {
+      ResidentGate gate(ctx->device, fit.share, fit.block);
+      femgpu::launch_res_impl<T>(ctx->dm, m, ctx->stream);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipStreamSynchronize(ctx->stream));
+    }
+    *done = ctx->h_sc->done;
+    if (*done == femgpu::RES_ABORTED) {
+      ctx->res_off = true;
+      ctx->res_np = 0;
+      *ok = false;
+      return FEMGPU_OK;
+    }
+    *steps += ctx->h_sc->par_final;
+    *iters += ctx->h_sc->iter_final;
+    m.fresh = 0;
+  }
+  return FEMGPU_OK;
+}
+
 // Explicit steps 1 .. n_steps in resident launches, from rest; d.d, d.v, d.a
 // end with the last state.  *ok as in run_resident (d.d, d.v, d.a are then
 // undefined).
@@ -2621,25 +2686,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
     r.c3 = T(C.c3);
     r.alpha = T(C.alpha);
     r.scale = T(C.expl_scale);
-    if (nrec && max_samples > 0) {
-      std::vector<int32_t> of(size_t(ctx->nn), -1), next(size_t(nrec), -1);
-      for (int i = nrec - 1; i >= 0; --i) {
-        int32_t &head = of[size_t(ctx->plan.node_inv[ctx->recv[i]])];
-        next[size_t(i)] = head;
-        head = i;
-      }
-      int32_t *pof, *pnext;
-      if ((st = upload(ctx, "recv_of", of, &pof)) || (st = upload(ctx, "recv_next", next, &pnext)))
-        return st;
-      HIPCHK(hipStreamSynchronize(ctx->stream));
-      r.rec_of = pof;
-      r.rec_next = pnext;
-      r.n_rec = nrec;
-      r.rec_every = every;
-      r.rec_samples = max_samples;
-      r.rec_quantity = ctx->recv_quantity;
-      r.traces = dtr;
-    }
+    if (nrec && max_samples > 0 && (st = res_receivers<T>(ctx, max_samples, dtr, &r))) return st;
     if ((st = run_resident_steps<T>(ctx, r, endnt, &resident))) return st;
     if (!resident) {
       for (T *p : {dd, dv, da}) femgpu::launch_fill<T>(p, int64_t(nd), T(0), ctx->stream);
@@ -2765,6 +2812,61 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       femgpu::launch_inv_diag<T>(ctx->dm, diagK_t, ceff, T(1), dmc, invA, ctx->stream);
     }
     w.invD = invA;
+    bool impl_resident = !ctx->res_off && femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit);
+    if (impl_resident) {
+      femgpu::ResImpl<T> m{};
+      m.d = dd;
+      m.v = dv;
+      m.a = da;
+      m.f_file = dff;
+      m.f_unit = dfu;
+      m.mlump = dml;
+      m.invA = invA;
+      m.coef_file = dcf;
+      m.coef_unit = dcu;
+      m.dt = T(C.dt);
+      m.c1 = T(C.c1);
+      m.c2 = T(C.c2);
+      m.c3 = T(C.c3);
+      m.c4 = T(C.c4);
+      m.alpha = T(C.alpha);
+      m.beta = T(beta_d);
+      m.cK = sh.cK;
+      m.cM = sh.m ? sh.cM : T(0);
+      m.eps = o.pcg_eps;
+      m.max_iter = 1000000;
+      m.fresh = 1;
+      if (nrec && max_samples > 0 && (st = res_receivers<T>(ctx, max_samples, dtr, &m))) return st;
+      // relaxation looks at max |v| after every step
+      const int chunk = relax ? 1 : endnt;
+      int last = 1, total = 0;
+      bool settled = false;
+      while (steps < endnt && last == 1 && impl_resident && !settled) {
+        int n = 0, it = 0;
+        if ((st = run_resident_implicit<T>(ctx, m, steps + 1, chunk, &last, &n, &it, &impl_resident)))
+          return st;
+        m.fresh = 0;
+        steps += n;
+        total += it;
+        if (relax && impl_resident && last == 1) {
+          double vm = 0.0;
+          if ((st = vmax(&vm))) return st;
+          settled = vm < eps_relax;
+        }
+      }
+      S.pcg_iterations = total;
+      if (impl_resident && last != 1) {
+        S.status = done_status(last);
+        ctx->err = "implicit step " + std::to_string(steps + 1) + ": PCG stopped with " + std::to_string(last);
+        if (stats) *stats = S;
+        return S.status;
+      }
+      if (!impl_resident) {
+        steps = 0;
+        for (T *q : {dd, dv, da}) femgpu::launch_fill<T>(q, int64_t(nd), T(0), ctx->stream);
+      }
+    }
+    if (!impl_resident) {
     CgScalars *sc;
     double *part_patch, *part_node;
     if ((st = dbuf(ctx, "sc_main", 1, &sc)) ||
@@ -2941,6 +3043,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
     HIPCHK(hipGetLastError());
     steps = nt - 1;
     S.pcg_iterations = total_it;
+    }
   }
   HIPCHK(hipEventRecord(ctx->ev1, ctx->stream));
   HIPCHK(hipEventSynchronize(ctx->ev1));

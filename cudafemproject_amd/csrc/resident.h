@@ -41,7 +41,6 @@ struct ResPcg {
   T *x, *p, *r_out;
   const T *invD;
   unsigned long long *entries;  // interface entries (res_entry_words)
-  OpShift<T> sh;
   unsigned long long *words;  // res_words(np)
   CgScalars *sc;              // the scalars at the end (host-visible memory)
   int fresh, kind;
@@ -74,11 +73,20 @@ bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit);
 template <typename T>
 void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &a, hipStream_t s);
 
+// Receivers of a resident run (rec_of null: none): per node its first receiver
+// or -1, the receivers of one node linked by rec_next.
+template <typename T>
+struct ResRecv {
+  const int32_t *rec_of, *rec_next;
+  int n_rec, rec_every, rec_samples, rec_quantity;
+  T *traces;
+};
+
 // Explicit GN22 steps step0 .. step0 + n_steps - 1 (1-based) in one launch;
 // from d = v = a = 0 when fresh, else from d, v, a, which hold the state at
 // the end.
 template <typename T>
-struct ResDyn {
+struct ResDyn : ResRecv<T> {
   T *d, *v, *a;
   const T *f_file, *f_unit, *invM;
   const double *coef_file, *coef_unit;   // per step
@@ -88,11 +96,6 @@ struct ResDyn {
   unsigned long long *abort;             // zero; nonzero after a launch that did not complete
   unsigned tag0;                         // tags tag0 .. tag0 + n_steps - 1, following the last launch's
   int fresh, step0, n_steps;
-  // receivers (rec_of null: none): per node its first receiver or -1, the
-  // receivers of one node linked by rec_next
-  const int32_t *rec_of, *rec_next;
-  int n_rec, rec_every, rec_samples, rec_quantity;
-  T *traces;
 };
 
 template <typename T>
@@ -100,6 +103,30 @@ bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit);
 
 template <typename T>
 void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &a, hipStream_t s);
+
+// Implicit GN22 steps in one launch, likewise; a launch ends early after the
+// step in which its PCG iterations reach it_budget.  At the end sc->done is 1,
+// or the done code of the step that failed, sc->par_final the steps done and
+// sc->iter_final the PCG iterations.
+template <typename T>
+struct ResImpl : ResRecv<T> {
+  T *d, *v, *a;
+  const T *f_file, *f_unit, *mlump, *invA;
+  const double *coef_file, *coef_unit;
+  T dt, c1, c2, c3, c4, alpha, beta;
+  T cK, cM;               // operator cK K + cM diag(mlump) (cM 0: no mass)
+  double eps;             // nested PCG: gamma < eps gamma0
+  int max_iter, it_budget;
+  unsigned long long *words, *entries;
+  CgScalars *sc;
+  int fresh, step0, n_steps;
+};
+
+template <typename T>
+bool res_impl_fit(const DevMesh &dm, int device, ResFit *fit);
+
+template <typename T>
+void launch_res_impl(const DevMesh &dm, const ResImpl<T> &a, hipStream_t s);
 
 hipError_t prepare_resident_kernels();
 

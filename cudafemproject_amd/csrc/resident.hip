@@ -1,5 +1,5 @@
-// resident.hip -- the PCG iteration (femfunc.cpp:59-111) and the explicit time
-// step (femfunc.cpp:247-343) as one launch per solve or run.
+// resident.hip -- the PCG iteration (femfunc.cpp:59-111) and the explicit and
+// implicit time steps (femfunc.cpp:247-343) as one launch per solve or run.
 //
 // A launch costs about 4 us on gfx950 even when it does nothing, and the
 // launch-per-kernel forms of kernels.hip pay it once a step and twice an
@@ -569,6 +569,123 @@ struct ResPatch {
   }
 };
 
+// The PCG of one workgroup (the recurrence of k_ebe_patch MODE 1 and
+// k_pcg_update): r, p, x of this thread's DOFs, the scalars the same in every
+// workgroup.
+template <typename T, int DIM, int PT, int NE>
+struct ResSolver {
+  using Patch = ResPatch<T, DIM, PT, NE>;
+  static constexpr int ND = Patch::ND;
+  Patch &P;
+  Exchange xpq, xrz;
+  u64 *entries;
+  unsigned tag, entry_tag;
+  int pid;
+  bool alone;            // one workgroup: no exchange
+  int *s_flag;           // LDS: a wait ran out
+  double *s_red, *s_bc;  // LDS: p'q (16); r'z and r'r (32); their totals (1 + 2)
+  double g, q2, g_prev;  // r'z, r'r; the r'z that p was formed with
+  int n_upd;
+
+  __device__ __forceinline__ ResSolver(Patch &patch, const ResMesh<T> &m, u64 *words, u64 *ent, int b,
+                                       int id, int *flag)
+      : P(patch), entries(ent), pid(id), alone(m.np == 1), s_flag(flag), s_red(patch.s_red),
+        s_bc(patch.s_red + 48), g(0.0), q2(0.0), g_prev(1.0), n_upd(0) {
+    const size_t stride = res_copy_words(m.np);
+    xpq = Exchange{words + RES_HEAD, stride, words + 1, m.np, b % EX_COPIES};
+    xrz = Exchange{xpq.words + size_t(2) * m.np, stride, words + 1, m.np, b % EX_COPIES};
+    // (workgroup 0 advances the tags at its end, after an exchange that every
+    // workgroup took part in with the tags it reads here)
+    tag = unsigned(ld_agent(words));
+    entry_tag = unsigned(ld_agent(words + 2 + (sizeof(T) == 8 ? 1 : 0)));
+  }
+
+  __device__ __forceinline__ void store_tags(u64 *words) const {
+    st_agent(words, u64(tag));
+    st_agent(words + 2 + (sizeof(T) == 8 ? 1 : 0), u64(entry_tag));
+  }
+
+  // g, q2 = r'z and r'r over all patches (z = invD r).
+  __device__ __forceinline__ bool dots(const T (&r)[ND], const T (&invd)[ND]) {
+    double v[2] = {0.0, 0.0};
+    if (P.first)
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        v[0] += double(r[i]) * double(mul_rn(invd[i], r[i]));
+        v[1] += double(r[i]) * double(r[i]);
+      }
+    sum_to_wave0<PT, 2>(v, s_red + 16);
+    ++tag;
+    if (!alone && threadIdx.x < 64) publish<2>(xrz, pid, tag, v);
+    const bool ok = gather<2>(xrz, tag, v, s_bc, s_flag, alone);
+    g = v[0];
+    q2 = v[1];
+    return ok;
+  }
+
+  // Iterates from r, p, x with g and q2 formed until a stop; returns the done
+  // code.  cMm: the mass shift of this thread's DOFs.
+  __device__ __forceinline__ int run(T (&r)[ND], T (&p)[ND], T (&x)[ND], const T (&invd)[ND], T cK,
+                                     const T (&cMm)[ND], int kind, double thresh, double pause,
+                                     int max_iter, int last) {
+    for (;;) {
+      if (n_upd >= 1) {
+        if (kind == 0 ? g < thresh : q2 <= thresh) return 1;
+      } else if (q2 == 0.0) {
+        return 1;
+      }
+      if (!isfinite(g)) return 2;
+      if (n_upd >= max_iter) return 4;
+      // (looked at every eighth iteration: r'r is not monotone, and a
+      // replacement at a single dip can cost directions -- a 160 x 80-class
+      // plate under body force took 3225 iterations with a look at every one,
+      // 1953 so, 1950 in the launch-per-kernel form)
+      if ((n_upd & 7) == 0 && q2 < pause) return 5;
+      if (n_upd >= last) return RES_CAP;
+      const T beta = T(g / g_prev);
+      g_prev = g;
+      if (P.has)
+#pragma unroll
+        for (int i = 0; i < ND; ++i) p[i] = pcg_dir(invd[i], r[i], beta, p[i]);
+      T q[ND];
+      P.product(p, q);
+      double vpq[1] = {0.0};
+      if (P.has)
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+          q[i] = cK * q[i];
+          if (P.own) q[i] += cMm[i] * p[i];
+          vpq[0] += double(p[i]) * double(q[i]);
+          // the mass shift belongs to the patch that accounts for the node
+          if (!P.own && P.first) vpq[0] += double(cMm[i]) * double(p[i]) * double(p[i]);
+        }
+      P.put(q);
+      ++tag;
+      ++entry_tag;
+      sum_to_wave0<PT, 1>(vpq, s_red);
+      if (!alone) {
+        if (threadIdx.x < 64) publish<1>(xpq, pid, tag, vpq);
+        if (!P.trade(entries, entry_tag, xpq.abort)) *s_flag = 1;
+      }
+      if (!gather<1>(xpq, tag, vpq, s_bc + 2, s_flag, alone)) return RES_ABORTED;
+      const double pq = vpq[0], alpha_d = g / pq;
+      // (no x or r has changed: the state of the last completed iteration)
+      if (!(pq > 0.0) || !isfinite(alpha_d)) return isfinite(pq) ? 3 : 2;
+      const T alpha = T(alpha_d);
+      P.collect(q);
+      if (P.has)
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+          if (!P.own) q[i] += cMm[i] * p[i];
+          x[i] = x[i] + alpha * p[i];
+          r[i] = r[i] - alpha * q[i];
+        }
+      if (!dots(r, invd)) return RES_ABORTED;
+      ++n_upd;
+    }
+  }
+};
+
 template <typename T>
 struct PcgArgs {
   ResMesh<T> m;
@@ -584,125 +701,36 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
   const int b = blockIdx.x;
   const int pid = (b & 7) * a.m.p8 + (b >> 3);
   if (pid >= a.m.np) return;
-  const bool alone = a.m.np == 1;  // no exchange
-  const int t = threadIdx.x;
-  if (t == 0) s_flag = 0;
+  if (threadIdx.x == 0) s_flag = 0;
   Patch P;
   P.load(a.m, pid, lds);
-  double *s_red = P.s_red;  // p'q; r'z and r'r
-  double *s_bc = s_red + 48;
-  T r[ND], p[ND], x[ND], d[ND], q[ND], cMm[ND];
+  T r[ND], p[ND], x[ND], d[ND], cMm[ND];
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     r[i] = p[i] = x[i] = d[i] = cMm[i] = T(0);
     if (P.has) {
       r[i] = a.s.r_in[P.go + i];
       d[i] = a.s.invD[P.go + i];
-      if (a.s.sh.m) cMm[i] = a.s.sh.cM * a.s.sh.m[P.go + i];
       if (!a.s.fresh) {
         p[i] = a.s.p[P.go + i];
         x[i] = a.s.x[P.go + i];
       }
     }
   }
-  const T cK = a.s.sh.cK;
-  // (workgroup 0 advances the tags at its end, after an exchange that every
-  // workgroup took part in with the tags it reads here)
-  u64 *const epoch = a.s.words;
-  const size_t stride = res_copy_words(a.m.np);
-  const Exchange xpq{a.s.words + RES_HEAD, stride, epoch + 1, a.m.np, b % EX_COPIES};
-  const Exchange xrz{xpq.words + size_t(2) * a.m.np, stride, epoch + 1, a.m.np, b % EX_COPIES};
-  u64 *const etag = epoch + 2 + (sizeof(T) == 8 ? 1 : 0);
-  unsigned tag = unsigned(ld_agent(epoch)), entry_tag = unsigned(ld_agent(etag));
-
-  // r'z and r'r over all patches
-  double g = 0.0, q2 = 0.0;
-  auto dots = [&]() -> bool {
-    double v[2] = {0.0, 0.0};
-    if (P.first)
-#pragma unroll
-      for (int i = 0; i < ND; ++i) {
-        v[0] += double(r[i]) * double(mul_rn(d[i], r[i]));
-        v[1] += double(r[i]) * double(r[i]);
-      }
-    sum_to_wave0<PT, 2>(v, s_red + 16);
-    ++tag;
-    if (!alone && t < 64) publish<2>(xrz, pid, tag, v);
-    const bool ok = gather<2>(xrz, tag, v, s_bc, &s_flag, alone);
-    g = v[0];
-    q2 = v[1];
-    return ok;
-  };
-
-  bool alive = dots();
-  double g_prev = a.s.fresh ? 1.0 : a.s.g_prev;
-  const double gamma0 = a.s.fresh ? g : a.s.gamma0, rr0 = a.s.fresh ? q2 : a.s.rr0;
-  const double pause = a.s.fresh ? a.s.pause * q2 : a.s.pause;
-  const double thresh = !a.s.fresh ? a.s.thresh : a.s.kind == 0 ? a.s.eps * g : a.s.eps * a.s.eps * q2;
-  int n_upd = a.s.it0;
+  ResSolver<T, DIM, PT, NE> S(P, a.m, a.s.words, a.s.entries, b, pid, &s_flag);
+  S.n_upd = a.s.it0;
   int done = RES_ABORTED;
-  while (alive) {
-    int stop = 0;
-    if (n_upd >= 1) {
-      if (a.s.kind == 0 ? g < thresh : q2 <= thresh) stop = 1;
-    } else if (q2 == 0.0) {
-      stop = 1;
+  double gamma0 = a.s.gamma0, rr0 = a.s.rr0, thresh = a.s.thresh, pause = a.s.pause;
+  if (S.dots(r, d)) {
+    if (a.s.fresh) {
+      gamma0 = S.g;
+      rr0 = S.q2;
+      thresh = a.s.kind == 0 ? a.s.eps * S.g : a.s.eps * a.s.eps * S.q2;
+      pause = a.s.pause * S.q2;
+    } else {
+      S.g_prev = a.s.g_prev;
     }
-    if (!stop && !isfinite(g)) stop = 2;
-    if (!stop && n_upd >= a.s.max_iter) stop = 4;
-    // (looked at every eighth iteration: r'r is not monotone, and a replacement
-    // at a single dip can cost directions -- a 160 x 80-class plate under body
-    // force took 3225 iterations with a look at every one, 1953 so, 1950 in the
-    // launch-per-kernel form)
-    if (!stop && (n_upd & 7) == 0 && q2 < pause) stop = 5;
-    if (!stop && n_upd - a.s.it0 >= a.s.cap) stop = RES_CAP;
-    if (stop) {
-      done = stop;
-      break;
-    }
-    const T beta = T(g / g_prev);
-    g_prev = g;
-    if (P.has)
-#pragma unroll
-      for (int i = 0; i < ND; ++i) p[i] = pcg_dir(d[i], r[i], beta, p[i]);
-    P.product(p, q);
-    double vpq[1] = {0.0};
-    if (P.has)
-#pragma unroll
-      for (int i = 0; i < ND; ++i) {
-        q[i] = cK * q[i];
-        if (P.own) q[i] += cMm[i] * p[i];
-        vpq[0] += double(p[i]) * double(q[i]);
-        // the mass shift belongs to the patch that accounts for the node
-        if (!P.own && P.first) vpq[0] += double(cMm[i]) * double(p[i]) * double(p[i]);
-      }
-    P.put(q);
-    ++tag;
-    ++entry_tag;
-    sum_to_wave0<PT, 1>(vpq, s_red);
-    if (!alone) {
-      if (t < 64) publish<1>(xpq, pid, tag, vpq);
-      if (!P.trade(a.s.entries, entry_tag, epoch + 1)) s_flag = 1;
-    }
-    alive = gather<1>(xpq, tag, vpq, s_bc + 2, &s_flag, alone);
-    if (!alive) break;
-    const double pq = vpq[0], alpha_d = g / pq;
-    if (!(pq > 0.0) || !isfinite(alpha_d)) {
-      // no x or r has changed: the state of the last completed iteration
-      done = isfinite(pq) ? 3 : 2;
-      break;
-    }
-    const T alpha = T(alpha_d);
-    P.collect(q);
-    if (P.has)
-#pragma unroll
-      for (int i = 0; i < ND; ++i) {
-        if (!P.own) q[i] += cMm[i] * p[i];
-        x[i] = x[i] + alpha * p[i];
-        r[i] = r[i] - alpha * q[i];
-      }
-    alive = dots();
-    ++n_upd;
+    done = S.run(r, p, x, d, T(1), cMm, a.s.kind, thresh, pause, a.s.max_iter, a.s.it0 + a.s.cap);
   }
   if (P.first)
 #pragma unroll
@@ -711,19 +739,133 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
       a.s.p[P.go + i] = p[i];
       a.s.r_out[P.go + i] = r[i];
     }
-  if (pid == 0 && t == 0) {
+  if (pid == 0 && threadIdx.x == 0) {
     CgScalars *sc = a.s.sc;
     sc->gamma0 = gamma0;
     sc->rr0 = rr0;
     sc->thresh = thresh;
-    sc->g[0] = sc->g[1] = g_prev;
-    sc->g_final = g;
-    sc->rr_final = q2;
-    sc->iter_final = n_upd;
+    sc->g[0] = sc->g[1] = S.g_prev;
+    sc->g_final = S.g;
+    sc->rr_final = S.q2;
+    sc->iter_final = S.n_upd;
     sc->pause = pause;
-    st_agent(epoch, u64(tag));
-    st_agent(etag, u64(entry_tag));
-    if (ld_agent(epoch + 1) != 0) done = RES_ABORTED;
+    S.store_tags(a.s.words);
+    if (ld_agent(a.s.words + 1) != 0) done = RES_ABORTED;
+    sc->done = done;
+  }
+}
+
+// Implicit GN22 steps: the predictor (k_dyn_predict), K (d~ + beta v~) and its
+// trade, the residual (k_dyn_correct), the nested PCG for the acceleration,
+// the corrector (k_dyn_implicit_post).
+template <typename T>
+struct ImplArgs {
+  ResMesh<T> m;
+  ResImpl<T> s;
+};
+
+// One receiver sample of this thread's DOFs, if its node has receivers.
+template <typename T, int DIM, typename Patch, typename R>
+__device__ __forceinline__ void record(const Patch &P, const R &s, int rec, int step, const T *d,
+                                       const T *v, const T *a) {
+  if (rec < 0 || step % s.rec_every != 0) return;
+  const int smp = step / s.rec_every - 1;
+  if (smp >= s.rec_samples) return;
+  const T *src = s.rec_quantity == 0 ? d : s.rec_quantity == 1 ? v : a;
+  for (int k = rec; k >= 0; k = s.rec_next[k])
+#pragma unroll
+    for (int i = 0; i < Patch::ND; ++i)
+      s.traces[(int64_t(smp) * s.n_rec + k) * DIM + P.comp(i)] = src[i];
+}
+
+template <typename T, int DIM, int PT, int NE>
+__global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
+  using Patch = ResPatch<T, DIM, PT, NE>;
+  constexpr int ND = Patch::ND;
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_flag;
+  const int b = blockIdx.x;
+  const int pid = (b & 7) * arg.m.p8 + (b >> 3);
+  if (pid >= arg.m.np) return;
+  if (threadIdx.x == 0) s_flag = 0;
+  Patch P;
+  P.load(arg.m, pid, lds);
+  const ResImpl<T> &s = arg.s;
+  T d[ND], v[ND], a[ND], invd[ND], cMm[ND], ml[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    d[i] = v[i] = a[i] = invd[i] = cMm[i] = ml[i] = T(0);
+    if (P.has) {
+      invd[i] = s.invA[P.go + i];
+      ml[i] = s.mlump[P.go + i];
+      if (s.cM != T(0)) cMm[i] = s.cM * ml[i];
+      if (!s.fresh) {
+        d[i] = s.d[P.go + i];
+        v[i] = s.v[P.go + i];
+        a[i] = s.a[P.go + i];
+      }
+    }
+  }
+  const int rec = s.rec_of && P.has && P.first ? s.rec_of[P.gid] : -1;
+  ResSolver<T, DIM, PT, NE> S(P, arg.m, s.words, s.entries, b, pid, &s_flag);
+  int done = 1, n = 0, total = 0;
+  for (; n < s.n_steps && total < s.it_budget; ++n) {
+    const int step = s.step0 + n;
+    const T cf = T(s.coef_file[step]), cu = T(s.coef_unit[step]);
+    T x[ND], r[ND], p[ND];
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      d[i] = d[i] + s.dt * v[i];
+      d[i] = d[i] + s.c1 * a[i];
+      v[i] = v[i] + s.c2 * a[i];
+      x[i] = s.beta != T(0) ? d[i] + s.beta * v[i] : d[i];
+    }
+    P.product(x, r);
+    if (!S.alone) {
+      P.put(r);
+      ++S.entry_tag;
+      __syncthreads();
+      if (!P.trade(S.entries, S.entry_tag, S.xpq.abort)) s_flag = 1;
+      __syncthreads();
+      P.collect(r);
+    }
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      const T kd = r[i];
+      p[i] = x[i] = r[i] = T(0);
+      if (P.has) {
+        const T f = cf * s.f_file[P.go + i] + cu * s.f_unit[P.go + i] - kd;
+        r[i] = s.alpha != T(0) ? f - s.alpha * ml[i] * v[i] : f;
+      }
+    }
+    S.n_upd = 0;
+    S.g_prev = 1.0;
+    done = RES_ABORTED;
+    if (S.dots(r, invd))
+      done = S.run(r, p, x, invd, s.cK, cMm, 0, s.eps * S.g, 0.0, s.max_iter, s.max_iter + 1);
+    total += S.n_upd;
+    if (done != 1) break;
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      a[i] = x[i];
+      v[i] = v[i] + s.c3 * a[i];
+      d[i] = d[i] + s.c4 * a[i];
+    }
+    record<T, DIM>(P, s, rec, step, d, v, a);
+  }
+  if (P.first && done == 1)
+#pragma unroll
+    for (int i = 0; i < ND; ++i) {
+      s.d[P.go + i] = d[i];
+      s.v[P.go + i] = v[i];
+      s.a[P.go + i] = a[i];
+    }
+  if (pid == 0 && threadIdx.x == 0) {
+    CgScalars *sc = s.sc;
+    sc->iter_final = total;
+    sc->par_final = n;
+    S.store_tags(s.words);
+    if (ld_agent(s.words + 1) != 0) done = RES_ABORTED;
     sc->done = done;
   }
 }
@@ -755,7 +897,6 @@ __global__ __launch_bounds__(PT) void k_dyn_resident(DynArgs<T> a) {
   P.load(a.m, pid, lds);
   const ResDyn<T> &s = a.s;
   T d[ND], v[ND], ac[ND], ff[ND], fu[ND], im[ND];
-  int rec = -1;
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
     d[i] = v[i] = ac[i] = ff[i] = fu[i] = im[i] = T(0);
@@ -770,7 +911,7 @@ __global__ __launch_bounds__(PT) void k_dyn_resident(DynArgs<T> a) {
       }
     }
   }
-  if (s.rec_of && P.has && P.first) rec = s.rec_of[P.gid];
+  const int rec = s.rec_of && P.has && P.first ? s.rec_of[P.gid] : -1;
   bool alive = true;
   for (int n = 0; n < s.n_steps; ++n) {
     const int step = s.step0 + n;
@@ -795,15 +936,7 @@ __global__ __launch_bounds__(PT) void k_dyn_resident(DynArgs<T> a) {
         gn22_correct<T>(cf, cu, ff[i], fu[i], kd[i], im[i], s.c2, s.c3, s.alpha, s.scale, ac[i], v[i]);
         d[i] = x[i];
       }
-    if (rec >= 0 && step % s.rec_every == 0) {
-      const int smp = step / s.rec_every - 1;
-      if (smp < s.rec_samples)
-        for (int k = rec; k >= 0; k = s.rec_next[k])
-#pragma unroll
-          for (int i = 0; i < ND; ++i)
-            s.traces[(int64_t(smp) * s.n_rec + k) * DIM + P.comp(i)] =
-                s.rec_quantity == 0 ? d[i] : s.rec_quantity == 1 ? v[i] : ac[i];
-    }
+    record<T, DIM>(P, s, rec, step, d, v, ac);
   }
   if (P.first && alive)
 #pragma unroll
@@ -877,6 +1010,8 @@ template <typename T>
 using PcgKernel = void (*)(PcgArgs<T>);
 template <typename T>
 using DynKernel = void (*)(DynArgs<T>);
+template <typename T>
+using ImplKernel = void (*)(ImplArgs<T>);
 
 #define FEMGPU_RES_KERNEL(NAME, KIND)                                                       \
   template <typename T>                                                                     \
@@ -887,6 +1022,7 @@ using DynKernel = void (*)(DynArgs<T>);
   }
 FEMGPU_RES_KERNEL(k_pcg_resident, PcgKernel)
 FEMGPU_RES_KERNEL(k_dyn_resident, DynKernel)
+FEMGPU_RES_KERNEL(k_impl_resident, ImplKernel)
 #undef FEMGPU_RES_KERNEL
 
 // Workgroups of a kernel that a compute unit holds, and the device's units
@@ -967,12 +1103,28 @@ void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &s, hipStream_t st) {
 }
 
 template <typename T>
+bool res_impl_fit(const DevMesh &dm, int device, ResFit *fit) {
+  const Form f = res_form(dm);
+  return dm.xpatch && f.ne && fits(dm, device, reinterpret_cast<const void *>(k_impl_resident_of<T>(dm.dim, f)),
+                                   res_lds_bytes(dm, int(sizeof(T))), fit);
+}
+
+template <typename T>
+void launch_res_impl(const DevMesh &dm, const ResImpl<T> &s, hipStream_t st) {
+  const ImplArgs<T> a{res_mesh<T>(dm), s};
+  const Form f = res_form(dm);
+  hipLaunchKernelGGL(k_impl_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
+                     res_lds_bytes(dm, int(sizeof(T))), st, a);
+}
+
+template <typename T>
 static hipError_t prepare_t() {
   hipError_t e = hipSuccess, r;
   for (int dim : {2, 3})
     for (Form f : {Form{512, 1}, Form{768, 1}, Form{768, 2}})
       for (const void *fn : {reinterpret_cast<const void *>(k_pcg_resident_of<T>(dim, f)),
-                             reinterpret_cast<const void *>(k_dyn_resident_of<T>(dim, f))})
+                             reinterpret_cast<const void *>(k_dyn_resident_of<T>(dim, f)),
+                             reinterpret_cast<const void *>(k_impl_resident_of<T>(dim, f))})
         if ((r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX)) !=
             hipSuccess)
           e = r;
@@ -988,7 +1140,9 @@ hipError_t prepare_resident_kernels() {
   template bool res_pcg_fit<T>(const DevMesh &, int, ResFit *);               \
   template void launch_res_pcg<T>(const DevMesh &, const ResPcg<T> &, hipStream_t); \
   template bool res_dyn_fit<T>(const DevMesh &, int, ResFit *);               \
-  template void launch_res_dyn<T>(const DevMesh &, const ResDyn<T> &, hipStream_t);
+  template void launch_res_dyn<T>(const DevMesh &, const ResDyn<T> &, hipStream_t); \
+  template bool res_impl_fit<T>(const DevMesh &, int, ResFit *);              \
+  template void launch_res_impl<T>(const DevMesh &, const ResImpl<T> &, hipStream_t);
 FEMGPU_RES_INST(double)
 FEMGPU_RES_INST(float)
 

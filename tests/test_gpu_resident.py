@@ -203,3 +203,30 @@ def test_resident_steps_past_one_launch(ctx):
     assert np.array_equal(tr[-1], u1)
     u2, _ = ctx.dyn_run(endtime=16000.5 * dt, **opts)
     assert np.array_equal(tr[159], u2) and np.isfinite(u1).all()
+
+
+@pytest.mark.parametrize("mode", [F.IMPLICIT_PHYSICAL, F.IMPLICIT_REFERENCE])
+@pytest.mark.parametrize("make", [lambda: cube_problem(9), lambda: plate_problem(70, 45)],
+                         ids=["cube9", "plate70x45"])
+def test_resident_implicit_matches_launches(ctx, make, mode):
+    """Implicit steps in one launch against a launch per kernel: Rayleigh
+    damping (physical operator), receivers, nested solves to 1e-24 on gamma."""
+    pb = make()
+    h = 1.0 / 9 if pb.dim == 3 else 1.0 / 70
+    dt = h / np.sqrt(3 * 2e7 / 2400.0)
+    opts = dict(rho=2400.0, beta2=0.5, dt=dt, endtime=7.5 * dt, wavelet_type=F.WAVELET_RICKER,
+                freq=1.0 / (3 * dt), ampl=1e3, mass_convention=F.MASS_PHYSICAL, implicit_mode=mode,
+                pcg_eps=1e-24)
+    if mode == F.IMPLICIT_PHYSICAL:
+        opts.update(damping_alpha=0.1 / dt, damping_beta=0.2 * dt)
+    nodes = np.linspace(0, pb.n_nodes - 1, 30).astype(np.int32)
+
+    def go():
+        ctx.set_receivers(nodes, F.RECV_VELOCITY, 2)
+        u, st = ctx.dyn_run(**opts)
+        assert st["steps"] == 7 and st["pcg_iterations"] > 7
+        return u, ctx.traces()
+
+    res = [_run_with(ctx, pb, t, go) for t in FORMS]
+    for u, tr in res[:2]:
+        assert rel(u, res[2][0]) <= 1e-9 and rel(tr, res[2][1]) <= 1e-9
