@@ -14,8 +14,11 @@
 
 #include "batch.h"
 #include "batch_ls.h"
+#include "batch_res.h"
 #include "femgpu.h"
 #include "kernels.h"
+#include "resident.h"
+#include "resident_gate.h"
 
 namespace femgpu {
 
@@ -36,6 +39,12 @@ struct BatchState {
   int bl_np = 0, bl_nblk = 0, bl_nif = 0, bl_ent = 0, bl_pn = 0;
   int64_t bl_slots = 0;
   int *h_count = nullptr;                // pinned
+  // resident form of the lockstep schedule (batch_res.h): br_np_max 0 where the
+  // plans don't suit it
+  int br_np_max = 0, br_in = 0, br_src = 0;  // most patches of an instance; exchange sizes of a patch
+  int64_t br_entries = 0;
+  int br_degree = BR_DEGREE;             // more once a launch found a node with more neighbours
+  bool br_off = false;                   // a launch did not complete
   std::map<std::string, std::pair<void *, size_t>> bufs;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_poll[2] = {nullptr, nullptr};
 };
@@ -117,6 +126,10 @@ std::string build_lockstep(BatchState *b, hipStream_t s, const int64_t *node_off
   std::vector<double> c64(size_t(b->total_nodes) * dim);
   int32_t E0 = 0, S0 = 0;
   int ent = 0, pn = 0;
+  bool resident = dim == 2;
+  std::vector<ExchangePatch> xpat;
+  std::vector<uint32_t> xout;
+  std::vector<uint16_t> xsrc, xin, xend, xown;
   for (int i = 0; i < b->n_inst; ++i) {
     const int64_t nn = node_off[i + 1] - node_off[i], ne = elem_off[i + 1] - elem_off[i];
     const double *nd = nodes + size_t(node_off[i]) * dim;
@@ -133,6 +146,26 @@ std::string build_lockstep(BatchState *b, hipStream_t s, const int64_t *node_off
     I.p0 = int32_t(pat.size());
     I.if0 = int32_t(iface.size() / 4);
     const int32_t SH0 = int32_t(shinfo.size() / 4), PN0 = int32_t(nend.size());
+    ExchangePlan X;
+    resident = resident && Q.emax_used <= BR_ELEMS && Q.pn_used <= BR_NODES && build_exchange(Q, X);
+    if (resident) {
+      const int32_t O0 = int32_t(xout.size());
+      for (ExchangePatch e : X.patches) {
+        e.in_start += int32_t(b->br_entries);
+        e.out_start += O0;
+        xpat.push_back(e);
+      }
+      for (uint32_t e : X.out_entry) xout.push_back(e + uint32_t(b->br_entries));
+      xsrc.insert(xsrc.end(), X.out_src.begin(), X.out_src.end());
+      xin.insert(xin.end(), X.in_pos.begin(), X.in_pos.end());
+      xend.insert(xend.end(), X.src_end.begin(), X.src_end.end());
+      xown.insert(xown.end(), X.own_pos.begin(), X.own_pos.end());
+      b->br_entries += (X.n_entries + 63) / 64 * 64;
+      b->br_in = std::max(b->br_in, X.n_in_max);
+      b->br_src = std::max(b->br_src, X.n_src_max);
+      b->br_np_max = std::max(b->br_np_max, int(Q.patches.size()));
+      resident = b->br_entries < (int64_t(1) << 31) / br_entry_words(4);
+    }
     for (PatchInfo pi : Q.patches) {
       pi.elem_start += E0;
       pi.own_start += N0;
@@ -201,7 +234,176 @@ std::string build_lockstep(BatchState *b, hipStream_t s, const int64_t *node_off
       (e = bup(b, s, "bl_c32", c32, &d8)) != hipSuccess ||
       (e = bup(b, s, "bl_fix", b->bl_fix, &d9)) != hipSuccess)
     return std::string("upload failed: ") + hipGetErrorString(e);
+  if (!resident) {
+    b->br_np_max = 0;
+    return "";
+  }
+  // tickets: instances with the most patches first (their solves take longest)
+  std::vector<int32_t> by_size(b->n_inst), tickets;
+  std::iota(by_size.begin(), by_size.end(), 0);
+  std::stable_sort(by_size.begin(), by_size.end(), [&](int x, int y) {
+    return b->bl_inst[x].p1 - b->bl_inst[x].p0 > b->bl_inst[y].p1 - b->bl_inst[y].p0;
+  });
+  for (int32_t i : by_size)
+    for (int32_t p = b->bl_inst[i].p0; p < b->bl_inst[i].p1; ++p) tickets.push_back(p);
+  ExchangePatch *x0;
+  uint32_t *x1;
+  uint16_t *x2;
+  int32_t *x3;
+  if ((e = bup(b, s, "br_patches", xpat, &x0)) != hipSuccess ||
+      (e = bup(b, s, "br_out", xout, &x1)) != hipSuccess ||
+      (e = bup(b, s, "br_src", xsrc, &x2)) != hipSuccess ||
+      (e = bup(b, s, "br_in", xin, &x2)) != hipSuccess ||
+      (e = bup(b, s, "br_end", xend, &x2)) != hipSuccess ||
+      (e = bup(b, s, "br_own", xown, &x2)) != hipSuccess ||
+      (e = bup(b, s, "br_tickets", tickets, &x3)) != hipSuccess ||
+      (e = bup(b, s, "br_perm", b->bl_perm, &x3)) != hipSuccess)
+    return std::string("upload failed: ") + hipGetErrorString(e);
   return "";
+}
+
+// Per-system results of a finished lockstep solve (hs: [instance][nr]).
+int report(femgpu_ctx *ctx, const BatchState *b, int n_rhs, int nr, const std::vector<BLState> &hs,
+           femgpu_batch_stat *stats) {
+  int worst = FEMGPU_OK;
+  for (int i = 0; i < b->n_inst; ++i)
+    for (int rr = 0; rr < n_rhs; ++rr) {
+      const BLState &x = hs[size_t(i) * nr + rr];
+      const int status = x.state == 3 ? x.status : FEMGPU_E_MAXIT;
+      if (stats) {
+        femgpu_batch_stat &o2 = stats[size_t(i) * n_rhs + rr];
+        o2.status = status;
+        o2.iterations = x.state == 3 ? x.iters : std::max(x.it[0], x.it[1]) + 1;
+        o2.replacements = std::max(x.nrep, 0);
+        o2.rel_res = x.ff > 0.0 ? std::sqrt(x.rr / x.ff) : 0.0;
+      }
+      if (status != FEMGPU_OK && worst == FEMGPU_OK) worst = status;
+    }
+  if (worst != FEMGPU_OK)
+    return ctx_fail(ctx, worst, "some batch systems did not converge (see stats)");
+  return FEMGPU_OK;
+}
+
+#define BCHK_(call)                                                                         \
+  do {                                                                                      \
+    hipError_t e_ = (call);                                                                 \
+    if (e_ != hipSuccess)                                                                   \
+      return ctx_fail(ctx, FEMGPU_E_HIP, (std::string(#call) + ": " + hipGetErrorString(e_)).c_str()); \
+  } while (0)
+
+// Resident lockstep solve (batch_res.h) where the instances fit the device;
+// *ran false: not run, or it did not complete.
+int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, const double *f,
+                         const femgpu_solve_opts &o, double *u_out, femgpu_batch_stat *stats,
+                         double *solve_ms, bool *ran) {
+  *ran = false;
+  if (!b->br_np_max || b->br_off) return FEMGPU_OK;
+  const int lds = br_lds_bytes(nr, b->bl_pn, b->bl_ent, b->br_in, b->br_src);
+  double block = 1.0;
+  const int capacity = br_capacity(nr, b->br_degree, lds, ctx_device(ctx), &block);
+  if (b->br_np_max > capacity) return FEMGPU_OK;
+  hipStream_t s = ctx_stream(ctx);
+  const int64_t N = b->total_nodes;
+  const size_t nd = size_t(N) * 2, nv = nd * nr, nu = nd * n_rhs;
+  const size_t n_state = size_t(b->n_inst) * nr;
+  // entries, exchange words, abort flag and ticket: zero before the launch
+  const size_t n_ent = size_t(b->br_entries) * br_entry_words(nr);
+  const size_t n_words = br_patch_words(nr) * size_t(b->bl_np);
+  double *d_user, *d_f, *d_x, *diag, *slots, *invD, *zero;
+  BLState *st;
+  BCHK_(bbuf(b, "br_user", nu, &d_user));
+  BCHK_(bbuf(b, "bl_f", nv, &d_f));
+  BCHK_(bbuf(b, "bl_x64", nv, &d_x));
+  BCHK_(bbuf(b, "bl_diag64", nd, &diag));
+  BCHK_(bbuf(b, "bl_s64", size_t(b->bl_slots) * nr * 2 + 1, &slots));
+  BCHK_(bbuf(b, "bl64_invD", nd, &invD));
+  BCHK_(bbuf(b, "br_words", n_ent + n_words + 3, &zero));
+  BCHK_(bbuf(b, "bl_state", n_state, &st));
+  auto *words = reinterpret_cast<unsigned long long *>(zero);
+  auto table = [&](const char *name) { return b->bufs[name].first; };
+  BRArgs a{};
+  a.patches = static_cast<const PatchInfo *>(table("bl_patches"));
+  a.erec = static_cast<const uint32_t *>(table("bl_erec"));
+  a.sh_info = static_cast<const int4 *>(table("bl_shinfo"));
+  a.node_end = static_cast<const uint16_t *>(table("bl_nodeend"));
+  a.fixmask = static_cast<const uint8_t *>(table("bl_fix"));
+  a.coords = static_cast<const double *>(table("bl_c64"));
+  a.diagK = diag;
+  a.inst = static_cast<const BLInst *>(table("bl_inst"));
+  a.xpatch = static_cast<const ExchangePatch *>(table("br_patches"));
+  a.out_entry = static_cast<const uint32_t *>(table("br_out"));
+  a.out_src = static_cast<const uint16_t *>(table("br_src"));
+  a.in_pos = static_cast<const uint16_t *>(table("br_in"));
+  a.src_end = static_cast<const uint16_t *>(table("br_end"));
+  a.own_pos = static_cast<const uint16_t *>(table("br_own"));
+  a.order = static_cast<const int32_t *>(table("br_tickets"));
+  a.np = b->bl_np;
+  a.ent = b->bl_ent;
+  a.pn = b->bl_pn;
+  a.n_in_max = b->br_in;
+  a.n_src_max = b->br_src;
+  a.f = d_f;
+  a.invD = invD;
+  a.x = d_x;
+  a.abort = words;
+  a.ticket = reinterpret_cast<unsigned *>(words + 1);
+  a.crowded = words + 2;
+  a.words = words + 3;
+  a.entries = a.words + n_words;
+  a.st = st;
+  a.max_iter = o.max_iter > 0 ? o.max_iter : 100000;
+  a.tol2 = o.tol * o.tol;
+  BLArgs<double> m{};
+  m.patches = a.patches;
+  m.erec = a.erec;
+  m.sh_info = a.sh_info;
+  m.node_end = a.node_end;
+  m.fixmask = a.fixmask;
+  m.coords = a.coords;
+  m.diagK = diag;
+  m.inst = a.inst;
+  m.iface = static_cast<const int4 *>(table("bl_iface"));
+  m.np = b->bl_np;
+  m.p8 = (b->bl_np + 7) / 8;
+  m.ent = b->bl_ent;
+  m.pn = b->bl_pn;
+  const int32_t *perm = static_cast<const int32_t *>(table("br_perm"));
+  std::vector<BLState> hs(n_state);
+  unsigned long long head[3];
+  BCHK_(hipMemcpyAsync(d_user, f, nu * sizeof(double), hipMemcpyHostToDevice, s));
+  {
+    const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(b->bl_np) / capacity), block);
+    BCHK_(hipEventRecord(b->ev0, s));
+    launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
+    bl_diag(2, m, b->bl_nif, diag, slots, s);
+    bl_inv_diag<double>(int64_t(nd), diag, invD, s);
+    launch_fill<double>(zero, int64_t(n_ent + n_words + 3), 0.0, s);
+    launch_fill<double>(d_x, int64_t(nv), 0.0, s);
+    launch_batch_resident(nr, b->br_degree, a, s);
+    BCHK_(hipGetLastError());
+    BCHK_(hipEventRecord(b->ev1, s));
+    launch_br_rhs_out(N, n_rhs, nr, perm, d_x, d_user, s);
+    BCHK_(hipMemcpyAsync(hs.data(), st, hs.size() * sizeof(BLState), hipMemcpyDeviceToHost, s));
+    BCHK_(hipMemcpyAsync(head, words, sizeof head, hipMemcpyDeviceToHost, s));
+    BCHK_(hipStreamSynchronize(s));
+  }
+  if (head[0]) {
+    if (!head[2] || b->br_degree == BR_DEGREE_MAX) {
+      b->br_off = true;
+      return FEMGPU_OK;
+    }
+    b->br_degree = BR_DEGREE_MAX;
+    return solve_resident_batch(ctx, b, n_rhs, nr, f, o, u_out, stats, solve_ms, ran);
+  }
+  *ran = true;
+  float ms = 0.f;
+  BCHK_(hipEventElapsedTime(&ms, b->ev0, b->ev1));
+  if (solve_ms) *solve_ms = ms;
+  if (u_out) {
+    BCHK_(hipMemcpyAsync(u_out, d_user, nu * sizeof(double), hipMemcpyDeviceToHost, s));
+    BCHK_(hipStreamSynchronize(s));
+  }
+  return report(ctx, b, n_rhs, nr, hs, stats);
 }
 
 // Lockstep solve (batch_ls.h) of n_rhs right-hand sides padded to nr.
@@ -232,12 +434,6 @@ int solve_lockstep(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, const doub
   int *d_count;
   const size_t ns = size_t(b->bl_slots) * nr * dim + 1;
 #define BL_BUF(name, n, ptr) BCHK_(bbuf(b, name, n, ptr))
-#define BCHK_(call)                                                                         \
-  do {                                                                                      \
-    hipError_t e_ = (call);                                                                 \
-    if (e_ != hipSuccess)                                                                   \
-      return ctx_fail(ctx, FEMGPU_E_HIP, (std::string(#call) + ": " + hipGetErrorString(e_)).c_str()); \
-  } while (0)
   BCHK_(bup(b, s, "bl_f", fi, &d_f));
   BL_BUF("bl_x64", nv, &x64);
   BL_BUF("bl_y64", nv, &y64);
@@ -355,7 +551,6 @@ int solve_lockstep(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, const doub
   BCHK_(hipMemcpyAsync(hs.data(), st, hs.size() * sizeof(BLState), hipMemcpyDeviceToHost, s));
   BCHK_(hipStreamSynchronize(s));
 #undef BL_BUF
-#undef BCHK_
   if (u_out)
     for (int64_t gq = 0; gq < b->total_nodes; ++gq) {
       const int64_t u = b->bl_perm[gq];
@@ -363,24 +558,10 @@ int solve_lockstep(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, const doub
         for (int c = 0; c < dim; ++c)
           u_out[(size_t(u) * n_rhs + rr) * dim + c] = xi[(size_t(gq) * nr + rr) * dim + c];
     }
-  int worst = FEMGPU_OK;
-  for (int i = 0; i < b->n_inst; ++i)
-    for (int rr = 0; rr < n_rhs; ++rr) {
-      const BLState &x = hs[size_t(i) * nr + rr];
-      const int status = x.state == 3 ? x.status : FEMGPU_E_MAXIT;
-      if (stats) {
-        femgpu_batch_stat &o2 = stats[size_t(i) * n_rhs + rr];
-        o2.status = status;
-        o2.iterations = x.state == 3 ? x.iters : std::max(x.it[0], x.it[1]) + 1;
-        o2.replacements = std::max(x.nrep, 0);
-        o2.rel_res = x.ff > 0.0 ? std::sqrt(x.rr / x.ff) : 0.0;
-      }
-      if (status != FEMGPU_OK && worst == FEMGPU_OK) worst = status;
-    }
-  if (worst != FEMGPU_OK)
-    return ctx_fail(ctx, worst, "some batch systems did not converge (see stats)");
-  return FEMGPU_OK;
+  return report(ctx, b, n_rhs, nr, hs, stats);
 }
+
+#undef BCHK_
 
 }  // namespace
 }  // namespace femgpu
@@ -613,6 +794,9 @@ int femgpu_batch_solve(femgpu_ctx *ctx, int n_rhs, const double *f, const femgpu
   hipStream_t s = femgpu::ctx_stream(ctx);
   BCHK(hipSetDevice(femgpu::ctx_device(ctx)));
   if (o.batch_schedule == FEMGPU_BATCH_LOCKSTEP) {
+    bool ran = false;
+    const int rc = femgpu::solve_resident_batch(ctx, b, n_rhs, nr, f, o, u_out, stats, solve_ms, &ran);
+    if (ran || rc != FEMGPU_OK) return rc;
     if (o.precision == FEMGPU_MIXED)
       return femgpu::solve_lockstep<float>(ctx, b, n_rhs, nr, f, o, u_out, stats, solve_ms);
     return femgpu::solve_lockstep<double>(ctx, b, n_rhs, nr, f, o, u_out, stats, solve_ms);

@@ -7,7 +7,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <condition_variable>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -23,16 +22,19 @@
 #include "femgpu.h"
 #include "batch.h"
 #include "batch_ls.h"
+#include "batch_res.h"
 #include "cg1.h"
 #include "femgpu_internal.h"
 #include "kernels.h"
 #include "noalloc.h"
 #include "resident.h"
+#include "resident_gate.h"
 
 using femgpu::CgScalars;
 using femgpu::DevMesh;
 using femgpu::MeshPlan;
 using femgpu::OpShift;
+using femgpu::ResidentGate;
 
 namespace {
 
@@ -705,49 +707,6 @@ int replay_until(femgpu_ctx *ctx, const Replay &exec, CgScalars *sc, int block, 
   return FEMGPU_OK;
 }
 
-// Resident launches (resident.h) wait for each other's workgroups, so all
-// workgroups of a launch must reach the device: alone they do when they fit
-// it; beside others they do while the launches' shares and the largest
-// workgroup together stay within it (then some compute unit always has room
-// for the next workgroup).  A launch that would not fit waits here for the
-// others to end.
-class ResidentGate {
- public:
-  ResidentGate(int device, double share, double block) : g_(gate(device)), share_(share) {
-    std::unique_lock<std::mutex> lock(g_.mu);
-    g_.cv.wait(lock, [&] {
-      return g_.n == 0 || g_.load + share + std::max(g_.block, block) <= 1.0;
-    });
-    ++g_.n;
-    g_.load += share;
-    g_.block = std::max(g_.block, block);
-  }
-  ~ResidentGate() {
-    {
-      std::lock_guard<std::mutex> lock(g_.mu);
-      g_.load -= share_;
-      if (--g_.n == 0) g_.load = g_.block = 0.0;
-    }
-    g_.cv.notify_all();
-  }
-
- private:
-  struct Gate {
-    std::mutex mu;
-    std::condition_variable cv;
-    int n = 0;
-    double load = 0.0, block = 0.0;
-  };
-  static Gate &gate(int device) {
-    static std::mutex mu;
-    static std::map<int, Gate> gates;
-    std::lock_guard<std::mutex> lock(mu);
-    return gates[device];
-  }
-  Gate &g_;
-  double share_;
-};
-
 // Whether this plan's PCG runs resident (all its workgroups on the chip).
 template <typename T>
 bool pcg_resident(const femgpu_ctx *ctx) {
@@ -1303,6 +1262,7 @@ int femgpu_create(femgpu_ctx **out, int device_ordinal) {
   HIPCHK(femgpu::prepare_cg1_kernels());
   HIPCHK(femgpu::prepare_bl_kernels());
   HIPCHK(femgpu::prepare_resident_kernels());
+  HIPCHK(femgpu::prepare_br_kernels());
   *out = c.release();
   return FEMGPU_OK;
 }

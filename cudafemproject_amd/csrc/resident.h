@@ -13,9 +13,10 @@ namespace femgpu {
 
 // The workgroups' exchange buffer for np patches, in 8-byte words: the tag of
 // the last exchange, the abort flag, the tags of the last trade of entries
-// (FP32, FP64; every launch advances its tags), and the tagged partials in EX_COPIES copies on pages of their own.  The interface
-// entries are tagged words too (res_entry_words).  Both are zeroed when they
-// are allocated or the plan changes, and after an aborted launch.
+// (FP32, FP64; every launch advances its tags), and the tagged partials in
+// EX_COPIES copies on pages of their own.  The interface entries are tagged
+// words too (res_entry_words).  Both are zeroed when they are allocated or the
+// plan changes, and after an aborted launch.
 constexpr int EX_COPIES = 8;
 constexpr size_t RES_HEAD = 512;
 __host__ __device__ inline size_t res_copy_words(int np) {
@@ -129,5 +130,10 @@ template <typename T>
 void launch_res_impl(const DevMesh &dm, const ResImpl<T> &a, hipStream_t s);
 
 hipError_t prepare_resident_kernels();
+
+// Workgroups of a kernel that a compute unit holds, and the device's units
+// (asked of the runtime once per kernel and LDS size).
+int blocks_per_cu(const void *fn, int threads, int lds);
+int compute_units(int device);
 
 }  // namespace femgpu

@@ -50,6 +50,7 @@
 #include "kernels.h"
 #include "patch_common.h"
 #include "resident.h"
+#include "resident_dev.h"
 
 namespace femgpu {
 
@@ -57,223 +58,7 @@ namespace {
 
 using namespace elem;
 using namespace patch;
-
-using u64 = unsigned long long;
-
-constexpr u64 WAIT_TICKS = 100000000ull;  // one second of the 100 MHz clock
-
-__device__ __forceinline__ void st_agent(u64 *p, u64 v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ u64 ld_agent(const u64 *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// A double as two tagged words, and back.
-__device__ __forceinline__ void tag_words(double v, unsigned tag, u64 (&w)[2]) {
-  const u64 b = static_cast<u64>(__double_as_longlong(v));
-  w[0] = (u64(tag) << 32) | (b & 0xffffffffull);
-  w[1] = (u64(tag) << 32) | (b >> 32);
-}
-__device__ __forceinline__ double untag(const u64 (&w)[2]) {
-  return __longlong_as_double(static_cast<long long>((w[1] << 32) | (w[0] & 0xffffffffull)));
-}
-
-// A bounded wait: true once the caller should give up (another workgroup
-// did, or WAIT_TICKS have passed since the 256th look).
-struct Patience {
-  u64 *abort;
-  u64 start = 0;
-  __device__ __forceinline__ bool over(int spin) {
-    if ((spin & 255) != 255) return false;
-    const u64 now = wall_clock64();
-    if (start == 0) start = now;
-    if (ld_agent(abort) == 0 && now - start <= WAIT_TICKS) return false;
-    st_agent(abort, 1);
-    return true;
-  }
-};
-
-// Interface sums travel as entries (femgpu_internal.h): the bits of DIM values
-// in words of 48 under a 16-bit tag (a third fewer words than 32 under 32;
-// the traffic of some hundred kilobytes a step per workgroup is what bounds a
-// trade).  The tag counts the trades through a set of entries, and every trade
-// writes them all: a stale word carries the tag before the one awaited.  Word
-// w of 64 consecutive entries lie together.
-template <typename T, int DIM>
-constexpr int EW = res_entry_size(DIM, int(sizeof(T)));
-
-template <typename T, int DIM>
-__device__ __forceinline__ size_t entry_word(unsigned e, int w) {
-  return (size_t(e >> 6) * EW<T, DIM> + w) * 64 + (e & 63u);
-}
-
-template <typename T>
-__device__ __forceinline__ void to_bits(T v, unsigned *u) {
-  if constexpr (sizeof(T) == 8) {
-    const u64 b = static_cast<u64>(__double_as_longlong(v));
-    u[0] = unsigned(b);
-    u[1] = unsigned(b >> 32);
-  } else {
-    u[0] = __float_as_uint(v);
-  }
-}
-template <typename T>
-__device__ __forceinline__ T from_bits(const unsigned *u) {
-  if constexpr (sizeof(T) == 8)
-    return __longlong_as_double(static_cast<long long>((u64(u[1]) << 32) | u[0]));
-  else
-    return __uint_as_float(u[0]);
-}
-
-template <typename T, int DIM>
-__device__ __forceinline__ void send_entry(u64 *entries, unsigned e, unsigned tag, const T *v) {
-  constexpr int W = EW<T, DIM>, U = sizeof(T) / 4;
-  unsigned u[DIM * U + 2];
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) to_bits<T>(v[c], &u[c * U]);
-  u[DIM * U] = u[DIM * U + 1] = 0u;
-  // 16-bit unit j of the payload: half j & 1 of u[j >> 1]
-  auto unit = [&](int j) { return j >= 2 * DIM * U ? 0u : (j & 1) ? u[j >> 1] >> 16 : u[j >> 1] & 0xffffu; };
-#pragma unroll
-  for (int w = 0; w < W; ++w)
-    st_agent(&entries[entry_word<T, DIM>(e, w)],
-             (u64((tag << 16) | unit(3 * w + 2)) << 32) | (unit(3 * w + 1) << 16) | unit(3 * w));
-}
-
-// Entry e into v; false when the wait ran out.
-template <typename T, int DIM>
-__device__ __forceinline__ bool recv_entry(const u64 *entries, unsigned e, unsigned tag, u64 *abort,
-                                           T *v) {
-  constexpr int W = EW<T, DIM>, U = sizeof(T) / 4;
-  u64 h[W];
-  Patience wait{abort};
-  for (int spin = 0;; ++spin) {
-    bool all = true;
-#pragma unroll
-    for (int w = 0; w < W; ++w) h[w] = ld_agent(&entries[entry_word<T, DIM>(e, w)]);
-#pragma unroll
-    for (int w = 0; w < W; ++w) all = all && unsigned(h[w] >> 48) == (tag & 0xffffu);
-    if (all) break;
-    if (wait.over(spin)) return false;
-  }
-  auto unit = [&](int j) { return unsigned(h[j / 3] >> (16 * (j % 3))) & 0xffffu; };
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) {
-    unsigned u[U];
-#pragma unroll
-    for (int i = 0; i < U; ++i) u[i] = unit(2 * (c * U + i)) | (unit(2 * (c * U + i) + 1) << 16);
-    v[c] = from_bits<T>(u);
-  }
-  return true;
-}
-
-// The exchange words lie in EX_COPIES copies, each read by every
-// EX_COPIES-th workgroup (a copy per XCD): all workgroups polling one copy
-// of a few kilobytes queue up at the memory channels that hold it.
-struct Exchange {
-  u64 *words;      // copy 0 of this exchange: [2 * NV][np]
-  size_t stride;   // words from copy to copy
-  u64 *abort;      // nonzero: a workgroup gave up waiting
-  int np, copy;    // copy: the one this workgroup reads
-};
-
-// Sums of NV values over the workgroup's threads, valid in wave 0 (the same
-// bits in every lane; fixed order).  s_red: NV * PT / 64 doubles that no
-// thread still reads or writes for another sum.
-template <int PT, int NV>
-__device__ __forceinline__ void sum_to_wave0(double (&v)[NV], double *s_red) {
-  constexpr int W = PT / 64;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
-  if (l == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) s_red[k * W + w] = v[k];
-  __syncthreads();
-  if (w == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      // (at most 16 waves: one row, its sum in every lane of the row)
-      double q = s_red[k * W + min(l & 15, W - 1)];
-      if ((l & 15) >= W) q = 0.0;
-      q += dpp_f64<0xB1>(q);
-      q += dpp_f64<0x4E>(q);
-      q += dpp_f64<0x141>(q);
-      q += dpp_f64<0x140>(q);
-      v[k] = q;
-    }
-}
-
-// Wave 0 publishes the workgroup's NV values under `tag`.
-template <int NV>
-__device__ __forceinline__ void publish(const Exchange &x, int pid, unsigned tag,
-                                        const double (&v)[NV]) {
-  const int t = threadIdx.x;
-  if (t < 2 * NV * EX_COPIES) {
-    const int k = t % (2 * NV), copy = t / (2 * NV);
-    double d = v[0];
-#pragma unroll
-    for (int i = 1; i < NV; ++i) d = (k >> 1) == i ? v[i] : d;
-    u64 w[2];
-    tag_words(d, tag, w);
-    st_agent(&x.words[copy * x.stride + size_t(k) * x.np + pid], (k & 1) ? w[1] : w[0]);
-  }
-}
-
-// Wave 0 gathers every workgroup's NV values of `tag` (NB loads of each lane
-// in flight) and sums them in a fixed order; the sums reach every thread
-// through s_bc (NV doubles) behind a barrier, which also ends the wait for
-// the entries.  alone: v is the sum already.  False when a workgroup gave up
-// (or *s_flag was set).
-template <int NV>
-__device__ __forceinline__ bool gather(const Exchange &x, unsigned tag, double (&v)[NV],
-                                       double *s_bc, int *s_flag, bool alone) {
-  constexpr int NB = 4;
-  if (threadIdx.x < 64 && !alone) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = 0.0;
-    const u64 *words = x.words + x.copy * x.stride;
-    bool ok = true;
-    for (int i0 = threadIdx.x; ok && i0 < x.np; i0 += 64 * NB) {
-      u64 h[NB][NV][2];
-      Patience wait{x.abort};
-      for (int spin = 0;; ++spin) {
-        bool all = true;
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int k = 0; k < 2 * NV; ++k)
-            if (i0 + 64 * i < x.np)
-              h[i][k >> 1][k & 1] = ld_agent(&words[size_t(k) * x.np + i0 + 64 * i]);
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int k = 0; k < 2 * NV; ++k)
-            if (i0 + 64 * i < x.np) all = all && unsigned(h[i][k >> 1][k & 1] >> 32) == tag;
-        if (all) break;
-        if (wait.over(spin)) {
-          ok = false;
-          break;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i0 + 64 * i < x.np)
-#pragma unroll
-          for (int k = 0; k < NV; ++k) v[k] += untag(h[i][k]);
-    }
-    if (!ok) *s_flag = 1;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
-  }
-  if (threadIdx.x == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) s_bc[k] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = s_bc[k];
-  return *s_flag == 0;
-}
+using namespace resident;
 
 // LDS of a resident workgroup: node coordinates and vector, `comps` components
 // of the node-sorted element entries, the interface nodes' contributions
@@ -314,30 +99,6 @@ struct ResMesh {
   const uint16_t *out_src, *in_pos, *src_end, *own_pos;
   int n_in_max, n_src_max;
 };
-
-// Sum of the entry run [b0, b1) (multiples of 4) in a fixed order.
-template <typename T>
-__device__ __forceinline__ T run_sum(const T *s_res, int b0, int b1) {
-  using V4 = typename Vec4<T>::type;
-  const V4 *rp = reinterpret_cast<const V4 *>(s_res) + (b0 >> 2);
-  T s0 = T(0), s1 = T(0), s2 = T(0), s3 = T(0);
-  const int n4 = (b1 - b0) >> 2;
-  for (int m = n4 >> 1; m > 0; --m, rp += 2) {
-    const V4 u = rp[0], v = rp[1];
-    s0 += Vec4<T>::get(u, 0) + Vec4<T>::get(v, 0);
-    s1 += Vec4<T>::get(u, 1) + Vec4<T>::get(v, 1);
-    s2 += Vec4<T>::get(u, 2) + Vec4<T>::get(v, 2);
-    s3 += Vec4<T>::get(u, 3) + Vec4<T>::get(v, 3);
-  }
-  if (n4 & 1) {
-    const V4 u = rp[0];
-    s0 += Vec4<T>::get(u, 0);
-    s1 += Vec4<T>::get(u, 1);
-    s2 += Vec4<T>::get(u, 2);
-    s3 += Vec4<T>::get(u, 3);
-  }
-  return (s0 + s1) + (s2 + s3);
-}
 
 // One patch in one workgroup of PT threads for a whole launch.  NE = 1: one
 // element and one DOF per thread (thread t: node t / DIM, component t % DIM),
@@ -1025,8 +786,20 @@ FEMGPU_RES_KERNEL(k_dyn_resident, DynKernel)
 FEMGPU_RES_KERNEL(k_impl_resident, ImplKernel)
 #undef FEMGPU_RES_KERNEL
 
-// Workgroups of a kernel that a compute unit holds, and the device's units
-// (asked of the runtime once per kernel and LDS size).
+// Whether a kernel of this form fits the plan, a workgroup per compute unit.
+bool fits(const DevMesh &dm, int device, const void *fn, int lds, ResFit *fit) {
+  const int cu = compute_units(device);
+  if (cu < 1 || lds > RES_LDS_MAX) return false;
+  const int per = blocks_per_cu(fn, res_form(dm).threads, lds);
+  const int grid = 8 * ((dm.np + 7) / 8);
+  if (per < 1 || grid > cu) return false;
+  fit->block = 1.0 / per;
+  fit->share = double(grid) / (double(per) * cu);
+  return true;
+}
+
+}  // namespace
+
 int blocks_per_cu(const void *fn, int threads, int lds) {
   static std::mutex mu;
   static std::map<std::tuple<const void *, int, int>, int> seen;
@@ -1057,20 +830,6 @@ int compute_units(int device) {
   seen[device] = n;
   return n;
 }
-
-// Whether a kernel of this form fits the plan, a workgroup per compute unit.
-bool fits(const DevMesh &dm, int device, const void *fn, int lds, ResFit *fit) {
-  const int cu = compute_units(device);
-  if (cu < 1 || lds > RES_LDS_MAX) return false;
-  const int per = blocks_per_cu(fn, res_form(dm).threads, lds);
-  const int grid = 8 * ((dm.np + 7) / 8);
-  if (per < 1 || grid > cu) return false;
-  fit->block = 1.0 / per;
-  fit->share = double(grid) / (double(per) * cu);
-  return true;
-}
-
-}  // namespace
 
 template <typename T>
 bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit) {

@@ -1,0 +1,54 @@
+// resident_gate.h -- admission of resident launches to a device.
+#pragma once
+
+#include <algorithm>
+#include <condition_variable>
+#include <map>
+#include <mutex>
+
+namespace femgpu {
+
+// Resident launches (resident.h) wait for each other's workgroups, so all
+// workgroups of a launch must reach the device: alone they do when they fit
+// it; beside others they do while the launches' shares and the largest
+// workgroup together stay within it (then some compute unit always has room
+// for the next workgroup).  A launch that would not fit waits here for the
+// others to end.
+class ResidentGate {
+ public:
+  ResidentGate(int device, double share, double block) : g_(gate(device)), share_(share) {
+    std::unique_lock<std::mutex> lock(g_.mu);
+    g_.cv.wait(lock, [&] {
+      return g_.n == 0 || g_.load + share + std::max(g_.block, block) <= 1.0;
+    });
+    ++g_.n;
+    g_.load += share;
+    g_.block = std::max(g_.block, block);
+  }
+  ~ResidentGate() {
+    {
+      std::lock_guard<std::mutex> lock(g_.mu);
+      g_.load -= share_;
+      if (--g_.n == 0) g_.load = g_.block = 0.0;
+    }
+    g_.cv.notify_all();
+  }
+
+ private:
+  struct Gate {
+    std::mutex mu;
+    std::condition_variable cv;
+    int n = 0;
+    double load = 0.0, block = 0.0;
+  };
+  static Gate &gate(int device) {
+    static std::mutex mu;
+    static std::map<int, Gate> gates;
+    std::lock_guard<std::mutex> lock(mu);
+    return gates[device];
+  }
+  Gate &g_;
+  double share_;
+};
+
+}  // namespace femgpu

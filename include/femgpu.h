@@ -66,9 +66,12 @@ enum {
 
 /* Schedules of femgpu_batch_solve (no counterpart in the reference). */
 enum {
-  FEMGPU_BATCH_LOCKSTEP = 0,   /* every iteration of every system in two
-                                  grid-wide launches (graph replays): each
-                                  instance spread over the whole GPU        */
+  FEMGPU_BATCH_LOCKSTEP = 0,   /* every instance spread over many compute
+                                  units: 2D, one launch in which an
+                                  instance's workgroups stay on the chip
+                                  until it is done (FP64 throughout, also
+                                  for MIXED); else every iteration of every
+                                  system in two grid-wide launches          */
   FEMGPU_BATCH_PERSISTENT = 1  /* one workgroup runs one instance's whole
                                   solve; the batch is one launch             */
 };
@@ -272,10 +275,9 @@ int femgpu_compliance_grad(femgpu_ctx *ctx, const femgpu_solve_opts *opts, doubl
 /* --- batched independent static solves ----------------------------------------
  * No counterpart in the reference (it solves one problem per process run).
  * Many small meshes ("instances"), each with its own material, constraints
- * and 1..4 right-hand sides, solved in ONE persistent launch: one workgroup
- * runs an instance's whole Jacobi-PCG (the algorithm of gpuPCG_EbE_vec,
- * femfunc.cpp:25-128, with the relative-residual stopping rule), largest
- * instances first.  Meshes are concatenated: instance i owns user nodes
+ * and 1..4 right-hand sides, solved together by Jacobi-PCG (the algorithm of
+ * gpuPCG_EbE_vec, femfunc.cpp:25-128, with the relative-residual stopping
+ * rule), largest instances first.  Meshes are concatenated: instance i owns user nodes
  * [node_off[i], node_off[i+1]) and elements [elem_off[i], elem_off[i+1]);
  * element node ids and constraint node ids are instance-local. */
 typedef struct {
