@@ -263,17 +263,6 @@ int upload(femgpu_ctx *ctx, const std::string &name, const std::vector<T> &h, T 
   return FEMGPU_OK;
 }
 
-// user node vector (nn x dim) -> internal order
-std::vector<double> to_internal(const femgpu_ctx *ctx, const double *u) {
-  const int d = ctx->dim;
-  std::vector<double> v(size_t(ctx->nn) * d);
-  for (int64_t i = 0; i < ctx->nn; ++i) {
-    const int64_t s = ctx->plan.node_perm[i];
-    for (int c = 0; c < d; ++c) v[size_t(i) * d + c] = u[size_t(s) * d + c];
-  }
-  return v;
-}
-
 // Host node vector (user order) -> device vector `name` in internal order,
 // permuted on the device.  The caller synchronises the stream before the
 // host vector may change.
@@ -2449,40 +2438,11 @@ int femgpu_get_traces(femgpu_ctx *ctx, double *out, int64_t capacity, int *n_sam
 
 namespace {
 
-// Per-DOF assembled mass (user order).  lumped: 2D rho A/3, 3D rho V/12
-// (reference) or rho V/4 (physical); consistent diagonal: 2D rho A/6, 3D rho V/24.
-std::vector<double> host_mass(const femgpu_ctx *ctx, double rho, bool lumped, int conv) {
-  const int d = ctx->dim, npe = d + 1;
-  std::vector<double> m(size_t(ctx->nn) * d, 0.0);
-  for (int64_t e = 0; e < ctx->ne; ++e) {
-    const int32_t *en = &ctx->elems[size_t(e) * npe];
-    double meas;
-    if (d == 2) {
-      const double *a = &ctx->nodes[size_t(en[0]) * 2], *b = &ctx->nodes[size_t(en[1]) * 2],
-                   *c = &ctx->nodes[size_t(en[2]) * 2];
-      meas = 0.5 * std::fabs((b[0] - a[0]) * (c[1] - a[1]) - (b[1] - a[1]) * (c[0] - a[0]));
-    } else {
-      const double *a = &ctx->nodes[size_t(en[0]) * 3], *b = &ctx->nodes[size_t(en[1]) * 3],
-                   *c = &ctx->nodes[size_t(en[2]) * 3], *q = &ctx->nodes[size_t(en[3]) * 3];
-      const double e1[3] = {b[0] - a[0], b[1] - a[1], b[2] - a[2]};
-      const double e2[3] = {c[0] - a[0], c[1] - a[1], c[2] - a[2]};
-      const double e3[3] = {q[0] - a[0], q[1] - a[1], q[2] - a[2]};
-      meas = std::fabs(e1[0] * (e2[1] * e3[2] - e2[2] * e3[1]) -
-                       e1[1] * (e2[0] * e3[2] - e2[2] * e3[0]) +
-                       e1[2] * (e2[0] * e3[1] - e2[1] * e3[0])) / 6.0;
-    }
-    const double mass = rho * meas;
-    double per;
-    if (d == 2)
-      per = lumped ? mass / 3.0 : mass / 6.0;
-    else if (lumped)
-      per = conv == FEMGPU_MASS_PHYSICAL ? mass / 4.0 : mass / 12.0;
-    else
-      per = mass / 24.0;
-    for (int a = 0; a < npe; ++a)
-      for (int c = 0; c < d; ++c) m[size_t(en[a]) * d + c] += per;
-  }
-  return m;
+// Divisor of an element's mass per corner.  lumped: 2D 3, 3D 12 (reference) or 4
+// (physical); consistent diagonal: 2D 6, 3D 24.
+double mass_div(int dim, bool lumped, int conv) {
+  if (dim == 2) return lumped ? 3.0 : 6.0;
+  return !lumped ? 24.0 : conv == FEMGPU_MASS_PHYSICAL ? 4.0 : 12.0;
 }
 
 template <typename T>
@@ -2536,30 +2496,26 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   std::vector<double> ffile, funit;
   host_rhs(ctx, false, ffile);
   host_rhs(ctx, true, funit);
-  std::vector<double> ff_i = to_internal(ctx, ffile.data()), fu_i = to_internal(ctx, funit.data());
-  std::vector<T> ff_t(ff_i.begin(), ff_i.end()), fu_t(fu_i.begin(), fu_i.end());
   const int mconv = o.mass_convention;
-  std::vector<double> mass_l = host_mass(ctx, o.rho, true, mconv);
-  std::vector<double> ml_i = to_internal(ctx, mass_l.data());
-  std::vector<T> invM(nd, T(0)), mlump(nd, T(0));
-  for (size_t i = 0; i < nd; ++i) {
-    mlump[i] = T(ml_i[i]);
-    invM[i] = ml_i[i] > 0 ? T(1.0 / ml_i[i]) : T(0);
-  }
   const std::string tg = sizeof(T) == 8 ? "d64" : "d32";
   T *dd, *dd2, *dv, *da, *dy, *dpart, *dff, *dfu, *dinvM, *dml;
-  double *dcf, *dcu, *dmaxp, *dmax;
+  double *dcf, *dcu, *dmaxp, *dmax, *dmass, *dmslots;
   int *dstep;
   if ((st = dbuf(ctx, tg + "d", nd, &dd)) || (st = dbuf(ctx, tg + "d2", nd, &dd2)) ||
       (st = dbuf(ctx, tg + "v", nd, &dv)) ||
       (st = dbuf(ctx, tg + "a", nd, &da)) || (st = dbuf(ctx, tg + "y", nd, &dy)) ||
       (st = dbuf(ctx, tg + "part", size_t(ctx->plan.n_slots) * d + 1, &dpart)) ||
-      (st = upload(ctx, tg + "ff", ff_t, &dff)) || (st = upload(ctx, tg + "fu", fu_t, &dfu)) ||
-      (st = upload(ctx, tg + "invM", invM, &dinvM)) || (st = upload(ctx, tg + "ml", mlump, &dml)) ||
+      (st = upload_nodes(ctx, tg + "ff", ffile.data(), &dff)) ||
+      (st = upload_nodes(ctx, tg + "fu", funit.data(), &dfu)) ||
+      (st = dbuf(ctx, tg + "invM", nd, &dinvM)) || (st = dbuf(ctx, tg + "ml", nd, &dml)) ||
+      (st = dbuf(ctx, "dyn_mass", size_t(ctx->nn), &dmass)) ||
+      (st = dbuf(ctx, "dyn_mslots", size_t(ctx->plan.n_slots) + 1, &dmslots)) ||
       (st = upload(ctx, "dyn_cf", cfile, &dcf)) || (st = upload(ctx, "dyn_cu", cunit, &dcu)) ||
       (st = dbuf(ctx, "dyn_step", 1, &dstep)) || (st = dbuf(ctx, "dyn_maxp", 256, &dmaxp)) ||
       (st = dbuf(ctx, "dyn_max", 1, &dmax)))
     return st;
+  femgpu::launch_mass<T>(ctx->dm, o.rho, mass_div(d, true, mconv), dmass, dmslots, dml, dinvM,
+                         ctx->stream);
   // receivers
   const int nrec = int(ctx->recv.size());
   const int every = ctx->recv_every;
@@ -2764,11 +2720,10 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       femgpu::launch_inv_diag<T>(ctx->dm, diagK_t, ceff, cmass, dml, invA, ctx->stream);
     } else {
       // reference: operator K, preconditioner cK diag(K) + diag(M_consistent)
-      std::vector<double> mc = host_mass(ctx, o.rho, false, mconv);
-      std::vector<double> mc_i = to_internal(ctx, mc.data());
-      std::vector<T> mc_t(mc_i.begin(), mc_i.end());
       T *dmc;
-      if ((st = upload(ctx, tg + "mc", mc_t, &dmc))) return st;
+      if ((st = dbuf(ctx, tg + "mc", nd, &dmc))) return st;
+      femgpu::launch_mass<T>(ctx->dm, o.rho, mass_div(d, false, mconv), dmass, dmslots, dmc,
+                             static_cast<T *>(nullptr), ctx->stream);
       femgpu::launch_inv_diag<T>(ctx->dm, diagK_t, ceff, T(1), dmc, invA, ctx->stream);
     }
     w.invD = invA;

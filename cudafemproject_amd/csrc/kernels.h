@@ -108,6 +108,12 @@ void launch_matvec_patch(const DevMesh &dm, const T *x, T *y, T *partial, hipStr
 template <typename T>
 void launch_diag(const DevMesh &dm, T *d, T *partial, hipStream_t s);
 
+// Assembled mass per DOF from element masses rho |e| / div per corner: lumped,
+// and its reciprocal into inv unless null.  mass (nodes), slots: FP64 scratch.
+template <typename T>
+void launch_mass(const DevMesh &dm, double rho, double div, double *mass, double *slots, T *lumped,
+                 T *inv, hipStream_t s);
+
 // invD = 1 / (cK*diag + cM*m) (0 where the sum is 0).
 template <typename T>
 void launch_inv_diag(const DevMesh &dm, const T *diag, T cK, T cM, const T *m, T *invD,
