@@ -215,12 +215,28 @@ int plan_default(int dim, int64_t n_nodes, const double *nodes, int64_t n_elems,
   // (a patch of 768 elements has more than 256 nodes in 2D and often in 3D:
   // from half the elements on, 256 threads may give more than NP patches)
   if (n_elems > NP * 768 / 2 && n_elems <= NP * 1536)
-    side = std::thread([&] {
-      std::string m;
-      wide_st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 512, wide, m);
-    });
-  const int st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 256, plan, msg);
-  if (side.joinable()) side.join();
+    try {
+      side = std::thread([&] {
+        std::string m;
+        try {
+          wide_st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 512, wide, m);
+        } catch (...) {
+          wide_st = FEMGPU_E_NOMEM;
+        }
+      });
+    } catch (...) {  // (no thread: one plan)
+    }
+  struct Join {
+    std::thread &t;
+    ~Join() {
+      if (t.joinable()) t.join();
+    }
+  };
+  int st;
+  {
+    const Join join{side};
+    st = plan_mesh(dim, n_nodes, nodes, n_elems, elems, 0, 256, plan, msg);
+  }
   *threads = 256;
   if (st == FEMGPU_OK && wide_st == FEMGPU_OK && int64_t(plan.patches.size()) > NP &&
       int64_t(wide.patches.size()) <= NP) {
