@@ -29,6 +29,7 @@
 #include "noalloc.h"
 #include "resident.h"
 #include "resident_gate.h"
+#include "strip.h"
 
 using femgpu::CgScalars;
 using femgpu::DevMesh;
@@ -117,6 +118,7 @@ struct femgpu_ctx {
   int recv_quantity = 0, recv_every = 1;
   std::vector<double> traces;           // last run: n_samples x n_recv x dim
   int n_samples = 0;
+  std::vector<int32_t> strip_elems;  // internal elements of the strips (StripPlan), empty: none
   MeshPlan plan;
   DevMesh dm;
   std::map<std::string, DevBuf> bufs;
@@ -242,6 +244,24 @@ int plan_default(int dim, int64_t n_nodes, const double *nodes, int64_t n_elems,
       int64_t(wide.patches.size()) <= NP) {
     plan = std::move(wide);
     *threads = 512;
+    return st;
+  }
+  // Launch-per-kernel plans: as many elements as leave every patch a strip per
+  // thread (strip.h).  Strips of a ragged or jittered grid are a tenth
+  // shorter than a regular one's; a fifth wave for the rest costs the FP64
+  // kernels the fourth workgroup per compute unit (use_strips; 47^3 hexes: FP64
+  // 25.0 -> 23.9 us per iteration, matvec 21.1 -> 15.8, planned twice in 242
+  // instead of 113 ms).
+  if (st == FEMGPU_OK && int64_t(plan.patches.size()) > NP) {
+    femgpu::StripPlan x;
+    const int stride = 256 / 4 * 5;
+    if (femgpu::build_strips(plan, 256, stride, x) && x.strips_used > 256) {
+      MeshPlan cut;
+      std::string m;
+      if (plan_mesh(dim, n_nodes, nodes, n_elems, elems, 768 * 256 / x.strips_used * 31 / 32, 256, cut, m) == FEMGPU_OK &&
+          femgpu::build_strips(cut, 256, stride, x) && x.strips_used <= 256)
+        plan = std::move(cut);
+    }
   }
   return st;
 }
@@ -324,6 +344,31 @@ void lame(int dim, double E, double nu, double &lam, double &mu) {
   lam = dim == 3 ? E * nu / ((1.0 + nu) * (1.0 - 2.0 * nu)) : E * nu / (1.0 - nu * nu);
 }
 
+// The element scales (internal order) strip by strip.
+int strip_scales(femgpu_ctx *ctx, const std::vector<double> &s64, const std::vector<float> &s32) {
+  if (!femgpu::has_strips(ctx->dm)) return FEMGPU_OK;
+  const size_t stride = size_t(ctx->dm.strip_stride);
+  std::vector<double> v64(ctx->strip_elems.size(), 1.0);
+  std::vector<float> v32(v64.size(), 1.f);
+  for (size_t p = 0; p < size_t(ctx->dm.np); ++p)
+    for (size_t i = 0; i < stride; ++i)
+      for (size_t k = 0; k < femgpu::STRIP_ELEMS; ++k) {
+        const int32_t e = ctx->strip_elems[(p * stride + i) * 3 + k];
+        if (e < 0) continue;
+        v64[(p * 3 + k) * stride + i] = s64[size_t(e)];
+        v32[(p * 3 + k) * stride + i] = s32[size_t(e)];
+      }
+  double *p64;
+  float *p32;
+  int st;
+  if ((st = upload(ctx, "strip_escale64", v64, &p64)) || (st = upload(ctx, "strip_escale32", v32, &p32)))
+    return st;
+  HIPCHK(hipStreamSynchronize(ctx->stream));  // v64, v32 go out of scope
+  ctx->dm.strip_escale64 = p64;
+  ctx->dm.strip_escale32 = p32;
+  return FEMGPU_OK;
+}
+
 int ensure_material(femgpu_ctx *ctx) {
   if (!ctx->dirty_mat) return FEMGPU_OK;
   lame(ctx->dim, ctx->E, ctx->nu, ctx->dm.lam, ctx->dm.mu);
@@ -341,9 +386,10 @@ int ensure_material(femgpu_ctx *ctx) {
     if (st) return st;
     ctx->dm.escale64 = p64;
     ctx->dm.escale32 = p32;
+    if ((st = strip_scales(ctx, s64, s32))) return st;
   } else {
-    ctx->dm.escale64 = nullptr;
-    ctx->dm.escale32 = nullptr;
+    ctx->dm.escale64 = ctx->dm.strip_escale64 = nullptr;
+    ctx->dm.escale32 = ctx->dm.strip_escale32 = nullptr;
   }
   ctx->dirty_mat = false;
   ctx->dirty_diag = true;
@@ -1095,6 +1141,12 @@ int matvec_noalloc_t(femgpu_ctx *ctx, const double *x, double *y) {
   T *xi = reinterpret_cast<T *>(base);
   T *yi = reinterpret_cast<T *>(base + vec);
   T *part = reinterpret_cast<T *>(base + 2 * vec);
+  // straight from x and to y where the plan has strips and the two don't overlap
+  if (femgpu::has_strips(ctx->dm) && (x + nd <= y || y + nd <= x)) {
+    femgpu::launch_strip_matvec_user<T>(ctx->dm, ctx->d_node_perm, x, y, part, ctx->stream);
+    HIPCHK(hipGetLastError());
+    return FEMGPU_OK;
+  }
   femgpu::launch_gather_user<T>(ctx->nn, ctx->dim, ctx->d_node_perm, x, xi, ctx->stream);
   femgpu::launch_matvec<T>(ctx->dm, xi, yi, part, ctx->stream);
   femgpu::launch_scatter_user<T>(ctx->nn, ctx->dm.n_active, ctx->dim, ctx->d_node_perm, yi, y,
@@ -1222,6 +1274,36 @@ int upload_plan(femgpu_ctx *ctx) {
       dm.x_entries = x.n_entries;
     }
   }
+  ctx->strip_elems.clear();
+  if (dm.np > femgpu::RES_PATCHES_MAX && threads <= 512) {
+    femgpu::StripPlan x;
+    const int stride = threads / 4 * 5;
+    if (femgpu::build_strips(P, threads, stride, x)) {
+      std::vector<int32_t> user(size_t(dm.np) * threads, 0);
+      for (size_t p = 0; p < P.patches.size(); ++p) {
+        const femgpu::PatchInfo &Q = P.patches[p];
+        for (int k = 0; k < Q.n_own + Q.n_sh; ++k)
+          user[p * threads + k] =
+              P.node_perm[k < Q.n_own ? Q.own_start + k : P.sh_gid[size_t(Q.sh_start + k - Q.n_own)]];
+      }
+      uint32_t *r, *r2;
+      uint16_t *pe;
+      int32_t *pu;
+      if ((st = upload(ctx, "strip_rec", x.rec, &r)) || (st = upload(ctx, "strip_rec2", x.rec2, &r2)) ||
+          (st = upload(ctx, "strip_pend", x.pend, &pe)) || (st = upload(ctx, "puser", user, &pu)))
+        return st;
+      HIPCHK(hipStreamSynchronize(ctx->stream));  // x, user go out of scope
+      ctx->strip_elems = std::move(x.elems);
+      dm.strip_rec = reinterpret_cast<const uint4 *>(r);
+      dm.strip_rec2 = r2;
+      dm.strip_pend = pe;
+      dm.puser = pu;
+      dm.strip_stride = stride;
+      // (a wave per 64 strips, and a thread per node)
+      dm.strip_threads = (std::max(x.strips_used, dm.pn) + 63) & ~63;
+      dm.strip_ent = (x.ent_used + 3) & ~3;
+    }
+  }
   std::vector<double> c64(size_t(n_nodes) * dim);
   std::vector<float> c32(c64.size());
   for (int64_t i = 0; i < n_nodes; ++i)
@@ -1268,6 +1350,7 @@ int femgpu_create(femgpu_ctx **out, int device_ordinal) {
   HIPCHK(femgpu::prepare_bl_kernels());
   HIPCHK(femgpu::prepare_resident_kernels());
   HIPCHK(femgpu::prepare_br_kernels());
+  HIPCHK(femgpu::prepare_strip_kernels());
   *out = c.release();
   return FEMGPU_OK;
 }

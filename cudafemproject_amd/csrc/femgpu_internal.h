@@ -99,6 +99,26 @@ bool stride_records(const MeshPlan &plan, std::vector<uint32_t> &rec,
 void pack_patch_nodes(const MeshPlan &plan, int stride, std::vector<int32_t> &pgid,
                       std::vector<int32_t> &pslot, std::vector<uint16_t> &pend);
 
+// Strips: runs of up to STRIP_ELEMS elements of a patch in which element k has
+// the strip's nodes k .. k + dim, so that consecutive elements share a face and
+// a strip of three tetrahedra has 6 nodes where its elements have 12 corners:
+// half of the LDS traffic of a patch product and half of its entries.  One
+// thread per strip.
+constexpr int STRIP_ELEMS = 3;
+struct StripPlan {
+  int strips_used = 0;            // most strips of a patch
+  int ent_used = 0;               // longest padded entry list of a patch
+  // strip s of patch p at p * stride + s, zero past
+  // the patch's strips.  Words: l0 | l1 << 10 | l2 << 20 | elements << 30,
+  // l3 | l4 << 10 | l5 << 20, then p0 | p1 << 14, p2 | p3 << 14 (rec, 4 words)
+  // and p4 | p5 << 14 (rec2): local nodes and entry positions of its nodes.
+  std::vector<uint32_t> rec, rec2;
+  std::vector<uint16_t> pend;     // per patch node at node_stride: end of its run
+  std::vector<int32_t> elems;     // internal elements, 3 per strip, -1 past its length
+};
+// False when a patch has more strips than `stride`.
+bool build_strips(const MeshPlan &plan, int node_stride, int stride, StripPlan &strips);
+
 // What a patch sends and receives when every patch finishes its own copy of
 // the interface nodes (resident.hip).  For every interface node each patch
 // holding it sends its partial sum to each of the others: one entry per

@@ -50,6 +50,15 @@ struct DevMesh {
   const uint16_t *x_src_end = nullptr, *x_own_pos = nullptr;
   int x_in_max = 0, x_src_max = 0;
   int64_t x_entries = 0;
+  // strips (StripPlan, strip.h; null: none): records, run ends, the element
+  // scales strip by strip, and the user's node ids per patch node
+  const uint4 *strip_rec = nullptr;
+  const uint32_t *strip_rec2 = nullptr;
+  const uint16_t *strip_pend = nullptr;
+  const double *strip_escale64 = nullptr;
+  const float *strip_escale32 = nullptr;
+  const int32_t *puser = nullptr;
+  int strip_stride = 0, strip_threads = 0, strip_ent = 0;
 };
 
 // Scalars of one PCG run, device resident.  Iteration j of the fused

@@ -29,6 +29,7 @@
 #include "element.h"
 #include "kernels.h"
 #include "patch_common.h"
+#include "strip.h"
 
 namespace femgpu {
 
@@ -1294,6 +1295,10 @@ int lds_bytes(int dim, int elem_bytes, int pn, int ent) {
 
 template <typename T>
 void launch_matvec_patch(const DevMesh &dm, const T *x, T *y, T *partial, hipStream_t s) {
+  if (use_strips<T>(dm)) {
+    launch_strip_matvec<T>(dm, x, y, partial, s);
+    return;
+  }
   PatchArgs<T> a = patch_args<T>(dm);
   a.x = x;
   a.y = y;
@@ -1373,23 +1378,29 @@ template <typename T>
 void launch_pcg_iter(const DevMesh &dm, T *x, T *r, T *p, T *q, T *partial, const T *invD,
                      OpShift<T> sh, CgScalars *sc, double *part_patch, double *part_node,
                      int parity, hipStream_t s) {
-  PatchArgs<T> a = patch_args<T>(dm);
-  a.x = r;
-  a.invD = invD;
-  a.xs = x;
-  a.p = p;
-  a.y = q;
-  a.partial = partial;
-  a.sh = sh;
-  a.sc = sc;
-  a.part = part_patch;
-  a.prz = part_node + (2 * (parity ^ 1) + 0) * NODE_PARTS;
-  a.prr = part_node + (2 * (parity ^ 1) + 1) * NODE_PARTS;
-  a.parity = parity;
-  if (dm.dim == 3)
-    launch_patch<T, 3, 1>(dm, a, s);
-  else
-    launch_patch<T, 2, 1>(dm, a, s);
+  const double *prz = part_node + (2 * (parity ^ 1) + 0) * NODE_PARTS;
+  const double *prr = part_node + (2 * (parity ^ 1) + 1) * NODE_PARTS;
+  if (use_strips<T>(dm)) {
+    launch_strip_pcg<T>(dm, {r, invD, x, p, q, partial, sh, sc, part_patch, prz, prr, parity}, s);
+  } else {
+    PatchArgs<T> a = patch_args<T>(dm);
+    a.x = r;
+    a.invD = invD;
+    a.xs = x;
+    a.p = p;
+    a.y = q;
+    a.partial = partial;
+    a.sh = sh;
+    a.sc = sc;
+    a.part = part_patch;
+    a.prz = prz;
+    a.prr = prr;
+    a.parity = parity;
+    if (dm.dim == 3)
+      launch_patch<T, 3, 1>(dm, a, s);
+    else
+      launch_patch<T, 2, 1>(dm, a, s);
+  }
   UpdArgs<T> u{};
   u.n_owned = dm.n_owned;
   u.n_active = dm.n_active;

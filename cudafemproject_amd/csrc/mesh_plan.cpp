@@ -57,29 +57,34 @@ struct BankScratch {
   std::vector<int16_t> c64, c32;
 };
 
-std::string spread_entry_banks(MeshPlan &plan, const PatchInfo &P, int npe, int pn_max,
-                               int32_t nloc, int32_t run, BankScratch &B) {
+// Items of up to `corners` entries (elements, strips), item i's local nodes at
+// lid[4 or more * i] (NO_NODE: none), one item per thread and round of pn_max.
+// node_end: ends of the nodes' runs.
+constexpr uint16_t NO_NODE = 0xffff;
+
+bool spread_entry_banks(const uint16_t *lid, uint16_t *epos, int stride, int corners, int32_t items,
+                        int pn_max, const uint16_t *node_end, int32_t nloc, int32_t run,
+                        BankScratch &B) {
   const int32_t nwave = (pn_max + 63) / 64;
-  const int32_t slots_e = (P.n_elem + pn_max - 1) / pn_max;
-  const int32_t n_w = slots_e * npe * nwave;
+  const int32_t slots_e = (items + pn_max - 1) / pn_max;
+  const int32_t n_w = slots_e * corners * nwave;
   B.occ.assign(size_t(run), -1);
   B.rstart.resize(nloc);
-  for (int32_t k = 0; k < nloc; ++k) B.rstart[k] = k ? int32_t(plan.node_end[P.pnode_start + k - 1]) : 0;
-  B.wid.assign(size_t(P.n_elem) * 4, 0);
-  B.half.assign(size_t(P.n_elem) * 4, 0);
+  for (int32_t k = 0; k < nloc; ++k) B.rstart[k] = k ? int32_t(node_end[k - 1]) : 0;
+  B.wid.assign(size_t(items) * stride, 0);
+  B.half.assign(size_t(items) * stride, 0);
   B.c64.assign(size_t(n_w) * 64, 0);
   B.c32.assign(size_t(n_w) * 64, 0);
-  uint16_t *epos = &plan.epos[size_t(P.elem_start) * 4];
-  const uint16_t *lid = &plan.elem_lid[size_t(P.elem_start) * 4];
   for (int32_t e = 0; e < slots_e; ++e)
-    for (int a = 0; a < npe; ++a)
+    for (int a = 0; a < corners; ++a)
       for (int32_t t = 0; t < pn_max; ++t) {
         const int32_t i = e * pn_max + t;
-        if (i >= P.n_elem) break;
-        const int32_t j = i * 4 + a, l = lid[j];
-        const int32_t W = (e * npe + a) * nwave + t / 64, h = (t & 63) >> 5;
+        if (i >= items) break;
+        const int32_t j = i * stride + a, l = lid[j];
+        if (l == NO_NODE) continue;
+        const int32_t W = (e * corners + a) * nwave + t / 64, h = (t & 63) >> 5;
         int16_t *u64 = &B.c64[size_t(W) * 64], *u32 = &B.c32[size_t(W) * 64 + h * 32];
-        const int32_t r1 = int32_t(plan.node_end[P.pnode_start + l]);
+        const int32_t r1 = int32_t(node_end[l]);
         int32_t best = -1, best_cost = INT32_MAX;
         for (int32_t p = B.rstart[l]; p < r1; ++p) {
           if (B.occ[p] >= 0) continue;
@@ -90,7 +95,7 @@ std::string spread_entry_banks(MeshPlan &plan, const PatchInfo &P, int npe, int 
             if (cost == 0) break;
           }
         }
-        if (best < 0) return "internal error: node run full";
+        if (best < 0) return false;  // (the run is full)
         B.occ[best] = j;
         B.wid[j] = W;
         B.half[j] = uint8_t(h);
@@ -116,7 +121,7 @@ std::string spread_entry_banks(MeshPlan &plan, const PatchInfo &P, int npe, int 
   for (int sweep = 0; sweep < 2; ++sweep) {
     int32_t improved = 0;
     for (int32_t k = 0; k < nloc; ++k) {
-      const int32_t r0 = B.rstart[k], r1 = int32_t(plan.node_end[P.pnode_start + k]);
+      const int32_t r0 = B.rstart[k], r1 = int32_t(node_end[k]);
       for (int32_t p = r0; p < r1; ++p)
         for (int32_t q = p + 1; q < r1; ++q) {
           const int32_t x = B.occ[p], y = B.occ[q];
@@ -138,7 +143,7 @@ std::string spread_entry_banks(MeshPlan &plan, const PatchInfo &P, int npe, int 
   }
   for (int32_t p = 0; p < run; ++p)
     if (B.occ[p] >= 0) epos[B.occ[p]] = uint16_t(p);
-  return "";
+  return true;
 }
 
 // fn(i) for i in [0, n) by up to 8 threads (fewer when the system gives fewer),
@@ -395,8 +400,9 @@ std::string build_plan(int dim, int64_t nn, const double *nodes, int64_t ne,
     return [&, bank = BankScratch()](int32_t p) mutable {
       const PatchInfo &P = plan.patches[p];
       const int32_t nloc = P.n_own + P.n_sh;
-      if (!spread_entry_banks(plan, P, npe, pn_max, nloc, plan.node_end[P.pnode_start + nloc - 1], bank)
-               .empty())
+      const uint16_t *end = &plan.node_end[P.pnode_start];
+      if (!spread_entry_banks(&plan.elem_lid[size_t(P.elem_start) * 4], &plan.epos[size_t(P.elem_start) * 4],
+                              4, npe, P.n_elem, pn_max, end, nloc, end[nloc - 1], bank))
         full = true;
     };
   });
@@ -458,6 +464,211 @@ void pack_patch_nodes(const MeshPlan &plan, int stride, std::vector<int32_t> &pg
       pend[i] = plan.node_end[size_t(Q.pnode_start + k)];
     }
   }
+}
+
+namespace {
+
+// The strips of one patch: elements joined across shared faces (2D: edges).
+struct StripScratch {
+  std::vector<std::pair<uint32_t, int32_t>> face;  // hash table: key + 1, element * 4 + face
+  std::vector<int32_t> adj;                        // 4 per element: neighbour * 4 + its face, or -1
+  std::vector<uint8_t> used;
+  std::vector<int32_t> deg, queue[5];              // free neighbours; elements by their number
+  std::vector<int32_t> strip;                      // 3 elements per strip, -1: none
+  std::vector<uint16_t> lid, epos, end;            // 6 per strip; per node
+  std::vector<int32_t> cnt;
+  BankScratch bank;
+};
+
+void strip_neighbours(const uint16_t *lid, int32_t n, int dim, StripScratch &S) {
+  size_t size = 64;
+  while (size < size_t(n) * 8) size *= 2;
+  S.face.assign(size, {0u, 0});
+  S.adj.assign(size_t(n) * 4, -1);
+  for (int32_t e = 0; e < n; ++e)
+    for (int f = 0; f <= dim; ++f) {  // the face opposite corner f
+      uint32_t v[3] = {0, 0, 0};
+      for (int a = 0, m = 0; a <= dim; ++a)
+        if (a != f) v[m++] = lid[size_t(e) * 4 + a];
+      if (v[0] > v[1]) std::swap(v[0], v[1]);
+      if (dim == 3) {
+        if (v[1] > v[2]) std::swap(v[1], v[2]);
+        if (v[0] > v[1]) std::swap(v[0], v[1]);
+      }
+      const uint32_t key = (v[0] | v[1] << 10 | v[2] << 20) + 1;
+      size_t h = (key * 2654435761u >> 8) & (size - 1);
+      while (S.face[h].first && S.face[h].first != key) h = (h + 1) & (size - 1);
+      if (!S.face[h].first) {
+        S.face[h] = {key, e * 4 + f};
+      } else if (S.face[h].second >= 0) {  // (of more than two elements at a face, the first two)
+        S.adj[size_t(e) * 4 + f] = S.face[h].second;
+        S.adj[size_t(S.face[h].second)] = e * 4 + f;
+        S.face[h].second = -1;
+      }
+    }
+}
+
+// Greedy strips, each begun at an element with the fewest free neighbours (it is
+// the first to be left alone) and continued to those with the fewest, among
+// equals the nearest in the order; or (!by_degree) in the order and to the
+// nearest.  The number of strips; S.strip: their elements, S.lid: their nodes.
+int32_t find_strips(const uint16_t *lid, int32_t n, int dim, bool by_degree, StripScratch &S) {
+  int32_t n_strips = 0;
+  S.strip.clear();
+  S.lid.clear();
+  auto out = [&](const int32_t *el, const uint16_t *nd) {
+    S.strip.insert(S.strip.end(), el, el + 3);
+    S.lid.insert(S.lid.end(), nd, nd + 6);
+    ++n_strips;
+  };
+  S.used.assign(size_t(n), 0);
+  S.deg.assign(size_t(n), 0);
+  for (auto &q : S.queue) q.clear();
+  for (int32_t e = 0; e < n; ++e) {
+    for (int f = 0; f <= dim; ++f) S.deg[e] += S.adj[size_t(e) * 4 + f] >= 0;
+    S.queue[by_degree ? S.deg[e] : 0].push_back(e);
+  }
+  size_t at[5] = {0, 0, 0, 0, 0};
+  // an element with the fewest free neighbours (entries may be out of date)
+  auto pick = [&]() -> int32_t {
+    for (int d = 0; d <= dim + 1; ++d)
+      while (at[d] < S.queue[d].size()) {
+        const int32_t e = S.queue[d][at[d]++];
+        if (!S.used[e] && (!by_degree || S.deg[e] == d)) return e;
+      }
+    return -1;
+  };
+  auto use = [&](int32_t e) {
+    S.used[e] = 1;
+    for (int f = 0; f <= dim; ++f) {
+      const int32_t a = S.adj[size_t(e) * 4 + f];
+      if (a < 0 || S.used[a >> 2]) continue;
+      const int32_t m = a >> 2;
+      if (!by_degree) continue;
+      S.queue[--S.deg[m]].push_back(m);
+      at[S.deg[m]] = std::min(at[S.deg[m]], S.queue[S.deg[m]].size() - 1);
+    }
+  };
+  // the face of e to the next element of its strip, or -1
+  auto next = [&](int32_t e) {
+    int best = -1, cost = INT32_MAX;
+    for (int f = 0; f <= dim; ++f) {
+      const int32_t a = S.adj[size_t(e) * 4 + f];
+      if (a < 0 || S.used[a >> 2]) continue;
+      const int c = (by_degree ? S.deg[a >> 2] * 65536 : 0) + std::abs((a >> 2) - e);
+      if (c < cost) {
+        cost = c;
+        best = f;
+      }
+    }
+    return best;
+  };
+  auto node = [&](int32_t e, int a) { return lid[size_t(e) * 4 + a]; };
+  for (int32_t e; (e = pick()) >= 0;) {
+    int32_t el[3] = {e, -1, -1};
+    uint16_t nd[6] = {NO_NODE, NO_NODE, NO_NODE, NO_NODE, NO_NODE, NO_NODE};
+    use(e);
+    const int f0 = next(e);
+    if (f0 < 0) {
+      for (int a = 0; a <= dim; ++a) nd[a] = node(e, a);
+      out(el, nd);
+      continue;
+    }
+    const int32_t mid = S.adj[size_t(e) * 4 + f0] >> 2, f1 = S.adj[size_t(e) * 4 + f0] & 3;
+    el[1] = mid;
+    use(mid);
+    const int f2 = next(mid);
+    // nodes: the first element's own, those of both or all, the last one's own
+    int m = 0;
+    nd[m++] = node(e, f0);
+    if (f2 >= 0) nd[m++] = node(mid, f2);
+    for (int a = 0; a <= dim; ++a)
+      if (a != f1 && a != f2) nd[m++] = node(mid, a);
+    nd[m++] = node(mid, f1);
+    if (f2 >= 0) {
+      const int32_t C = S.adj[size_t(mid) * 4 + f2];
+      el[2] = C >> 2;
+      use(C >> 2);
+      nd[m++] = node(C >> 2, C & 3);
+    }
+    out(el, nd);
+  }
+  return n_strips;
+}
+
+}  // namespace
+
+bool build_strips(const MeshPlan &plan, int node_stride, int stride, StripPlan &x) {
+  const size_t np = plan.patches.size();
+  x = StripPlan();
+  x.rec.assign(np * size_t(stride) * 4, 0u);
+  x.rec2.assign(np * size_t(stride), 0u);
+  x.pend.assign(np * size_t(node_stride), 0);
+  x.elems.assign(np * size_t(stride) * STRIP_ELEMS, -1);
+  std::vector<int32_t> n_strips(np), n_ent(np);
+  std::atomic<bool> failed{false};
+  for_each_patch(int32_t(np), [&] {
+    return [&, S = StripScratch()](int32_t p) mutable {
+      const PatchInfo &P = plan.patches[p];
+      const int32_t nloc = P.n_own + P.n_sh;
+      const size_t base = size_t(p) * stride;
+      const uint16_t *lid = &plan.elem_lid[size_t(P.elem_start) * 4];
+      strip_neighbours(lid, P.n_elem, plan.dim, S);
+      // (in the order a regular grid divides without remainder; elsewhere by
+      // degree leaves a tenth fewer strips)
+      int32_t n = find_strips(lid, P.n_elem, plan.dim, false, S);
+      if (n > (P.n_elem + 2) / 3) n = find_strips(lid, P.n_elem, plan.dim, true, S);
+      n_strips[p] = n;
+      if (n > stride) {
+        failed = true;
+        return;
+      }
+      for (int32_t s = 0; s < n; ++s) {
+        uint32_t count = 0;
+        for (int k = 0; k < STRIP_ELEMS; ++k)
+          if (S.strip[size_t(s) * 3 + k] >= 0) {
+            x.elems[(base + s) * 3 + k] = P.elem_start + S.strip[size_t(s) * 3 + k];
+            ++count;
+          }
+        x.rec[(base + s) * 4] = count << 30;
+      }
+      S.cnt.assign(nloc, 0);
+      for (uint16_t l : S.lid)
+        if (l != NO_NODE) ++S.cnt[l];
+      S.end.resize(nloc);
+      int32_t run = 0;
+      for (int32_t k = 0; k < nloc; ++k) {
+        run = (run + S.cnt[k] + 3) & ~3;
+        S.end[k] = x.pend[size_t(p) * node_stride + k] = uint16_t(run);
+      }
+      n_ent[p] = run;
+      S.epos.assign(S.lid.size(), 0);
+      if (!spread_entry_banks(S.lid.data(), S.epos.data(), 6, plan.dim + STRIP_ELEMS, n, stride,
+                              S.end.data(), nloc, run, S.bank)) {
+        failed = true;
+        return;
+      }
+      for (int32_t s = 0; s < n; ++s) {
+        uint32_t l[6], q[6];
+        for (int a = 0; a < 6; ++a) {
+          const uint16_t v = S.lid[size_t(s) * 6 + a];
+          l[a] = v == NO_NODE ? 0u : v;
+          q[a] = S.epos[size_t(s) * 6 + a];
+        }
+        uint32_t *r = &x.rec[(base + s) * 4];
+        r[0] |= l[0] | l[1] << 10 | l[2] << 20;
+        r[1] = l[3] | l[4] << 10 | l[5] << 20;
+        r[2] = q[0] | q[1] << 14;
+        r[3] = q[2] | q[3] << 14;
+        x.rec2[base + s] = q[4] | q[5] << 14;
+      }
+    };
+  });
+  for (size_t p = 0; p < np; ++p) {
+    x.strips_used = std::max(x.strips_used, int(n_strips[p]));
+    x.ent_used = std::max(x.ent_used, int(n_ent[p]));
+  }
+  return !failed;
 }
 
 bool build_exchange(const MeshPlan &plan, ExchangePlan &x) {
