@@ -768,20 +768,23 @@ bool pcg_resident(const femgpu_ctx *ctx) {
 // The exchange words and this precision's entries, zeroed for this plan (an
 // entry's tag is short: words of another precision's layout would not do).
 template <typename T>
-int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long **entries) {
+int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long **entries,
+                size_t *entry_words) {
   const size_t n = femgpu::res_words(ctx->dm.np);
   const size_t n64 = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
   const size_t n32 = femgpu::res_entry_words<float>(ctx->dm.x_entries, ctx->dim);
   double *w, *e;
   int st;
-  if ((st = dbuf(ctx, "res_words", n, &w)) || (st = dbuf(ctx, "res_entries", n64 + n32, &e))) return st;
+  if ((st = dbuf(ctx, "res_words", n, &w)) || (st = dbuf(ctx, "res_entries", 2 * (n64 + n32), &e)))
+    return st;
   if (ctx->res_np != ctx->dm.np) {
     femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
-    femgpu::launch_fill<double>(e, int64_t(n64 + n32), 0.0, ctx->stream);
+    femgpu::launch_fill<double>(e, int64_t(2 * (n64 + n32)), 0.0, ctx->stream);
     ctx->res_np = ctx->dm.np;
   }
   *words = reinterpret_cast<unsigned long long *>(w);
-  *entries = reinterpret_cast<unsigned long long *>(e) + (sizeof(T) == 8 ? 0 : n64);
+  *entries = reinterpret_cast<unsigned long long *>(e) + (sizeof(T) == 8 ? 0 : 2 * n64);
+  *entry_words = sizeof(T) == 8 ? n64 : n32;
   return FEMGPU_OK;
 }
 
@@ -795,7 +798,7 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
   int st;
   if (!femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit))
     return fail(ctx, FEMGPU_E_STATE, "internal error: resident PCG does not fit");
-  if ((st = res_buffers<T>(ctx, &a.words, &a.entries))) return st;
+  if ((st = res_buffers<T>(ctx, &a.words, &a.entries, &a.entry_words))) return st;
   a.sc = ctx->h_sc;
   a.cap = RES_ITER_CAP;
   for (;;) {
@@ -862,7 +865,7 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
   int st;
   if (!femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit))
     return fail(ctx, FEMGPU_E_STATE, "internal error: resident steps do not fit");
-  if ((st = res_buffers<T>(ctx, &m.words, &m.entries))) return st;
+  if ((st = res_buffers<T>(ctx, &m.words, &m.entries, &m.entry_words))) return st;
   m.sc = ctx->h_sc;
   m.it_budget = 4 * RES_ITER_CAP;
   *done = 1;

@@ -19,8 +19,9 @@ namespace femgpu {
 // plan changes, and after an aborted launch.
 constexpr int EX_COPIES = 8;
 constexpr size_t RES_HEAD = 512;
+constexpr int RES_SUMS = 5;  // sums of a PCG iteration, in two places in turn
 __host__ __device__ inline size_t res_copy_words(int np) {
-  return (size_t(6) * size_t(np) + 511) & ~size_t(511);
+  return (size_t(4 * RES_SUMS) * size_t(np) + 511) & ~size_t(511);
 }
 inline size_t res_words(int np) { return RES_HEAD + EX_COPIES * res_copy_words(np); }
 // Words of an entry: dim values of tb bytes, 48 bits to a word.
@@ -41,8 +42,9 @@ struct ResPcg {
   const T *r_in;
   T *x, *p, *r_out;
   const T *invD;
-  unsigned long long *entries;  // interface entries (res_entry_words)
-  unsigned long long *words;  // res_words(np)
+  unsigned long long *entries;  // two sets of interface entries
+  size_t entry_words;           // of a set (res_entry_words)
+  unsigned long long *words;    // res_words(np)
   CgScalars *sc;              // the scalars at the end (host-visible memory)
   int fresh, kind;
   double eps;             // fresh: tolerance (threshold formed from the initial residual)
@@ -65,9 +67,10 @@ struct ResFit {
 // Whether the plan's PCG runs resident: patches of up to 512 nodes and 1536
 // elements, every workgroup on a compute unit of its own.  Several workgroups
 // per unit would fit, and lose to the launch-per-kernel form (a 40^3-hex cube
-// in 500 patches: FP64 32.3 against 18.1 us per iteration, mixed 20.4 against
-// 15.3), whose launches cost less the more work there is between them; in 256
-// patches of twice the size the resident form is ahead, 16.7 and 12.5 us.
+// in 500 patches, with two trips per iteration: FP64 32.3 against 18.1 us, mixed
+// 20.4 against 15.3), whose launches cost less the more work there is between
+// them; in 256 patches of twice the size the resident form is ahead, 14.5 and
+// 9.9 us.
 template <typename T>
 bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit);
 
@@ -119,6 +122,7 @@ struct ResImpl : ResRecv<T> {
   double eps;             // nested PCG: gamma < eps gamma0
   int max_iter, it_budget;
   unsigned long long *words, *entries;
+  size_t entry_words;     // as ResPcg
   CgScalars *sc;
   int fresh, step0, n_steps;
 };

@@ -9,18 +9,21 @@
 // registers and LDS; between workgroups only the interface nodes' partial
 // sums and the dot products' partials travel, through memory, at agent scope.
 //
-// What bounds it, in kcycles of 2.4 GHz: an iteration's two trips through
-// memory (3.5 each from the first store to the last load at 10 workgroups, 4
-// to 7 at 100; a step's one: 2.6 at 10, 6 at 229) and the element phase of one
-// patch on one compute unit (FP64 tets: 4 for 768 elements, 12 for 1536, bound
-// by LDS traffic and FP64 issue).  Measured, launch per kernel -> resident:
-//   us per PCG iteration: 12x7 plate FP64 10.2 -> 1.9 (one workgroup, no
-//   trips), 64x32 plate FP64 10.2 -> 5.3, 24^3 hexes FP64 14.0 -> 9.0 and mixed
-//   14.0 -> 8.2, 40^3 hexes (1536 elements per patch) FP64 18.1 -> 16.7 and
-//   mixed 15.3 -> 12.5;
+// What bounds it, in kcycles of 2.4 GHz: an iteration's (a step's) trip through
+// memory (from the first store to the last load 3.5 at 10 workgroups, 4 to 7 at
+// 100 to 230) and the element phase of one patch on one compute unit (FP64
+// tets: 4 for 768 elements, 12 for 1536, bound by LDS traffic and FP64 issue).
+// Measured, launch per kernel -> resident:
+//   us per PCG iteration: 12x7 plate FP64 10.2 -> 1.7 (one workgroup, no
+//   trip), 64x32 plate FP64 10.2 -> 3.7, 24^3 hexes FP64 14.0 -> 6.9 and mixed
+//   14.0 -> 6.6, 40^3 hexes (1536 elements per patch) FP64 18.1 -> 14.5 and
+//   mixed 15.3 -> 9.9; with a trip for p'K p and one for r'z, as the
+//   launch-per-kernel recurrence has it, 5.3 for the 64x32 plate, 9.0 and 8.2,
+//   16.7 and 12.5;
 //   us per explicit step: 63x31 plate FP32 with receivers 9.1 -> 2.0, 160x80
 //   plate FP64 5.7 -> 2.3, 16x16x256 column FP64 15.5 -> 10.1 and FP32
-//   10.7 -> 6.3.
+//   10.7 -> 6.3;
+//   20 implicit steps of an 11x11x80 column (870 iterations) 13.4 -> 5.7 ms.
 //
 // Every workgroup forms every scalar itself from all partials in the same
 // order, and every patch holding an interface node carries its own copy of
@@ -30,14 +33,14 @@
 // Exchange: a workgroup's partials and its interface sums are published as
 // 8-byte words, 32 bits of payload under a 32-bit tag (the number of the
 // exchange), so that a value and its arrival are one load and nothing has to
-// be ordered: an iteration is two trips through memory.  Every workgroup has
-// read an exchange's words before it publishes in the next one, so each word
-// has one place.  Stores and loads of shared data are relaxed agent-scope
+// be ordered.  A workgroup that has everyone's words of one exchange knows that
+// everyone has read those of the one before, so two places (and, for the
+// interface sums, two sets of entries) take turns.  Stores and loads of shared data are relaxed agent-scope
 // atomics (written through, not served from a stale cache); an agent-scope
 // fence would write the XCD's L2 back, some 40 us.
 //
 // Waiting needs all workgroups on the chip: the host launches this form only
-// where they fit (res_pcg_fits), and a wait is bounded (WAIT_TICKS): past it
+// where they fit (res_pcg_fit), and a wait is bounded (WAIT_TICKS): past it
 // the launch ends with an abort flag and the host runs the launch-per-kernel
 // form instead.
 #include <hip/hip_runtime.h>
@@ -77,7 +80,7 @@ __host__ __device__ inline ResLds res_lds(int dim, int tb, int pn, int ent, int 
   L.off_os = L.off_oe + al32(n_in * 4);
   L.off_ip = L.off_os + al32(n_in * 2);
   L.off_red = L.off_ip + al32(n_in * 2);
-  L.total = L.off_red + (3 * 16 + 4) * 8;
+  L.total = L.off_red + (16 * RES_SUMS + 8) * 8;
   return L;
 }
 
@@ -330,31 +333,44 @@ struct ResPatch {
   }
 };
 
-// The PCG of one workgroup (the recurrence of k_ebe_patch MODE 1 and
-// k_pcg_update): r, p, x of this thread's DOFs, the scalars the same in every
-// workgroup.
+// The PCG of one workgroup: r, p, x of this thread's DOFs, the scalars the same in
+// every workgroup.  One trip through memory per iteration: K z (z = invD r) is
+// formed and traded instead of K p, s = K p follows from the recurrence
+// s = K z + beta s (Chronopoulos and Gear, J. Comput. Appl. Math. 25 (1989)), and
+//   p'Kp = z'Kz + 2 beta z's + beta^2 p's  (p, s of the last iteration)
+// from sums that travel beside r'z and r'r.  Neither beta nor the step length
+// uses an orthogonality that rounding loses, and every RENEW iterations (or
+// where the sums cancel) s = K p and p's are formed anew, so r keeps to f - K x
+// as it does with a product K p in every iteration: iterations and errors are
+// those of that recurrence (64 x 32 plate, FP64 to 1e-10: 620 both, error
+// 6.9e-12 both).
+// (Mixed solves of the batch workload's plates and of cubes: 98.7, 93.9 and
+// 91.1 ms in all with 8, 16 and 32; iterations within 3 %.)
+constexpr int RENEW = 32;
+
 template <typename T, int DIM, int PT, int NE>
 struct ResSolver {
   using Patch = ResPatch<T, DIM, PT, NE>;
   static constexpr int ND = Patch::ND;
   Patch &P;
-  Exchange xpq, xrz;
+  Exchange ex;
   u64 *entries;
+  size_t entry_words;
   unsigned tag, entry_tag;
   int pid;
   bool alone;            // one workgroup: no exchange
   int *s_flag;           // LDS: a wait ran out
-  double *s_red, *s_bc;  // LDS: p'q (16); r'z and r'r (32); their totals (1 + 2)
+  double *s_red, *s_bc;  // LDS: the waves' sums; the totals
   double g, q2, g_prev;  // r'z, r'r; the r'z that p was formed with
+  double gamma0, rr0, thresh, pause;
   int n_upd;
 
-  __device__ __forceinline__ ResSolver(Patch &patch, const ResMesh<T> &m, u64 *words, u64 *ent, int b,
-                                       int id, int *flag)
-      : P(patch), entries(ent), pid(id), alone(m.np == 1), s_flag(flag), s_red(patch.s_red),
-        s_bc(patch.s_red + 48), g(0.0), q2(0.0), g_prev(1.0), n_upd(0) {
-    const size_t stride = res_copy_words(m.np);
-    xpq = Exchange{words + RES_HEAD, stride, words + 1, m.np, b % EX_COPIES};
-    xrz = Exchange{xpq.words + size_t(2) * m.np, stride, words + 1, m.np, b % EX_COPIES};
+  __device__ __forceinline__ ResSolver(Patch &patch, const ResMesh<T> &m, u64 *words, u64 *ent,
+                                       size_t ent_words, int b, int id, int *flag)
+      : P(patch), entries(ent), entry_words(ent_words), pid(id), alone(m.np == 1), s_flag(flag),
+        s_red(patch.s_red), s_bc(patch.s_red + 16 * RES_SUMS), g(0.0), q2(0.0), g_prev(1.0),
+        n_upd(0) {
+    ex = Exchange{words + RES_HEAD, res_copy_words(m.np), words + 1, m.np, b % EX_COPIES};
     // (workgroup 0 advances the tags at its end, after an exchange that every
     // workgroup took part in with the tags it reads here)
     tag = unsigned(ld_agent(words));
@@ -366,30 +382,94 @@ struct ResSolver {
     st_agent(words + 2 + (sizeof(T) == 8 ? 1 : 0), u64(entry_tag));
   }
 
-  // g, q2 = r'z and r'r over all patches (z = invD r).
-  __device__ __forceinline__ bool dots(const T (&r)[ND], const T (&invd)[ND]) {
-    double v[2] = {0.0, 0.0};
-    if (P.first)
-#pragma unroll
-      for (int i = 0; i < ND; ++i) {
-        v[0] += double(r[i]) * double(mul_rn(invd[i], r[i]));
-        v[1] += double(r[i]) * double(r[i]);
-      }
-    sum_to_wave0<PT, 2>(v, s_red + 16);
+  // A trade; the sets of entries take turns, as in the explicit steps: a
+  // neighbour may still be reading the last trade's.
+  __device__ __forceinline__ void trade() {
+    ++entry_tag;
+    if (!P.trade(entries + (entry_tag & 1u) * entry_words, entry_tag, ex.abort)) *s_flag = 1;
+  }
+
+  // y = K x, complete.  False: a wait ran out.
+  __device__ __forceinline__ bool apply(const T (&x)[ND], T (&y)[ND]) {
+    P.product(x, y);
+    if (alone) return true;
+    P.put(y);
+    __syncthreads();
+    trade();
+    __syncthreads();
+    P.collect(y);
+    return *s_flag == 0;
+  }
+
+  // v summed over all workgroups; with_trade: the trade of what was put beside
+  // it.  False: a wait ran out.
+  __device__ __forceinline__ bool sums(double (&v)[RES_SUMS], bool with_trade = false) {
     ++tag;
-    if (!alone && threadIdx.x < 64) publish<2>(xrz, pid, tag, v);
-    const bool ok = gather<2>(xrz, tag, v, s_bc, s_flag, alone);
-    g = v[0];
-    q2 = v[1];
+    const double sum = sum_by_wave<PT>(v, s_red);
+    Exchange e = ex;
+    e.words += (tag & 1u) * size_t(2 * RES_SUMS) * ex.np;
+    if (!alone) {
+      publish(e, pid, tag, sum);
+      if (with_trade) trade();
+    }
+    return gather(e, tag, sum, v, s_bc, s_flag, alone);
+  }
+
+  // s = (cK K + diag(cMm)) p.
+  __device__ __forceinline__ bool refresh(const T (&p)[ND], T (&s)[ND], T cK, const T (&cMm)[ND]) {
+    const bool ok = apply(p, s);
+#pragma unroll
+    for (int i = 0; i < ND; ++i) s[i] = cK * s[i] + cMm[i] * p[i];
     return ok;
   }
 
-  // Iterates from r, p, x with g and q2 formed until a stop; returns the done
-  // code.  cMm: the mass shift of this thread's DOFs.
+  // Iterates from r, p, x until a stop; returns the done code.  fresh: p = 0,
+  // and the threshold and the pause are formed from the first sums (eps, and
+  // pause relative to r'r); else p, g_prev, thresh and pause are an earlier
+  // run's.  cMm: the mass shift of this thread's DOFs.
   __device__ __forceinline__ int run(T (&r)[ND], T (&p)[ND], T (&x)[ND], const T (&invd)[ND], T cK,
-                                     const T (&cMm)[ND], int kind, double thresh, double pause,
+                                     const T (&cMm)[ND], bool fresh, int kind, double eps,
                                      int max_iter, int last) {
+    T s[ND];
+    if (fresh) {
+#pragma unroll
+      for (int i = 0; i < ND; ++i) s[i] = T(0);
+    } else if (!refresh(p, s, cK, cMm)) {
+      return RES_ABORTED;
+    }
     for (;;) {
+      T z[ND], w[ND];
+#pragma unroll
+      for (int i = 0; i < ND; ++i) z[i] = mul_rn(invd[i], r[i]);
+      P.product(z, w);
+      double v[RES_SUMS] = {0.0, 0.0, 0.0, 0.0, 0.0};
+      if (P.has)
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+          w[i] = cK * w[i];
+          if (P.own) w[i] += cMm[i] * z[i];
+          const double zi = double(z[i]);
+          v[2] += zi * double(w[i]);
+          if (P.first) {
+            v[0] += double(r[i]) * zi;
+            v[1] += double(r[i]) * double(r[i]);
+            v[3] += zi * double(s[i]);
+            v[4] += double(p[i]) * double(s[i]);
+            // the mass shift belongs to the patch that accounts for the node
+            if (!P.own) v[2] += double(cMm[i]) * zi * zi;
+          }
+        }
+      P.put(w);
+      if (!sums(v, true)) return RES_ABORTED;
+      g = v[0];
+      q2 = v[1];
+      if (fresh) {
+        fresh = false;
+        gamma0 = g;
+        rr0 = q2;
+        thresh = kind == 0 ? eps * g : eps * eps * q2;
+        pause *= q2;
+      }
       if (n_upd >= 1) {
         if (kind == 0 ? g < thresh : q2 <= thresh) return 1;
       } else if (q2 == 0.0) {
@@ -403,45 +483,42 @@ struct ResSolver {
       // 1953 so, 1950 in the launch-per-kernel form)
       if ((n_upd & 7) == 0 && q2 < pause) return 5;
       if (n_upd >= last) return RES_CAP;
-      const T beta = T(g / g_prev);
-      g_prev = g;
-      if (P.has)
-#pragma unroll
-        for (int i = 0; i < ND; ++i) p[i] = pcg_dir(invd[i], r[i], beta, p[i]);
-      T q[ND];
-      P.product(p, q);
-      double vpq[1] = {0.0};
-      if (P.has)
-#pragma unroll
-        for (int i = 0; i < ND; ++i) {
-          q[i] = cK * q[i];
-          if (P.own) q[i] += cMm[i] * p[i];
-          vpq[0] += double(p[i]) * double(q[i]);
-          // the mass shift belongs to the patch that accounts for the node
-          if (!P.own && P.first) vpq[0] += double(cMm[i]) * double(p[i]) * double(p[i]);
-        }
-      P.put(q);
-      ++tag;
-      ++entry_tag;
-      sum_to_wave0<PT, 1>(vpq, s_red);
-      if (!alone) {
-        if (threadIdx.x < 64) publish<1>(xpq, pid, tag, vpq);
-        if (!P.trade(entries, entry_tag, xpq.abort)) *s_flag = 1;
+      if (fabs(g) < 0x1p-1000) {
+        // (tolerance 0: the sums underflow, which is no breakdown; nothing is left
+        // to change)
+        ++n_upd;
+        continue;
       }
-      if (!gather<1>(xpq, tag, vpq, s_bc + 2, s_flag, alone)) return RES_ABORTED;
-      const double pq = vpq[0], alpha_d = g / pq;
+      const double beta_d = g / g_prev, own = v[2] + beta_d * beta_d * v[4];
+      double pq = v[2] + beta_d * (2.0 * v[3] + beta_d * v[4]);
+      const T beta = T(beta_d);
+      P.collect(w);
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        if (P.has && !P.own) w[i] += cMm[i] * z[i];
+        p[i] = fma(beta, p[i], z[i]);
+        s[i] = fma(beta, s[i], w[i]);
+      }
+      if (n_upd % RENEW == RENEW - 1 || !(pq > 0x1p-10 * own)) {
+        // (or where the sums cancel)
+        if (!refresh(p, s, cK, cMm)) return RES_ABORTED;
+        double u[RES_SUMS] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        if (P.first)
+#pragma unroll
+          for (int i = 0; i < ND; ++i) u[0] += double(p[i]) * double(s[i]);
+        if (!sums(u)) return RES_ABORTED;
+        pq = u[0];
+      }
+      const double alpha_d = g / pq;
       // (no x or r has changed: the state of the last completed iteration)
       if (!(pq > 0.0) || !isfinite(alpha_d)) return isfinite(pq) ? 3 : 2;
+      g_prev = g;
       const T alpha = T(alpha_d);
-      P.collect(q);
-      if (P.has)
 #pragma unroll
-        for (int i = 0; i < ND; ++i) {
-          if (!P.own) q[i] += cMm[i] * p[i];
-          x[i] = x[i] + alpha * p[i];
-          r[i] = r[i] - alpha * q[i];
-        }
-      if (!dots(r, invd)) return RES_ABORTED;
+      for (int i = 0; i < ND; ++i) {
+        x[i] = x[i] + alpha * p[i];
+        r[i] = r[i] - alpha * s[i];
+      }
       ++n_upd;
     }
   }
@@ -478,21 +555,15 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
       }
     }
   }
-  ResSolver<T, DIM, PT, NE> S(P, a.m, a.s.words, a.s.entries, b, pid, &s_flag);
+  ResSolver<T, DIM, PT, NE> S(P, a.m, a.s.words, a.s.entries, a.s.entry_words, b, pid, &s_flag);
   S.n_upd = a.s.it0;
-  int done = RES_ABORTED;
-  double gamma0 = a.s.gamma0, rr0 = a.s.rr0, thresh = a.s.thresh, pause = a.s.pause;
-  if (S.dots(r, d)) {
-    if (a.s.fresh) {
-      gamma0 = S.g;
-      rr0 = S.q2;
-      thresh = a.s.kind == 0 ? a.s.eps * S.g : a.s.eps * a.s.eps * S.q2;
-      pause = a.s.pause * S.q2;
-    } else {
-      S.g_prev = a.s.g_prev;
-    }
-    done = S.run(r, p, x, d, T(1), cMm, a.s.kind, thresh, pause, a.s.max_iter, a.s.it0 + a.s.cap);
-  }
+  S.gamma0 = a.s.gamma0;
+  S.rr0 = a.s.rr0;
+  S.thresh = a.s.thresh;
+  S.pause = a.s.pause;
+  if (!a.s.fresh) S.g_prev = a.s.g_prev;
+  int done = S.run(r, p, x, d, T(1), cMm, a.s.fresh != 0, a.s.kind, a.s.eps, a.s.max_iter,
+                   a.s.it0 + a.s.cap);
   if (P.first)
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -502,14 +573,14 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
     }
   if (pid == 0 && threadIdx.x == 0) {
     CgScalars *sc = a.s.sc;
-    sc->gamma0 = gamma0;
-    sc->rr0 = rr0;
-    sc->thresh = thresh;
+    sc->gamma0 = S.gamma0;
+    sc->rr0 = S.rr0;
+    sc->thresh = S.thresh;
     sc->g[0] = sc->g[1] = S.g_prev;
     sc->g_final = S.g;
     sc->rr_final = S.q2;
     sc->iter_final = S.n_upd;
-    sc->pause = pause;
+    sc->pause = S.pause;
     S.store_tags(a.s.words);
     if (ld_agent(a.s.words + 1) != 0) done = RES_ABORTED;
     sc->done = done;
@@ -568,7 +639,7 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
     }
   }
   const int rec = s.rec_of && P.has && P.first ? s.rec_of[P.gid] : -1;
-  ResSolver<T, DIM, PT, NE> S(P, arg.m, s.words, s.entries, b, pid, &s_flag);
+  ResSolver<T, DIM, PT, NE> S(P, arg.m, s.words, s.entries, s.entry_words, b, pid, &s_flag);
   int done = 1, n = 0, total = 0;
   for (; n < s.n_steps && total < s.it_budget; ++n) {
     const int step = s.step0 + n;
@@ -581,15 +652,8 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
       v[i] = v[i] + s.c2 * a[i];
       x[i] = s.beta != T(0) ? d[i] + s.beta * v[i] : d[i];
     }
-    P.product(x, r);
-    if (!S.alone) {
-      P.put(r);
-      ++S.entry_tag;
-      __syncthreads();
-      if (!P.trade(S.entries, S.entry_tag, S.xpq.abort)) s_flag = 1;
-      __syncthreads();
-      P.collect(r);
-    }
+    done = RES_ABORTED;
+    if (!S.apply(x, r)) break;
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
       const T kd = r[i];
@@ -601,9 +665,8 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
     }
     S.n_upd = 0;
     S.g_prev = 1.0;
-    done = RES_ABORTED;
-    if (S.dots(r, invd))
-      done = S.run(r, p, x, invd, s.cK, cMm, 0, s.eps * S.g, 0.0, s.max_iter, s.max_iter + 1);
+    S.pause = 0.0;
+    done = S.run(r, p, x, invd, s.cK, cMm, true, 0, s.eps, s.max_iter, s.max_iter + 1);
     total += S.n_upd;
     if (done != 1) break;
 #pragma unroll

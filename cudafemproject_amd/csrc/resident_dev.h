@@ -128,109 +128,11 @@ __device__ __forceinline__ bool recv_entry(const u64 *entries, unsigned e, unsig
 // EX_COPIES-th workgroup (a copy per XCD): all workgroups polling one copy
 // of a few kilobytes queue up at the memory channels that hold it.
 struct Exchange {
-  u64 *words;      // copy 0 of this exchange: [2 * NV][np]
+  u64 *words;      // copy 0 of this exchange: [2 * RES_SUMS][np]
   size_t stride;   // words from copy to copy
   u64 *abort;      // nonzero: a workgroup gave up waiting
   int np, copy;    // copy: the one this workgroup reads
 };
-
-// Sums of NV values over the workgroup's threads, valid in wave 0 (the same
-// bits in every lane; fixed order).  s_red: NV * PT / 64 doubles that no
-// thread still reads or writes for another sum.
-template <int PT, int NV>
-__device__ __forceinline__ void sum_to_wave0(double (&v)[NV], double *s_red) {
-  constexpr int W = PT / 64;
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
-  if (l == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) s_red[k * W + w] = v[k];
-  __syncthreads();
-  if (w == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      // (at most 16 waves: one row, its sum in every lane of the row)
-      double q = s_red[k * W + min(l & 15, W - 1)];
-      if ((l & 15) >= W) q = 0.0;
-      q += dpp_f64<0xB1>(q);
-      q += dpp_f64<0x4E>(q);
-      q += dpp_f64<0x141>(q);
-      q += dpp_f64<0x140>(q);
-      v[k] = q;
-    }
-}
-
-// Wave 0 publishes the workgroup's NV values under `tag`.
-template <int NV>
-__device__ __forceinline__ void publish(const Exchange &x, int pid, unsigned tag,
-                                        const double (&v)[NV]) {
-  const int t = threadIdx.x;
-  if (t < 2 * NV * EX_COPIES) {
-    const int k = t % (2 * NV), copy = t / (2 * NV);
-    double d = v[0];
-#pragma unroll
-    for (int i = 1; i < NV; ++i) d = (k >> 1) == i ? v[i] : d;
-    u64 w[2];
-    tag_words(d, tag, w);
-    st_agent(&x.words[copy * x.stride + size_t(k) * x.np + pid], (k & 1) ? w[1] : w[0]);
-  }
-}
-
-// Wave 0 gathers every workgroup's NV values of `tag` (NB loads of each lane
-// in flight) and sums them in a fixed order; the sums reach every thread
-// through s_bc (NV doubles) behind a barrier, which also ends the wait for
-// the entries.  alone: v is the sum already.  False when a workgroup gave up
-// (or *s_flag was set).
-template <int NV>
-__device__ __forceinline__ bool gather(const Exchange &x, unsigned tag, double (&v)[NV],
-                                       double *s_bc, int *s_flag, bool alone) {
-  constexpr int NB = 4;
-  if (threadIdx.x < 64 && !alone) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = 0.0;
-    const u64 *words = x.words + x.copy * x.stride;
-    bool ok = true;
-    for (int i0 = threadIdx.x; ok && i0 < x.np; i0 += 64 * NB) {
-      u64 h[NB][NV][2];
-      Patience wait{x.abort};
-      for (int spin = 0;; ++spin) {
-        bool all = true;
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int k = 0; k < 2 * NV; ++k)
-            if (i0 + 64 * i < x.np)
-              h[i][k >> 1][k & 1] = ld_agent(&words[size_t(k) * x.np + i0 + 64 * i]);
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int k = 0; k < 2 * NV; ++k)
-            if (i0 + 64 * i < x.np) all = all && unsigned(h[i][k >> 1][k & 1] >> 32) == tag;
-        if (all) break;
-        if (wait.over(spin)) {
-          ok = false;
-          break;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < NB; ++i)
-        if (i0 + 64 * i < x.np)
-#pragma unroll
-          for (int k = 0; k < NV; ++k) v[k] += untag(h[i][k]);
-    }
-    if (!ok) *s_flag = 1;
-#pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
-  }
-  if (threadIdx.x == 0)
-#pragma unroll
-    for (int k = 0; k < NV; ++k) s_bc[k] = v[k];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k) v[k] = s_bc[k];
-  return *s_flag == 0;
-}
 
 // Sum of the entry run [b0, b1) (multiples of 4) in a fixed order.
 template <typename T>
@@ -447,6 +349,87 @@ __device__ __forceinline__ double wave_sums(const double (&v)[NV]) {
     }
     return sum8(s + lane_xor<8>(s));
   }
+}
+
+// Sums of RES_SUMS values over the workgroup's threads: wave v < RES_SUMS gets value
+// v's in every lane of its first row (fixed order).  s_red: RES_SUMS * 16 doubles
+// that no thread still reads or writes.
+template <int PT>
+__device__ __forceinline__ double sum_by_wave(const double (&v)[RES_SUMS], double *s_red) {
+  constexpr int W = PT / 64;
+  static_assert(RES_SUMS <= 8 && W >= RES_SUMS && W <= 16, "");
+  double v8[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) v8[k] = k < RES_SUMS ? v[k < RES_SUMS ? k : 0] : 0.0;
+  const double s = wave_sums<8>(v8);
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  if ((l & 7) == 0 && l < 8 * RES_SUMS) s_red[(l >> 3) * 16 + w] = s;
+  __syncthreads();
+  double q = w < RES_SUMS && l < W ? s_red[w * 16 + l] : 0.0;
+  q += dpp_f64<0xB1>(q);
+  q += dpp_f64<0x4E>(q);
+  q += dpp_f64<0x141>(q);
+  return q + dpp_f64<0x140>(q);
+}
+
+// Wave v publishes the workgroup's value v under `tag`, a copy to two lanes.
+__device__ __forceinline__ void publish(const Exchange &x, int pid, unsigned tag, double v) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  if (w < RES_SUMS && l < 2 * EX_COPIES) {
+    u64 h[2];
+    tag_words(v, tag, h);
+    st_agent(&x.words[(l >> 1) * x.stride + size_t(2 * w + (l & 1)) * x.np + pid], h[l & 1]);
+  }
+}
+
+// Wave v gathers every workgroup's value v of `tag` (NB loads of each lane in
+// flight) and sums them in a fixed order; the sums reach every thread through
+// s_bc (RES_SUMS doubles) behind a barrier, which also ends the wait for the
+// entries.  alone: v is the sum already.  False when a workgroup gave up (or
+// *s_flag was set).
+__device__ __forceinline__ bool gather(const Exchange &x, unsigned tag, double v,
+                                       double (&sums)[RES_SUMS], double *s_bc, int *s_flag,
+                                       bool alone) {
+  constexpr int NB = 4;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  if (w < RES_SUMS) {
+    if (!alone) {
+      v = 0.0;
+      const u64 *words = x.words + x.copy * x.stride + size_t(2 * w) * x.np;
+      bool ok = true;
+      for (int i0 = l; ok && i0 < x.np; i0 += 64 * NB) {
+        u64 h[NB][2];
+        Patience wait{x.abort};
+        for (int spin = 0;; ++spin) {
+          bool all = true;
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+              if (i0 + 64 * i < x.np) h[i][k] = ld_agent(&words[size_t(k) * x.np + i0 + 64 * i]);
+#pragma unroll
+          for (int i = 0; i < NB; ++i)
+            if (i0 + 64 * i < x.np)
+              all = all && unsigned(h[i][0] >> 32) == tag && unsigned(h[i][1] >> 32) == tag;
+          if (all) break;
+          if (wait.over(spin)) {
+            ok = false;
+            break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+          if (i0 + 64 * i < x.np) v += untag(h[i]);
+      }
+      if (!ok) *s_flag = 1;
+      v = wave_sum(v);
+    }
+    if (l == 0) s_bc[w] = v;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < RES_SUMS; ++k) sums[k] = s_bc[k];
+  return *s_flag == 0;
 }
 
 }  // namespace resident

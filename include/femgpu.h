@@ -80,7 +80,10 @@ enum {
 enum {
   FEMGPU_CG_STANDARD = 0,         /* the reference's recurrence
                                      (femfunc.cpp:59-111): two reductions
-                                     per iteration, two launches           */
+                                     per iteration, two launches; where the
+                                     whole solve is one launch, s = A p is
+                                     carried between products that renew it
+                                     every 32 iterations                    */
   FEMGPU_CG_SINGLE_REDUCTION = 1  /* Chronopoulos-Gear form: s = A p and
                                      w = A M^-1 r carried as recurrences,
                                      one reduction and one launch per
