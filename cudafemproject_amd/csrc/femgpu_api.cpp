@@ -1278,7 +1278,7 @@ int upload_plan(femgpu_ctx *ctx) {
     }
   }
   ctx->strip_elems.clear();
-  if (dm.np > femgpu::RES_PATCHES_MAX && threads <= 512) {
+  if (threads == 512 || (dm.np > femgpu::RES_PATCHES_MAX && threads == 256)) {
     femgpu::StripPlan x;
     const int stride = threads / 4 * 5;
     if (femgpu::build_strips(P, threads, stride, x)) {

@@ -75,6 +75,15 @@ __device__ __forceinline__ void decode_rec(uint3 r, int *l, int *q) {
   q[3] = int(r.z >> 18);
 }
 
+// Node n of a strip (StripPlan) and the position of its entry; n known to the
+// compiler.
+__device__ __forceinline__ unsigned strip_node(const uint4 &rec, int n) {
+  return ((n < 3 ? rec.x : rec.y) >> (10 * (n % 3))) & 1023u;
+}
+__device__ __forceinline__ unsigned strip_entry(const uint4 &rec, uint32_t rec2, int n) {
+  return ((n < 2 ? rec.z : n < 4 ? rec.w : rec2) >> (14 * (n % 2))) & 16383u;
+}
+
 // Zero the LDS entry list: the padding entries of the node runs (never
 // written by an element) must read as zero.
 template <typename T, int PT>

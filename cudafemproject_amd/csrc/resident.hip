@@ -12,7 +12,8 @@
 // What bounds it, in kcycles of 2.4 GHz: an iteration's (a step's) trip through
 // memory (from the first store to the last load 3.5 at 10 workgroups, 4 to 7 at
 // 100 to 230) and the element phase of one patch on one compute unit (FP64
-// tets: 4 for 768 elements, 12 for 1536, bound by LDS traffic and FP64 issue).
+// tets: 4 for 768 elements; for 1536 12 one by one, 8 in strips; bound by LDS
+// traffic and FP64 issue).
 // Measured, launch per kernel -> resident:
 //   us per PCG iteration: 12x7 plate FP64 10.2 -> 1.7 (one workgroup, no
 //   trip), 64x32 plate FP64 10.2 -> 3.7, 24^3 hexes FP64 14.0 -> 6.9 and mixed
@@ -21,8 +22,8 @@
 //   launch-per-kernel recurrence has it, 5.3 for the 64x32 plate, 9.0 and 8.2,
 //   16.7 and 12.5;
 //   us per explicit step: 63x31 plate FP32 with receivers 9.1 -> 2.0, 160x80
-//   plate FP64 5.7 -> 2.3, 16x16x256 column FP64 15.5 -> 10.1 and FP32
-//   10.7 -> 6.3;
+//   plate FP64 5.7 -> 2.3, 16x16x256 column FP64 15.5 -> 8.2 and FP32
+//   10.7 -> 5.9;
 //   20 implicit steps of an 11x11x80 column (870 iterations) 13.4 -> 5.7 ms.
 //
 // Every workgroup forms every scalar itself from all partials in the same
@@ -54,6 +55,7 @@
 #include "patch_common.h"
 #include "resident.h"
 #include "resident_dev.h"
+#include "strip.h"
 
 namespace femgpu {
 
@@ -90,6 +92,9 @@ struct ResMesh {
   const PatchInfo *patches;
   const uint32_t *erec_s;
   int emax;
+  const uint4 *strip_rec;  // strips (NE = 3)
+  const uint32_t *strip_rec2;
+  int strip_stride;
   const int32_t *pgid, *pslot;
   const uint16_t *pend;
   int pstride;             // of pgid, pslot, pend
@@ -106,18 +111,20 @@ struct ResMesh {
 // One patch in one workgroup of PT threads for a whole launch.  NE = 1: one
 // element and one DOF per thread (thread t: node t / DIM, component t % DIM),
 // the element entries of every component in LDS at once, one barrier instead
-// of 2 DIM - 1 per product.  NE = 2 (patches of up to 512 nodes): two elements
-// per thread, a node with its DIM DOFs in each of the first threads, the
-// components' entries in turn through one list.
+// of 2 DIM - 1 per product.  Else (patches of up to 512 nodes) a node with its
+// DIM DOFs in each of the first threads and the components' entries in turn
+// through one list, with NE = 3 a strip of up to three elements per thread
+// (StripPlan), with NE = 2 two elements one by one.
 template <typename T, int DIM, int PT, int NE>
 struct ResPatch {
-  static constexpr bool DOF = NE == 1;
+  static constexpr bool DOF = NE == 1, STRIPS = NE == 3;
   static constexpr int ND = DOF ? 1 : DIM;     // DOFs per thread
   static constexpr int COMPS = DOF ? DIM : 1;  // components in the entry list
   static constexpr int NPE = DIM + 1, NDE = DIM * NPE;
+  static constexpr int NS = DIM + STRIP_ELEMS;  // nodes of a full strip
   // the elements' geometry in registers for the whole launch, where they hold
   // it (FP64 with two elements per thread: formed again in every product)
-  static constexpr bool GEOM = DOF || sizeof(T) == 4;
+  static constexpr bool GEOM = NE != 2 || sizeof(T) == 4;
   static constexpr int NGEO = GEOM ? DIM * DIM + 1 : 1;
 
   T *s_c, *s_x, *s_res, *s_in;
@@ -126,7 +133,9 @@ struct ResPatch {
   double *s_red;
   int ent, n_elem, n_in, in_start;
   T lam, mu;
-  uint3 rec[NE];
+  uint3 rec[STRIPS ? 1 : NE];  // elements
+  uint4 srec;                  // the strip
+  uint32_t srec2;
   T esc[NE];
   bool has, own, first;  // first: this patch accounts for the node
   unsigned fm;           // fixed DOFs of this thread
@@ -163,12 +172,21 @@ struct ResPatch {
     in_start = E.in_start;
     lam = a.lam;
     mu = a.mu;
-    const uint3 *prec = reinterpret_cast<const uint3 *>(a.erec_s) + size_t(pid) * unsigned(a.emax);
+    if constexpr (STRIPS) {
+      const size_t i = size_t(pid) * a.strip_stride + t;
+      srec = a.strip_rec[i];
+      srec2 = a.strip_rec2[i];
 #pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      const int i = t + e * PT;
-      rec[e] = prec[unsigned(min(i, a.emax - 1))];
-      esc[e] = a.escale && i < n_elem ? a.escale[P.elem_start + i] : T(1);
+      for (int e = 0; e < NE; ++e)
+        esc[e] = a.escale ? a.escale[(size_t(pid) * NE + e) * a.strip_stride + t] : T(1);
+    } else {
+      const uint3 *prec = reinterpret_cast<const uint3 *>(a.erec_s) + size_t(pid) * unsigned(a.emax);
+#pragma unroll
+      for (int e = 0; e < NE; ++e) {
+        const int i = t + e * PT;
+        rec[e] = prec[unsigned(min(i, a.emax - 1))];
+        esc[e] = a.escale && i < n_elem ? a.escale[P.elem_start + i] : T(1);
+      }
     }
     clear_entries<T, PT>(s_res, COMPS * ent);
     const int k = DOF ? t / DIM : t;
@@ -203,8 +221,14 @@ struct ResPatch {
     if constexpr (GEOM) {
 #pragma unroll
       for (int e = 0; e < NE; ++e) {
-        int l[4], q[4];
-        decode_rec(rec[e], l, q);
+        int l[4] = {0, 0, 0, 0}, q[4];
+        if constexpr (STRIPS) {
+          // (node 0 past a strip's end: its elements are not formed)
+#pragma unroll
+          for (int n = 0; n < NPE; ++n) l[n] = int(strip_node(srec, e + n));
+        } else {
+          decode_rec(rec[e], l, q);
+        }
         T X[NDE];
 #pragma unroll
         for (int n = 0; n < NPE; ++n)
@@ -261,6 +285,42 @@ struct ResPatch {
       }
       __syncthreads();
       y[0] = run_sum<T>(s_res + (t % DIM) * ent, b0, b1);
+    } else if constexpr (STRIPS) {
+      const int count = int(srec.x >> 30);
+      T F[NS * DIM];
+      if (count) {
+        T U[NS * DIM];
+        auto load = [&](int n) {
+          const unsigned l = strip_node(srec, n) * unsigned(DIM);
+#pragma unroll
+          for (int c = 0; c < DIM; ++c) U[n * DIM + c] = s_x[l + c];
+        };
+#pragma unroll
+        for (int n = 0; n < DIM; ++n) load(n);
+#pragma unroll
+        for (int k = 0; k < STRIP_ELEMS; ++k) {
+#pragma unroll
+          for (int c = 0; c < DIM; ++c) F[(k + DIM) * DIM + c] = T(0);
+          if (k < count) {
+            load(k + DIM);
+            T f[NDE];
+            (void)elem_force_geo<T, DIM>(geo[k], U + k * DIM, lam, mu, f);
+#pragma unroll
+            for (int i = 0; i < NDE; ++i)
+              F[k * DIM + i] = k == 0 || i >= DIM * DIM ? f[i] : F[k * DIM + i] + f[i];
+          }
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        if (c) __syncthreads();
+        if (count)
+#pragma unroll
+          for (int n = 0; n < NS; ++n)
+            if (n <= DIM || n < count + DIM) s_res[strip_entry(srec, srec2, n)] = F[n * DIM + c];
+        __syncthreads();
+        y[c] = run_sum<T>(s_res, b0, b1);
+      }
     } else {
       // (corner 0's force is minus the others', formed again at the scatter:
       // fewer live registers)
@@ -771,6 +831,27 @@ __global__ __launch_bounds__(PT) void k_dyn_resident(DynArgs<T> a) {
     }
 }
 
+// The kernels' forms: 768 threads with one element and one DOF each (patches
+// of up to 256 nodes and 768 elements; 512 threads hold the 2D patches, which
+// mostly run into the node limit first); patches of up to 512 nodes: 512 threads
+// with a strip and a node each, whose registers hold the strips' geometry, else
+// 768 with two elements each (us per explicit step of the 16x16x256 column FP64
+// 10.2 -> 8.4 and FP32 6.3 -> 5.8, per implicit iteration 15.2 -> 12.0; with 640
+// threads for more strips a 40^3 cube slows from 14.5 to 15.4 us per iteration).
+struct Form {
+  int threads, ne;
+};
+constexpr int RES_NODES[] = {0, 256, 512}, RES_THREADS = 768, RES_STRIPS = 512;
+constexpr int RES_LDS_MAX = 160 * 1024 - 256;
+
+Form res_form(const DevMesh &dm) {
+  if (dm.pn <= RES_NODES[1] && dm.emax <= RES_THREADS)
+    return {dm.dim == 2 && dm.emax <= 512 ? 512 : RES_THREADS, 1};
+  if (dm.pn > RES_NODES[2]) return {0, 0};
+  if (has_strips(dm) && dm.strip_threads <= RES_STRIPS) return {RES_STRIPS, 3};
+  return dm.emax <= 2 * RES_THREADS ? Form{RES_THREADS, 2} : Form{0, 0};
+}
+
 template <typename T>
 ResMesh<T> res_mesh(const DevMesh &dm) {
   ResMesh<T> a{};
@@ -779,23 +860,27 @@ ResMesh<T> res_mesh(const DevMesh &dm) {
   a.emax = dm.emax;
   a.pgid = dm.pgid;
   a.pslot = dm.pslot;
-  a.pend = dm.pend;
+  const bool strips = res_form(dm).ne == 3;
+  a.pend = strips ? dm.strip_pend : dm.pend;
+  a.strip_rec = dm.strip_rec;
+  a.strip_rec2 = dm.strip_rec2;
+  a.strip_stride = dm.strip_stride;
   a.pstride = dm.patch_threads;
   a.fixmask = dm.fixmask;
   if constexpr (sizeof(T) == 8) {
     a.coords = reinterpret_cast<const T *>(dm.coords64);
-    a.escale = reinterpret_cast<const T *>(dm.escale64);
+    a.escale = strips ? dm.strip_escale64 : dm.escale64;
     a.diagK = reinterpret_cast<const T *>(dm.diag64);
   } else {
     a.coords = reinterpret_cast<const T *>(dm.coords32);
-    a.escale = reinterpret_cast<const T *>(dm.escale32);
+    a.escale = strips ? dm.strip_escale32 : dm.escale32;
     a.diagK = reinterpret_cast<const T *>(dm.diag32);
   }
   a.lam = T(dm.lam);
   a.mu = T(dm.mu);
   a.np = dm.np;
   a.p8 = (dm.np + 7) / 8;
-  a.ent = dm.ent;
+  a.ent = strips ? dm.strip_ent : dm.ent;
   a.pn = dm.pn;
   a.xpatch = dm.xpatch;
   a.out_entry = dm.x_out_entry;
@@ -808,25 +893,10 @@ ResMesh<T> res_mesh(const DevMesh &dm) {
   return a;
 }
 
-// The kernels' forms: 768 threads with one element and one DOF each (patches
-// of up to 256 nodes and 768 elements; 512 threads hold the 2D patches, which
-// mostly run into the node limit first), else two elements each and a node per
-// thread (up to 512 nodes and 1536 elements).
-struct Form {
-  int threads, ne;
-};
-constexpr int RES_NODES[] = {0, 256, 512}, RES_THREADS = 768;
-constexpr int RES_LDS_MAX = 160 * 1024 - 256;
-
-Form res_form(const DevMesh &dm) {
-  if (dm.pn <= RES_NODES[1] && dm.emax <= RES_THREADS)
-    return {dm.dim == 2 && dm.emax <= 512 ? 512 : RES_THREADS, 1};
-  if (dm.pn <= RES_NODES[2] && dm.emax <= 2 * RES_THREADS) return {RES_THREADS, 2};
-  return {0, 0};
-}
-
 int res_lds_bytes(const DevMesh &dm, int tb) {
-  return res_lds(dm.dim, tb, dm.pn, dm.ent, res_form(dm).ne == 1 ? dm.dim : 1, dm.x_in_max, dm.x_src_max)
+  const bool strips = res_form(dm).ne == 3;
+  return res_lds(dm.dim, tb, dm.pn, strips ? dm.strip_ent : dm.ent,
+                 res_form(dm).ne == 1 ? dm.dim : 1, dm.x_in_max, dm.x_src_max)
       .total;
 }
 
@@ -840,6 +910,7 @@ using ImplKernel = void (*)(ImplArgs<T>);
 #define FEMGPU_RES_KERNEL(NAME, KIND)                                                       \
   template <typename T>                                                                     \
   KIND<T> NAME##_of(int dim, Form f) {                                                      \
+    if (f.ne == 3) return dim == 3 ? KIND<T>(NAME<T, 3, 512, 3>) : KIND<T>(NAME<T, 2, 512, 3>); \
     if (f.ne == 2) return dim == 3 ? KIND<T>(NAME<T, 3, 768, 2>) : KIND<T>(NAME<T, 2, 768, 2>); \
     if (dim == 3) return NAME<T, 3, 768, 1>;                                                \
     return f.threads == 512 ? KIND<T>(NAME<T, 2, 512, 1>) : KIND<T>(NAME<T, 2, 768, 1>);    \
@@ -943,7 +1014,7 @@ template <typename T>
 static hipError_t prepare_t() {
   hipError_t e = hipSuccess, r;
   for (int dim : {2, 3})
-    for (Form f : {Form{512, 1}, Form{768, 1}, Form{768, 2}})
+    for (Form f : {Form{512, 1}, Form{768, 1}, Form{512, 3}, Form{768, 2}})
       for (const void *fn : {reinterpret_cast<const void *>(k_pcg_resident_of<T>(dim, f)),
                              reinterpret_cast<const void *>(k_dyn_resident_of<T>(dim, f)),
                              reinterpret_cast<const void *>(k_impl_resident_of<T>(dim, f))})

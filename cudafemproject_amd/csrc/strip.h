@@ -14,9 +14,9 @@ namespace femgpu {
 // Threads of a strip workgroup: at most a quarter more than the patch's nodes.
 constexpr int STRIP_THREADS_MAX = 640;
 
-// Strips are planned for plans of more than RES_PATCHES_MAX patches of up to 512
-// threads (the others run resident, resident.h) where every patch has at most
-// 5/4 as many strips as threads.
+// Strips are planned for plans of 512 threads and for those of 256 with more than
+// RES_PATCHES_MAX patches (the others run resident with an element per thread,
+// resident.h), where every patch has at most 5/4 as many strips as threads.
 inline bool has_strips(const DevMesh &dm) { return dm.strip_rec != nullptr; }
 
 // Whether the kernels of arithmetic T take strips.  In FP64 not with a wave more

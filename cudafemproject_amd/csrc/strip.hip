@@ -219,8 +219,7 @@ __global__ __launch_bounds__(STRIP_THREADS_MAX)
   if (count) {
     T X[NS * DIM], U[NS * DIM];
     auto load = [&](int n) {
-      const uint32_t w = n < 3 ? rec.x : rec.y;
-      const unsigned l = ((w >> (10 * (n % 3))) & 1023u) * unsigned(DIM);
+      const unsigned l = strip_node(rec, n) * unsigned(DIM);
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
         X[n * DIM + c] = s_c[l + c];
@@ -251,11 +250,8 @@ __global__ __launch_bounds__(STRIP_THREADS_MAX)
     if (c) lds_barrier();
     if (count) {
 #pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        const uint32_t w = n < 2 ? rec.z : n < 4 ? rec.w : rec2;
-        const unsigned q = (w >> (14 * (n % 2))) & 16383u;
-        if (n <= DIM || n < count + DIM) s_res[q] = F[n * DIM + c];
-      }
+      for (int n = 0; n < NS; ++n)
+        if (n <= DIM || n < count + DIM) s_res[strip_entry(rec, rec2, n)] = F[n * DIM + c];
     }
     lds_barrier();
     using V4 = typename Vec4<T>::type;
