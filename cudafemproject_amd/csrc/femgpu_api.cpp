@@ -1144,9 +1144,9 @@ int matvec_noalloc_t(femgpu_ctx *ctx, const double *x, double *y) {
   T *xi = reinterpret_cast<T *>(base);
   T *yi = reinterpret_cast<T *>(base + vec);
   T *part = reinterpret_cast<T *>(base + 2 * vec);
-  // straight from x and to y where the plan has strips and the two don't overlap
-  if (femgpu::has_strips(ctx->dm) && (x + nd <= y || y + nd <= x)) {
-    femgpu::launch_strip_matvec_user<T>(ctx->dm, ctx->d_node_perm, x, y, part, ctx->stream);
+  // straight from x and to y where the two don't overlap
+  if (x + nd <= y || y + nd <= x) {
+    femgpu::launch_matvec_user<T>(ctx->dm, ctx->d_node_perm, x, y, part, ctx->stream);
     HIPCHK(hipGetLastError());
     return FEMGPU_OK;
   }

@@ -107,6 +107,12 @@ int grid_blocks(int64_t n);
 // before any launch or capture.
 hipError_t prepare_kernels();
 
+// y = K x on FP64 vectors in user order (not overlapping; 0 at nodes no element
+// references), in arithmetic T.
+template <typename T>
+void launch_matvec_user(const DevMesh &dm, const int32_t *node_perm, const double *x, double *y,
+                        T *partial, hipStream_t s);
+
 // y = K x (standalone: patch kernel + interface gather).
 template <typename T>
 void launch_matvec(const DevMesh &dm, const T *x, T *y, T *partial, hipStream_t s);

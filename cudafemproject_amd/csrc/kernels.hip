@@ -49,7 +49,10 @@ using namespace patch;
 // explicit step in one launch: MODE 3, then the corrector of the owned nodes
 // from their complete K d~; an interface node is corrected one launch late,
 // by every patch that holds it, from the previous launch's slots (the first
-// patch stores the result).
+// patch stores the result).  MODE 5: MODE 0 on FP64 vectors in user order,
+// through the node ids, which saves the two launches that permute (FP64 product
+// on device vectors, us: 12x7 plate 10.9 -> 3.4, 64x32 plate 12.8 -> 5.9, 24^3
+// hexes 13.5 -> 9.4).
 
 // FP64 PCG: x += alpha p in the next iteration's patch kernel (k_ebe_patch
 // MODE 1); FP32: in the update kernel.
@@ -96,6 +99,9 @@ struct PatchArgs {
   int step_off;
   const T *invM;            // lumped inverse mass
   T c2, c3, alpha, scale;   // GN22 corrector and mass-damping coefficients
+  const int32_t *perm;      // MODE 5: user node of a node; x and y
+  const double *xu;
+  double *yu;
 };
 
 // One workgroup per patch, one patch node per thread (phases A and C), up to
@@ -109,7 +115,7 @@ struct PatchArgs {
 // and is slower; everything else keeps the allocator's choice.
 template <typename T, int MODE, int PT>
 struct PatchWaves {
-  static constexpr int value = PT == 256 && sizeof(T) == 8 && (MODE == 0 || MODE == 1) ? 4 : 1;
+  static constexpr int value = PT == 256 && sizeof(T) == 8 && (MODE == 0 || MODE == 1 || MODE == 5) ? 4 : 1;
 };
 
 template <typename T, int DIM, int MODE, int PT>
@@ -219,7 +225,7 @@ void k_ebe_patch(PatchArgs<T> a) {
   // element's record here and the others after the node loads: every
   // workgroup stages its nodes at the same time, bandwidth-bound, and the
   // later records arrive while the first element is computed.
-  constexpr bool LATE_REC = MODE == 0 || MODE == 1;
+  constexpr bool LATE_REC = MODE == 0 || MODE == 1 || MODE == 5;
   uint3 rec[EPT];
   T esc[EPT];
   // per-patch bases (uniform) and small unsigned thread offsets: scalar
@@ -252,7 +258,7 @@ void k_ebe_patch(PatchArgs<T> a) {
   // element offsets of the node and its slot, 32-bit (few live registers);
   // the node's signed, so that its components' accesses merge into one
   // vector access (the slot's stay apart: one register fewer at the peak)
-  int go = 0;
+  int go = 0, uo = 0;
   unsigned so = 0;
   int b0 = 0, b1 = 0;
   unsigned fm = 0;
@@ -276,9 +282,10 @@ void k_ebe_patch(PatchArgs<T> a) {
 #pragma unroll
     for (int c = 0; c < DIM; ++c) s_c[k * DIM + c] = a.coords[go + c];
     if constexpr (MODE != 2) fm = a.fixmask[gid] & FMASK;
-    if constexpr (MODE == 0) {
+    if constexpr (MODE == 5) uo = a.perm[gid] * DIM;
+    if constexpr (MODE == 0 || MODE == 5) {
 #pragma unroll
-      for (int c = 0; c < DIM; ++c) xin[c] = a.x[go + c];
+      for (int c = 0; c < DIM; ++c) xin[c] = MODE == 5 ? T(a.xu[uo + c]) : a.x[go + c];
     } else if constexpr (MODE == 1) {
       T pv[DIM];
 #pragma unroll
@@ -364,7 +371,7 @@ void k_ebe_patch(PatchArgs<T> a) {
   const unsigned fm = fmf & FMASK;
   const bool first = (fmf & 0x10u) != 0u;
 
-  if constexpr (MODE == 0 || MODE == 1) {
+  if constexpr (MODE == 0 || MODE == 1 || MODE == 5) {
     if (has_node) {
 #pragma unroll
       for (int c = 0; c < DIM; ++c) xin[c] = s_x[k * DIM + c];
@@ -374,6 +381,8 @@ void k_ebe_patch(PatchArgs<T> a) {
           if ((fm >> c) & 1u) {
             if constexpr (MODE == 0)
               xin[c] = a.x[go + c];
+            else if constexpr (MODE == 5)
+              xin[c] = T(a.xu[uo + c]);
             else if (own)
               xin[c] = a.p[go + c];
             else
@@ -431,7 +440,10 @@ void k_ebe_patch(PatchArgs<T> a) {
           if (a.sh.m) v += cM * a.sh.m[go + c] * xin[c];
           acc_en += double(xin[c]) * double(v);
         }
-        a.y[go + c] = v;
+        if constexpr (MODE == 5)
+          a.yu[uo + c] = double(v);
+        else
+          a.y[go + c] = v;
       }
     } else {
 #pragma unroll
@@ -468,6 +480,26 @@ __global__ __launch_bounds__(NT) void k_iface_gather(int64_t n_owned, int64_t n_
   add_slots<T, DIM>(partial, slot_start[s], slot_start[s + 1], acc);
 #pragma unroll
   for (int c = 0; c < DIM; ++c) y[(n_owned + s) * DIM + c] = acc[c];
+}
+
+// Interface nodes of a user-order product, and 0 at nodes no element references.
+template <typename T>
+__global__ __launch_bounds__(NT) void k_iface_user(int64_t n_owned, int64_t n_active, int64_t nn, int dim,
+                                                   const int32_t *slot_start, const int32_t *perm,
+                                                   const T *partial, double *y) {
+  const int64_t n = n_owned + int64_t(blockIdx.x) * NT + threadIdx.x;
+  if (n >= nn) return;
+  const int64_t s = n - n_owned, u = int64_t(perm[n]) * dim;
+  const int j0 = n < n_active ? slot_start[s] : 0, j1 = n < n_active ? slot_start[s + 1] : 0;
+  if (dim == 3) {
+    T acc[3] = {T(0), T(0), T(0)};
+    add_slots<T, 3>(partial, j0, j1, acc);
+    for (int c = 0; c < 3; ++c) y[u + c] = double(acc[c]);
+  } else {
+    T acc[2] = {T(0), T(0)};
+    add_slots<T, 2>(partial, j0, j1, acc);
+    for (int c = 0; c < 2; ++c) y[u + c] = double(acc[c]);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1272,7 +1304,8 @@ hipError_t prepare_kernels() {
   FEMGPU_ATTR(T, D, 3, 256) FEMGPU_ATTR(T, D, 0, 512) FEMGPU_ATTR(T, D, 1, 512)                \
   FEMGPU_ATTR(T, D, 2, 512) FEMGPU_ATTR(T, D, 3, 512) FEMGPU_ATTR(T, D, 0, 1024)               \
   FEMGPU_ATTR(T, D, 1, 1024) FEMGPU_ATTR(T, D, 2, 1024) FEMGPU_ATTR(T, D, 3, 1024)          \
-  FEMGPU_ATTR(T, D, 4, 256) FEMGPU_ATTR(T, D, 4, 512) FEMGPU_ATTR(T, D, 4, 1024)
+  FEMGPU_ATTR(T, D, 4, 256) FEMGPU_ATTR(T, D, 4, 512) FEMGPU_ATTR(T, D, 4, 1024)          \
+  FEMGPU_ATTR(T, D, 5, 256) FEMGPU_ATTR(T, D, 5, 512) FEMGPU_ATTR(T, D, 5, 1024)
   FEMGPU_ATTR_TD(double, 3)
   FEMGPU_ATTR_TD(double, 2)
   FEMGPU_ATTR_TD(float, 3)
@@ -1321,6 +1354,28 @@ void launch_matvec(const DevMesh &dm, const T *x, T *y, T *partial, hipStream_t 
       hipLaunchKernelGGL((k_iface_gather<T, 2>), dim3(g), dim3(NT), 0, s, dm.n_owned, dm.n_iface,
                          dm.slot_start, partial, y);
   }
+}
+
+template <typename T>
+void launch_matvec_user(const DevMesh &dm, const int32_t *node_perm, const double *x, double *y,
+                        T *partial, hipStream_t s) {
+  if (has_strips(dm)) {
+    launch_strip_matvec_user<T>(dm, x, y, partial, s);
+  } else {
+    PatchArgs<T> a = patch_args<T>(dm);
+    a.perm = node_perm;
+    a.xu = x;
+    a.yu = y;
+    a.partial = partial;
+    if (dm.dim == 3)
+      launch_patch<T, 3, 5>(dm, a, s);
+    else
+      launch_patch<T, 2, 5>(dm, a, s);
+  }
+  const int64_t n = dm.nn - dm.n_owned;
+  if (n > 0)
+    hipLaunchKernelGGL((k_iface_user<T>), dim3(int((n + NT - 1) / NT)), dim3(NT), 0, s, dm.n_owned,
+                       dm.n_active, dm.nn, dm.dim, dm.slot_start, node_perm, partial, y);
 }
 
 template <typename T>
@@ -1639,6 +1694,8 @@ void launch_reset_scalars(CgScalars *sc, int kind, double eps, int max_iter, hip
 #define FEMGPU_INST(T)                                                                          \
   template void launch_matvec<T>(const DevMesh &, const T *, T *, T *, hipStream_t);           \
   template void launch_matvec_patch<T>(const DevMesh &, const T *, T *, T *, hipStream_t);     \
+  template void launch_matvec_user<T>(const DevMesh &, const int32_t *, const double *,       \
+                                      double *, T *, hipStream_t);                             \
   template void launch_diag<T>(const DevMesh &, T *, T *, hipStream_t);                        \
   template void launch_mass<T>(const DevMesh &, double, double, double *, double *, T *, T *,  \
                                hipStream_t);                                                   \

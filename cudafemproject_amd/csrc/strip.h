@@ -32,10 +32,10 @@ inline bool use_strips(const DevMesh &dm) {
 template <typename T>
 void launch_strip_matvec(const DevMesh &dm, const T *x, T *y, T *partial, hipStream_t s);
 
-// y = K x on FP64 vectors in user order (not overlapping), in arithmetic T.
+// The same on FP64 vectors in user order (launch_matvec_user).
 template <typename T>
-void launch_strip_matvec_user(const DevMesh &dm, const int32_t *node_perm, const double *x, double *y,
-                              T *partial, hipStream_t s);
+void launch_strip_matvec_user(const DevMesh &dm, const double *x, double *y, T *partial,
+                              hipStream_t s);
 
 // The patch kernel of a PCG iteration (launch_pcg_iter).
 template <typename T>

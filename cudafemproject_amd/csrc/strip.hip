@@ -29,8 +29,6 @@ namespace {
 using namespace elem;
 using namespace patch;
 
-constexpr int NT = 256;
-
 enum { MATVEC = 0, PCG = 1, USER = 2 };
 
 template <typename T>
@@ -317,26 +315,6 @@ __global__ __launch_bounds__(STRIP_THREADS_MAX)
   }
 }
 
-// Interface nodes of a user-order product, and 0 at nodes no element references.
-template <typename T>
-__global__ __launch_bounds__(NT) void k_iface_user(int64_t n_owned, int64_t n_active, int64_t nn, int dim,
-                                                   const int32_t *slot_start, const int32_t *perm,
-                                                   const T *partial, double *y) {
-  const int64_t n = n_owned + int64_t(blockIdx.x) * NT + threadIdx.x;
-  if (n >= nn) return;
-  const int64_t s = n - n_owned, u = int64_t(perm[n]) * dim;
-  const int j0 = n < n_active ? slot_start[s] : 0, j1 = n < n_active ? slot_start[s + 1] : 0;
-  if (dim == 3) {
-    T acc[3] = {T(0), T(0), T(0)};
-    add_slots<T, 3>(partial, j0, j1, acc);
-    for (int c = 0; c < 3; ++c) y[u + c] = double(acc[c]);
-  } else {
-    T acc[2] = {T(0), T(0)};
-    add_slots<T, 2>(partial, j0, j1, acc);
-    for (int c = 0; c < 2; ++c) y[u + c] = double(acc[c]);
-  }
-}
-
 template <typename T>
 StripArgs<T> strip_args(const DevMesh &dm) {
   StripArgs<T> a{};
@@ -389,17 +367,13 @@ void launch_strip_matvec(const DevMesh &dm, const T *x, T *y, T *partial, hipStr
 }
 
 template <typename T>
-void launch_strip_matvec_user(const DevMesh &dm, const int32_t *node_perm, const double *x, double *y,
-                              T *partial, hipStream_t s) {
+void launch_strip_matvec_user(const DevMesh &dm, const double *x, double *y, T *partial,
+                              hipStream_t s) {
   StripArgs<T> a = strip_args<T>(dm);
   a.xu = x;
   a.yu = y;
   a.partial = partial;
   launch<T, USER>(dm, a, s);
-  const int64_t n = dm.nn - dm.n_owned;
-  if (n > 0)
-    hipLaunchKernelGGL((k_iface_user<T>), dim3(int((n + NT - 1) / NT)), dim3(NT), 0, s, dm.n_owned,
-                       dm.n_active, dm.nn, dm.dim, dm.slot_start, node_perm, partial, y);
 }
 
 template <typename T>
@@ -430,8 +404,8 @@ hipError_t prepare_strip_kernels() {
 
 #define FEMGPU_STRIP_INST(T)                                                                       \
   template void launch_strip_matvec<T>(const DevMesh &, const T *, T *, T *, hipStream_t);         \
-  template void launch_strip_matvec_user<T>(const DevMesh &, const int32_t *, const double *,      \
-                                            double *, T *, hipStream_t);                           \
+  template void launch_strip_matvec_user<T>(const DevMesh &, const double *, double *, T *,        \
+                                            hipStream_t);                                          \
   template void launch_strip_pcg<T>(const DevMesh &, const StripPcg<T> &, hipStream_t);
 FEMGPU_STRIP_INST(double)
 FEMGPU_STRIP_INST(float)
