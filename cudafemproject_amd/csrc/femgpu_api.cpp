@@ -1258,20 +1258,25 @@ int upload_plan(femgpu_ctx *ctx) {
   if (dm.np <= femgpu::RES_PATCHES_MAX) {
     femgpu::ExchangePlan x;
     if (femgpu::build_exchange(P, x)) {
-      femgpu::ExchangePatch *xp;
-      uint32_t *oe;
-      uint16_t *os, *ip, *se, *op;
-      if ((st = upload(ctx, "x_patch", x.patches, &xp)) || (st = upload(ctx, "x_oe", x.out_entry, &oe)) ||
-          (st = upload(ctx, "x_os", x.out_src, &os)) || (st = upload(ctx, "x_ip", x.in_pos, &ip)) ||
-          (st = upload(ctx, "x_se", x.src_end, &se)) || (st = upload(ctx, "x_op", x.own_pos, &op)))
-        return st;
-      HIPCHK(hipStreamSynchronize(ctx->stream));  // x goes out of scope
-      dm.xpatch = xp;
-      dm.x_out_entry = oe;
-      dm.x_out_src = os;
-      dm.x_in_pos = ip;
-      dm.x_src_end = se;
-      dm.x_own_pos = op;
+      // (one buffer and one copy: each costs a small mesh some 10 us)
+      std::vector<uint8_t> all;
+      auto add = [&](const auto &v) {
+        const size_t at = (all.size() + 15) & ~size_t(15);
+        all.resize(at + v.size() * sizeof(v[0]));
+        if (!v.empty()) std::memcpy(all.data() + at, v.data(), v.size() * sizeof(v[0]));
+        return at;
+      };
+      const size_t xp = add(x.patches), oe = add(x.out_entry), os = add(x.out_src), ip = add(x.in_pos),
+                   se = add(x.src_end), op = add(x.own_pos);
+      uint8_t *t;
+      if ((st = upload(ctx, "x_tables", all, &t))) return st;
+      HIPCHK(hipStreamSynchronize(ctx->stream));  // all goes out of scope
+      dm.xpatch = reinterpret_cast<const femgpu::ExchangePatch *>(t + xp);
+      dm.x_out_entry = reinterpret_cast<const uint32_t *>(t + oe);
+      dm.x_out_src = reinterpret_cast<const uint16_t *>(t + os);
+      dm.x_in_pos = reinterpret_cast<const uint16_t *>(t + ip);
+      dm.x_src_end = reinterpret_cast<const uint16_t *>(t + se);
+      dm.x_own_pos = reinterpret_cast<const uint16_t *>(t + op);
       dm.x_in_max = x.n_in_max;
       dm.x_src_max = x.n_src_max;
       dm.x_entries = x.n_entries;
@@ -1327,6 +1332,25 @@ int upload_plan(femgpu_ctx *ctx) {
   return ensure_fix(ctx);
 }
 
+// The kernels' LDS limits, once per device: more than a hundred calls of the
+// runtime, a quarter of the time that a context of a small mesh takes to set
+// up.
+hipError_t prepare_device(int device) {
+  static std::mutex mu;
+  static std::map<int, bool> ready;
+  std::lock_guard<std::mutex> lock(mu);
+  if (ready[device]) return hipSuccess;
+  hipError_t e;
+  if ((e = femgpu::prepare_kernels()) != hipSuccess || (e = femgpu::prepare_cg1_kernels()) != hipSuccess ||
+      (e = femgpu::prepare_bl_kernels()) != hipSuccess ||
+      (e = femgpu::prepare_resident_kernels()) != hipSuccess ||
+      (e = femgpu::prepare_br_kernels()) != hipSuccess ||
+      (e = femgpu::prepare_strip_kernels()) != hipSuccess)
+    return e;
+  ready[device] = true;
+  return hipSuccess;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1348,12 +1372,7 @@ int femgpu_create(femgpu_ctx **out, int device_ordinal) {
   for (auto &e : ctx->ev_poll) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCHK(hipEventCreate(&ctx->ev0));
   HIPCHK(hipEventCreate(&ctx->ev1));
-  HIPCHK(femgpu::prepare_kernels());
-  HIPCHK(femgpu::prepare_cg1_kernels());
-  HIPCHK(femgpu::prepare_bl_kernels());
-  HIPCHK(femgpu::prepare_resident_kernels());
-  HIPCHK(femgpu::prepare_br_kernels());
-  HIPCHK(femgpu::prepare_strip_kernels());
+  HIPCHK(prepare_device(device_ordinal));
   *out = c.release();
   return FEMGPU_OK;
 }
