@@ -204,7 +204,7 @@ def bench_column(args, F):
         "fp32_vs_fp64_rel_displacement_diff": float(np.linalg.norm(u32 - u64) / np.linalg.norm(u64)),
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "one explicit step fp64 (k_ebe_patch MODE 4: predictor, EbE matvec, corrector)",
+                     "kernel": "one explicit step fp64 (k_dyn_resident: predictor, EbE matvec, corrector)",
                      "bytes_per_launch": b64},
         "fp32_step_gbs": b32 / (us32 * 1e-6) / 1e9,
         "cpu_baseline": None,
@@ -415,7 +415,7 @@ def bench_batch(args, F):
         "mixed_vs_fp64_max_rel_diff": diff, "vs_single_solver_max_rel_diff": max(chk),
         "roofline": {"bound": "hbm", "achieved": ach, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": ach / HBM_PEAK_GBS, "traffic": None,
-                     "kernel": "k_bl_patch<float,2,4,1> + k_bl_update<float,2,4> (all iterations)",
+                     "kernel": "k_batch_resident<4,8> (all iterations; bytes as the launch-per-iteration form streams them)",
                      "bytes_per_launch": tot},
         "cpu_baseline": None,
     }
