@@ -684,7 +684,7 @@ def main():
     achieved = b32 / mv32 / 1e9
     roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-                "kernel": f"EbE matvec fp32 (k_ebe_patch + k_iface_gather), cube64, "
+                "kernel": f"EbE matvec fp32 (k_strip + k_iface_gather), cube64, "
                           f"{t32[0]}-thread patches of {t32[1]} elements",
                 "bytes_per_launch": b32}
 
