@@ -844,6 +844,13 @@ int res_receivers(femgpu_ctx *ctx, int max_samples, T *traces, femgpu::ResRecv<T
   int st;
   if ((st = upload(ctx, "recv_of", of, &pof)) || (st = upload(ctx, "recv_next", next, &pnext))) return st;
   HIPCHK(hipStreamSynchronize(ctx->stream));  // the vectors go out of scope
+  // no patch holds a node that no element references: its samples are the
+  // state's, zero
+  const bool live = std::all_of(ctx->recv.begin(), ctx->recv.end(), [&](int32_t v) {
+    return ctx->plan.node_inv[size_t(v)] < ctx->dm.n_active;
+  });
+  if (!live)
+    femgpu::launch_fill<T>(traces, int64_t(max_samples) * int64_t(n) * ctx->dim, T(0), ctx->stream);
   r->rec_of = pof;
   r->rec_next = pnext;
   r->n_rec = int(n);
