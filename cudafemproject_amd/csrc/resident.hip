@@ -552,6 +552,8 @@ struct ResSolver {
       const double beta_d = g / g_prev, own = v[2] + beta_d * beta_d * v[4];
       double pq = v[2] + beta_d * (2.0 * v[3] + beta_d * v[4]);
       const T beta = T(beta_d);
+      // (beyond the range of T: the state of the last completed iteration)
+      if (!isfinite(beta)) return 2;
       P.collect(w);
 #pragma unroll
       for (int i = 0; i < ND; ++i) {
@@ -571,7 +573,7 @@ struct ResSolver {
       }
       const double alpha_d = g / pq;
       // (no x or r has changed: the state of the last completed iteration)
-      if (!(pq > 0.0) || !isfinite(alpha_d)) return isfinite(pq) ? 3 : 2;
+      if (!(pq > 0.0) || !isfinite(pq) || !isfinite(alpha_d)) return isfinite(pq) ? 3 : 2;
       g_prev = g;
       const T alpha = T(alpha_d);
 #pragma unroll

@@ -40,3 +40,19 @@ def test_trace_of_a_node_without_elements(ctx, beta2, precision):
             assert np.all(tr[:, 0] == 0.0) and np.all(tr[:, 2] == 0.0)
     finally:
         ctx.set_receivers([], F.RECV_DISPLACEMENT, 1)
+
+
+@pytest.mark.parametrize("precision", [F.FP32, F.MIXED])
+@pytest.mark.parametrize("make", [lambda: plate_problem(12, 7), lambda: plate_problem(40, 20),
+                                  lambda: cube_problem(9)], ids=["plate12x7", "plate40x20", "cube9"])
+def test_loads_beyond_the_range_of_fp32(ctx, make, precision):
+    """r'z of these loads does not fit a float: the solve says so and leaves
+    the last completed iteration's state, which is x = 0."""
+    pb = make()
+    ctx.set_problem(pb)
+    f = ctx.rhs()
+    for e in (80, 100):
+        u, st = ctx.solve_rhs(f * 2.0 ** e, precision, tol=1e-5, tol_kind=F.TOL_REL_RES, max_iter=2000,
+                              raise_on_error=False)
+        assert st["status"] == -3 and st["iterations"] == 0
+        assert np.all(u == 0.0)
