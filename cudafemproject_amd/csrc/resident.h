@@ -55,8 +55,9 @@ struct ResPcg {
 };
 
 // done codes of a resident launch besides CgScalars': 6 the launch did not
-// complete (its workgroups were not on the chip together), 7 cap reached.
-constexpr int RES_ABORTED = 6, RES_CAP = 7;
+// complete (its workgroups were not on the chip together), 7 cap reached; within
+// the kernels 8 the sums underflowed (3 or 4 to the host).
+constexpr int RES_ABORTED = 6, RES_CAP = 7, RES_FAINT = 8;
 
 // The part of the device that a resident launch takes, and of one compute
 // unit that a workgroup takes.

@@ -408,6 +408,15 @@ struct ResPatch {
 // 91.1 ms in all with 8, 16 and 32; iterations within 3 %.)
 constexpr int RENEW = 32;
 
+// Below this r'z every iteration forms s = K p and p's, as the two-trip form
+// does: its own rounding, at the end of the number range no longer relative to the
+// values, would stay in a recurrence.  FP32: z or r of some 2^-100 (a solve of a 9^3
+// cube run on at tolerance 0 left that floor again and was at 1e24 ||f|| after
+// 12000 iterations; so it stays at the floor, as there).  FP64: the sums
+// themselves end at 2^-1074.
+template <typename T>
+constexpr double FAINT = sizeof(T) == 8 ? 0x1p-1000 : 0x1p-160;
+
 template <typename T, int DIM, int PT, int NE>
 struct ResSolver {
   using Patch = ResPatch<T, DIM, PT, NE>;
@@ -543,12 +552,6 @@ struct ResSolver {
       // 1953 so, 1950 in the launch-per-kernel form)
       if ((n_upd & 7) == 0 && q2 < pause) return 5;
       if (n_upd >= last) return RES_CAP;
-      if (fabs(g) < 0x1p-1000) {
-        // (tolerance 0: the sums underflow, which is no breakdown; nothing is left
-        // to change)
-        ++n_upd;
-        continue;
-      }
       const double beta_d = g / g_prev, own = v[2] + beta_d * beta_d * v[4];
       double pq = v[2] + beta_d * (2.0 * v[3] + beta_d * v[4]);
       const T beta = T(beta_d);
@@ -561,7 +564,8 @@ struct ResSolver {
         p[i] = fma(beta, p[i], z[i]);
         s[i] = fma(beta, s[i], w[i]);
       }
-      if (n_upd % RENEW == RENEW - 1 || !(pq > 0x1p-10 * own)) {
+      const bool faint = fabs(g) < FAINT<T>;
+      if (faint || n_upd % RENEW == RENEW - 1 || !(pq > 0x1p-10 * own)) {
         // (or where the sums cancel)
         if (!refresh(p, s, cK, cMm)) return RES_ABORTED;
         double u[RES_SUMS] = {0.0, 0.0, 0.0, 0.0, 0.0};
@@ -573,7 +577,8 @@ struct ResSolver {
       }
       const double alpha_d = g / pq;
       // (no x or r has changed: the state of the last completed iteration)
-      if (!(pq > 0.0) || !isfinite(pq) || !isfinite(alpha_d)) return isfinite(pq) ? 3 : 2;
+      if (!(pq > 0.0) || !isfinite(pq) || !isfinite(alpha_d))
+        return faint ? RES_FAINT : isfinite(pq) ? 3 : 2;
       g_prev = g;
       const T alpha = T(alpha_d);
 #pragma unroll
@@ -626,6 +631,11 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
   if (!a.s.fresh) S.g_prev = a.s.g_prev;
   int done = S.run(r, p, x, d, T(1), cMm, a.s.fresh != 0, a.s.kind, a.s.eps, a.s.max_iter,
                    a.s.it0 + a.s.cap);
+  if (done == RES_FAINT) {
+    // (without a tolerance a solve goes on to its cap, and changes nothing more)
+    if (!(a.s.eps > 0.0)) S.n_upd = a.s.max_iter;
+    done = a.s.eps > 0.0 ? 3 : 4;
+  }
   if (P.first)
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -730,6 +740,7 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
     S.pause = 0.0;
     done = S.run(r, p, x, invd, s.cK, cMm, true, 0, s.eps, s.max_iter, s.max_iter + 1);
     total += S.n_upd;
+    if (done == RES_FAINT) done = 3;
     if (done != 1) break;
 #pragma unroll
     for (int i = 0; i < ND; ++i) {

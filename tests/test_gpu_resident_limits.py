@@ -56,3 +56,55 @@ def test_loads_beyond_the_range_of_fp32(ctx, make, precision):
                               raise_on_error=False)
         assert st["status"] == -3 and st["iterations"] == 0
         assert np.all(u == 0.0)
+
+
+@pytest.mark.parametrize("make", [lambda: plate_problem(40, 20), lambda: cube_problem(9)],
+                         ids=["plate40x20", "cube9"])
+def test_fp32_iterations_past_convergence(ctx, make):
+    """A solve without a tolerance stays where it has converged: thousands of
+    iterations at the floor of the number range leave the residual as it is
+    (to the rounding of its own evaluation: within a factor of two)."""
+    pb = make()
+    ctx.set_problem(pb)
+    f = ctx.rhs()
+    floor = ctx.solve_rhs(f, F.FP32, tol=0.0, max_iter=1000, raise_on_error=False)[1]["rel_res"]
+    assert floor < 1e-2
+    for cap in (5000, 12000, 20000):
+        u, st = ctx.solve_rhs(f, F.FP32, tol=0.0, max_iter=cap, raise_on_error=False)
+        assert st["status"] == -4 and st["iterations"] == cap
+        assert np.isfinite(u).all() and st["rel_res"] <= 2 * floor, (cap, st["rel_res"], floor)
+
+
+@pytest.mark.parametrize("kind", [F.TOL_REL_RES, F.TOL_REF_GAMMA])
+@pytest.mark.parametrize("exponent", [-472, -480, -488])
+def test_faint_loads_converge(ctx, exponent, kind):
+    """r'z of 2^-1074 to 2^-1000 at the end of the solve: a load of 2^exponent
+    times the size gives that displacement (both within the tolerance's 1e-8
+    times the condition number, below 1e4)."""
+    pb = plate_problem(40, 20, convention=F.LOADS_PHYSICAL)
+    ctx.set_problem(pb)
+    f = ctx.rhs()
+    opts = dict(tol=1e-8 if kind == F.TOL_REL_RES else 1e-16, tol_kind=kind)
+    u0, s0 = ctx.solve_rhs(f, F.FP64, **opts)
+    u, st = ctx.solve_rhs(f * 2.0 ** exponent, F.FP64, max_iter=4000, **opts)
+    assert abs(st["iterations"] - s0["iterations"]) <= 5
+    assert rel(u * 2.0 ** -exponent, u0) <= 1e-4
+
+
+def test_underflow_ends_a_solve(ctx):
+    """Sums that underflow to nothing: a breakdown where there is a tolerance
+    that is not met, also within an implicit step; without one the cap."""
+    pb = plate_problem(12, 7, convention=F.LOADS_PHYSICAL)
+    ctx.set_problem(pb)
+    f = ctx.rhs()
+    u, st = ctx.solve_rhs(f, F.FP64, tol=0.0, max_iter=1000000, raise_on_error=False)
+    assert st["status"] == -4 and st["iterations"] == 1000000 and st["solve_ms"] < 100.0
+    u, st = ctx.solve_rhs(f * 1e-160, F.FP64, tol=1e-8, tol_kind=F.TOL_REL_RES, max_iter=100000,
+                          raise_on_error=False)
+    assert st["status"] == -5 and st["iterations"] < 1000
+    dt = 1e-4
+    u, st = ctx.dyn_run(rho=2400.0, beta2=0.5, dt=dt, endtime=1.5 * dt, ampl=1e3,
+                        wavelet_type=F.WAVELET_RICKER, freq=1.0 / (3 * dt), pcg_eps=0.0,
+                        mass_convention=F.MASS_PHYSICAL, implicit_mode=F.IMPLICIT_PHYSICAL,
+                        raise_on_error=False)
+    assert st["status"] == -5 and st["steps"] == 0 and st["pcg_iterations"] < 10000
