@@ -27,6 +27,7 @@ FP64, FP32, MIXED = 0, 1, 2
 TOL_REF_GAMMA, TOL_REL_RES = 0, 1
 CG_STANDARD, CG_SINGLE_REDUCTION = 0, 1
 BATCH_LOCKSTEP, BATCH_PERSISTENT = 0, 1
+RESIDENT_AUTO, RESIDENT_OFF = 0, 1
 LOADS_REFERENCE, LOADS_PHYSICAL = 0, 1
 MASS_REFERENCE, MASS_PHYSICAL = 0, 1
 WAVELET_NONE, WAVELET_RICKER, WAVELET_BERLAGE = 0, 1, 2
@@ -78,6 +79,8 @@ SIGNATURES = {
     "femgpu_last_error": (C.c_char_p, [_P]),
     "femgpu_set_stream": (C.c_int, [_P, _P]),
     "femgpu_sync": (C.c_int, [_P]),
+    "femgpu_set_resident": (C.c_int, [_P, C.c_int]),
+    "femgpu_resident_info": (C.c_int, [_P, _L]),
     "femgpu_set_mesh": (C.c_int, [_P, C.c_int, C.c_int64, _D, C.c_int64, _I]),
     "femgpu_set_tuning": (C.c_int, [_P, C.c_int, C.c_int]),
     "femgpu_autotune": (C.c_int, [_P, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
@@ -314,6 +317,15 @@ class Context:
 
     def sync(self):
         self._check(self.lib.femgpu_sync(self.h), "sync")
+
+    def set_resident(self, mode: int = RESIDENT_AUTO):
+        self._check(self.lib.femgpu_set_resident(self.h, mode), "set_resident")
+
+    def resident_info(self) -> tuple[int, int]:
+        """Launches that stayed on the chip: (completed, given up)."""
+        n = (C.c_int64 * 2)()
+        self._check(self.lib.femgpu_resident_info(self.h, n), "resident_info")
+        return n[0], n[1]
 
     # --- solves ----------------------------------------------------------------
     def _opts(self, precision, tol, tol_kind, max_iter, inner_tol, check_every,

@@ -297,7 +297,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
                          const femgpu_solve_opts &o, double *u_out, femgpu_batch_stat *stats,
                          double *solve_ms, bool *ran) {
   *ran = false;
-  if (!b->br_np_max || b->br_off) return FEMGPU_OK;
+  if (!b->br_np_max || b->br_off || !ctx_resident(ctx).on()) return FEMGPU_OK;
   const int lds = br_lds_bytes(nr, b->bl_pn, b->bl_ent, b->br_in, b->br_src);
   double block = 1.0;
   const int capacity = br_capacity(nr, b->br_degree, lds, ctx_device(ctx), &block);
@@ -387,6 +387,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     BCHK_(hipMemcpyAsync(head, words, sizeof head, hipMemcpyDeviceToHost, s));
     BCHK_(hipStreamSynchronize(s));
   }
+  ++(head[0] ? ctx_resident(ctx).given_up : ctx_resident(ctx).completed);
   if (head[0]) {
     if (!head[2] || b->br_degree == BR_DEGREE_MAX) {
       b->br_off = true;

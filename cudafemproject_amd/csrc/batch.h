@@ -86,5 +86,7 @@ hipStream_t ctx_stream(femgpu_ctx *c);
 int ctx_device(femgpu_ctx *c);
 int ctx_fail(femgpu_ctx *c, int code, const char *msg);
 BatchState *&ctx_batch(femgpu_ctx *c);
+struct ResidentUse;
+ResidentUse &ctx_resident(femgpu_ctx *c);
 
 }  // namespace femgpu

@@ -139,12 +139,11 @@ struct femgpu_ctx {
   uint64_t buf_gen = 0;
   uint64_t graph_gen = 0;
 
-  // resident solves (resident.h): patches the exchange words are zeroed for;
-  // off after a launch that did not complete
+  // resident solves (resident.h): patches the exchange words are zeroed for
   int res_np = 0;
   int dyn_np = 0;                // the same for the time steps' entries
   unsigned dyn_tag[2] = {0, 0};  // and the last tags used in them (FP32, FP64)
-  bool res_off = false;
+  femgpu::ResidentUse res;
 
   // femgpu_matvec_noalloc: this device's fixed scratch array (device
   // address from hipGetSymbolAddress) and the internal -> user node map
@@ -160,6 +159,7 @@ int ctx_fail(femgpu_ctx *c, int code, const char *msg) {
   return code;
 }
 BatchState *&ctx_batch(femgpu_ctx *c) { return c->batch; }
+ResidentUse &ctx_resident(femgpu_ctx *c) { return c->res; }
 }  // namespace femgpu
 
 namespace {
@@ -762,7 +762,7 @@ int replay_until(femgpu_ctx *ctx, const Replay &exec, CgScalars *sc, int block, 
 template <typename T>
 bool pcg_resident(const femgpu_ctx *ctx) {
   femgpu::ResFit fit;
-  return !ctx->res_off && femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit);
+  return ctx->res.on() && femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit);
 }
 
 // The exchange words and this precision's entries, zeroed for this plan (an
@@ -811,11 +811,13 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
     }
     const CgScalars &h = *ctx->h_sc;
     if (h.done == femgpu::RES_ABORTED) {
-      ctx->res_off = true;
+      ++ctx->res.given_up;
+      ctx->res.off = true;
       ctx->res_np = 0;
       *ok = false;
       return FEMGPU_OK;
     }
+    ++ctx->res.completed;
     if (h.done != femgpu::RES_CAP) break;
     a.fresh = 0;
     a.r_in = a.r_out;
@@ -890,11 +892,13 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     }
     *done = ctx->h_sc->done;
     if (*done == femgpu::RES_ABORTED) {
-      ctx->res_off = true;
+      ++ctx->res.given_up;
+      ctx->res.off = true;
       ctx->res_np = 0;
       *ok = false;
       return FEMGPU_OK;
     }
+    ++ctx->res.completed;
     *steps += ctx->h_sc->par_final;
     *iters += ctx->h_sc->iter_final;
     m.fresh = 0;
@@ -942,10 +946,11 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
     *ok = *gave_up == 0;
+    ++(*ok ? ctx->res.completed : ctx->res.given_up);
     d.fresh = 0;
   }
   if (!*ok) {
-    ctx->res_off = true;
+    ctx->res.off = true;
     ctx->dyn_np = 0;
   }
   return FEMGPU_OK;
@@ -1423,6 +1428,21 @@ int femgpu_set_stream(femgpu_ctx *ctx, void *hip_stream) {
 int femgpu_sync(femgpu_ctx *ctx) {
   if (!ctx) return FEMGPU_E_ARG;
   HIPCHK(hipStreamSynchronize(ctx->stream));
+  return FEMGPU_OK;
+}
+
+int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
+  if (!ctx) return FEMGPU_E_ARG;
+  if (mode != FEMGPU_RESIDENT_AUTO && mode != FEMGPU_RESIDENT_OFF)
+    return fail(ctx, FEMGPU_E_ARG, "set_resident: unknown mode");
+  ctx->res.mode = mode;
+  return FEMGPU_OK;
+}
+
+int femgpu_resident_info(const femgpu_ctx *ctx, int64_t *info) {
+  if (!ctx || !info) return FEMGPU_E_ARG;
+  info[0] = ctx->res.completed;
+  info[1] = ctx->res.given_up;
   return FEMGPU_OK;
 }
 
@@ -2717,7 +2737,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   // lag one step (the displacement does not).
   const bool one_launch = expl && nrec == 0 && !relax;
   femgpu::ResFit fit;
-  bool resident = expl && !relax && !ctx->res_off &&
+  bool resident = expl && !relax && ctx->res.on() &&
                   femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit);
   if (resident) {
     femgpu::ResDyn<T> r{};
@@ -2860,7 +2880,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       femgpu::launch_inv_diag<T>(ctx->dm, diagK_t, ceff, T(1), dmc, invA, ctx->stream);
     }
     w.invD = invA;
-    bool impl_resident = !ctx->res_off && femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit);
+    bool impl_resident = ctx->res.on() && femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit);
     if (impl_resident) {
       femgpu::ResImpl<T> m{};
       m.d = dd;

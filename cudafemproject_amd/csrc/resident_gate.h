@@ -3,10 +3,19 @@
 
 #include <algorithm>
 #include <condition_variable>
+#include <cstdint>
 #include <map>
 #include <mutex>
 
 namespace femgpu {
+
+// A context's use of the forms that stay on the chip (femgpu_set_resident).
+struct ResidentUse {
+  int mode = 0;                 // FEMGPU_RESIDENT_*
+  bool off = false;             // a launch did not complete: launches from then on
+  int64_t completed = 0, given_up = 0;
+  bool on() const { return mode == 0 && !off; }
+};
 
 // Resident launches (resident.h) wait for each other's workgroups, so all
 // workgroups of a launch must reach the device: alone they do when they fit

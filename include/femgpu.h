@@ -124,6 +124,17 @@ int femgpu_set_stream(femgpu_ctx *ctx, void *hip_stream);
 /* Synchronise the context's stream. */
 int femgpu_sync(femgpu_ctx *ctx);
 
+/* Solves with the standard recurrence, time steps and 2D batches of meshes
+ * that fit the device run in launches whose workgroups stay on the chip and
+ * wait for each other (AUTO, the default); everything else, and with OFF
+ * these too, in a launch per kernel.  No counterpart in the reference; for
+ * tests and measurements of either form. */
+enum { FEMGPU_RESIDENT_AUTO = 0, FEMGPU_RESIDENT_OFF = 1 };
+int femgpu_set_resident(femgpu_ctx *ctx, int mode);
+/* Launches of this context that stayed on the chip: info[0] completed,
+ * info[1] given up (a wait ran out; the call then went on in launches). */
+int femgpu_resident_info(const femgpu_ctx *ctx, int64_t *info);
+
 /* --- problem definition ---------------------------------------------------
  * Replaces: the dataKeeper readers (DataKeeper/src/datakeeper.cpp:116-213)
  * and the ElementsData constructor's host->device copies
