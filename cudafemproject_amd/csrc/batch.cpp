@@ -317,7 +317,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   BCHK_(bbuf(b, "bl_diag64", nd, &diag));
   BCHK_(bbuf(b, "bl_s64", size_t(b->bl_slots) * nr * 2 + 1, &slots));
   BCHK_(bbuf(b, "bl64_invD", nd, &invD));
-  BCHK_(bbuf(b, "br_words", n_ent + n_words + 3, &zero));
+  BCHK_(bbuf(b, "br_words", n_ent + n_words + 4, &zero));
   BCHK_(bbuf(b, "bl_state", n_state, &st));
   auto *words = reinterpret_cast<unsigned long long *>(zero);
   auto table = [&](const char *name) { return b->bufs[name].first; };
@@ -346,9 +346,9 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   a.invD = invD;
   a.x = d_x;
   a.abort = words;
-  a.ticket = reinterpret_cast<unsigned *>(words + 1);
-  a.crowded = words + 2;
-  a.words = words + 3;
+  a.ticket = reinterpret_cast<unsigned *>(words + 2);
+  a.crowded = words + 3;
+  a.words = words + 4;
   a.entries = a.words + n_words;
   a.st = st;
   a.max_iter = o.max_iter > 0 ? o.max_iter : 100000;
@@ -369,7 +369,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   m.pn = b->bl_pn;
   const int32_t *perm = static_cast<const int32_t *>(table("br_perm"));
   std::vector<BLState> hs(n_state);
-  unsigned long long head[3];
+  unsigned long long head[4];
   BCHK_(hipMemcpyAsync(d_user, f, nu * sizeof(double), hipMemcpyHostToDevice, s));
   {
     const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(b->bl_np) / capacity), block);
@@ -377,9 +377,10 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
     bl_diag(2, m, b->bl_nif, diag, slots, s);
     bl_inv_diag<double>(int64_t(nd), diag, invD, s);
-    launch_fill<double>(zero, int64_t(n_ent + n_words + 3), 0.0, s);
+    launch_fill<double>(zero, int64_t(n_ent + n_words + 4), 0.0, s);
+    if (ctx_resident(ctx).lose_from >= 0) launch_fill<double>(zero + 1, 1, test_wait(), s);
     launch_fill<double>(d_x, int64_t(nv), 0.0, s);
-    launch_batch_resident(nr, b->br_degree, a, s);
+    launch_batch_resident(nr, b->br_degree, a, s, ctx_resident(ctx).lose());
     BCHK_(hipGetLastError());
     BCHK_(hipEventRecord(b->ev1, s));
     launch_br_rhs_out(N, n_rhs, nr, perm, d_x, d_user, s);
@@ -389,7 +390,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   }
   ++(head[0] ? ctx_resident(ctx).given_up : ctx_resident(ctx).completed);
   if (head[0]) {
-    if (!head[2] || b->br_degree == BR_DEGREE_MAX) {
+    if (!head[3] || b->br_degree == BR_DEGREE_MAX) {
       b->br_off = true;
       return FEMGPU_OK;
     }

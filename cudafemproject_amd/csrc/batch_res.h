@@ -42,8 +42,9 @@ struct BRArgs {
   const double *f, *invD;              // [node][rhs][2], [node][2]
   double *x;                           // solution, likewise
   unsigned long long *entries, *words; // zero before the launch
-  unsigned long long *abort, *crowded; // zero; nonzero after a launch that did not complete,
-                                       // for a node with too many neighbours
+  unsigned long long *abort;           // zero, then the bound of a wait (0: a second); nonzero
+                                       // after a launch that did not complete
+  unsigned long long *crowded;         // zero; nonzero for a node with too many neighbours
   unsigned *ticket;                    // zero
   BLState *st;                         // per (instance, rhs), written at the end
   int max_iter;
@@ -55,7 +56,8 @@ struct BRArgs {
 int br_lds_bytes(int nr, int pn, int ent, int n_in, int n_src);
 int br_capacity(int nr, int degree, int lds, int device, double *block);
 
-void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s);
+// (short_grid: tests; without the last ticket)
+void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s, bool short_grid);
 
 // Right-hand sides to internal node order padded to nr, and solutions back.
 void launch_br_rhs_in(int64_t n, int n_rhs, int nr, const int32_t *perm, const double *user,

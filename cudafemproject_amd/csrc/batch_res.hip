@@ -532,9 +532,9 @@ int br_capacity(int nr, int degree, int lds, int device, double *block) {
   return per * cu;
 }
 
-void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s) {
+void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s, bool short_grid) {
   const int lds = br_lds_bytes(nr, a.pn, a.ent, a.n_in_max, a.n_src_max);
-  hipLaunchKernelGGL(kernel_of(nr, degree), dim3(a.np), dim3(PT), lds, s, a);
+  hipLaunchKernelGGL(kernel_of(nr, degree), dim3(a.np - (short_grid && a.np > 1)), dim3(PT), lds, s, a);
 }
 
 void launch_br_rhs_in(int64_t n, int n_rhs, int nr, const int32_t *perm, const double *user,

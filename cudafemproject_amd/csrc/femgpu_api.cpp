@@ -780,6 +780,8 @@ int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long 
   if (ctx->res_np != ctx->dm.np) {
     femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
     femgpu::launch_fill<double>(e, int64_t(2 * (n64 + n32)), 0.0, ctx->stream);
+    if (ctx->res.lose_from >= 0)
+      femgpu::launch_fill<double>(w + 2, 1, femgpu::test_wait(), ctx->stream);
     ctx->res_np = ctx->dm.np;
   }
   *words = reinterpret_cast<unsigned long long *>(w);
@@ -805,7 +807,7 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
     ctx->h_sc->done = femgpu::RES_ABORTED;
     {
       ResidentGate gate(ctx->device, fit.share, fit.block);
-      femgpu::launch_res_pcg<T>(ctx->dm, a, ctx->stream);
+      femgpu::launch_res_pcg<T>(ctx->dm, a, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
@@ -886,7 +888,7 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     ctx->h_sc->done = femgpu::RES_ABORTED;
     {
       ResidentGate gate(ctx->device, fit.share, fit.block);
-      femgpu::launch_res_impl<T>(ctx->dm, m, ctx->stream);
+      femgpu::launch_res_impl<T>(ctx->dm, m, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
@@ -915,21 +917,23 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
   int st;
   if (!femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit))
     return fail(ctx, FEMGPU_E_STATE, "internal error: resident steps do not fit");
-  // two sets of entries per precision, then the abort flag
+  // two sets of entries per precision, then the abort flag and the bound of a wait
   const size_t n64 = femgpu::res_entry_words<double>(ctx->dm.x_entries, ctx->dim);
   const size_t n32 = femgpu::res_entry_words<float>(ctx->dm.x_entries, ctx->dim);
-  const size_t n = 2 * (n64 + n32) + 1;
+  const size_t n = 2 * (n64 + n32) + 2;
   double *w;
   if ((st = dbuf(ctx, "dyn_entries", n, &w))) return st;
   d.entries = reinterpret_cast<unsigned long long *>(w) + (sizeof(T) == 8 ? 0 : 2 * n64);
   d.entry_words = sizeof(T) == 8 ? n64 : n32;
-  d.abort = reinterpret_cast<unsigned long long *>(w) + n - 1;
+  d.abort = reinterpret_cast<unsigned long long *>(w) + n - 2;
   d.fresh = 1;
   *ok = true;
   for (int done = 0; done < n_steps && *ok; done += d.n_steps) {
     d.n_steps = std::min(n_steps - done, RES_STEP_CAP);
     if (ctx->dyn_np != ctx->dm.np) {
       femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
+      if (ctx->res.lose_from >= 0)
+        femgpu::launch_fill<double>(w + n - 1, 1, femgpu::test_wait(), ctx->stream);
       ctx->dyn_np = ctx->dm.np;
       ctx->dyn_tag[0] = ctx->dyn_tag[1] = 0;
     }
@@ -940,7 +944,7 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
     unsigned long long *gave_up = reinterpret_cast<unsigned long long *>(&ctx->h_sc[3]);
     {
       ResidentGate gate(ctx->device, fit.share, fit.block);
-      femgpu::launch_res_dyn<T>(ctx->dm, d, ctx->stream);
+      femgpu::launch_res_dyn<T>(ctx->dm, d, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipMemcpyAsync(gave_up, d.abort, sizeof(*gave_up), hipMemcpyDeviceToHost, ctx->stream));
       HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -1433,9 +1437,14 @@ int femgpu_sync(femgpu_ctx *ctx) {
 
 int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
   if (!ctx) return FEMGPU_E_ARG;
-  if (mode != FEMGPU_RESIDENT_AUTO && mode != FEMGPU_RESIDENT_OFF)
+  if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_LOSE_LATER)
     return fail(ctx, FEMGPU_E_ARG, "set_resident: unknown mode");
   ctx->res.mode = mode;
+  ctx->res.off = false;
+  ctx->res.lose_from = mode == FEMGPU_RESIDENT_TEST_LOSE         ? ctx->res.completed
+                       : mode == FEMGPU_RESIDENT_TEST_LOSE_LATER ? ctx->res.completed + 2
+                                                                 : -1;
+  ctx->res_np = ctx->dyn_np = 0;  // (the exchange words are made again)
   return FEMGPU_OK;
 }
 

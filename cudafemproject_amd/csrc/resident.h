@@ -12,9 +12,9 @@
 namespace femgpu {
 
 // The workgroups' exchange buffer for np patches, in 8-byte words: the tag of
-// the last exchange, the abort flag, the tags of the last trade of entries
-// (FP32, FP64; every launch advances its tags), and the tagged partials in
-// EX_COPIES copies on pages of their own.  The interface entries are tagged
+// the last exchange, the abort flag, the bound of a wait (0: a second), the tags
+// of the last trade of entries (FP32, FP64; every launch advances its tags), and
+// the tagged partials in EX_COPIES copies on pages of their own.  The interface entries are tagged
 // words too (res_entry_words).  Both are zeroed when they are allocated or the
 // plan changes, and after an aborted launch.
 constexpr int EX_COPIES = 8;
@@ -75,8 +75,9 @@ struct ResFit {
 template <typename T>
 bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit);
 
+// (short_grid: tests; a workgroup that others wait for is left out)
 template <typename T>
-void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &a, hipStream_t s);
+void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &a, hipStream_t s, bool short_grid);
 
 // Receivers of a resident run (rec_of null: none): per node its first receiver
 // or -1, the receivers of one node linked by rec_next.
@@ -98,7 +99,8 @@ struct ResDyn : ResRecv<T> {
   T dt, c1, c2, c3, alpha, scale;        // DynCoeffs
   unsigned long long *entries;           // two sets of entry_words
   size_t entry_words;
-  unsigned long long *abort;             // zero; nonzero after a launch that did not complete
+  unsigned long long *abort;             // zero; nonzero after a launch that did not complete;
+                                         // then the bound of a wait (0: a second)
   unsigned tag0;                         // tags tag0 .. tag0 + n_steps - 1, following the last launch's
   int fresh, step0, n_steps;
 };
@@ -107,7 +109,7 @@ template <typename T>
 bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit);
 
 template <typename T>
-void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &a, hipStream_t s);
+void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &a, hipStream_t s, bool short_grid);
 
 // Implicit GN22 steps in one launch, likewise; a launch ends early after the
 // step in which its PCG iterations reach it_budget.  At the end sc->done is 1,
@@ -132,7 +134,7 @@ template <typename T>
 bool res_impl_fit(const DevMesh &dm, int device, ResFit *fit);
 
 template <typename T>
-void launch_res_impl(const DevMesh &dm, const ResImpl<T> &a, hipStream_t s);
+void launch_res_impl(const DevMesh &dm, const ResImpl<T> &a, hipStream_t s, bool short_grid);
 
 hipError_t prepare_resident_kernels();
 

@@ -443,12 +443,12 @@ struct ResSolver {
     // (workgroup 0 advances the tags at its end, after an exchange that every
     // workgroup took part in with the tags it reads here)
     tag = unsigned(ld_agent(words));
-    entry_tag = unsigned(ld_agent(words + 2 + (sizeof(T) == 8 ? 1 : 0)));
+    entry_tag = unsigned(ld_agent(words + 3 + (sizeof(T) == 8 ? 1 : 0)));
   }
 
   __device__ __forceinline__ void store_tags(u64 *words) const {
     st_agent(words, u64(tag));
-    st_agent(words + 2 + (sizeof(T) == 8 ? 1 : 0), u64(entry_tag));
+    st_agent(words + 3 + (sizeof(T) == 8 ? 1 : 0), u64(entry_tag));
   }
 
   // A trade; the sets of entries take turns, as in the explicit steps: a
@@ -933,6 +933,14 @@ FEMGPU_RES_KERNEL(k_dyn_resident, DynKernel)
 FEMGPU_RES_KERNEL(k_impl_resident, ImplKernel)
 #undef FEMGPU_RES_KERNEL
 
+// Workgroups of a launch (short_grid: up to the last patch's, and without it).
+int grid_of(int np, int p8, bool short_grid) {
+  int n = 8 * p8;
+  if (short_grid && np > 1)
+    while (((n - 1) & 7) * p8 + ((n - 1) >> 3) >= np) --n;
+  return short_grid && np > 1 ? n - 1 : n;
+}
+
 // Whether a kernel of this form fits the plan, a workgroup per compute unit.
 bool fits(const DevMesh &dm, int device, const void *fn, int lds, ResFit *fit) {
   const int cu = compute_units(device);
@@ -986,10 +994,11 @@ bool res_pcg_fit(const DevMesh &dm, int device, ResFit *fit) {
 }
 
 template <typename T>
-void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &s, hipStream_t st) {
+void launch_res_pcg(const DevMesh &dm, const ResPcg<T> &s, hipStream_t st, bool short_grid) {
   const PcgArgs<T> a{res_mesh<T>(dm), s};
   const Form f = res_form(dm);
-  hipLaunchKernelGGL(k_pcg_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
+  hipLaunchKernelGGL(k_pcg_resident_of<T>(dm.dim, f), dim3(grid_of(a.m.np, a.m.p8, short_grid)),
+                     dim3(f.threads),
                      res_lds_bytes(dm, int(sizeof(T))), st, a);
 }
 
@@ -1001,10 +1010,11 @@ bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit) {
 }
 
 template <typename T>
-void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &s, hipStream_t st) {
+void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &s, hipStream_t st, bool short_grid) {
   const DynArgs<T> a{res_mesh<T>(dm), s};
   const Form f = res_form(dm);
-  hipLaunchKernelGGL(k_dyn_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
+  hipLaunchKernelGGL(k_dyn_resident_of<T>(dm.dim, f), dim3(grid_of(a.m.np, a.m.p8, short_grid)),
+                     dim3(f.threads),
                      res_lds_bytes(dm, int(sizeof(T))), st, a);
 }
 
@@ -1016,10 +1026,11 @@ bool res_impl_fit(const DevMesh &dm, int device, ResFit *fit) {
 }
 
 template <typename T>
-void launch_res_impl(const DevMesh &dm, const ResImpl<T> &s, hipStream_t st) {
+void launch_res_impl(const DevMesh &dm, const ResImpl<T> &s, hipStream_t st, bool short_grid) {
   const ImplArgs<T> a{res_mesh<T>(dm), s};
   const Form f = res_form(dm);
-  hipLaunchKernelGGL(k_impl_resident_of<T>(dm.dim, f), dim3(8 * a.m.p8), dim3(f.threads),
+  hipLaunchKernelGGL(k_impl_resident_of<T>(dm.dim, f), dim3(grid_of(a.m.np, a.m.p8, short_grid)),
+                     dim3(f.threads),
                      res_lds_bytes(dm, int(sizeof(T))), st, a);
 }
 
@@ -1044,11 +1055,11 @@ hipError_t prepare_resident_kernels() {
 
 #define FEMGPU_RES_INST(T)                                                    \
   template bool res_pcg_fit<T>(const DevMesh &, int, ResFit *);               \
-  template void launch_res_pcg<T>(const DevMesh &, const ResPcg<T> &, hipStream_t); \
+  template void launch_res_pcg<T>(const DevMesh &, const ResPcg<T> &, hipStream_t, bool); \
   template bool res_dyn_fit<T>(const DevMesh &, int, ResFit *);               \
-  template void launch_res_dyn<T>(const DevMesh &, const ResDyn<T> &, hipStream_t); \
+  template void launch_res_dyn<T>(const DevMesh &, const ResDyn<T> &, hipStream_t, bool); \
   template bool res_impl_fit<T>(const DevMesh &, int, ResFit *);              \
-  template void launch_res_impl<T>(const DevMesh &, const ResImpl<T> &, hipStream_t);
+  template void launch_res_impl<T>(const DevMesh &, const ResImpl<T> &, hipStream_t, bool);
 FEMGPU_RES_INST(double)
 FEMGPU_RES_INST(float)
 

@@ -36,7 +36,8 @@ __device__ __forceinline__ double untag(const u64 (&w)[2]) {
 }
 
 // A bounded wait: true once the caller should give up (another workgroup
-// did, or WAIT_TICKS have passed since the 256th look).
+// did, or WAIT_TICKS -- or what the host put beside the abort word -- have
+// passed since the 256th look).
 struct Patience {
   u64 *abort;
   u64 start = 0;
@@ -44,7 +45,8 @@ struct Patience {
     if ((spin & 255) != 255) return false;
     const u64 now = wall_clock64();
     if (start == 0) start = now;
-    if (ld_agent(abort) == 0 && now - start <= WAIT_TICKS) return false;
+    const u64 limit = ld_agent(abort + 1);
+    if (ld_agent(abort) == 0 && now - start <= (limit ? limit : WAIT_TICKS)) return false;
     st_agent(abort, 1);
     return true;
   }

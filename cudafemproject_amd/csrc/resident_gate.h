@@ -4,6 +4,7 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <mutex>
 
@@ -14,8 +15,19 @@ struct ResidentUse {
   int mode = 0;                 // FEMGPU_RESIDENT_*
   bool off = false;             // a launch did not complete: launches from then on
   int64_t completed = 0, given_up = 0;
-  bool on() const { return mode == 0 && !off; }
+  int64_t lose_from = -1;       // tests: launches from this one on lack a workgroup
+  bool on() const { return mode != 1 && !off; }
+  bool lose() const { return lose_from >= 0 && completed >= lose_from; }
 };
+
+// The bound of a wait in such tests, 2 ms, as the word that the kernels read.
+constexpr uint64_t TEST_WAIT_TICKS = 200000;
+inline double test_wait() {
+  double v;
+  static_assert(sizeof v == sizeof TEST_WAIT_TICKS, "");
+  std::memcpy(&v, &TEST_WAIT_TICKS, sizeof v);
+  return v;
+}
 
 // Resident launches (resident.h) wait for each other's workgroups, so all
 // workgroups of a launch must reach the device: alone they do when they fit

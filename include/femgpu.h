@@ -128,8 +128,15 @@ int femgpu_sync(femgpu_ctx *ctx);
  * that fit the device run in launches whose workgroups stay on the chip and
  * wait for each other (AUTO, the default); everything else, and with OFF
  * these too, in a launch per kernel.  No counterpart in the reference; for
- * tests and measurements of either form. */
-enum { FEMGPU_RESIDENT_AUTO = 0, FEMGPU_RESIDENT_OFF = 1 };
+ * tests and measurements of either form.  Tests of what follows a launch that
+ * does not complete: every such launch (LOSE), or every one from the third on
+ * (LOSE_LATER), lacks a workgroup, and the others' waits run out after 2 ms. */
+enum {
+  FEMGPU_RESIDENT_AUTO = 0,
+  FEMGPU_RESIDENT_OFF = 1,
+  FEMGPU_RESIDENT_TEST_LOSE = 2,
+  FEMGPU_RESIDENT_TEST_LOSE_LATER = 3
+};
 int femgpu_set_resident(femgpu_ctx *ctx, int mode);
 /* Launches of this context that stayed on the chip: info[0] completed,
  * info[1] given up (a wait ran out; the call then went on in launches). */

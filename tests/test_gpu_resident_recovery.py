@@ -1,0 +1,92 @@
+"""GPU: resident launches that do not complete.  The host leaves a workgroup out
+of a launch, the others give up waiting for it (after 2 ms), every kernel ends,
+and the call goes on in launches: the results are the launch form's, bit for
+bit, also where the launch that failed continued earlier ones."""
+import numpy as np
+import pytest
+
+import cudafemproject_amd as F
+from cudafemproject_amd.problem import cube_problem, load_batch, plate_batch, plate_problem
+
+pytestmark = pytest.mark.gpu
+
+STEP = dict(rho=2400.0, wavelet_type=F.WAVELET_RICKER, ampl=1e3, mass_convention=F.MASS_PHYSICAL)
+
+
+def _solve(precision, **kw):
+    def run(c):
+        c.set_problem(cube_problem(9))
+        u, st = c.solve(precision, raise_on_error=False, **kw)
+        return [u, st["status"], st["iterations"], st["outer_iterations"]]
+    return run
+
+
+def _steps(beta2, steps, precision=F.FP64, receivers=(), make=lambda: plate_problem(70, 45), dt=1e-5,
+           tuning=(0, 0), **kw):
+    def run(c):
+        c.set_tuning(*tuning)
+        c.set_problem(make())
+        c.set_tuning(0, 0)
+        c.set_receivers(list(receivers), F.RECV_VELOCITY, 3)
+        u, st = c.dyn_run(beta2=beta2, dt=dt, endtime=(steps + 0.5) * dt if steps > 0 else -1e-30,
+                          freq=1.0 / (20 * dt), precision=precision, raise_on_error=False,
+                          **dict(STEP, **kw))
+        tr = c.traces() if len(receivers) else 0
+        c.set_receivers([], F.RECV_VELOCITY, 1)
+        return [u, st["status"], st["steps"], st["pcg_iterations"], tr]
+    return run
+
+
+def _batch(precision):
+    insts = plate_batch(3, seed=3, nx_range=(30, 40), ny_range=(20, 30))
+
+    def run(c):
+        load_batch(c, insts)
+        us, st, _ = c.batch_solve([b.f for b in insts], precision=precision, tol=1e-9)
+        return us + [st["status"], st["iterations"]]
+    return run
+
+
+IMPL = dict(implicit_mode=F.IMPLICIT_PHYSICAL, pcg_eps=1e-20)
+REL = dict(tol=1e-9, tol_kind=F.TOL_REL_RES)
+FIRST = {
+    "fp64": _solve(F.FP64, **REL),
+    "fp32": _solve(F.FP32, tol=1e-4, tol_kind=F.TOL_REL_RES),
+    "mixed": _solve(F.MIXED, **REL),
+    "explicit": _steps(0.0, 60),
+    "explicit-traces": _steps(0.0, 60, F.FP32, receivers=(0, 700, 3000)),
+    "implicit": _steps(0.5, 5, **IMPL),
+    "implicit-traces": _steps(0.5, 6, receivers=(0, 700, 3000), **IMPL),
+    "batch": _batch(F.FP64),
+    "batch-mixed": _batch(F.MIXED),
+}
+# in the third launch
+LATER = {
+    "fp32-capped": _solve(F.FP32, tol=0.0, max_iter=12500),
+    "mixed": _solve(F.MIXED, tol=1e-12, tol_kind=F.TOL_REL_RES),
+    "explicit": _steps(0.0, 40000, make=lambda: plate_problem(6, 4), tuning=(16, 256)),
+    "implicit-relaxation": _steps(0.5, 0, make=lambda: plate_problem(12, 7), tuning=(16, 256), dt=1e-4,
+                                  relax_reference=0, max_steps=8, **IMPL),
+}
+
+
+@pytest.mark.parametrize("mode,name", [(F.RESIDENT_TEST_LOSE, n) for n in FIRST] +
+                         [(F.RESIDENT_TEST_LOSE_LATER, n) for n in LATER])
+def test_lost_workgroup(mode, name):
+    run = (FIRST if mode == F.RESIDENT_TEST_LOSE else LATER)[name]
+    print(f"[lost] {name}", flush=True)
+    with F.Context(0) as c:
+        c.set_resident(F.RESIDENT_OFF)
+        want = run(c)
+        assert c.resident_info() == (0, 0)
+    with F.Context(0) as c:
+        c.set_resident(mode)
+        for _ in range(2):
+            got = run(c)
+            assert all(np.array_equal(a, b) for a, b in zip(got, want))
+        done, lost = c.resident_info()
+        assert lost >= 1 and done == (0 if mode == F.RESIDENT_TEST_LOSE else 2)
+        c.set_resident(F.RESIDENT_AUTO)
+        again = run(c)
+        assert c.resident_info()[0] > done and c.resident_info()[1] == lost
+        assert all(np.all(np.isfinite(np.asarray(a, float))) for a in again)
