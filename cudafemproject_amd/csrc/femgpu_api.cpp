@@ -803,8 +803,10 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
   if ((st = res_buffers<T>(ctx, &a.words, &a.entries, &a.entry_words))) return st;
   a.sc = ctx->h_sc;
   a.cap = RES_ITER_CAP;
+  a.late = ctx->res.late;
   for (;;) {
     ctx->h_sc->done = femgpu::RES_ABORTED;
+    ctx->h_sc->gave_up = 0;
     {
       ResidentGate gate(ctx->device, fit.share, fit.block);
       femgpu::launch_res_pcg<T>(ctx->dm, a, ctx->stream, ctx->res.lose());
@@ -812,7 +814,7 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
     const CgScalars &h = *ctx->h_sc;
-    if (h.done == femgpu::RES_ABORTED) {
+    if (h.done == femgpu::RES_ABORTED || h.gave_up) {
       ++ctx->res.given_up;
       ctx->res.off = true;
       ctx->res_np = 0;
@@ -878,6 +880,7 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     return fail(ctx, FEMGPU_E_STATE, "internal error: resident steps do not fit");
   if ((st = res_buffers<T>(ctx, &m.words, &m.entries, &m.entry_words))) return st;
   m.sc = ctx->h_sc;
+  m.late = ctx->res.late;
   m.it_budget = 4 * RES_ITER_CAP;
   *done = 1;
   *steps = *iters = 0;
@@ -886,13 +889,14 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     m.step0 = step0 + *steps;
     m.n_steps = n_steps - *steps;
     ctx->h_sc->done = femgpu::RES_ABORTED;
+    ctx->h_sc->gave_up = 0;
     {
       ResidentGate gate(ctx->device, fit.share, fit.block);
       femgpu::launch_res_impl<T>(ctx->dm, m, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
-    *done = ctx->h_sc->done;
+    *done = ctx->h_sc->gave_up ? femgpu::RES_ABORTED : ctx->h_sc->done;
     if (*done == femgpu::RES_ABORTED) {
       ++ctx->res.given_up;
       ctx->res.off = true;
@@ -1437,13 +1441,14 @@ int femgpu_sync(femgpu_ctx *ctx) {
 
 int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
   if (!ctx) return FEMGPU_E_ARG;
-  if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_LOSE_LATER)
+  if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_LATE)
     return fail(ctx, FEMGPU_E_ARG, "set_resident: unknown mode");
   ctx->res.mode = mode;
   ctx->res.off = false;
   ctx->res.lose_from = mode == FEMGPU_RESIDENT_TEST_LOSE         ? ctx->res.completed
                        : mode == FEMGPU_RESIDENT_TEST_LOSE_LATER ? ctx->res.completed + 2
                                                                  : -1;
+  ctx->res.late = mode == FEMGPU_RESIDENT_TEST_LATE;
   ctx->res_np = ctx->dyn_np = 0;  // (the exchange words are made again)
   return FEMGPU_OK;
 }

@@ -90,6 +90,7 @@ struct CgScalars {
   int done;            // 0 running, 1 converged, 2 non-finite, 3 breakdown, 4 max-iter,
                        // 5 paused for a residual replacement (single-reduction PCG)
   int max_iter;
+  int gave_up;         // resident launches: a workgroup gave up waiting
 };
 
 // Optional mass shift of the operator: y = cK*K x + cM*diag(m) x.

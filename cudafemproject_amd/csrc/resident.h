@@ -49,6 +49,7 @@ struct ResPcg {
   int fresh, kind;
   double eps;             // fresh: tolerance (threshold formed from the initial residual)
   double gamma0, rr0, thresh, g_prev;  // not fresh
+  int late;               // tests: the last patch's workgroup gives up at its end
   double pause;           // stop with done = 5 once r'r < pause (fresh: times
                           // the initial r'r; 0: never)
   int it0, max_iter, cap; // updates done before, in all, and at most in this launch
@@ -56,7 +57,9 @@ struct ResPcg {
 
 // done codes of a resident launch besides CgScalars': 6 the launch did not
 // complete (its workgroups were not on the chip together), 7 cap reached; within
-// the kernels 8 the sums underflowed (3 or 4 to the host).
+// the kernels 8 the sums underflowed (3 or 4 to the host).  Every workgroup that
+// gives up sets gave_up itself: it may be after the one that writes the scalars
+// has ended, in the last exchange.
 constexpr int RES_ABORTED = 6, RES_CAP = 7, RES_FAINT = 8;
 
 // The part of the device that a resident launch takes, and of one compute
@@ -127,6 +130,7 @@ struct ResImpl : ResRecv<T> {
   unsigned long long *words, *entries;
   size_t entry_words;     // as ResPcg
   CgScalars *sc;
+  int late;               // as ResPcg
   int fresh, step0, n_steps;
 };
 

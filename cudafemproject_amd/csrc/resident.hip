@@ -636,6 +636,11 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
     if (!(a.s.eps > 0.0)) S.n_upd = a.s.max_iter;
     done = a.s.eps > 0.0 ? 3 : 4;
   }
+  if (a.s.late && pid == a.m.np - 1) done = RES_ABORTED;
+  if (done == RES_ABORTED) {
+    if (threadIdx.x == 0) a.s.sc->gave_up = 1;
+    return;
+  }
   if (P.first)
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -654,7 +659,6 @@ __global__ __launch_bounds__(PT) void k_pcg_resident(PcgArgs<T> a) {
     sc->iter_final = S.n_upd;
     sc->pause = S.pause;
     S.store_tags(a.s.words);
-    if (ld_agent(a.s.words + 1) != 0) done = RES_ABORTED;
     sc->done = done;
   }
 }
@@ -750,6 +754,11 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
     }
     record<T, DIM>(P, s, rec, step, d, v, a);
   }
+  if (s.late && pid == arg.m.np - 1) done = RES_ABORTED;
+  if (done == RES_ABORTED) {
+    if (threadIdx.x == 0) s.sc->gave_up = 1;
+    return;
+  }
   if (P.first && done == 1)
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
@@ -762,7 +771,6 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
     sc->iter_final = total;
     sc->par_final = n;
     S.store_tags(s.words);
-    if (ld_agent(s.words + 1) != 0) done = RES_ABORTED;
     sc->done = done;
   }
 }

@@ -16,6 +16,7 @@ struct ResidentUse {
   bool off = false;             // a launch did not complete: launches from then on
   int64_t completed = 0, given_up = 0;
   int64_t lose_from = -1;       // tests: launches from this one on lack a workgroup
+  bool late = false;            // tests: one gives up at its end
   bool on() const { return mode != 1 && !off; }
   bool lose() const { return lose_from >= 0 && completed >= lose_from; }
 };

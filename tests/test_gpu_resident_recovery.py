@@ -90,3 +90,20 @@ def test_lost_workgroup(mode, name):
         again = run(c)
         assert c.resident_info()[0] > done and c.resident_info()[1] == lost
         assert all(np.all(np.isfinite(np.asarray(a, float))) for a in again)
+
+
+@pytest.mark.parametrize("name", ["fp64", "fp32", "mixed", "implicit", "implicit-traces"])
+def test_late_abort(name):
+    """A workgroup that gives up in the last exchange, when the one that reports
+    the scalars has them all and has ended: its part of the result is missing,
+    and the host is told."""
+    run = FIRST[name]
+    print(f"[late] {name}", flush=True)
+    with F.Context(0) as c:
+        c.set_resident(F.RESIDENT_OFF)
+        want = run(c)
+    with F.Context(0) as c:
+        c.set_resident(F.RESIDENT_TEST_LATE)
+        got = run(c)
+        assert c.resident_info() == (0, 1)
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
