@@ -43,7 +43,8 @@ struct BatchState {
   // plans don't suit it
   int br_np_max = 0, br_in = 0, br_src = 0;  // most patches of an instance; exchange sizes of a patch
   int64_t br_entries = 0;
-  int br_degree = BR_DEGREE;             // more once a launch found a node with more neighbours
+  // nodes with more than BR_DEGREE neighbours in a patch, and how many
+  std::vector<std::pair<int32_t, int>> br_crowded;
   bool br_off = false;                   // a launch did not complete
   std::map<std::string, std::pair<void *, size_t>> bufs;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_poll[2] = {nullptr, nullptr};
@@ -109,6 +110,27 @@ double elem_det(int dim, const double *nodes, const int32_t *en) {
          e1[2] * (e2[0] * e3[1] - e2[1] * e3[0]);
 }
 
+// Nodes of a 2D plan with more than BR_DEGREE neighbours in a patch (internal
+// node, the most in one).
+void find_crowded(const MeshPlan &Q, int32_t first_node, std::vector<std::pair<int32_t, int>> &out) {
+  std::vector<std::vector<uint16_t>> near;
+  for (const PatchInfo &P : Q.patches) {
+    near.assign(size_t(P.n_own + P.n_sh), {});
+    for (int32_t e = P.elem_start; e < P.elem_start + P.n_elem; ++e)
+      for (int a = 0; a < 3; ++a)
+        for (int b = 0; b < 3; ++b) {
+          const uint16_t m = Q.elem_lid[size_t(e) * 4 + b];
+          auto &list = near[Q.elem_lid[size_t(e) * 4 + a]];
+          if (a != b && std::find(list.begin(), list.end(), m) == list.end()) list.push_back(m);
+        }
+    for (int32_t k = 0; k < P.n_own + P.n_sh; ++k)
+      if (near[size_t(k)].size() > size_t(BR_DEGREE))
+        out.emplace_back(first_node + (k < P.n_own ? P.own_start + k
+                                                   : Q.sh_gid[size_t(P.sh_start + k - P.n_own)]),
+                         int(near[size_t(k)].size()));
+  }
+}
+
 // Lockstep plans (batch_ls.h): every instance planned with the
 // single-problem patch limits, plans concatenated, tables uploaded.
 std::string build_lockstep(BatchState *b, hipStream_t s, const int64_t *node_off,
@@ -149,6 +171,7 @@ std::string build_lockstep(BatchState *b, hipStream_t s, const int64_t *node_off
     ExchangePlan X;
     resident = resident && Q.emax_used <= BR_ELEMS && Q.pn_used <= BR_NODES && build_exchange(Q, X);
     if (resident) {
+      find_crowded(Q, N0, b->br_crowded);
       const int32_t O0 = int32_t(xout.size());
       for (ExchangePatch e : X.patches) {
         e.in_start += int32_t(b->br_entries);
@@ -300,7 +323,13 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   if (!b->br_np_max || b->br_off || !ctx_resident(ctx).on()) return FEMGPU_OK;
   const int lds = br_lds_bytes(nr, b->bl_pn, b->bl_ent, b->br_in, b->br_src);
   double block = 1.0;
-  const int capacity = br_capacity(nr, b->br_degree, lds, ctx_device(ctx), &block);
+  // (a constrained row has no neighbours)
+  int most = 0;
+  for (const auto &c : b->br_crowded)
+    if ((b->bl_fix[size_t(c.first)] & 3) != 3) most = std::max(most, c.second);
+  if (most > BR_DEGREE_MAX) return FEMGPU_OK;
+  const int degree = most > BR_DEGREE ? BR_DEGREE_MAX : BR_DEGREE;
+  const int capacity = br_capacity(nr, degree, lds, ctx_device(ctx), &block);
   if (b->br_np_max > capacity) return FEMGPU_OK;
   hipStream_t s = ctx_stream(ctx);
   const int64_t N = b->total_nodes;
@@ -317,7 +346,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   BCHK_(bbuf(b, "bl_diag64", nd, &diag));
   BCHK_(bbuf(b, "bl_s64", size_t(b->bl_slots) * nr * 2 + 1, &slots));
   BCHK_(bbuf(b, "bl64_invD", nd, &invD));
-  BCHK_(bbuf(b, "br_words", n_ent + n_words + 4, &zero));
+  BCHK_(bbuf(b, "br_words", n_ent + n_words + 3, &zero));
   BCHK_(bbuf(b, "bl_state", n_state, &st));
   auto *words = reinterpret_cast<unsigned long long *>(zero);
   auto table = [&](const char *name) { return b->bufs[name].first; };
@@ -347,8 +376,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   a.x = d_x;
   a.abort = words;
   a.ticket = reinterpret_cast<unsigned *>(words + 2);
-  a.crowded = words + 3;
-  a.words = words + 4;
+  a.words = words + 3;
   a.entries = a.words + n_words;
   a.st = st;
   a.max_iter = o.max_iter > 0 ? o.max_iter : 100000;
@@ -369,7 +397,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   m.pn = b->bl_pn;
   const int32_t *perm = static_cast<const int32_t *>(table("br_perm"));
   std::vector<BLState> hs(n_state);
-  unsigned long long head[4];
+  unsigned long long gave_up;
   BCHK_(hipMemcpyAsync(d_user, f, nu * sizeof(double), hipMemcpyHostToDevice, s));
   {
     const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(b->bl_np) / capacity), block);
@@ -377,25 +405,21 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
     bl_diag(2, m, b->bl_nif, diag, slots, s);
     bl_inv_diag<double>(int64_t(nd), diag, invD, s);
-    launch_fill<double>(zero, int64_t(n_ent + n_words + 4), 0.0, s);
+    launch_fill<double>(zero, int64_t(n_ent + n_words + 3), 0.0, s);
     if (ctx_resident(ctx).lose_from >= 0) launch_fill<double>(zero + 1, 1, test_wait(), s);
     launch_fill<double>(d_x, int64_t(nv), 0.0, s);
-    launch_batch_resident(nr, b->br_degree, a, s, ctx_resident(ctx).lose());
+    launch_batch_resident(nr, degree, a, s, ctx_resident(ctx).lose());
     BCHK_(hipGetLastError());
     BCHK_(hipEventRecord(b->ev1, s));
     launch_br_rhs_out(N, n_rhs, nr, perm, d_x, d_user, s);
     BCHK_(hipMemcpyAsync(hs.data(), st, hs.size() * sizeof(BLState), hipMemcpyDeviceToHost, s));
-    BCHK_(hipMemcpyAsync(head, words, sizeof head, hipMemcpyDeviceToHost, s));
+    BCHK_(hipMemcpyAsync(&gave_up, words, sizeof gave_up, hipMemcpyDeviceToHost, s));
     BCHK_(hipStreamSynchronize(s));
   }
-  ++(head[0] ? ctx_resident(ctx).given_up : ctx_resident(ctx).completed);
-  if (head[0]) {
-    if (!head[3] || b->br_degree == BR_DEGREE_MAX) {
-      b->br_off = true;
-      return FEMGPU_OK;
-    }
-    b->br_degree = BR_DEGREE_MAX;
-    return solve_resident_batch(ctx, b, n_rhs, nr, f, o, u_out, stats, solve_ms, ran);
+  ++(gave_up ? ctx_resident(ctx).given_up : ctx_resident(ctx).completed);
+  if (gave_up) {
+    b->br_off = true;
+    return FEMGPU_OK;
   }
   *ran = true;
   float ms = 0.f;

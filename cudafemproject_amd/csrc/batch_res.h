@@ -17,8 +17,9 @@ constexpr int BR_ELEMS = BR_THREADS;
 
 // Most neighbours of a node within its patch: regular triangulations have six,
 // and with 8 the rows of four systems fit the registers of two workgroups per
-// compute unit; a mesh with more runs with 12, which spill (60 plates of
-// 80 x 40, four load cases, FP64: 21.9 against 24.7 ms).
+// compute unit; a mesh with more (counted on the host when it is loaded) runs
+// with 12, which spill (60 plates of 80 x 40, four load cases, FP64: 21.9
+// against 24.7 ms).
 constexpr int BR_DEGREE = 8, BR_DEGREE_MAX = 12;
 
 // Words of a patch in its instance's exchange (three places of 2 nr values).
@@ -44,7 +45,6 @@ struct BRArgs {
   unsigned long long *entries, *words; // zero before the launch
   unsigned long long *abort;           // zero, then the bound of a wait (0: a second); nonzero
                                        // after a launch that did not complete
-  unsigned long long *crowded;         // zero; nonzero for a node with too many neighbours
   unsigned *ticket;                    // zero
   BLState *st;                         // per (instance, rhs), written at the end
   int max_iter;

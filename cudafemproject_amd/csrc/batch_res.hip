@@ -280,10 +280,11 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
     }
     __syncthreads();
     if (!row.build(has ? k : 0, c, b0, b1, s_ent, s_el, s_fix, s_c, diag, I.lam, I.mu)) {
-      st_agent(a.crowded, 1);
-      st_agent(a.abort, 1);
+      st_agent(a.abort, 1);  // (the host counted wrongly)
+      s_flag = 1;
     }
     __syncthreads();
+    if (s_flag) return;
   }
   const int node = has ? k : 0;
   constexpr int sv = BR_NODES * DIM;  // a system's stride in s_p, s_x

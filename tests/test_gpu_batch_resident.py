@@ -125,3 +125,19 @@ def test_two_batches_at_once():
     for k in (0, 1):
         for a, b in zip(want[k], got[k]):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("degree,fixed,resident", [(8, False, 1), (9, False, 1), (12, False, 1),
+                                                   (13, False, 0), (13, True, 1), (40, True, 1)])
+def test_form_by_neighbour_count(degree, fixed, resident):
+    """The rows are chosen before the launch: no launch runs in vain, and none
+    on rows that lack a neighbour (a constrained node's hold none)."""
+    nodes, elems = fan(degree)
+    rng = np.random.default_rng(degree)
+    b = instance(nodes, elems, rng, 2)
+    con = np.union1d(b.constr_node, [0]) if fixed else np.setdiff1d(b.constr_node, [0])
+    b.constr_node = con.astype(np.int32)
+    b.constr_code = np.full(len(con), 3, np.int32)
+    with F.Context(0) as c:
+        check(c, [b, instance(*fan(5), rng, 2)])
+        assert c.resident_info() == (2 * resident, 0)
