@@ -6,7 +6,7 @@ kernels for gfx950 behind the C-ABI of include/femgpu.h.
 """
 from ._lib import (BATCH_LOCKSTEP, BATCH_PERSISTENT, CG_SINGLE_REDUCTION, CG_STANDARD, FP32, FP64, MIXED, IMPLICIT_PHYSICAL, IMPLICIT_REFERENCE, LOADS_PHYSICAL,
                    LOADS_REFERENCE, MASS_PHYSICAL, MASS_REFERENCE, TOL_REF_GAMMA, TOL_REL_RES,
-                   RECV_ACCELERATION, RECV_DISPLACEMENT, RECV_VELOCITY, RESIDENT_AUTO, RESIDENT_OFF, RESIDENT_TEST_LATE, RESIDENT_TEST_LOSE, RESIDENT_TEST_LOSE_LATER, WAVELET_BERLAGE,
+                   RECV_ACCELERATION, RECV_DISPLACEMENT, RECV_VELOCITY, RESIDENT_AUTO, RESIDENT_OFF, RESIDENT_TEST_LATE, RESIDENT_TEST_LOSE, RESIDENT_TEST_LOSE_LATER, RESIDENT_TEST_SHORT_WAITS, WAVELET_BERLAGE,
                    WAVELET_NONE, WAVELET_RICKER, Context, FemGpuError,
                    load_library, plan_info)
 from .problem import Problem
@@ -17,4 +17,4 @@ __all__ = ["Context", "FemGpuError", "Problem", "load_library", "plan_info", "FP
            "WAVELET_BERLAGE", "IMPLICIT_REFERENCE", "IMPLICIT_PHYSICAL", "CG_STANDARD",
            "CG_SINGLE_REDUCTION", "BATCH_LOCKSTEP", "BATCH_PERSISTENT", "RECV_DISPLACEMENT", "RECV_VELOCITY", "RECV_ACCELERATION",
            "RESIDENT_AUTO", "RESIDENT_OFF", "RESIDENT_TEST_LOSE", "RESIDENT_TEST_LOSE_LATER",
-           "RESIDENT_TEST_LATE"]
+           "RESIDENT_TEST_LATE", "RESIDENT_TEST_SHORT_WAITS"]

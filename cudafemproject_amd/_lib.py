@@ -27,7 +27,8 @@ FP64, FP32, MIXED = 0, 1, 2
 TOL_REF_GAMMA, TOL_REL_RES = 0, 1
 CG_STANDARD, CG_SINGLE_REDUCTION = 0, 1
 BATCH_LOCKSTEP, BATCH_PERSISTENT = 0, 1
-RESIDENT_AUTO, RESIDENT_OFF, RESIDENT_TEST_LOSE, RESIDENT_TEST_LOSE_LATER, RESIDENT_TEST_LATE = 0, 1, 2, 3, 4
+RESIDENT_AUTO, RESIDENT_OFF = 0, 1
+RESIDENT_TEST_LOSE, RESIDENT_TEST_LOSE_LATER, RESIDENT_TEST_LATE, RESIDENT_TEST_SHORT_WAITS = 2, 3, 4, 5
 LOADS_REFERENCE, LOADS_PHYSICAL = 0, 1
 MASS_REFERENCE, MASS_PHYSICAL = 0, 1
 WAVELET_NONE, WAVELET_RICKER, WAVELET_BERLAGE = 0, 1, 2

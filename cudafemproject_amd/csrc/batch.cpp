@@ -335,7 +335,8 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   const int64_t N = b->total_nodes;
   const size_t nd = size_t(N) * 2, nv = nd * nr, nu = nd * n_rhs;
   const size_t n_state = size_t(b->n_inst) * nr;
-  // entries, exchange words, abort flag and ticket: zero before the launch
+  // abort word, bound of a wait, tickets, signs of progress, exchange words,
+  // entries: zero before the launch
   const size_t n_ent = size_t(b->br_entries) * br_entry_words(nr);
   const size_t n_words = br_patch_words(nr) * size_t(b->bl_np);
   double *d_user, *d_f, *d_x, *diag, *slots, *invD, *zero;
@@ -346,7 +347,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   BCHK_(bbuf(b, "bl_diag64", nd, &diag));
   BCHK_(bbuf(b, "bl_s64", size_t(b->bl_slots) * nr * 2 + 1, &slots));
   BCHK_(bbuf(b, "bl64_invD", nd, &invD));
-  BCHK_(bbuf(b, "br_words", n_ent + n_words + 3, &zero));
+  BCHK_(bbuf(b, "br_words", n_ent + n_words + 4, &zero));
   BCHK_(bbuf(b, "bl_state", n_state, &st));
   auto *words = reinterpret_cast<unsigned long long *>(zero);
   auto table = [&](const char *name) { return b->bufs[name].first; };
@@ -375,8 +376,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   a.invD = invD;
   a.x = d_x;
   a.abort = words;
-  a.ticket = reinterpret_cast<unsigned *>(words + 2);
-  a.words = words + 3;
+  a.words = words + 4;
   a.entries = a.words + n_words;
   a.st = st;
   a.max_iter = o.max_iter > 0 ? o.max_iter : 100000;
@@ -405,8 +405,8 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
     bl_diag(2, m, b->bl_nif, diag, slots, s);
     bl_inv_diag<double>(int64_t(nd), diag, invD, s);
-    launch_fill<double>(zero, int64_t(n_ent + n_words + 3), 0.0, s);
-    if (ctx_resident(ctx).lose_from >= 0) launch_fill<double>(zero + 1, 1, test_wait(), s);
+    launch_fill<double>(zero, int64_t(n_ent + n_words + 4), 0.0, s);
+    if (ctx_resident(ctx).impatient()) launch_fill<double>(zero + 1, 1, test_wait(), s);
     launch_fill<double>(d_x, int64_t(nv), 0.0, s);
     launch_batch_resident(nr, degree, a, s, ctx_resident(ctx).lose());
     BCHK_(hipGetLastError());

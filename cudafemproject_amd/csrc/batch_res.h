@@ -43,9 +43,9 @@ struct BRArgs {
   const double *f, *invD;              // [node][rhs][2], [node][2]
   double *x;                           // solution, likewise
   unsigned long long *entries, *words; // zero before the launch
-  unsigned long long *abort;           // zero, then the bound of a wait (0: a second); nonzero
-                                       // after a launch that did not complete
-  unsigned *ticket;                    // zero
+  unsigned long long *abort;           // zero; nonzero after a launch that did not complete; then
+                                       // the bound of a wait (0: a second), the ticket counter,
+                                       // the signs of progress (zero both)
   BLState *st;                         // per (instance, rhs), written at the end
   int max_iter;
   double tol2;

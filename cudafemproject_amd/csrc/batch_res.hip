@@ -26,7 +26,9 @@
 // instance: when a workgroup waits for a peer that has not started, only
 // earlier instances and its own are on the chip, and the earlier ones end, so
 // it starts in the end, in whatever order the hardware starts workgroups, as
-// long as one instance fits the chip.  (Waits are bounded all the same.)
+// long as one instance fits the chip.  Waits are bounded all the same, for a
+// peer that has started from the wait's begin, else from the last sign of
+// progress of an earlier instance.
 //
 // All arithmetic is FP64.  A system ends on its FP64 residual f - K x, formed
 // when the recurrence's meets the tolerance.
@@ -99,14 +101,14 @@ __device__ __forceinline__ void publish_lanes(u64 *words, int i, unsigned tag, d
 }
 template <int NV>
 __device__ __forceinline__ bool gather_lanes(const u64 *words, int np, unsigned tag, u64 *abort,
-                                             double &sum) {
+                                             unsigned last, double &sum) {
   constexpr int G = 64 / NV, NB = 4;
   const int l = fresh(threadIdx.x), v = (l >> 3) % NV;
   sum = 0.0;
   bool ok = true;
   for (int i0 = (l & 7) + 8 * ((l >> 3) / NV); ok && i0 < np; i0 += G * NB) {
     u64 h[NB][2];
-    Patience wait{abort};
+    QueuePatience wait{abort, last};
     for (int spin = 0;; ++spin) {
       bool all = true;
 #pragma unroll
@@ -202,7 +204,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
   const int t = threadIdx.x;
   if (t == 0) {
     s_flag = 0;
-    s_ticket = int(atomicAdd(a.ticket, 1u));
+    s_ticket = int(atomicAdd(reinterpret_cast<unsigned *>(a.abort + 2), 1u));
   }
   __syncthreads();
   const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
@@ -228,6 +230,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
   const BLInst I = a.inst[P.pad];
   const int np = I.p1 - I.p0, lp = pid - I.p0;
   const bool alone = np == 1;
+  const unsigned last = unsigned(ticket - lp + np - 1);  // the instance's last ticket
   // p'q, r'z and r'r, the same of a replaced residual (three places: one is
   // written again only after two exchanges that every workgroup took part in)
   u64 *xpq = a.words + br_patch_words(NR) * size_t(I.p0);
@@ -319,8 +322,8 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
     for (int i = t % TV; i < E.n_in; i += TV)
       send_entry<double, DIM>(a.entries, at(s_oe[i]), entry_tag, &s_in[int(s_os[i]) * NX + v * DIM]);
     for (int i = t % TV; i < E.n_in; i += TV)
-      if (!recv_entry<double, DIM>(a.entries, at(unsigned(E.in_start + i)), entry_tag, a.abort,
-                                   &s_in[int(s_ip[i]) * NX + v * DIM]))
+      if (!recv_entry<double, DIM>(a.entries, at(unsigned(E.in_start + i)), entry_tag,
+                                   QueuePatience{a.abort, last}, &s_in[int(s_ip[i]) * NX + v * DIM]))
         s_flag = 1;
   };
   auto collect = [&](double (&y)[NR]) {
@@ -345,7 +348,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
     if (t < 64) {
       if (!alone) {
         publish_lanes<2 * NR>(ex, lp, tag, s);
-        if (!gather_lanes<2 * NR>(ex, np, tag, a.abort, s)) s_flag = 1;
+        if (!gather_lanes<2 * NR>(ex, np, tag, a.abort, last, s)) s_flag = 1;
       }
       const double o = lane_xor<8 * NR>(s);
       const bool second = t & (8 * NR);
@@ -383,6 +386,10 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
   }
   bool ok = s_flag == 0;
   while (ok) {
+    // a sign of progress to the instances that wait for room (some every 32
+    // iterations)
+    if (lp == 0 && t == 0 && ((tag >> 1) & 31u) == 0)
+      (void)__hip_atomic_fetch_add(a.abort + 3, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned iter = __builtin_amdgcn_readfirstlane(s_iter);
     const unsigned want = __builtin_amdgcn_readfirstlane(s_want);
     if (!(iter | want)) break;
@@ -429,7 +436,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
       trade(iter);
     }
     if (t < 64) {
-      if (!alone && !gather_lanes<NR>(xpq, np, tag, a.abort, d)) s_flag = 1;
+      if (!alone && !gather_lanes<NR>(xpq, np, tag, a.abort, last, d)) s_flag = 1;
       double alpha = 0.0;
       if (S.state == 0) {
         alpha = S.g / d;

@@ -780,7 +780,7 @@ int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long 
   if (ctx->res_np != ctx->dm.np) {
     femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
     femgpu::launch_fill<double>(e, int64_t(2 * (n64 + n32)), 0.0, ctx->stream);
-    if (ctx->res.lose_from >= 0)
+    if (ctx->res.impatient())
       femgpu::launch_fill<double>(w + 2, 1, femgpu::test_wait(), ctx->stream);
     ctx->res_np = ctx->dm.np;
   }
@@ -936,7 +936,7 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
     d.n_steps = std::min(n_steps - done, RES_STEP_CAP);
     if (ctx->dyn_np != ctx->dm.np) {
       femgpu::launch_fill<double>(w, int64_t(n), 0.0, ctx->stream);
-      if (ctx->res.lose_from >= 0)
+      if (ctx->res.impatient())
         femgpu::launch_fill<double>(w + n - 1, 1, femgpu::test_wait(), ctx->stream);
       ctx->dyn_np = ctx->dm.np;
       ctx->dyn_tag[0] = ctx->dyn_tag[1] = 0;
@@ -1441,7 +1441,7 @@ int femgpu_sync(femgpu_ctx *ctx) {
 
 int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
   if (!ctx) return FEMGPU_E_ARG;
-  if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_LATE)
+  if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_SHORT_WAITS)
     return fail(ctx, FEMGPU_E_ARG, "set_resident: unknown mode");
   ctx->res.mode = mode;
   ctx->res.off = false;
@@ -1449,6 +1449,7 @@ int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
                        : mode == FEMGPU_RESIDENT_TEST_LOSE_LATER ? ctx->res.completed + 2
                                                                  : -1;
   ctx->res.late = mode == FEMGPU_RESIDENT_TEST_LATE;
+  ctx->res.short_waits = mode == FEMGPU_RESIDENT_TEST_SHORT_WAITS;
   ctx->res_np = ctx->dyn_np = 0;  // (the exchange words are made again)
   return FEMGPU_OK;
 }

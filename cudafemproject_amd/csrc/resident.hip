@@ -376,7 +376,7 @@ struct ResPatch {
     for (int i = threadIdx.x; i < n_in; i += PT)
       send_entry<T, DIM>(entries, s_oe[i], tag, &s_in[int(s_os[i]) * DIM]);
     for (int i = threadIdx.x; i < n_in; i += PT)
-      if (!recv_entry<T, DIM>(entries, unsigned(in_start + i), tag, abort, &s_in[int(s_ip[i]) * DIM]))
+      if (!recv_entry<T, DIM>(entries, unsigned(in_start + i), tag, Patience{abort}, &s_in[int(s_ip[i]) * DIM]))
         return false;
     return true;
   }

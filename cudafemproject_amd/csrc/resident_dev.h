@@ -52,6 +52,27 @@ struct Patience {
   }
 };
 
+// The same in a launch whose workgroups take tickets: while the peers waited
+// for may not have started (the ticket counter, abort[2], has not passed `last`),
+// the bound runs from the last sign of progress of any workgroup (abort[3]):
+// they start when earlier instances end, which may take long, but ends.
+struct QueuePatience {
+  u64 *abort;
+  unsigned last;
+  u64 start = 0, seen = 0;
+  __device__ __forceinline__ bool over(int spin) {
+    if ((spin & 255) != 255) return false;
+    const u64 now = wall_clock64();
+    const u64 signs = ld_agent(abort + 3);
+    if (start == 0 || (signs != seen && unsigned(ld_agent(abort + 2)) <= last)) start = now;
+    seen = signs;
+    const u64 limit = ld_agent(abort + 1);
+    if (ld_agent(abort) == 0 && now - start <= (limit ? limit : WAIT_TICKS)) return false;
+    st_agent(abort, 1);
+    return true;
+  }
+};
+
 // Interface sums travel as entries (femgpu_internal.h): the bits of DIM values
 // in words of 48 under a 16-bit tag (a third fewer words than 32 under 32;
 // the traffic of some hundred kilobytes a step per workgroup is what bounds a
@@ -100,12 +121,11 @@ __device__ __forceinline__ void send_entry(u64 *entries, unsigned e, unsigned ta
 }
 
 // Entry e into v; false when the wait ran out.
-template <typename T, int DIM>
-__device__ __forceinline__ bool recv_entry(const u64 *entries, unsigned e, unsigned tag, u64 *abort,
+template <typename T, int DIM, typename Wait>
+__device__ __forceinline__ bool recv_entry(const u64 *entries, unsigned e, unsigned tag, Wait wait,
                                            T *v) {
   constexpr int W = EW<T, DIM>, U = sizeof(T) / 4;
   u64 h[W];
-  Patience wait{abort};
   for (int spin = 0;; ++spin) {
     bool all = true;
 #pragma unroll

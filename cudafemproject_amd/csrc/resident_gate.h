@@ -18,6 +18,8 @@ struct ResidentUse {
   int64_t lose_from = -1;       // tests: launches from this one on lack a workgroup
   bool late = false;            // tests: one gives up at its end
   bool on() const { return mode != 1 && !off; }
+  bool short_waits = false;     // tests: waits run out after 2 ms, nothing is lost
+  bool impatient() const { return short_waits || lose_from >= 0; }
   bool lose() const { return lose_from >= 0 && completed >= lose_from; }
 };
 

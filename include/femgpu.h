@@ -131,13 +131,15 @@ int femgpu_sync(femgpu_ctx *ctx);
  * tests and measurements of either form.  Tests of what follows a launch that
  * does not complete: every such launch (LOSE), or every one from the third on
  * (LOSE_LATER), lacks a workgroup, and the others' waits run out after 2 ms;
- * or a workgroup of a solve gives up when all others have ended (LATE). */
+ * or a workgroup of a solve gives up when all others have ended (LATE); or
+ * waits run out after 2 ms and nothing else is changed (SHORT_WAITS). */
 enum {
   FEMGPU_RESIDENT_AUTO = 0,
   FEMGPU_RESIDENT_OFF = 1,
   FEMGPU_RESIDENT_TEST_LOSE = 2,
   FEMGPU_RESIDENT_TEST_LOSE_LATER = 3,
-  FEMGPU_RESIDENT_TEST_LATE = 4
+  FEMGPU_RESIDENT_TEST_LATE = 4,
+  FEMGPU_RESIDENT_TEST_SHORT_WAITS = 5
 };
 int femgpu_set_resident(femgpu_ctx *ctx, int mode);
 /* Launches of this context that stayed on the chip: info[0] completed,

@@ -141,3 +141,22 @@ def test_form_by_neighbour_count(degree, fixed, resident):
     with F.Context(0) as c:
         check(c, [b, instance(*fan(5), rng, 2)])
         assert c.resident_info() == (2 * resident, 0)
+
+
+def test_patience_with_queued_peers():
+    """Instances of more than half the device each: the second one's first
+    workgroups wait for the rest of it until the first one ends, here some ten
+    times the bound of a wait (2 ms).  Nobody gives up, and the bits are those
+    with the usual bound."""
+    insts = plate_batch(3, seed=5, nx_range=(255, 260), ny_range=(255, 260))
+    rhs = [b.f[:, :1] for b in insts]
+    with F.Context(0) as c:
+        load_batch(c, insts)
+        us, st, ms = c.batch_solve(rhs, precision=F.FP64, tol=1e-8)
+        print(f"[patience] {ms:.1f} ms, {st['iterations'].ravel()} iterations", flush=True)
+        assert np.all(st["status"] == 0) and c.resident_info() == (1, 0)
+        assert ms > 40.0  # (three instances in turn: each waits some 10 ms)
+        c.set_resident(F.RESIDENT_TEST_SHORT_WAITS)
+        us2, st2, _ = c.batch_solve(rhs, precision=F.FP64, tol=1e-8)
+        assert c.resident_info() == (2, 0)
+        assert np.array_equal(st, st2) and all(np.array_equal(a, b) for a, b in zip(us, us2))
