@@ -397,10 +397,14 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   m.pn = b->bl_pn;
   const int32_t *perm = static_cast<const int32_t *>(table("br_perm"));
   std::vector<BLState> hs(n_state);
+  // (tests: fewer than the largest instance needs)
+  const int groups = ctx_resident(ctx).lose() && b->br_np_max > 1
+                         ? b->br_np_max - 1
+                         : std::min(b->bl_np, br_groups_max(ctx_device(ctx)));
   unsigned long long gave_up;
   BCHK_(hipMemcpyAsync(d_user, f, nu * sizeof(double), hipMemcpyHostToDevice, s));
   {
-    const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(b->bl_np) / capacity), block);
+    const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(groups) / capacity), block);
     BCHK_(hipEventRecord(b->ev0, s));
     launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
     bl_diag(2, m, b->bl_nif, diag, slots, s);
@@ -408,7 +412,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     launch_fill<double>(zero, int64_t(n_ent + n_words + 4), 0.0, s);
     if (ctx_resident(ctx).impatient()) launch_fill<double>(zero + 1, 1, test_wait(), s);
     launch_fill<double>(d_x, int64_t(nv), 0.0, s);
-    launch_batch_resident(nr, degree, a, s, ctx_resident(ctx).lose());
+    launch_batch_resident(nr, degree, a, groups, s);
     BCHK_(hipGetLastError());
     BCHK_(hipEventRecord(b->ev1, s));
     launch_br_rhs_out(N, n_rhs, nr, perm, d_x, d_user, s);

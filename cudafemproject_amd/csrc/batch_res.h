@@ -45,7 +45,7 @@ struct BRArgs {
   unsigned long long *entries, *words; // zero before the launch
   unsigned long long *abort;           // zero; nonzero after a launch that did not complete; then
                                        // the bound of a wait (0: a second), the ticket counter,
-                                       // the signs of progress (zero both)
+                                       // the time of the last sign of progress (zero both)
   BLState *st;                         // per (instance, rhs), written at the end
   int max_iter;
   double tol2;
@@ -56,8 +56,11 @@ struct BRArgs {
 int br_lds_bytes(int nr, int pn, int ent, int n_in, int n_src);
 int br_capacity(int nr, int degree, int lds, int device, double *block);
 
-// (short_grid: tests; without the last ticket)
-void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s, bool short_grid);
+// groups: at least as many as the patches of any instance, and at most
+// br_groups_max, what the registers let the device hold (those that start late
+// find no ticket left, so more would do no harm).
+int br_groups_max(int device);
+void launch_batch_resident(int nr, int degree, const BRArgs &a, int groups, hipStream_t s);
 
 // Right-hand sides to internal node order padded to nr, and solutions back.
 void launch_br_rhs_in(int64_t n, int n_rhs, int nr, const int32_t *perm, const double *user,

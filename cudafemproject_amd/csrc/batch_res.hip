@@ -22,13 +22,16 @@
 // one workgroup: the products 4.2, two trips through memory 3.6 + 2.2 and 4.6,
 // interface sums 1.9, block sums 2; two workgroups per compute unit overlap.
 //
-// Workgroups take tickets as they start and the tickets run instance by
-// instance: when a workgroup waits for a peer that has not started, only
-// earlier instances and its own are on the chip, and the earlier ones end, so
-// it starts in the end, in whatever order the hardware starts workgroups, as
-// long as one instance fits the chip.  Waits are bounded all the same, for a
-// peer that has started from the wait's begin, else from the last sign of
-// progress of an earlier instance.
+// Workgroups take tickets, a patch each, and the tickets run instance by instance;
+// one that is done takes the next.  Whoever waits for a ticket that nobody has
+// taken waits for earlier instances only, and those end: the earliest one that
+// has not ended has all its patches in hand, as long as as many workgroups as
+// its patches are on the chip.  A launch has no more workgroups than the chip
+// holds.  (With a workgroup per ticket the later ones start when places become
+// free, and the hardware does not always start the next one that some compute
+// unit has room for: three plates of some 320 patches each stood still in one
+// run of three, some 100 places empty, until the waits ran out.)  Waits are
+// bounded all the same, from the launch's last sign of progress.
 //
 // All arithmetic is FP64.  A system ends on its FP64 residual f - K x, formed
 // when the recurrence's meets the tolerance.
@@ -83,7 +86,7 @@ template <int NV>
 __device__ __forceinline__ double block_sums(const double (&v)[NV], double *s_red) {
   static_assert(PT == 512, "eight waves: a value's in eight lanes");
   const double s = wave_sums<NV>(v);
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int tx = fresh(threadIdx.x), w = tx >> 6, l = tx & 63;
   if (l % (64 / NV) == 0) s_red[(l / (64 / NV)) * 8 + w] = s;
   __syncthreads();
   return w == 0 ? sum8(s_red[((l >> 3) % NV) * 8 + (l & 7)]) : 0.0;
@@ -94,21 +97,21 @@ __device__ __forceinline__ double block_sums(const double (&v)[NV], double *s_re
 // order.  False when a workgroup gave up.
 template <int NV>
 __device__ __forceinline__ void publish_lanes(u64 *words, int i, unsigned tag, double v) {
-  const int l = threadIdx.x;
+  const int l = fresh(threadIdx.x);
   u64 w[2];
   tag_words(v, tag, w);
   if (l < 8 * NV && (l & 7) < 2) st_agent(&words[(size_t(i) * NV + (l >> 3)) * 2 + (l & 1)], l & 1 ? w[1] : w[0]);
 }
 template <int NV>
 __device__ __forceinline__ bool gather_lanes(const u64 *words, int np, unsigned tag, u64 *abort,
-                                             unsigned last, double &sum) {
+                                             double &sum) {
   constexpr int G = 64 / NV, NB = 4;
   const int l = fresh(threadIdx.x), v = (l >> 3) % NV;
   sum = 0.0;
   bool ok = true;
   for (int i0 = (l & 7) + 8 * ((l >> 3) / NV); ok && i0 < np; i0 += G * NB) {
     u64 h[NB][2];
-    QueuePatience wait{abort, last};
+    QueuePatience wait{abort};
     for (int spin = 0;; ++spin) {
       bool all = true;
 #pragma unroll
@@ -193,24 +196,15 @@ struct BRSystem {
   }
 };
 
+// One patch from the first residual to the end of its instance's systems.
+// s_flag: 0; false: a wait ran out.
 template <int NR, int DEGREE>
-__global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
+__device__ __forceinline__ bool solve_patch(const BRArgs &a, int pid, unsigned char *lds, int &s_flag) {
   constexpr int W = PT / 64;
   constexpr int NPE = DIM + 1, NX = DIM * NR;
-  extern __shared__ __align__(16) unsigned char lds[];
   __shared__ BRRest s_rest[NR];
-  __shared__ int s_flag, s_ticket, s_iter, s_want;  // s_iter, s_want: systems that iterate, whose
-                                                    // residual is wanted
-  const int t = threadIdx.x;
-  if (t == 0) {
-    s_flag = 0;
-    s_ticket = int(atomicAdd(reinterpret_cast<unsigned *>(a.abort + 2), 1u));
-  }
-  __syncthreads();
-  const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
-  if (ticket >= a.np) return;
-  const int pid = a.order[ticket];
-
+  __shared__ int s_iter, s_want;  // systems that iterate, whose residual is wanted
+  const int t = fresh(threadIdx.x);  // (nothing of a patch is kept for the next)
   const BRLds L = br_lds(NR, a.pn, a.ent, a.n_in_max, a.n_src_max);
   double *s_p = reinterpret_cast<double *>(lds);
   uint16_t *s_ent = reinterpret_cast<uint16_t *>(lds);
@@ -230,7 +224,6 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
   const BLInst I = a.inst[P.pad];
   const int np = I.p1 - I.p0, lp = pid - I.p0;
   const bool alone = np == 1;
-  const unsigned last = unsigned(ticket - lp + np - 1);  // the instance's last ticket
   // p'q, r'z and r'r, the same of a replaced residual (three places: one is
   // written again only after two exchanges that every workgroup took part in)
   u64 *xpq = a.words + br_patch_words(NR) * size_t(I.p0);
@@ -287,7 +280,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
       s_flag = 1;
     }
     __syncthreads();
-    if (s_flag) return;
+    if (s_flag) return false;
   }
   const int node = has ? k : 0;
   constexpr int sv = BR_NODES * DIM;  // a system's stride in s_p, s_x
@@ -323,7 +316,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
       send_entry<double, DIM>(a.entries, at(s_oe[i]), entry_tag, &s_in[int(s_os[i]) * NX + v * DIM]);
     for (int i = t % TV; i < E.n_in; i += TV)
       if (!recv_entry<double, DIM>(a.entries, at(unsigned(E.in_start + i)), entry_tag,
-                                   QueuePatience{a.abort, last}, &s_in[int(s_ip[i]) * NX + v * DIM]))
+                                   QueuePatience{a.abort}, &s_in[int(s_ip[i]) * NX + v * DIM]))
         s_flag = 1;
   };
   auto collect = [&](double (&y)[NR]) {
@@ -348,7 +341,7 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
     if (t < 64) {
       if (!alone) {
         publish_lanes<2 * NR>(ex, lp, tag, s);
-        if (!gather_lanes<2 * NR>(ex, np, tag, a.abort, last, s)) s_flag = 1;
+        if (!gather_lanes<2 * NR>(ex, np, tag, a.abort, s)) s_flag = 1;
       }
       const double o = lane_xor<8 * NR>(s);
       const bool second = t & (8 * NR);
@@ -386,10 +379,6 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
   }
   bool ok = s_flag == 0;
   while (ok) {
-    // a sign of progress to the instances that wait for room (some every 32
-    // iterations)
-    if (lp == 0 && t == 0 && ((tag >> 1) & 31u) == 0)
-      (void)__hip_atomic_fetch_add(a.abort + 3, u64(1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     unsigned iter = __builtin_amdgcn_readfirstlane(s_iter);
     const unsigned want = __builtin_amdgcn_readfirstlane(s_want);
     if (!(iter | want)) break;
@@ -436,7 +425,11 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
       trade(iter);
     }
     if (t < 64) {
-      if (!alone && !gather_lanes<NR>(xpq, np, tag, a.abort, last, d)) s_flag = 1;
+      if (!alone && !gather_lanes<NR>(xpq, np, tag, a.abort, d)) s_flag = 1;
+      // every 32 iterations a sign of progress to those who wait (here: at the
+      // loop's begin it moved the spills about, and four systems took 6 %
+      // longer)
+      if ((tag & 62u) == 0 && t == 0) st_agent(a.abort + 3, wall_clock64());
       double alpha = 0.0;
       if (S.state == 0) {
         alpha = S.g / d;
@@ -490,6 +483,21 @@ __global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
     o.ff = R.ff;
     o.rr = R.rr;
   }
+  return ok;
+}
+
+template <int NR, int DEGREE>
+__global__ __launch_bounds__(PT, 4) void k_batch_resident(BRArgs a) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  __shared__ int s_flag, s_ticket;
+  if (threadIdx.x == 0) s_flag = 0;
+  for (;;) {
+    __syncthreads();  // (the last patch's values are read)
+    if (threadIdx.x == 0) s_ticket = int(atomicAdd(reinterpret_cast<unsigned *>(a.abort + 2), 1u));
+    __syncthreads();
+    const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+    if (ticket >= a.np || !solve_patch<NR, DEGREE>(a, a.order[ticket], lds, s_flag)) return;
+  }
 }
 
 // One value per thread: node, rhs, component.
@@ -540,9 +548,11 @@ int br_capacity(int nr, int degree, int lds, int device, double *block) {
   return per * cu;
 }
 
-void launch_batch_resident(int nr, int degree, const BRArgs &a, hipStream_t s, bool short_grid) {
+int br_groups_max(int device) { return 2 * compute_units(device); }
+
+void launch_batch_resident(int nr, int degree, const BRArgs &a, int groups, hipStream_t s) {
   const int lds = br_lds_bytes(nr, a.pn, a.ent, a.n_in_max, a.n_src_max);
-  hipLaunchKernelGGL(kernel_of(nr, degree), dim3(a.np - (short_grid && a.np > 1)), dim3(PT), lds, s, a);
+  hipLaunchKernelGGL(kernel_of(nr, degree), dim3(groups), dim3(PT), lds, s, a);
 }
 
 void launch_br_rhs_in(int64_t n, int n_rhs, int nr, const int32_t *perm, const double *user,

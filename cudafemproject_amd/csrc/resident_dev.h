@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
+
 #include "element.h"
 #include "patch_common.h"
 #include "resident.h"
@@ -17,7 +19,7 @@ using namespace patch;
 
 using u64 = unsigned long long;
 
-constexpr u64 WAIT_TICKS = 100000000ull;  // one second of the 100 MHz clock
+constexpr int WAIT_TICKS = 100000000;  // one second of the 100 MHz clock
 
 __device__ __forceinline__ void st_agent(u64 *p, u64 v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -37,39 +39,37 @@ __device__ __forceinline__ double untag(const u64 (&w)[2]) {
 
 // A bounded wait: true once the caller should give up (another workgroup
 // did, or WAIT_TICKS -- or what the host put beside the abort word -- have
-// passed since the 256th look).
+// passed since the 256th look).  (Times in 32 bits, 42 s round: the wait loops
+// stand where registers are short.)
 struct Patience {
   u64 *abort;
-  u64 start = 0;
+  unsigned start = 0;
   __device__ __forceinline__ bool over(int spin) {
     if ((spin & 255) != 255) return false;
-    const u64 now = wall_clock64();
-    if (start == 0) start = now;
-    const u64 limit = ld_agent(abort + 1);
-    if (ld_agent(abort) == 0 && now - start <= (limit ? limit : WAIT_TICKS)) return false;
+    const unsigned now = unsigned(wall_clock64());
+    if (start == 0) start = now | 1u;
+    return expired(abort, int(now - start));
+  }
+  static __device__ __forceinline__ bool expired(u64 *abort, int waited) {
+    const int limit = int(ld_agent(abort + 1));
+    if (ld_agent(abort) == 0 && waited <= (limit ? limit : WAIT_TICKS)) return false;
     st_agent(abort, 1);
     return true;
   }
 };
 
-// The same in a launch whose workgroups take tickets: while the peers waited
-// for may not have started (the ticket counter, abort[2], has not passed `last`),
-// the bound runs from the last sign of progress of any workgroup (abort[3]):
-// they start when earlier instances end, which may take long, but ends.
+// The same in a launch whose workgroups take tickets: the bound runs from the
+// last sign of progress of any workgroup (its time, in abort[3]).  The peers waited
+// for may still be busy with earlier instances, which may take long, but ends.
 struct QueuePatience {
   u64 *abort;
-  unsigned last;
-  u64 start = 0, seen = 0;
+  unsigned start = 0;
   __device__ __forceinline__ bool over(int spin) {
     if ((spin & 255) != 255) return false;
-    const u64 now = wall_clock64();
-    const u64 signs = ld_agent(abort + 3);
-    if (start == 0 || (signs != seen && unsigned(ld_agent(abort + 2)) <= last)) start = now;
-    seen = signs;
-    const u64 limit = ld_agent(abort + 1);
-    if (ld_agent(abort) == 0 && now - start <= (limit ? limit : WAIT_TICKS)) return false;
-    st_agent(abort, 1);
-    return true;
+    const unsigned now = unsigned(wall_clock64());
+    if (start == 0) start = now | 1u;
+    const unsigned sign = unsigned(ld_agent(abort + 3));
+    return Patience::expired(abort, min(int(now - start), sign ? int(now - sign) : INT_MAX));
   }
 };
 
@@ -316,10 +316,10 @@ __device__ __forceinline__ unsigned lane_xor(unsigned v) {
     return unsigned(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xf, 0xf, false));
   } else if constexpr (O == 16) {
     const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return threadIdx.x & 16u ? r[0] : r[1];
+    return fresh(threadIdx.x) & 16u ? r[0] : r[1];
   } else {
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return threadIdx.x & 32u ? r[0] : r[1];
+    return fresh(threadIdx.x) & 32u ? r[0] : r[1];
   }
 }
 template <int O>
@@ -359,7 +359,7 @@ __device__ __forceinline__ double wave_sums(const double (&v)[NV]) {
   if constexpr (NV == 8) {
     const double s0 = fold<16>(fold<32>(v[0], v[4]), fold<32>(v[2], v[6]));
     const double s1 = fold<16>(fold<32>(v[1], v[5]), fold<32>(v[3], v[7]));
-    const bool hi = threadIdx.x & 8u;
+    const bool hi = fresh(threadIdx.x) & 8u;
     return sum8((hi ? s1 : s0) + lane_xor<8>(hi ? s0 : s1));
   } else {
     double s;

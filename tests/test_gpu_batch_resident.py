@@ -160,3 +160,23 @@ def test_patience_with_queued_peers():
         us2, st2, _ = c.batch_solve(rhs, precision=F.FP64, tol=1e-8)
         assert c.resident_info() == (2, 0)
         assert np.array_equal(st, st2) and all(np.array_equal(a, b) for a, b in zip(us, us2))
+
+
+@pytest.mark.parametrize("nr,n,count", [(1, 258, 3), (4, 175, 4), (2, 120, 9)])
+def test_large_instances_take_turns(nr, n, count):
+    """More patches than the device holds, in instances of up to two thirds of
+    it: every launch completes (in fresh contexts: the hardware starts a launch's
+    workgroups differently from one to the next), with the same bits."""
+    insts = plate_batch(count, seed=7, nx_range=(n - 3, n + 3), ny_range=(n - 3, n + 3))
+    rhs = [b.f[:, :nr] for b in insts]
+    first = None
+    for k in range(3):
+        print(f"[turns] {nr} {n} {count} context {k}", flush=True)
+        with F.Context(0) as c:
+            load_batch(c, insts)
+            for _ in range(2):
+                us, st, _ = c.batch_solve(rhs, precision=F.FP64, tol=1e-6)
+                assert np.all(st["status"] == 0)
+                first = us if first is None else first
+                assert all(np.array_equal(a, b) for a, b in zip(us, first))
+            assert c.resident_info() == (2, 0)
