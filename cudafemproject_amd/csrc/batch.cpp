@@ -404,7 +404,10 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   unsigned long long gave_up;
   BCHK_(hipMemcpyAsync(d_user, f, nu * sizeof(double), hipMemcpyHostToDevice, s));
   {
-    const ResidentGate gate(ctx_device(ctx), std::min(1.0, double(groups) / capacity), block);
+    // (in eights: the hardware deals them out to 8 XCDs)
+    const int dealt = (groups + 7) & ~7;
+    const ResFit fit{std::min(1.0, double(dealt) / capacity), block, dealt};
+    const ResidentGate gate(ctx_device(ctx), compute_units(ctx_device(ctx)), fit);
     BCHK_(hipEventRecord(b->ev0, s));
     launch_br_rhs_in(N, n_rhs, nr, perm, d_user, d_f, s);
     bl_diag(2, m, b->bl_nif, diag, slots, s);

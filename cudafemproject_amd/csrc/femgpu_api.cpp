@@ -808,7 +808,7 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
     ctx->h_sc->done = femgpu::RES_ABORTED;
     ctx->h_sc->gave_up = 0;
     {
-      ResidentGate gate(ctx->device, fit.share, fit.block);
+      ResidentGate gate(ctx->device, femgpu::compute_units(ctx->device), fit);
       femgpu::launch_res_pcg<T>(ctx->dm, a, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -891,7 +891,7 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     ctx->h_sc->done = femgpu::RES_ABORTED;
     ctx->h_sc->gave_up = 0;
     {
-      ResidentGate gate(ctx->device, fit.share, fit.block);
+      ResidentGate gate(ctx->device, femgpu::compute_units(ctx->device), fit);
       femgpu::launch_res_impl<T>(ctx->dm, m, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -947,7 +947,7 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
     last_tag += unsigned(d.n_steps);
     unsigned long long *gave_up = reinterpret_cast<unsigned long long *>(&ctx->h_sc[3]);
     {
-      ResidentGate gate(ctx->device, fit.share, fit.block);
+      ResidentGate gate(ctx->device, femgpu::compute_units(ctx->device), fit);
       femgpu::launch_res_dyn<T>(ctx->dm, d, ctx->stream, ctx->res.lose());
       HIPCHK(hipGetLastError());
       HIPCHK(hipMemcpyAsync(gave_up, d.abort, sizeof(*gave_up), hipMemcpyDeviceToHost, ctx->stream));

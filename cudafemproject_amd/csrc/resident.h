@@ -8,6 +8,7 @@
 #include <cstdint>
 
 #include "kernels.h"
+#include "resident_gate.h"
 
 namespace femgpu {
 
@@ -61,12 +62,6 @@ struct ResPcg {
 // gives up sets gave_up itself: it may be after the one that writes the scalars
 // has ended, in the last exchange.
 constexpr int RES_ABORTED = 6, RES_CAP = 7, RES_FAINT = 8;
-
-// The part of the device that a resident launch takes, and of one compute
-// unit that a workgroup takes.
-struct ResFit {
-  double share = 0.0, block = 0.0;
-};
 
 // Whether the plan's PCG runs resident: patches of up to 512 nodes and 1536
 // elements, every workgroup on a compute unit of its own.  Several workgroups

@@ -958,6 +958,7 @@ bool fits(const DevMesh &dm, int device, const void *fn, int lds, ResFit *fit) {
   if (per < 1 || grid > cu) return false;
   fit->block = 1.0 / per;
   fit->share = double(grid) / (double(per) * cu);
+  fit->groups = grid;
   return true;
 }
 

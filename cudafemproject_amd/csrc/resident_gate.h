@@ -32,27 +32,40 @@ inline double test_wait() {
   return v;
 }
 
+// The part of the device that a resident launch takes, of one compute unit that
+// a workgroup takes, and its workgroups.
+struct ResFit {
+  double share = 0.0, block = 0.0;
+  int groups = 0;
+};
+
 // Resident launches (resident.h) wait for each other's workgroups, so all
 // workgroups of a launch must reach the device: alone they do when they fit
-// it; beside others they do while the launches' shares and the largest
-// workgroup together stay within it (then some compute unit always has room
-// for the next workgroup).  A launch that would not fit waits here for the
-// others to end.
+// it; beside others they do while some compute unit always has room for the next
+// workgroup.  It has while the launches' shares and the largest workgroup
+// together stay within the device, and also while the launches have no more
+// workgroups than the device has units (wherever they are, a unit without any is
+// left for the next): where a unit holds one workgroup, only the second lets
+// two small launches run together.  A launch that would not fit waits here for
+// the others to end.
 class ResidentGate {
  public:
-  ResidentGate(int device, double share, double block) : g_(gate(device)), share_(share) {
+  ResidentGate(int device, int units, const ResFit &fit) : g_(gate(device)), fit_(fit) {
     std::unique_lock<std::mutex> lock(g_.mu);
     g_.cv.wait(lock, [&] {
-      return g_.n == 0 || g_.load + share + std::max(g_.block, block) <= 1.0;
+      return g_.n == 0 || g_.load + fit.share + std::max(g_.block, fit.block) <= 1.0 ||
+             g_.groups + fit.groups <= units;
     });
     ++g_.n;
-    g_.load += share;
-    g_.block = std::max(g_.block, block);
+    g_.load += fit.share;
+    g_.groups += fit.groups;
+    g_.block = std::max(g_.block, fit.block);
   }
   ~ResidentGate() {
     {
       std::lock_guard<std::mutex> lock(g_.mu);
-      g_.load -= share_;
+      g_.load -= fit_.share;
+      g_.groups -= fit_.groups;
       if (--g_.n == 0) g_.load = g_.block = 0.0;
     }
     g_.cv.notify_all();
@@ -62,7 +75,7 @@ class ResidentGate {
   struct Gate {
     std::mutex mu;
     std::condition_variable cv;
-    int n = 0;
+    int n = 0, groups = 0;
     double load = 0.0, block = 0.0;
   };
   static Gate &gate(int device) {
@@ -72,7 +85,7 @@ class ResidentGate {
     return gates[device];
   }
   Gate &g_;
-  double share_;
+  const ResFit fit_;
 };
 
 }  // namespace femgpu

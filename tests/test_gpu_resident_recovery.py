@@ -107,3 +107,42 @@ def test_late_abort(name):
         got = run(c)
         assert c.resident_info() == (0, 1)
         assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+def test_small_launches_side_by_side():
+    """Four contexts whose launches take some 60 units each are admitted together:
+    solves, explicit and implicit steps in four threads give the bits that each
+    gives alone, and no launch is given up."""
+    import threading
+    jobs = [("fp64", lambda: cube_problem(17)), ("mixed", lambda: cube_problem(18)),
+            ("explicit", lambda: cube_problem(16)), ("implicit", lambda: cube_problem(15))]
+
+    def run(c, kind):
+        if kind in ("fp64", "mixed"):
+            return c.solve(F.FP64 if kind == "fp64" else F.MIXED, **REL)[0]
+        dt = 2e-5
+        return c.dyn_run(beta2=0.5 if kind == "implicit" else 0.0, dt=dt, freq=1.0 / (20 * dt),
+                         endtime=(8 if kind == "implicit" else 400.5) * dt, **dict(STEP, **IMPL))[0]
+
+    ctxs = [F.Context(0) for _ in jobs]
+    try:
+        for c, (_, make) in zip(ctxs, jobs):
+            c.set_problem(make())
+        want = [run(c, k) for c, (k, _) in zip(ctxs, jobs)]
+        got = [[] for _ in jobs]
+
+        def work(i):
+            for _ in range(6):
+                got[i].append(run(ctxs[i], jobs[i][0]))
+
+        ts = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+        for t in ts:
+            t.start()
+        for t in ts:
+            t.join()
+        for i, c in enumerate(ctxs):
+            assert len(got[i]) == 6 and all(np.array_equal(u, want[i]) for u in got[i])
+            assert c.resident_info()[1] == 0
+    finally:
+        for c in ctxs:
+            c.close()
