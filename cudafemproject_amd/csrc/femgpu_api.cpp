@@ -40,10 +40,10 @@ using femgpu::ResidentGate;
 namespace {
 
 constexpr int NODE_PART = 4 * femgpu::NODE_PARTS;  // partials of node kernels (4 arrays)
-// Iterations of one resident launch (a few ms to tens of ms of device time;
-// a longer solve continues in further launches)
+// Iterations of one resident launch (7 to 60 ms of device time; a longer solve or
+// run continues in further launches)
 constexpr int RES_ITER_CAP = 4096;
-constexpr int RES_STEP_CAP = 16384;  // the same for explicit steps
+constexpr int RES_STEP_CAP = 16384;  // the same for explicit steps (30 to 130 ms)
 
 struct DevBuf {
   void *p = nullptr;
@@ -881,11 +881,12 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
   if ((st = res_buffers<T>(ctx, &m.words, &m.entries, &m.entry_words))) return st;
   m.sc = ctx->h_sc;
   m.late = ctx->res.late;
-  m.it_budget = 4 * RES_ITER_CAP;
+  m.it_budget = RES_ITER_CAP;
+  m.mid = m.it0 = 0;
   *done = 1;
   *steps = *iters = 0;
   *ok = true;
-  while (*steps < n_steps && *done == 1) {
+  while (*steps < n_steps && (*done == 1 || *done == femgpu::RES_CAP)) {
     m.step0 = step0 + *steps;
     m.n_steps = n_steps - *steps;
     ctx->h_sc->done = femgpu::RES_ABORTED;
@@ -905,9 +906,16 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
       return FEMGPU_OK;
     }
     ++ctx->res.completed;
-    *steps += ctx->h_sc->par_final;
-    *iters += ctx->h_sc->iter_final;
+    const CgScalars &h = *ctx->h_sc;
+    *steps += h.par_final;
+    *iters += h.it[0];
     m.fresh = 0;
+    m.mid = *done == femgpu::RES_CAP;
+    m.it0 = h.iter_final;
+    m.gamma0 = h.gamma0;
+    m.rr0 = h.rr0;
+    m.thresh = h.thresh;
+    m.g_prev = h.g[1];
   }
   return FEMGPU_OK;
 }
@@ -2905,6 +2913,8 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       m.f_unit = dfu;
       m.mlump = dml;
       m.invA = invA;
+      m.r = w.r;
+      m.p = w.p;
       m.coef_file = dcf;
       m.coef_unit = dcu;
       m.dt = T(C.dt);

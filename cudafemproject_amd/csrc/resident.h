@@ -109,13 +109,14 @@ bool res_dyn_fit(const DevMesh &dm, int device, ResFit *fit);
 template <typename T>
 void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &a, hipStream_t s, bool short_grid);
 
-// Implicit GN22 steps in one launch, likewise; a launch ends early after the
-// step in which its PCG iterations reach it_budget.  At the end sc->done is 1,
-// or the done code of the step that failed, sc->par_final the steps done and
-// sc->iter_final the PCG iterations.
+// Implicit GN22 steps in one launch, likewise; a launch ends early when its PCG
+// iterations reach it_budget, within a step's solve (sc->done RES_CAP: d, v, a, r, p
+// and the scalars are the solve's, the next launch continues it, mid) or between
+// two.  At the end sc->done is 1, RES_CAP or the done code of the step that failed,
+// sc->par_final the steps completed and sc->it[0] the launch's PCG iterations.
 template <typename T>
 struct ResImpl : ResRecv<T> {
-  T *d, *v, *a;
+  T *d, *v, *a, *r, *p;
   const T *f_file, *f_unit, *mlump, *invA;
   const double *coef_file, *coef_unit;
   T dt, c1, c2, c3, c4, alpha, beta;
@@ -127,6 +128,8 @@ struct ResImpl : ResRecv<T> {
   CgScalars *sc;
   int late;               // as ResPcg
   int fresh, step0, n_steps;
+  int mid, it0;           // mid: the launch before ended in step0's solve after it0 iterations
+  double gamma0, rr0, thresh, g_prev;  // and these are its scalars
 };
 
 template <typename T>

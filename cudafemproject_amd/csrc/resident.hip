@@ -717,33 +717,52 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
   const int rec = s.rec_of && P.has && P.first ? s.rec_of[P.gid] : -1;
   ResSolver<T, DIM, PT, NE> S(P, arg.m, s.words, s.entries, s.entry_words, b, pid, &s_flag);
   int done = 1, n = 0, total = 0;
+  bool mid = s.mid != 0;
+  T x[ND], r[ND], p[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    x[i] = r[i] = p[i] = T(0);
+    if (P.has && mid) {
+      x[i] = a[i];
+      r[i] = s.r[P.go + i];
+      p[i] = s.p[P.go + i];
+    }
+  }
+  S.n_upd = s.it0;
+  S.gamma0 = s.gamma0;
+  S.rr0 = s.rr0;
+  S.thresh = s.thresh;
+  S.g_prev = s.g_prev;
+  S.pause = 0.0;
   for (; n < s.n_steps && total < s.it_budget; ++n) {
-    const int step = s.step0 + n;
-    const T cf = T(s.coef_file[step]), cu = T(s.coef_unit[step]);
-    T x[ND], r[ND], p[ND];
+    if (!mid) {
+      const int step = s.step0 + n;
+      const T cf = T(s.coef_file[step]), cu = T(s.coef_unit[step]);
 #pragma unroll
-    for (int i = 0; i < ND; ++i) {
-      d[i] = d[i] + s.dt * v[i];
-      d[i] = d[i] + s.c1 * a[i];
-      v[i] = v[i] + s.c2 * a[i];
-      x[i] = s.beta != T(0) ? d[i] + s.beta * v[i] : d[i];
-    }
-    done = RES_ABORTED;
-    if (!S.apply(x, r)) break;
-#pragma unroll
-    for (int i = 0; i < ND; ++i) {
-      const T kd = r[i];
-      p[i] = x[i] = r[i] = T(0);
-      if (P.has) {
-        const T f = cf * s.f_file[P.go + i] + cu * s.f_unit[P.go + i] - kd;
-        r[i] = s.alpha != T(0) ? f - s.alpha * ml[i] * v[i] : f;
+      for (int i = 0; i < ND; ++i) {
+        d[i] = d[i] + s.dt * v[i];
+        d[i] = d[i] + s.c1 * a[i];
+        v[i] = v[i] + s.c2 * a[i];
+        x[i] = s.beta != T(0) ? d[i] + s.beta * v[i] : d[i];
       }
+      done = RES_ABORTED;
+      if (!S.apply(x, r)) break;
+#pragma unroll
+      for (int i = 0; i < ND; ++i) {
+        const T kd = r[i];
+        p[i] = x[i] = r[i] = T(0);
+        if (P.has) {
+          const T f = cf * s.f_file[P.go + i] + cu * s.f_unit[P.go + i] - kd;
+          r[i] = s.alpha != T(0) ? f - s.alpha * ml[i] * v[i] : f;
+        }
+      }
+      S.n_upd = 0;
+      S.g_prev = 1.0;
     }
-    S.n_upd = 0;
-    S.g_prev = 1.0;
-    S.pause = 0.0;
-    done = S.run(r, p, x, invd, s.cK, cMm, true, 0, s.eps, s.max_iter, s.max_iter + 1);
-    total += S.n_upd;
+    const int it0 = S.n_upd;
+    done = S.run(r, p, x, invd, s.cK, cMm, !mid, 0, s.eps, s.max_iter, it0 + s.it_budget - total);
+    total += S.n_upd - it0;
+    mid = false;
     if (done == RES_FAINT) done = 3;
     if (done != 1) break;
 #pragma unroll
@@ -752,23 +771,32 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
       v[i] = v[i] + s.c3 * a[i];
       d[i] = d[i] + s.c4 * a[i];
     }
-    record<T, DIM>(P, s, rec, step, d, v, a);
+    record<T, DIM>(P, s, rec, s.step0 + n, d, v, a);
   }
   if (s.late && pid == arg.m.np - 1) done = RES_ABORTED;
   if (done == RES_ABORTED) {
     if (threadIdx.x == 0) s.sc->gave_up = 1;
     return;
   }
-  if (P.first && done == 1)
+  if (P.first && (done == 1 || done == RES_CAP))
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
       s.d[P.go + i] = d[i];
       s.v[P.go + i] = v[i];
-      s.a[P.go + i] = a[i];
+      s.a[P.go + i] = done == RES_CAP ? x[i] : a[i];
+      if (done == RES_CAP) {
+        s.r[P.go + i] = r[i];
+        s.p[P.go + i] = p[i];
+      }
     }
   if (pid == 0 && threadIdx.x == 0) {
     CgScalars *sc = s.sc;
-    sc->iter_final = total;
+    sc->gamma0 = S.gamma0;
+    sc->rr0 = S.rr0;
+    sc->thresh = S.thresh;
+    sc->g[1] = S.g_prev;
+    sc->iter_final = S.n_upd;
+    sc->it[0] = total;
     sc->par_final = n;
     S.store_tags(s.words);
     sc->done = done;

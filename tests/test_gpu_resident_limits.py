@@ -108,3 +108,35 @@ def test_underflow_ends_a_solve(ctx):
                         mass_convention=F.MASS_PHYSICAL, implicit_mode=F.IMPLICIT_PHYSICAL,
                         raise_on_error=False)
     assert st["status"] == -5 and st["steps"] == 0 and st["pcg_iterations"] < 10000
+
+
+@pytest.mark.parametrize("damping", [0.0, 0.1])
+def test_implicit_launches_are_bounded(ctx, damping):
+    """Quasi-static steps of a slender plate take some 4000 iterations each: a
+    launch ends after 4096, within a step's solve too, and the next one goes on.
+    r'z drops by 1e-20, so 1e-10 in energy and, with a condition number of 1e8,
+    1e-6 on the displacements against the launch form."""
+    pb = plate_problem(300, 3, 100.0, 1.0, convention=F.LOADS_PHYSICAL)
+    ctx.set_problem(pb)
+    dt = 1e2
+    out = []
+    try:
+        for mode in (F.RESIDENT_AUTO, F.RESIDENT_OFF):
+            ctx.set_resident(mode)
+            ctx.set_receivers([5, pb.n_nodes - 1], F.RECV_DISPLACEMENT, 1)
+            before = ctx.resident_info()
+            u, st = ctx.dyn_run(rho=2400.0, beta2=0.5, dt=dt, endtime=3.5 * dt, ampl=1e3,
+                                wavelet_type=F.WAVELET_RICKER, freq=1.0 / (3 * dt), pcg_eps=1e-20,
+                                mass_convention=F.MASS_PHYSICAL, implicit_mode=F.IMPLICIT_PHYSICAL,
+                                damping_beta=damping * dt)
+            after = ctx.resident_info()
+            assert st["steps"] == 3 and st["pcg_iterations"] > 8192 and after[1] == before[1]
+            if mode == F.RESIDENT_AUTO:
+                assert after[0] - before[0] >= -(-st["pcg_iterations"] // 4096)
+            else:
+                assert after == before
+            out.append((u, ctx.traces()))
+    finally:
+        ctx.set_resident(F.RESIDENT_AUTO)
+        ctx.set_receivers([], F.RECV_DISPLACEMENT, 1)
+    assert rel(out[0][0], out[1][0]) <= 1e-6 and rel(out[0][1], out[1][1]) <= 1e-6
