@@ -85,7 +85,7 @@ __host__ __device__ inline BRLds br_lds(int nr, int pn, int ent, int n_in, int n
 template <int NV>
 __device__ __forceinline__ double block_sums(const double (&v)[NV], double *s_red) {
   static_assert(PT == 512, "eight waves: a value's in eight lanes");
-  const double s = wave_sums<NV>(v);
+  const double s = wave_sums<NV>(v, fresh(threadIdx.x));
   const int tx = fresh(threadIdx.x), w = tx >> 6, l = tx & 63;
   if (l % (64 / NV) == 0) s_red[(l / (64 / NV)) * 8 + w] = s;
   __syncthreads();
@@ -134,9 +134,9 @@ __device__ __forceinline__ bool gather_lanes(const u64 *words, int np, unsigned 
       if (i0 + G * b < np) sum += untag(h[b]);
   }
   sum = sum8(sum);
-  if constexpr (NV == 1) sum += lane_xor<8>(sum);
-  if constexpr (NV <= 2) sum += lane_xor<16>(sum);
-  if constexpr (NV <= 4) sum += lane_xor<32>(sum);
+  if constexpr (NV == 1) sum += lane_xor<8>(sum, l);
+  if constexpr (NV <= 2) sum += lane_xor<16>(sum, l);
+  if constexpr (NV <= 4) sum += lane_xor<32>(sum, l);
   return __all(ok);
 }
 
@@ -343,7 +343,7 @@ __device__ __forceinline__ bool solve_patch(const BRArgs &a, int pid, unsigned c
         publish_lanes<2 * NR>(ex, lp, tag, s);
         if (!gather_lanes<2 * NR>(ex, np, tag, a.abort, s)) s_flag = 1;
       }
-      const double o = lane_xor<8 * NR>(s);
+      const double o = lane_xor<8 * NR>(s, fresh(threadIdx.x));
       const bool second = t & (8 * NR);
       g = second ? o : s;
       rr = second ? s : o;

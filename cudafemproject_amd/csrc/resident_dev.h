@@ -308,24 +308,25 @@ struct PatchRow {
   }
 };
 
-// Value of the lane 8, 16 or 32 away (xor).
+// Value of the lane 8, 16 or 32 away (xor); t: the thread (a caller without
+// registers to spare passes it formed anew, fresh(threadIdx.x)).
 template <int O>
-__device__ __forceinline__ unsigned lane_xor(unsigned v) {
+__device__ __forceinline__ unsigned lane_xor(unsigned v, unsigned t) {
   static_assert(O == 8 || O == 16 || O == 32, "");
   if constexpr (O == 8) {
     return unsigned(__builtin_amdgcn_update_dpp(0, int(v), 0x128, 0xf, 0xf, false));
   } else if constexpr (O == 16) {
     const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return fresh(threadIdx.x) & 16u ? r[0] : r[1];
+    return t & 16u ? r[0] : r[1];
   } else {
     const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-    return fresh(threadIdx.x) & 32u ? r[0] : r[1];
+    return t & 32u ? r[0] : r[1];
   }
 }
 template <int O>
-__device__ __forceinline__ double lane_xor(double v) {
-  return __hiloint2double(int(lane_xor<O>(unsigned(__double2hiint(v)))),
-                          int(lane_xor<O>(unsigned(__double2loint(v)))));
+__device__ __forceinline__ double lane_xor(double v, unsigned t) {
+  return __hiloint2double(int(lane_xor<O>(unsigned(__double2hiint(v)), t)),
+                          int(lane_xor<O>(unsigned(__double2loint(v)), t)));
 }
 // a + (a's partner) in the lower half (of 32: rows 0, 2), b + (b's partner) in the
 // upper (rows 1, 3).
@@ -355,21 +356,21 @@ __device__ __forceinline__ double sum8(double v) {
 // halves the values with the lanes that hold them: 8 values in 10 additions
 // instead of 48.
 template <int NV>
-__device__ __forceinline__ double wave_sums(const double (&v)[NV]) {
+__device__ __forceinline__ double wave_sums(const double (&v)[NV], unsigned t) {
   if constexpr (NV == 8) {
     const double s0 = fold<16>(fold<32>(v[0], v[4]), fold<32>(v[2], v[6]));
     const double s1 = fold<16>(fold<32>(v[1], v[5]), fold<32>(v[3], v[7]));
-    const bool hi = fresh(threadIdx.x) & 8u;
-    return sum8((hi ? s1 : s0) + lane_xor<8>(hi ? s0 : s1));
+    const bool hi = t & 8u;
+    return sum8((hi ? s1 : s0) + lane_xor<8>(hi ? s0 : s1, t));
   } else {
     double s;
     if constexpr (NV == 4) {
       s = fold<16>(fold<32>(v[0], v[2]), fold<32>(v[1], v[3]));
     } else {
       s = fold<32>(v[0], v[NV - 1]);
-      s += lane_xor<16>(s);
+      s += lane_xor<16>(s, t);
     }
-    return sum8(s + lane_xor<8>(s));
+    return sum8(s + lane_xor<8>(s, t));
   }
 }
 
@@ -383,7 +384,7 @@ __device__ __forceinline__ double sum_by_wave(const double (&v)[RES_SUMS], doubl
   double v8[8];
 #pragma unroll
   for (int k = 0; k < 8; ++k) v8[k] = k < RES_SUMS ? v[k < RES_SUMS ? k : 0] : 0.0;
-  const double s = wave_sums<8>(v8);
+  const double s = wave_sums<8>(v8, threadIdx.x);
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   if ((l & 7) == 0 && l < 8 * RES_SUMS) s_red[(l >> 3) * 16 + w] = s;
   __syncthreads();
