@@ -45,7 +45,6 @@ struct BatchState {
   int64_t br_entries = 0;
   // nodes with more than BR_DEGREE neighbours in a patch, and how many
   std::vector<std::pair<int32_t, int>> br_crowded;
-  bool br_off = false;                   // a launch did not complete
   std::map<std::string, std::pair<void *, size_t>> bufs;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_poll[2] = {nullptr, nullptr};
 };
@@ -320,7 +319,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
                          const femgpu_solve_opts &o, double *u_out, femgpu_batch_stat *stats,
                          double *solve_ms, bool *ran) {
   *ran = false;
-  if (!b->br_np_max || b->br_off || !ctx_resident(ctx).on()) return FEMGPU_OK;
+  if (!b->br_np_max) return FEMGPU_OK;
   const int lds = br_lds_bytes(nr, b->bl_pn, b->bl_ent, b->br_in, b->br_src);
   double block = 1.0;
   // (a constrained row has no neighbours)
@@ -330,7 +329,7 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
   if (most > BR_DEGREE_MAX) return FEMGPU_OK;
   const int degree = most > BR_DEGREE ? BR_DEGREE_MAX : BR_DEGREE;
   const int capacity = br_capacity(nr, degree, lds, ctx_device(ctx), &block);
-  if (b->br_np_max > capacity) return FEMGPU_OK;
+  if (b->br_np_max > capacity || !ctx_resident(ctx).on()) return FEMGPU_OK;
   hipStream_t s = ctx_stream(ctx);
   const int64_t N = b->total_nodes;
   const size_t nd = size_t(N) * 2, nv = nd * nr, nu = nd * n_rhs;
@@ -423,11 +422,8 @@ int solve_resident_batch(femgpu_ctx *ctx, BatchState *b, int n_rhs, int nr, cons
     BCHK_(hipMemcpyAsync(&gave_up, words, sizeof gave_up, hipMemcpyDeviceToHost, s));
     BCHK_(hipStreamSynchronize(s));
   }
-  ++(gave_up ? ctx_resident(ctx).given_up : ctx_resident(ctx).completed);
-  if (gave_up) {
-    b->br_off = true;
-    return FEMGPU_OK;
-  }
+  ctx_resident(ctx).ended(gave_up == 0);
+  if (gave_up) return FEMGPU_OK;
   *ran = true;
   float ms = 0.f;
   BCHK_(hipEventElapsedTime(&ms, b->ev0, b->ev1));

@@ -760,9 +760,9 @@ int replay_until(femgpu_ctx *ctx, const Replay &exec, CgScalars *sc, int block, 
 
 // Whether this plan's PCG runs resident (all its workgroups on the chip).
 template <typename T>
-bool pcg_resident(const femgpu_ctx *ctx) {
+bool pcg_resident(femgpu_ctx *ctx) {
   femgpu::ResFit fit;
-  return ctx->res.on() && femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit);
+  return femgpu::res_pcg_fit<T>(ctx->dm, ctx->device, &fit) && ctx->res.on();
 }
 
 // The exchange words and this precision's entries, zeroed for this plan (an
@@ -792,8 +792,7 @@ int res_buffers(femgpu_ctx *ctx, unsigned long long **words, unsigned long long 
 
 // Runs a resident PCG until it stops; on return the stream is idle and
 // h_sc[0] holds the scalars.  *ok = false: the launch did not complete (its
-// workgroups did not come together); this context then stays with the
-// launch-per-kernel form.
+// workgroups did not come together); the call goes on in launches.
 template <typename T>
 int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
   femgpu::ResFit fit;
@@ -815,13 +814,12 @@ int run_resident(femgpu_ctx *ctx, femgpu::ResPcg<T> a, bool *ok) {
     }
     const CgScalars &h = *ctx->h_sc;
     if (h.done == femgpu::RES_ABORTED || h.gave_up) {
-      ++ctx->res.given_up;
-      ctx->res.off = true;
+      ctx->res.ended(false);
       ctx->res_np = 0;
       *ok = false;
       return FEMGPU_OK;
     }
-    ++ctx->res.completed;
+    ctx->res.ended(true);
     if (h.done != femgpu::RES_CAP) break;
     a.fresh = 0;
     a.r_in = a.r_out;
@@ -899,13 +897,12 @@ int run_resident_implicit(femgpu_ctx *ctx, femgpu::ResImpl<T> m, int step0, int 
     }
     *done = ctx->h_sc->gave_up ? femgpu::RES_ABORTED : ctx->h_sc->done;
     if (*done == femgpu::RES_ABORTED) {
-      ++ctx->res.given_up;
-      ctx->res.off = true;
+      ctx->res.ended(false);
       ctx->res_np = 0;
       *ok = false;
       return FEMGPU_OK;
     }
-    ++ctx->res.completed;
+    ctx->res.ended(true);
     const CgScalars &h = *ctx->h_sc;
     *steps += h.par_final;
     *iters += h.it[0];
@@ -962,13 +959,10 @@ int run_resident_steps(femgpu_ctx *ctx, femgpu::ResDyn<T> d, int n_steps, bool *
       HIPCHK(hipStreamSynchronize(ctx->stream));
     }
     *ok = *gave_up == 0;
-    ++(*ok ? ctx->res.completed : ctx->res.given_up);
+    ctx->res.ended(*ok);
     d.fresh = 0;
   }
-  if (!*ok) {
-    ctx->res.off = true;
-    ctx->dyn_np = 0;
-  }
+  if (!*ok) ctx->dyn_np = 0;
   return FEMGPU_OK;
 }
 
@@ -1452,7 +1446,7 @@ int femgpu_set_resident(femgpu_ctx *ctx, int mode) {
   if (mode < FEMGPU_RESIDENT_AUTO || mode > FEMGPU_RESIDENT_TEST_SHORT_WAITS)
     return fail(ctx, FEMGPU_E_ARG, "set_resident: unknown mode");
   ctx->res.mode = mode;
-  ctx->res.off = false;
+  ctx->res.skip = ctx->res.back_off = 0;
   ctx->res.lose_from = mode == FEMGPU_RESIDENT_TEST_LOSE         ? ctx->res.completed
                        : mode == FEMGPU_RESIDENT_TEST_LOSE_LATER ? ctx->res.completed + 2
                                                                  : -1;
@@ -2760,8 +2754,8 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
   // lag one step (the displacement does not).
   const bool one_launch = expl && nrec == 0 && !relax;
   femgpu::ResFit fit;
-  bool resident = expl && !relax && ctx->res.on() &&
-                  femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit);
+  bool resident = expl && !relax && femgpu::res_dyn_fit<T>(ctx->dm, ctx->device, &fit) &&
+                  ctx->res.on();
   if (resident) {
     femgpu::ResDyn<T> r{};
     r.d = dd;
@@ -2903,7 +2897,7 @@ int dyn_run_t(femgpu_ctx *ctx, const femgpu_dyn_opts &o, double *u_out, femgpu_d
       femgpu::launch_inv_diag<T>(ctx->dm, diagK_t, ceff, T(1), dmc, invA, ctx->stream);
     }
     w.invD = invA;
-    bool impl_resident = ctx->res.on() && femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit);
+    bool impl_resident = femgpu::res_impl_fit<T>(ctx->dm, ctx->device, &fit) && ctx->res.on();
     if (impl_resident) {
       femgpu::ResImpl<T> m{};
       m.d = dd;

@@ -13,11 +13,25 @@ namespace femgpu {
 // A context's use of the forms that stay on the chip (femgpu_set_resident).
 struct ResidentUse {
   int mode = 0;                 // FEMGPU_RESIDENT_*
-  bool off = false;             // a launch did not complete: launches from then on
   int64_t completed = 0, given_up = 0;
+  int skip = 0, back_off = 0;   // calls left in the launch form; their number last time
   int64_t lose_from = -1;       // tests: launches from this one on lack a workgroup
   bool late = false;            // tests: one gives up at its end
-  bool on() const { return mode != 1 && !off; }
+  // Whether a call should try the resident form (asked once per call).  A launch
+  // that did not complete cost a wait of a second, most likely for another
+  // process's workgroups: the next 64 calls go without, twice as many after
+  // another in a row, at most 4096.
+  bool on() {
+    if (mode == 1) return false;
+    if (skip == 0) return true;
+    --skip;
+    return false;
+  }
+  void ended(bool complete) {
+    ++(complete ? completed : given_up);
+    back_off = complete ? 0 : std::min(std::max(64, 2 * back_off), 4096);
+    if (!complete) skip = back_off;
+  }
   bool short_waits = false;     // tests: waits run out after 2 ms, nothing is lost
   bool impatient() const { return short_waits || lose_from >= 0; }
   bool lose() const { return lose_from >= 0 && completed >= lose_from; }

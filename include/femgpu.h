@@ -143,7 +143,9 @@ enum {
 };
 int femgpu_set_resident(femgpu_ctx *ctx, int mode);
 /* Launches of this context that stayed on the chip: info[0] completed,
- * info[1] given up (a wait ran out; the call then went on in launches). */
+ * info[1] given up (a wait ran out, most likely because another process's
+ * workgroups held the device; the call then went on in launches, and so do the
+ * next 64, after another in a row 128, ..., at most 4096 calls). */
 int femgpu_resident_info(const femgpu_ctx *ctx, int64_t *info);
 
 /* --- problem definition ---------------------------------------------------

@@ -146,3 +146,28 @@ def test_small_launches_side_by_side():
     finally:
         for c in ctxs:
             c.close()
+
+
+def test_way_back():
+    """After a launch that was given up 64 calls of any kind go in launches, then
+    one tries again; after the second 128."""
+    small = plate_batch(1, seed=1, nx_range=(30, 31), ny_range=(20, 21))
+    with F.Context(0) as c:
+        c.set_problem(plate_problem(40, 20))
+        load_batch(c, small)
+        calls = [lambda: c.solve(F.FP64, **REL), lambda: c.solve(F.MIXED, **REL),
+                 lambda: c.dyn_run(dt=1e-5, endtime=3.5e-5, **STEP),
+                 lambda: c.dyn_run(dt=1e-5, endtime=3.5e-5, beta2=0.5, **dict(STEP, **IMPL)),
+                 lambda: c.batch_solve([small[0].f], precision=F.FP64, tol=1e-6)]
+        for f in calls:
+            f()
+        assert c.resident_info()[1] == 0
+        done = c.resident_info()[0]
+        c.set_resident(F.RESIDENT_TEST_LOSE)
+        lost = []
+        for k in range(200):
+            before = c.resident_info()[1]
+            calls[k % 5]()
+            if c.resident_info()[1] > before:
+                lost.append(k)
+        assert lost == [0, 65, 194] and c.resident_info() == (done, 3)
