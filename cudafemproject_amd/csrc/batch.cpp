@@ -110,23 +110,28 @@ double elem_det(int dim, const double *nodes, const int32_t *en) {
 }
 
 // Nodes of a 2D plan with more than BR_DEGREE neighbours in a patch (internal
-// node, the most in one).
+// node, the most in one; BR_DEGREE_MAX + 1: that many or more).
 void find_crowded(const MeshPlan &Q, int32_t first_node, std::vector<std::pair<int32_t, int>> &out) {
-  std::vector<std::vector<uint16_t>> near;
+  constexpr int CAP = BR_DEGREE_MAX + 1;
+  std::vector<uint16_t> near(size_t(BR_NODES) * CAP);
+  std::vector<int> count(BR_NODES);
   for (const PatchInfo &P : Q.patches) {
-    near.assign(size_t(P.n_own + P.n_sh), {});
+    std::fill(count.begin(), count.end(), 0);
     for (int32_t e = P.elem_start; e < P.elem_start + P.n_elem; ++e)
-      for (int a = 0; a < 3; ++a)
+      for (int a = 0; a < 3; ++a) {
+        const size_t l = Q.elem_lid[size_t(e) * 4 + a];
+        uint16_t *list = &near[l * CAP];
+        int &n = count[l];
         for (int b = 0; b < 3; ++b) {
           const uint16_t m = Q.elem_lid[size_t(e) * 4 + b];
-          auto &list = near[Q.elem_lid[size_t(e) * 4 + a]];
-          if (a != b && std::find(list.begin(), list.end(), m) == list.end()) list.push_back(m);
+          if (a != b && n < CAP && std::find(list, list + n, m) == list + n) list[n++] = m;
         }
+      }
     for (int32_t k = 0; k < P.n_own + P.n_sh; ++k)
-      if (near[size_t(k)].size() > size_t(BR_DEGREE))
+      if (count[size_t(k)] > BR_DEGREE)
         out.emplace_back(first_node + (k < P.n_own ? P.own_start + k
                                                    : Q.sh_gid[size_t(P.sh_start + k - P.n_own)]),
-                         int(near[size_t(k)].size()));
+                         count[size_t(k)]);
   }
 }
 
