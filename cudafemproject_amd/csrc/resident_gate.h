@@ -61,19 +61,25 @@ struct ResFit {
 // workgroups than the device has units (wherever they are, a unit without any is
 // left for the next): where a unit holds one workgroup, only the second lets
 // two small launches run together.  A launch that would not fit waits here for
-// the others to end.
+// the others to end, and those that come after it wait behind it (a stream of
+// small ones would keep a large one out for good).
 class ResidentGate {
  public:
   ResidentGate(int device, int units, const ResFit &fit) : g_(gate(device)), fit_(fit) {
     std::unique_lock<std::mutex> lock(g_.mu);
+    const uint64_t turn = g_.last++;
     g_.cv.wait(lock, [&] {
-      return g_.n == 0 || g_.load + fit.share + std::max(g_.block, fit.block) <= 1.0 ||
-             g_.groups + fit.groups <= units;
+      return turn == g_.next &&
+             (g_.n == 0 || g_.load + fit.share + std::max(g_.block, fit.block) <= 1.0 ||
+              g_.groups + fit.groups <= units);
     });
+    ++g_.next;
     ++g_.n;
     g_.load += fit.share;
     g_.groups += fit.groups;
     g_.block = std::max(g_.block, fit.block);
+    lock.unlock();
+    g_.cv.notify_all();  // (the next in turn may fit too)
   }
   ~ResidentGate() {
     {
@@ -89,6 +95,7 @@ class ResidentGate {
   struct Gate {
     std::mutex mu;
     std::condition_variable cv;
+    uint64_t last = 0, next = 0;  // turns given out and taken
     int n = 0, groups = 0;
     double load = 0.0, block = 0.0;
   };

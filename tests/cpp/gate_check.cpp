@@ -54,5 +54,39 @@ int main() {
         std::printf("FAIL %s (%d): expected %d\n", c.what, swap, c.both);
         ++bad;
       }
+  // A launch of the whole device comes to its turn while two threads keep small
+  // launches coming, at least one of them running at any time.
+  {
+    const int d = 1000;
+    std::atomic<bool> stop{false}, in{false};
+    std::atomic<int> running{0};
+    auto small = [&] {
+      while (!stop) {
+        ResidentGate g(d, 256, fit(10, 1));
+        ++running;
+        const auto t0 = std::chrono::steady_clock::now();
+        // (until the other one runs too, or 50 ms)
+        while (running < 2 && !stop && std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(50))
+          std::this_thread::yield();
+        std::this_thread::sleep_for(std::chrono::milliseconds(1));
+        --running;
+      }
+    };
+    std::thread a(small), b(small);
+    std::this_thread::sleep_for(std::chrono::milliseconds(20));
+    std::thread big([&] {
+      ResidentGate g(d, 256, fit(256, 1));
+      in = true;
+    });
+    for (int i = 0; i < 1000 && !in; ++i) std::this_thread::sleep_for(std::chrono::milliseconds(2));
+    if (!in) {
+      std::printf("FAIL a large launch is kept out\n");
+      ++bad;
+    }
+    stop = true;
+    a.join();
+    b.join();
+    big.join();
+  }
   return bad != 0;
 }
