@@ -18,8 +18,8 @@ constexpr int BR_ELEMS = BR_THREADS;
 // Most neighbours of a node within its patch: regular triangulations have six,
 // and with 8 the rows of four systems fit the registers of two workgroups per
 // compute unit; a mesh with more (counted on the host when it is loaded) runs
-// with 12, which spill (60 plates of 80 x 40, four load cases, FP64: 21.9
-// against 24.7 ms).
+// with 12, which spill (60 plates of 80 x 40, four load cases, FP64, all with 8
+// or all with 12: 21.9 against 24.7 ms).
 constexpr int BR_DEGREE = 8, BR_DEGREE_MAX = 12;
 
 // Words of a patch in its instance's exchange (three places of 2 nr values).

@@ -8,11 +8,12 @@
 // its residual replacement idles to the end of the replay.  Here matrix rows
 // and residuals stay in registers, directions and solutions in LDS, an
 // instance waits only for its own workgroups, replaces a residual at once and
-// makes room for the next when it is done.  Measured, FP64 to 1e-10, launch
-// per iteration -> resident: 60 plates of 80 x 40 with four load cases 45.3 ->
-// 21.9 ms (832 iterations), with one 16.5 -> 10.9; one plate of 160 x 80, four
-// load cases, 34.7 -> 16.9; one of 300 x 220 125.5 -> 81.7; 200 plates of
-// [16, 160] x [16, 80] 251 -> 155 ms (mixed 207).
+// makes room for the next when it is done.  Measured, device time of FP64
+// solves to 1e-10, launch per iteration -> resident: 60 equal plates of 80 x 40
+// with four load cases 44.7 -> 21.2 ms (830 iterations), with one 16.2 -> 10.0;
+// one plate of 160 x 80, four load cases, 33.9 -> 16.3; one of 300 x 220 to 1e-8
+// 110 -> 71; 200 plates of [16, 160] x [16, 80] to 1e-9 230 -> 127 ms (mixed in
+// launches 192).
 //
 // The patch's part of K is applied by rows (PatchRow) instead of element by
 // element: a product is the patch's 7 neighbour reads per DOF and system with

@@ -32,20 +32,22 @@
 // another's decision, and all copies have the same bits.
 //
 // Exchange: a workgroup's partials and its interface sums are published as
-// 8-byte words, 32 bits of payload under a 32-bit tag (the number of the
-// exchange), so that a value and its arrival are one load and nothing has to
-// be ordered.  A workgroup that has everyone's words of one exchange knows that
-// everyone has read those of the one before, so two places (and, for the
-// interface sums, two sets of entries) take turns.  Stores and loads of shared data are relaxed agent-scope
-// atomics (written through, not served from a stale cache); an agent-scope
-// fence would write the XCD's L2 back, some 40 us.
+// 8-byte words that carry the number of the exchange beside their payload
+// (partials: 32 bits under a 32-bit tag, interface sums: 48 under 16), so that a
+// value and its arrival are one load and nothing has to be ordered.  A
+// workgroup that has everyone's words of one exchange knows that everyone has
+// read those of the one before, so two places (and, for the interface sums, two
+// sets of entries) take turns.  Stores and loads of shared data are relaxed
+// agent-scope atomics (written through, not served from a stale cache); an
+// agent-scope fence would write the XCD's L2 back, some 40 us.
 //
 // Waiting needs all workgroups on the chip: the host launches this form only
 // where they fit (res_pcg_fit), and a wait is bounded (WAIT_TICKS): past it
-// the launch ends with an abort flag and the host runs the launch-per-kernel
-// form instead.
+// the launch ends, every workgroup that gave up says so to the host, and the
+// call goes on in the launch-per-kernel form.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -686,7 +688,10 @@ __device__ __forceinline__ void record(const Patch &P, const R &s, int rec, int 
       s.traces[(int64_t(smp) * s.n_rec + k) * DIM + P.comp(i)] = src[i];
 }
 
-template <typename T, int DIM, int PT, int NE>
+// MID: the launch begins within a step's solve.  Not a run-time flag: with both
+// entries to run() in one kernel, a column of 11 x 11 x 80 hexes took 6.29 ms
+// for 20 steps, in a kernel of its own 6.14.
+template <typename T, int DIM, int PT, int NE, bool MID>
 __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
   using Patch = ResPatch<T, DIM, PT, NE>;
   constexpr int ND = Patch::ND;
@@ -717,7 +722,7 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
   const int rec = s.rec_of && P.has && P.first ? s.rec_of[P.gid] : -1;
   ResSolver<T, DIM, PT, NE> S(P, arg.m, s.words, s.entries, s.entry_words, b, pid, &s_flag);
   int done = 1, n = 0, total = 0;
-  bool mid = s.mid != 0;
+  bool mid = MID;
   T x[ND], r[ND], p[ND];
 #pragma unroll
   for (int i = 0; i < ND; ++i) {
@@ -728,11 +733,13 @@ __global__ __launch_bounds__(PT) void k_impl_resident(ImplArgs<T> arg) {
       p[i] = s.p[P.go + i];
     }
   }
-  S.n_upd = s.it0;
-  S.gamma0 = s.gamma0;
-  S.rr0 = s.rr0;
-  S.thresh = s.thresh;
-  S.g_prev = s.g_prev;
+  if (mid) {
+    S.n_upd = s.it0;
+    S.gamma0 = s.gamma0;
+    S.rr0 = s.rr0;
+    S.thresh = s.thresh;
+    S.g_prev = s.g_prev;
+  }
   S.pause = 0.0;
   for (; n < s.n_steps && total < s.it_budget; ++n) {
     if (!mid) {
@@ -956,17 +963,23 @@ using DynKernel = void (*)(DynArgs<T>);
 template <typename T>
 using ImplKernel = void (*)(ImplArgs<T>);
 
-#define FEMGPU_RES_KERNEL(NAME, KIND)                                                       \
+#define FEMGPU_RES_KERNEL(OF, KIND, NAME, ...)                                              \
   template <typename T>                                                                     \
-  KIND<T> NAME##_of(int dim, Form f) {                                                      \
-    if (f.ne == 3) return dim == 3 ? KIND<T>(NAME<T, 3, 512, 3>) : KIND<T>(NAME<T, 2, 512, 3>); \
-    if (f.ne == 2) return dim == 3 ? KIND<T>(NAME<T, 3, 768, 2>) : KIND<T>(NAME<T, 2, 768, 2>); \
-    if (dim == 3) return NAME<T, 3, 768, 1>;                                                \
-    return f.threads == 512 ? KIND<T>(NAME<T, 2, 512, 1>) : KIND<T>(NAME<T, 2, 768, 1>);    \
+  KIND<T> OF(int dim, Form f) {                                                             \
+    if (f.ne == 3)                                                                          \
+      return dim == 3 ? KIND<T>(NAME<T, 3, 512, 3 __VA_ARGS__>)                             \
+                      : KIND<T>(NAME<T, 2, 512, 3 __VA_ARGS__>);                            \
+    if (f.ne == 2)                                                                          \
+      return dim == 3 ? KIND<T>(NAME<T, 3, 768, 2 __VA_ARGS__>)                             \
+                      : KIND<T>(NAME<T, 2, 768, 2 __VA_ARGS__>);                            \
+    if (dim == 3) return NAME<T, 3, 768, 1 __VA_ARGS__>;                                    \
+    return f.threads == 512 ? KIND<T>(NAME<T, 2, 512, 1 __VA_ARGS__>)                       \
+                            : KIND<T>(NAME<T, 2, 768, 1 __VA_ARGS__>);                      \
   }
-FEMGPU_RES_KERNEL(k_pcg_resident, PcgKernel)
-FEMGPU_RES_KERNEL(k_dyn_resident, DynKernel)
-FEMGPU_RES_KERNEL(k_impl_resident, ImplKernel)
+FEMGPU_RES_KERNEL(k_pcg_resident_of, PcgKernel, k_pcg_resident)
+FEMGPU_RES_KERNEL(k_dyn_resident_of, DynKernel, k_dyn_resident)
+FEMGPU_RES_KERNEL(k_impl_resident_of, ImplKernel, k_impl_resident, , false)
+FEMGPU_RES_KERNEL(k_impl_mid_resident_of, ImplKernel, k_impl_resident, , true)
 #undef FEMGPU_RES_KERNEL
 
 // Workgroups of a launch (short_grid: up to the last patch's, and without it).
@@ -1058,16 +1071,24 @@ void launch_res_dyn(const DevMesh &dm, const ResDyn<T> &s, hipStream_t st, bool 
 template <typename T>
 bool res_impl_fit(const DevMesh &dm, int device, ResFit *fit) {
   const Form f = res_form(dm);
-  return dm.xpatch && f.ne && fits(dm, device, reinterpret_cast<const void *>(k_impl_resident_of<T>(dm.dim, f)),
-                                   res_lds_bytes(dm, int(sizeof(T))), fit);
+  const int lds = res_lds_bytes(dm, int(sizeof(T)));
+  ResFit mid;
+  if (!dm.xpatch || !f.ne ||
+      !fits(dm, device, reinterpret_cast<const void *>(k_impl_resident_of<T>(dm.dim, f)), lds, fit) ||
+      !fits(dm, device, reinterpret_cast<const void *>(k_impl_mid_resident_of<T>(dm.dim, f)), lds, &mid))
+    return false;
+  // (either may be launched under one turn)
+  fit->share = std::max(fit->share, mid.share);
+  fit->block = std::max(fit->block, mid.block);
+  return true;
 }
 
 template <typename T>
 void launch_res_impl(const DevMesh &dm, const ResImpl<T> &s, hipStream_t st, bool short_grid) {
   const ImplArgs<T> a{res_mesh<T>(dm), s};
   const Form f = res_form(dm);
-  hipLaunchKernelGGL(k_impl_resident_of<T>(dm.dim, f), dim3(grid_of(a.m.np, a.m.p8, short_grid)),
-                     dim3(f.threads),
+  hipLaunchKernelGGL(s.mid ? k_impl_mid_resident_of<T>(dm.dim, f) : k_impl_resident_of<T>(dm.dim, f),
+                     dim3(grid_of(a.m.np, a.m.p8, short_grid)), dim3(f.threads),
                      res_lds_bytes(dm, int(sizeof(T))), st, a);
 }
 
@@ -1078,7 +1099,8 @@ static hipError_t prepare_t() {
     for (Form f : {Form{512, 1}, Form{768, 1}, Form{512, 3}, Form{768, 2}})
       for (const void *fn : {reinterpret_cast<const void *>(k_pcg_resident_of<T>(dim, f)),
                              reinterpret_cast<const void *>(k_dyn_resident_of<T>(dim, f)),
-                             reinterpret_cast<const void *>(k_impl_resident_of<T>(dim, f))})
+                             reinterpret_cast<const void *>(k_impl_resident_of<T>(dim, f)),
+                             reinterpret_cast<const void *>(k_impl_mid_resident_of<T>(dim, f))})
         if ((r = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, RES_LDS_MAX)) !=
             hipSuccess)
           e = r;

@@ -142,8 +142,9 @@ def _run_with(ctx, pb, tuning, fn):
     return fn()
 
 
-# patches of more than 256 nodes (two elements per thread), small ones, and
-# more than 256 patches (a launch per kernel)
+# patches of more than 256 nodes (a strip per thread where every patch has at most
+# 512 strips, else two elements), small ones, and more than 256 patches (a launch
+# per kernel)
 FORMS = [(1536, 512), (64, 256), (16, 256)]
 
 
