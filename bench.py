@@ -405,7 +405,7 @@ def bench_batch(args, F):
                    "n_elems": int(sum(len(b.elems) for b in insts)),
                    "n_dof": int(sum(2 * len(b.nodes) for b in insts)), "tol": 1e-8},
         "fp64_s": t64 / 1e3, "speedup_mixed_vs_fp64": t64 / tmx,
-        "schedule": "lockstep (every system over the whole GPU, graph replays)",
+        "schedule": "lockstep (2D: one resident launch)",
         "persistent_schedule_s": ({k: res[k][0] / 1e3 for k in ("mixed_persistent", "fp64_persistent")}
                                   if "mixed_persistent" in res else None),
         "systems_per_s_mixed": n_sys / (tmx * 1e-3),
